@@ -729,6 +729,11 @@ hn_status degree_prefix(hn_graph* g, int64_t* d_eoff, hipStream_t st) {
     return exclusive_scan<int64_t>(DegIn{g->rec}, d_eoff, g->nv, g->s_scan.ptr, st);
 }
 
+bool graph_known_symmetric(hn_graph* g) {
+    std::lock_guard<std::mutex> lock(g->sym_mu);   // another slot's thread may be checking
+    return g->sym == 1;
+}
+
 hn_status graph_is_symmetric(hn_graph* g, hipStream_t st, bool* yes) {
     // the serving loop's slot threads call this concurrently on one graph: the
     // check (which reserves the shared s_misc scratch) runs under a lock

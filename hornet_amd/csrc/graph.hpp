@@ -182,9 +182,9 @@ struct hn_graph {
     hn::Scratch s_mstage;             // staging of edge meta-data during updates
     hn::Scratch s_stamp;              // per vertex: its source segment in the current batch (unchecked)
     uint64_t* h_pinned = nullptr;     // small pinned readback area
-    // levels + 1 of the last single-source BFS: when its level loop first
-    // polls for the end (serving slots run BFS concurrently, hence atomic)
-    std::atomic<int> bfs_last_levels{0};
+    // whole-device rounds of the last single-source BFS (-1: none yet): how many
+    // the next one queues at first (serving slots run BFS concurrently, hence atomic)
+    std::atomic<int> bfs_last_rounds{-1};
     // timing events of the BFS expansion (one pair per queued level), created
     // on the first timed traversal
     static constexpr int BFS_EVENTS = 64;
@@ -256,6 +256,8 @@ hn_status ms_run_engine(MsEngine* e, const int32_t* sources, int32_t k, const in
 // whether the adjacency is symmetric (checked once per graph version when
 // not known; the multi-source BFS pulls only over symmetric graphs)
 hn_status graph_is_symmetric(hn_graph* g, hipStream_t st, bool* yes);
+// whether it is known to be, without a check
+bool graph_known_symmetric(hn_graph* g);
 // Multi-version windows (one launch serving queries of several graph
 // versions).  begin: before the window's updates are applied, with every
 // update entry on the device (d_tt[i] = update index 1..63 << 1 | 1 for an insert);

@@ -150,7 +150,7 @@ static void worker_loop(hn_server* s, ServeSlot* slot) {
         if (single) {
             bfs_layout(g->nv, g->ne, slot->bfs_scratch, &bb);
             for (int32_t i = 0; i < k; i++) {
-                hn_status st = bfs_run(g, srcs[i], slot->dist, nullptr, slot->stream, bb, false,
+                hn_status st = bfs_run(g, srcs[i], nullptr, nullptr, slot->stream, bb, false,
                                        reinterpret_cast<uint64_t*>(slot->h_digest), limits[i]);
                 // the digest from the level counters bfs_run read back into
                 // h_digest: every frontier expanded adds its size and its
@@ -164,7 +164,7 @@ static void worker_loop(hn_server* s, ServeSlot* slot) {
                     dg[1] = c.dsum;
                     dg[2] = c.levels > 0 ? c.levels - 1 : 0;
                     if (limits[i] > 0 && (int64_t)c.levels == (int64_t)limits[i]) {
-                        const uint64_t fn = c.fc[(c.levels + 1) & 1] >> 32;
+                        const uint64_t fn = c.left;
                         dg[0] += fn;
                         dg[1] += fn * c.levels;
                         if (fn) dg[2] = c.levels;
