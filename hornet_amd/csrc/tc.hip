@@ -12,457 +12,847 @@
 // (hornetsnest/test/TriangleTest2.cu:86-87, xlib/src/Graph/GraphStd.cpp:247-304),
 // so the sum is the triangle count.
 //
-// Here:
-//   * orientation of the symmetric storage is a flag + scan compaction (no
-//     atomics): keep (u,v) iff (deg u, u) < (deg v, v); the oriented offsets
-//     are the scan positions at the symmetric offsets;
-//   * intersection work min(d(u), d(v)) splits every edge into one of three
-//     wave64 classes: one lane per edge (<= 16 entries in the shorter list),
-//     sixteen lanes per edge (<= 128), where each lane binary-searches
-//     entries of the shorter list in the longer one, or a whole wave per edge
-//     intersecting 64-entry windows of both lists (tc_window_kernel; both
-//     equal the merge count on simple graphs);
-//   * the two deferred classes are queued by the one-lane pass; their waves
-//     claim 16 queued edges at a time from a ticket, which keeps the waves
-//     busy to the end of the skewed queues;
-//   * counts are reduced per wave; the total takes one 64-bit atomicAdd per
-//     wave, per-vertex credits (optional) one per edge with a non-zero count.
+// Here an edge is intersected where its longer list is: the owner of an edge is
+// the endpoint with the longer list, a workgroup puts the owner's list into LDS
+// once, and then walks the shorter lists of the owner's edges, one LDS test per
+// entry and no search.  Over an R-MAT s22 orientation (64 M edges) that is
+// 11.8 G tests of streamed entries; binary searches and 64-entry windows of both
+// lists, one edge at a time, took 75 ms for them; here 7.4.
+//   * The LDS set is exact: the most frequent vertices (hubs, up to 65,535 of
+//     them) have 16-bit codes and one bit each in an 8 KB bitmap; the others are
+//     hashed.  A list is two rows, its hubs' codes and the others' ids, each
+//     16-byte aligned and padded, so a lane loads eight codes at once and a test
+//     is one LDS word and a bit-field extract.  Skewed graphs put nearly all
+//     entries on hubs (R-MAT s22: 96 % of the tests), and an owner that is a hub
+//     of a degree orientation has nothing but hubs in its list, so that its
+//     other tests are skipped altogether.
+//   * The orientation keeps (u, v) iff (deg u, u) < (deg v, v): one pass over the
+//     stored entries that compacts every row into its own place (the order
+//     within a row does not matter to an LDS set).
+//   * An owner's edges: on simple symmetric storage its stored row, of which it
+//     takes the neighbours with shorter lists.  Otherwise (stored graphs, repeated
+//     entries, symmetry not known) its own list, and the sources of the edges
+//     whose longer list is the destination's, grouped by it first.
+//   * Owners are cut into tasks of up to TC_CAND candidates, which resident
+//     workgroups take from a ticket.  Edges between lists of at most TC_SMALL
+//     entries are compared in registers by one thread per source.
+//   * The count of an edge is credited to the shorter list's vertex with one
+//     atomic; the total is summed per workgroup.
 #include "graph.hpp"
 #include "prims.hpp"
 
 namespace hn {
 namespace {
 
-constexpr int TC_IPT = 2;
+constexpr int TC_G = 8;                        // entries per group: 16 bytes of hub codes, 32 of ids
+constexpr uint32_t TC_HUBS = 65535;            // hubs at most
+constexpr uint32_t TC_PAD16 = 0xFFFF;          // fills the last group of a row of codes: a bit never set
+constexpr uint32_t TC_PAD = 0xFFFFFFFFu;       // ... of a row of ids
+constexpr uint32_t TC_ID = 0x80000000u;        // (in a vertex's code) no hub: TC_ID | id
+constexpr int TC_BINS = 4096;
+constexpr uint32_t TC_SMALL = 16;              // lists up to this long are compared in registers
+constexpr uint32_t TC_CAND = 1024;             // candidates per task
+constexpr int TC_STEP = 2 * BLOCK;             // ... listed at a time
+constexpr uint32_t TC_TAIL = 256;              // ids hashed at a time
+constexpr uint32_t TC_HASH = 2 * TC_TAIL;
+constexpr int TC_TEAM = 8;                     // lanes per shorter list
+constexpr int TC_DEPTH = 4;                    // groups per lane in flight (2 and 8: 3 and 2 % slower on R-MAT s22)
+constexpr int TC_ORDER = 32;                   // classes of list lengths that a step is sorted by
+constexpr int TC_IPT = 2;                      // groups per lane of the passes over rows
 constexpr int TC_TILE = BLOCK * TC_IPT;
-constexpr int LIGHT_MAX = 16;
-// class limits on the shorter list: one lane per edge up to LIGHT_MAX
-// entries, MEDIUM_LANES lanes up to MEDIUM_MAX, the window intersection
-// above; measured on R-MAT s24 with binary searches in every class (16 / 256:
-// 783 ms per recount; 8 / 512: 819 ms; 8 / 256: 805 ms; 32 / 512: 784 ms;
-// 4 / 512: 1057 ms), then with the window class (window from 257 entries:
-// 451 ms, from 129: 431 ms, from 193: 448 ms; from 97 or 65 when the longer
-// list is at most 8 or 16 times longer: 430-435 ms)
-constexpr int MEDIUM_MAX = 128;
-constexpr int MEDIUM_LANES = 16;
 
-__device__ __forceinline__ bool bsearch_has(const int32_t* __restrict__ a, int64_t n, int32_t x) {
-    int64_t lo = 0, hi = n;
-    while (lo < hi) {
-        int64_t mid = (lo + hi) >> 1;
-        int32_t y = a[mid];
-        if (y < x) lo = mid + 1;
-        else if (y > x) hi = mid;
-        else return true;
-    }
-    return false;
+// A list: its rows' place in groups, the hubs' and the others' number.
+struct __attribute__((aligned(16))) TcRow {
+    uint32_t base;
+    uint32_t pad;
+    uint32_t n16;
+    uint32_t n32;
+    __device__ __forceinline__ uint32_t len() const { return n16 + n32; }
+};
+
+// Atomics on one address take 10 ns each, whoever makes them: the sums and the
+// tasks' tickets are spread over lines of their own.
+constexpr int TC_SUMS = 32, TC_LANES = 8;
+struct alignas(128) TcSum {
+    unsigned long long v;
+};
+struct alignas(128) TcTicket {
+    uint32_t v;
+};
+struct TcCtl {
+    TcSum total[TC_SUMS];
+    TcTicket ticket[TC_LANES];
+    uint32_t cut;        // bins from this one on are hubs
+    uint32_t ntask;
+    uint32_t hubs;
+    uint32_t repeats;    // some row stores an entry twice
+};
+
+// monotone in d: exponent and seven bits of mantissa
+__device__ __forceinline__ uint32_t tc_bin(uint32_t d) {
+    if (d == 0) return 0;
+    const int e = 31 - __clz((int)d);
+    return (uint32_t)e * 128u + (uint32_t)(((uint64_t)d << 7 >> e) & 127u);
 }
 
-struct TcCsr {
-    const int64_t* off;
-    const int32_t* adj;
+// ---- hubs: the weights' histogram, the bin from which at most TC_HUBS vertices
+// lie, and every vertex's code
+__global__ __launch_bounds__(BLOCK) void tc_hist_kernel(int64_t nv, const uint32_t* __restrict__ weight,
+                                                        uint32_t* __restrict__ hist) {
+    __shared__ uint32_t h[TC_BINS];
+    for (int i = threadIdx.x; i < TC_BINS; i += BLOCK) h[i] = 0;
+    __syncthreads();
+    for (int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x; v < nv; v += (int64_t)gridDim.x * BLOCK) {
+        const uint32_t w = weight[v];
+        if (w > 1) atomicAdd(&h[tc_bin(w)], 1u);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < TC_BINS; i += BLOCK)
+        if (h[i]) atomicAdd(hist + i, h[i]);
+}
+
+__global__ __launch_bounds__(BLOCK) void tc_cut_kernel(const uint32_t* __restrict__ hist, TcCtl* __restrict__ ctl) {
+    __shared__ uint32_t sc[NWAVES + 1];
+    __shared__ uint32_t cut;
+    if (threadIdx.x == 0) cut = TC_BINS;
+    __syncthreads();
+    constexpr int K = TC_BINS / BLOCK;
+    // thread t sums bins from the top: t * K .. t * K + K - 1 below TC_BINS
+    uint32_t x[K], sum = 0;
+    for (int k = 0; k < K; k++) {
+        x[k] = hist[TC_BINS - 1 - (threadIdx.x * K + k)];
+        sum += x[k];
+    }
+    uint32_t tot;
+    uint32_t run = block_exclusive_scan(sum, sc, &tot), mine = TC_BINS;
+    for (int k = 0; k < K; k++) {
+        run += x[k];
+        if (run <= TC_HUBS) mine = (uint32_t)(TC_BINS - 1 - (threadIdx.x * K + k));
+    }
+    if (mine < TC_BINS) atomicMin(&cut, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) ctl->cut = cut;
+}
+
+struct HubIn {
+    const uint32_t* weight;
+    const TcCtl* ctl;
+    __device__ __forceinline__ uint32_t operator()(int64_t v) const {
+        const uint32_t w = weight[v];
+        return w > 1 && tc_bin(w) >= ctl->cut ? 1u : 0u;
+    }
+};
+// (weight, code) side by side: the orientation looks up both of every entry
+struct HubOut {
+    const uint32_t* weight;
+    uint2* wc;
+    uint32_t* hub;
+    __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t is) const {
+        wc[v] = make_uint2(weight[v], is ? ex : (TC_ID | (uint32_t)v));
+        if (is) hub[ex] = (uint32_t)v;
+    }
 };
 
-struct TcOut {
-    unsigned long long* total;
-    unsigned long long* per_vertex;   // may be null
-    uint32_t* med_q;                  // edge ids for the medium class
-    uint32_t* heavy_q;                // edge ids for the heavy class
-    uint32_t* cnt;                    // [0] medium, [1] heavy, [2] heavy ticket, [3] medium ticket
-    int32_t* src_of;                  // edge -> source (written by the light pass)
+__global__ void tc_weight_deg_kernel(int64_t nv, const hn_vrec* __restrict__ rec, uint32_t* __restrict__ weight) {
+    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v < nv) weight[v] = (uint32_t)rec[v].deg;
+}
+
+// Where every vertex can have a bit there is nothing to choose: codes are the
+// ids.  One launch in place of six (weights, histogram, cut and codes), 110 us of
+// the 590 that a stored graph of 6 K vertices and 100 K entries took.
+__global__ void tc_all_hubs_kernel(int64_t nv, const hn_vrec* __restrict__ rec, uint2* __restrict__ wc,
+                                   uint32_t* __restrict__ hub) {
+    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= nv) return;
+    wc[v] = make_uint2((uint32_t)rec[v].deg, (uint32_t)v);
+    hub[v] = (uint32_t)v;
+}
+
+// ---- rows
+// groups of the stored rows, prefix summed: a row's place (its list is no
+// longer), and the partition for the pass over the entries
+struct StoredGroupsIn {
+    const hn_vrec* rec;
+    __device__ __forceinline__ uint32_t operator()(int64_t v) const { return ((uint32_t)rec[v].deg + TC_G - 1) / TC_G; }
+};
+__device__ __forceinline__ void tc_tiles(uint32_t* __restrict__ tile_lo, int64_t v, uint32_t ex, uint32_t x) {
+    if (x)
+        for (uint32_t t = (ex + TC_TILE - 1) / TC_TILE; (uint64_t)t * TC_TILE < (uint64_t)ex + x; t++)
+            tile_lo[t] = (uint32_t)v;
+}
+struct StoredGroupsOut {
+    TcRow* row;
+    uint32_t* P;
+    uint32_t* tile_lo;
+    __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t x) const {
+        row[v] = TcRow{ex, 0u, 0u, 0u};
+        P[v] = ex;
+        tc_tiles(tile_lo, v, ex, x);
+    }
 };
 
-// The light edges of one tile (at most LIGHT_MAX entries in the shorter
-// list): their lists, and one work item per entry of the shorter list.
-struct LightShared {
-    uint32_t s[TC_TILE];        // first entry of the shorter list in adj
-    uint32_t l[TC_TILE];        // first entry of the longer list
-    int32_t ln[TC_TILE];        // length of the longer list
-    int32_t credit[TC_TILE];    // the vertex credited
-    uint32_t pre[TC_TILE + 1];  // shorter-list lengths, then their exclusive prefix
-    uint32_t cnt[TC_TILE];      // matches per light edge
-    uint32_t sc[NWAVES + 1];
-    uint32_t n;
-};
+using TcLb = LbShared<TC_IPT, uint32_t, uint32_t>;
 
-// Light pass over all stored edges: defers medium / heavy edges to queues and
-// counts the light ones.  A light edge's up to LIGHT_MAX binary searches are
-// spread over the workgroup (one search per lane, the tile's light edges
-// flattened into one item list), not run one after another by the lane that
-// found the edge: the slowest lane of a wave had chained up to
-// TC_IPT x LIGHT_MAX searches.
-__global__ __launch_bounds__(BLOCK) void tc_light_kernel(int32_t nv, int64_t ne, TcCsr g, TcOut o) {
-    __shared__ LbShared<TC_IPT, int64_t> sh;
-    __shared__ LightShared ls;
-    unsigned long long acc = 0;
-    const uint64_t lt = lanemask_lt();
-    for (int64_t w0 = (int64_t)blockIdx.x * TC_TILE; w0 < ne; w0 += (int64_t)gridDim.x * TC_TILE) {
-        if (threadIdx.x == 0) ls.n = 0;   // lb_tile synchronises before it calls the items
-        lb_tile<TC_IPT>(
-            g.off, (int64_t)nv, w0, ne, sh, [&](int64_t s) { return (int64_t)0; },
-            [&](int64_t s, int64_t e, int64_t) {
-                const int32_t u0 = (int32_t)s;
-                const int32_t v0 = g.adj[e];
-                const int64_t su = g.off[u0], du = g.off[u0 + 1] - su;
-                const int64_t sv = g.off[v0], dv = g.off[v0 + 1] - sv;
-                int cls = 0;   // 0 done here, 1 medium, 2 heavy
-                o.src_of[e] = u0;
-                if (u0 != v0 && du >= 2) {
-                    const bool src_smaller = du < dv;
-                    const int64_t sn = src_smaller ? du : dv;
-                    if (sn <= LIGHT_MAX) {
-                        if (sn > 0) {
-                            const uint32_t k = atomicAdd(&ls.n, 1u);
-                            ls.s[k] = (uint32_t)(src_smaller ? su : sv);
-                            ls.l[k] = (uint32_t)(src_smaller ? sv : su);
-                            ls.ln[k] = (int32_t)(src_smaller ? dv : du);
-                            ls.credit[k] = src_smaller ? u0 : v0;
-                            ls.pre[k] = (uint32_t)sn;
-                            ls.cnt[k] = 0;
-                        }
-                    } else {
-                        cls = sn <= MEDIUM_MAX ? 1 : 2;
-                    }
-                }
-                // wave-aggregated queue appends for deferred edges
-                for (int q = 1; q <= 2; q++) {
-                    const uint64_t m = __ballot(cls == q);
-                    if (m) {
-                        const int leader = __ffsll((unsigned long long)m) - 1;
-                        uint32_t b = 0;
-                        if (__lane_id() == leader) b = atomicAdd(o.cnt + (q - 1), (uint32_t)__popcll(m));
-                        b = __shfl(b, leader, WAVE);
-                        if (cls == q) (q == 1 ? o.med_q : o.heavy_q)[b + (uint32_t)__popcll(m & lt)] = (uint32_t)e;
-                    }
-                }
-            });
-        __syncthreads();
-        // exclusive prefix of the shorter-list lengths (thread t owns entries
-        // t * TC_IPT .. t * TC_IPT + TC_IPT - 1)
-        const uint32_t n = ls.n;
-        uint32_t len[TC_IPT], sum = 0;
+// A tile's rows staged and its groups located: group j of the lane is the k-th
+// of row seg (seg < 0 past the end).
+struct TcLoc {
+    int64_t seg[TC_IPT];
+    uint32_t k[TC_IPT];
+};
+template <typename BaseFn>
+__device__ __forceinline__ TcLoc tc_locate(const uint32_t* __restrict__ P, int64_t nv, uint32_t total,
+                                           const uint32_t* __restrict__ tile_lo, int64_t t, int64_t ntiles, TcLb& sh,
+                                           BaseFn base, uint32_t (&b)[TC_IPT]) {
+    const int64_t lo = tile_lo[t], hi = t + 1 < ntiles ? (int64_t)tile_lo[t + 1] : nv - 1;
+    const int64_t span = hi - lo + 1;
+    const bool staged = span <= TcLb::CAP;
+    if (staged)
+        for (int i = threadIdx.x; i < (int)span; i += BLOCK) {
+            sh.pref[i] = P[lo + i];
+            sh.base[i] = base(lo + i);
+        }
+    __syncthreads();
+    TcLoc c;
+#pragma unroll
+    for (int j = 0; j < TC_IPT; j++) {
+        const int64_t w = t * TC_TILE + (int64_t)j * BLOCK + threadIdx.x;
+        c.seg[j] = -1;
+        c.k[j] = 0;
+        b[j] = 0;
+        if (w < (int64_t)total) {
+            if (staged) {
+                const int s = lb_locate(sh, (int)span, w);
+                c.seg[j] = lo + s;
+                c.k[j] = (uint32_t)w - sh.pref[s];
+                b[j] = sh.base[s];
+            } else {
+                const int64_t s = upper_bound_m1<int64_t>(P, lo, hi + 1, w);
+                c.seg[j] = s;
+                c.k[j] = (uint32_t)w - P[s];
+                b[j] = base(s);
+            }
+        }
+    }
+    return c;
+}
+
+// How often a vertex is an entry, from every `step`-th tile of the stored rows
+// (any choice of hubs gives the same counts).
+__global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
+                                                               const uint32_t* __restrict__ P,
+                                                               const uint32_t* __restrict__ tile_lo,
+                                                               const hn_vrec* __restrict__ rec,
+                                                               const int32_t* __restrict__ arena, int step,
+                                                               uint32_t* __restrict__ weight) {
+    __shared__ TcLb sh;
+    const uint32_t total = *ngroups;
+    const int64_t ntiles = ((int64_t)total + TC_TILE - 1) / TC_TILE;
+    for (int64_t t = (int64_t)blockIdx.x * step; t < ntiles; t += (int64_t)gridDim.x * step) {
+        uint32_t unit[TC_IPT];
+        const TcLoc c = tc_locate(P, nv, total, tile_lo, t, ntiles, sh,
+                                  [&](int64_t s) { return (uint32_t)(rec[s].off / UNIT_SLOTS); }, unit);
 #pragma unroll
         for (int j = 0; j < TC_IPT; j++) {
-            const uint32_t k = (uint32_t)threadIdx.x * TC_IPT + j;
-            len[j] = k < n ? ls.pre[k] : 0u;
-            sum += len[j];
-        }
-        uint32_t items;
-        uint32_t run = block_exclusive_scan(sum, ls.sc, &items);
-#pragma unroll
-        for (int j = 0; j < TC_IPT; j++) {
-            const uint32_t k = (uint32_t)threadIdx.x * TC_IPT + j;
-            if (k < n) ls.pre[k] = run;
-            run += len[j];
+            if (c.seg[j] < 0) continue;
+            const int64_t at = (int64_t)unit[j] * UNIT_SLOTS + (int64_t)c.k[j] * TC_G;
+            const int64_t n = min((int64_t)TC_G, (int64_t)rec[c.seg[j]].deg - (int64_t)c.k[j] * TC_G);
+            for (int64_t e = 0; e < n; e++) atomicAdd(weight + arena[at + e], 1u);
         }
         __syncthreads();
-        // one binary search per item: item t is entry t - pre[k] of light edge k
-        for (uint32_t t = threadIdx.x; t < items; t += BLOCK) {
-            uint32_t lo = 0, hi = n;   // largest k with pre[k] <= t (pre strictly increasing)
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (ls.pre[mid] <= t) lo = mid; else hi = mid;
-            }
-            const int32_t x = g.adj[(int64_t)ls.s[lo] + (t - ls.pre[lo])];
-            if (bsearch_has(g.adj + ls.l[lo], ls.ln[lo], x)) atomicAdd(&ls.cnt[lo], 1u);
-        }
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < n; k += BLOCK) {
-            const uint32_t c = ls.cnt[k];
-            if (c) {
-                if (o.per_vertex) atomicAdd(o.per_vertex + ls.credit[k], (unsigned long long)c);
-                acc += c;
-            }
-        }
-        __syncthreads();   // the next tile reuses ls
     }
-    acc = wave_reduce_sum(acc);
-    if (__lane_id() == 0 && acc) atomicAdd(o.total, acc);
 }
 
-// `lanes` lanes cooperate on one deferred edge
-constexpr int64_t TC_CHUNK = 16;
-template <int LANES>
-__global__ __launch_bounds__(BLOCK) void tc_group_kernel(TcCsr g, const uint32_t* __restrict__ q,
-                                                         const uint32_t* __restrict__ qcount,
-                                                         const int32_t* __restrict__ src_of, TcOut o) {
-    const uint32_t n = *qcount;
-    const int sub = threadIdx.x % LANES;
-    unsigned long long acc = 0;
-    // one deferred edge; the LANES lanes of a group share k, so a group is
-    // either wholly active or wholly done and the group shuffles never read an
-    // exited lane
-    auto one = [&](int64_t k) {
-        const int64_t e = q[k];
-        const int32_t u0 = src_of[e];
-        const int32_t v0 = g.adj[e];
-        const int64_t su = g.off[u0], du = g.off[u0 + 1] - su;
-        const int64_t sv = g.off[v0], dv = g.off[v0 + 1] - sv;
-        const bool src_smaller = du < dv;
-        const int32_t* sp = g.adj + (src_smaller ? su : sv);
-        const int64_t sn = src_smaller ? du : dv;
-        const int32_t* lp = g.adj + (src_smaller ? sv : su);
-        const int64_t ln = src_smaller ? dv : du;
-        uint32_t c = 0;
-        for (int64_t i = sub; i < sn; i += LANES) c += bsearch_has(lp, ln, sp[i]) ? 1u : 0u;
-        const int32_t credit = src_smaller ? u0 : v0;
-        // reduce over the group
-#pragma unroll
-        for (int d = LANES / 2; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
-        if (sub == 0 && c && o.per_vertex) atomicAdd(o.per_vertex + credit, (unsigned long long)c);
-        if (sub == 0) acc += c;
-    };
-    // edges differ widely in work: each wave claims TC_CHUNK edges per group
-    // at a time from its class's ticket until the queue is drained; the
-    // groups of a wave take the claimed edges in turn
-    constexpr int G = WAVE / LANES;
-    const int grp = (int)(__lane_id() / LANES);
-    uint32_t* ticket = o.cnt + (LANES == WAVE ? 2 : 3);
-    for (;;) {
-        uint32_t t = 0;
-        if (__lane_id() == 0) t = atomicAdd(ticket, 1u);
-        t = __shfl(t, 0, WAVE);
-        const int64_t k0 = (int64_t)t * TC_CHUNK * G;
-        if (k0 >= (int64_t)n) break;
-        const int64_t k1 = k0 + TC_CHUNK * G < (int64_t)n ? k0 + TC_CHUNK * G : (int64_t)n;
-        for (int64_t k = k0 + grp; k < k1; k += G) one(k);
-    }
-    acc = wave_reduce_sum(acc);
-    if (__lane_id() == 0 && acc) atomicAdd(o.total, acc);
-}
-
-// A whole wave per deferred edge, intersecting by sorted windows: lane l
-// holds element l of a 64-entry window of the shorter list S and of the
-// longer list L; each lane finds its S element in the L window with six
-// cross-lane steps, then the S window moves on if its last element is not
-// above the L window's, else the L window does.  Every load is one coalesced
-// 256-byte window, where the binary searches scatter their lanes over a
-// list's cache lines.  Once the L window has moved past an S window, the
-// S entries up to the old L window's last element were already checked, so
-// they count only above it: each S entry counts once if L holds it, as with
-// the binary searches, repeated entries of a multigraph included (a host
-// model of this loop was checked against per-entry binary searches on random
-// lists with and without repeats).
-//
-// A wave runs TC_SLOTS edges at once, each in its own slot, so that the
-// slots' dependent cross-lane steps and window loads overlap; a slot whose
-// edge is done takes the next one.  Windows past a list's end repeat its last
-// entry (they stay sorted and their last lane holds their largest entry),
-// and every iteration loads the next window of both lists of every slot (the
-// same one again when a list does not move on), so the loads need no
-// selects and are in flight while the slots are matched.
-// (R-MAT s24 recount: 1 slot 472 ms, 2 slots 450 ms, 4 slots 490 ms, whose
-// registers leave half the waves per SIMD)
-constexpr int SLOTS = 2;
-
-struct WinSlot {
-    const int32_t* sp;   // shorter list
-    const int32_t* lp;   // longer list
-    int64_t sn, ln;      // their lengths (>= 1 while live)
-    int64_t i, j;        // window starts
-    int32_t a, b;        // this lane's entry of the current windows
-    int32_t an, bn;      // ... of the next windows
-    int32_t lim;         // S entries up to lim were checked against an earlier L window
-    int32_t credit;      // vertex credited with the count
-    uint32_t c;          // this lane's matches
-    bool live;
-};
-
-__device__ __forceinline__ int32_t window_entry(const int32_t* __restrict__ x, int64_t n, int64_t k) {
-    return x[k < n ? k : n - 1];
-}
-
-__global__ __launch_bounds__(BLOCK) void tc_window_kernel(TcCsr g, const uint32_t* __restrict__ q,
-                                                          const uint32_t* __restrict__ qcount,
-                                                          const int32_t* __restrict__ src_of, TcOut o) {
-    const uint32_t n = *qcount;
+// Stored rows -> lists (ORIENT: only the entries up the degree order).  A lane
+// holds eight entries of one row; the lanes of a wave that hold the same row
+// claim its next places, in both of its rows, with one atomic.
+typedef int32_t TcVec __attribute__((ext_vector_type(4)));
+template <bool ORIENT>
+__global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
+                                                        const uint32_t* __restrict__ P,
+                                                        const uint32_t* __restrict__ tile_lo,
+                                                        const hn_vrec* __restrict__ rec,
+                                                        const int32_t* __restrict__ arena,
+                                                        const uint2* __restrict__ wc, TcRow* __restrict__ row,
+                                                        uint16_t* __restrict__ codes, uint32_t* __restrict__ ids,
+                                                        TcCtl* __restrict__ ctl) {
+    __shared__ TcLb sh;
+    const uint32_t total = *ngroups;
+    const int64_t ntiles = ((int64_t)total + TC_TILE - 1) / TC_TILE;
     const int lane = __lane_id();
-    unsigned long long acc = 0;
-    uint32_t* ticket = o.cnt + 2;
-    int64_t k = 0, k1 = 0;   // the wave's claimed edges [k, k1)
-    bool drained = false;
-    // the next queued edge into slot w (or the slot goes idle)
-    auto fetch = [&](WinSlot& w) {
-        if (k >= k1 && !drained) {
-            uint32_t t = 0;
-            if (lane == 0) t = atomicAdd(ticket, 1u);
-            t = __shfl(t, 0, WAVE);
-            k = (int64_t)t * TC_CHUNK;
-            k1 = k + TC_CHUNK < (int64_t)n ? k + TC_CHUNK : (int64_t)n;
-            drained = k >= (int64_t)n;
-        }
-        if (drained || k >= k1) {
-            w.live = false;
-            w.sp = w.lp = g.adj;   // an idle slot keeps loading one valid entry
-            w.sn = w.ln = 1;
-            w.i = w.j = 0;
-            w.a = w.b = w.an = w.bn = 0;
-            w.lim = -1;
-            w.c = 0;
-            w.credit = 0;
-            return;
-        }
-        const int64_t e = q[k++];
-        const int32_t u0 = src_of[e];
-        const int32_t v0 = g.adj[e];
-        const int64_t su = g.off[u0], du = g.off[u0 + 1] - su;
-        const int64_t sv = g.off[v0], dv = g.off[v0 + 1] - sv;
-        const bool src_smaller = du < dv;
-        w.sp = g.adj + (src_smaller ? su : sv);
-        w.sn = src_smaller ? du : dv;
-        w.lp = g.adj + (src_smaller ? sv : su);
-        w.ln = src_smaller ? dv : du;
-        w.credit = src_smaller ? u0 : v0;
-        w.live = true;   // a deferred edge has both lists above LIGHT_MAX entries
-        w.i = w.j = 0;
-        w.a = window_entry(w.sp, w.sn, lane);
-        w.b = window_entry(w.lp, w.ln, lane);
-        w.an = window_entry(w.sp, w.sn, WAVE + lane);
-        w.bn = window_entry(w.lp, w.ln, WAVE + lane);
-        w.lim = -1;
-        w.c = 0;
-    };
-    WinSlot ws[SLOTS];
+    bool twice = false;
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        uint32_t unit[TC_IPT];
+        const TcLoc c = tc_locate(P, nv, total, tile_lo, t, ntiles, sh,
+                                  [&](int64_t s) { return (uint32_t)(rec[s].off / UNIT_SLOTS); }, unit);
+        int32_t a[TC_IPT][TC_G], prev[TC_IPT], deg[TC_IPT];
 #pragma unroll
-    for (int s = 0; s < SLOTS; s++) fetch(ws[s]);
-    for (;;) {
-        bool any = false;
+        for (int j = 0; j < TC_IPT; j++) {
+            const int64_t at = (int64_t)unit[j] * UNIT_SLOTS + (int64_t)c.k[j] * TC_G;
+            const TcVec p = *reinterpret_cast<const TcVec*>(arena + at), q = *reinterpret_cast<const TcVec*>(arena + at + 4);
 #pragma unroll
-        for (int s = 0; s < SLOTS; s++) any = any || ws[s].live;
-        if (!any) break;
-        // first index p of each L window with b[p] >= a, the slots interleaved
-        int p[SLOTS];
-#pragma unroll
-        for (int s = 0; s < SLOTS; s++) p[s] = 0;
-#pragma unroll
-        for (int st = 32; st > 0; st >>= 1)
-#pragma unroll
-            for (int s = 0; s < SLOTS; s++) {
-                const int32_t x = __shfl(ws[s].b, p[s] + st - 1, WAVE);
-                p[s] += x < ws[s].a ? st : 0;
+            for (int e = 0; e < 4; e++) {
+                a[j][e] = p[e];
+                a[j][4 + e] = q[e];
             }
-#pragma unroll
-        for (int s = 0; s < SLOTS; s++) {
-            WinSlot& w = ws[s];
-            const int32_t y = __shfl(w.b, p[s] & (WAVE - 1), WAVE);
-            w.c += (w.live && p[s] < WAVE && y == w.a && w.i + lane < w.sn && w.a > w.lim) ? 1u : 0u;
-            const int32_t amax = __builtin_amdgcn_readlane(w.a, WAVE - 1);
-            const int32_t bmax = __builtin_amdgcn_readlane(w.b, WAVE - 1);
-            const bool adv_a = amax <= bmax;
-            w.i += adv_a ? WAVE : 0;
-            w.j += adv_a ? 0 : WAVE;
-            w.a = adv_a ? w.an : w.a;
-            w.b = adv_a ? w.b : w.bn;
-            w.lim = adv_a ? -1 : bmax;
-            w.an = window_entry(w.sp, w.sn, w.i + WAVE + lane);
-            w.bn = window_entry(w.lp, w.ln, w.j + WAVE + lane);
+            prev[j] = c.k[j] ? arena[at - 1] : -1;
+            deg[j] = rec[c.seg[j] >= 0 ? c.seg[j] : 0].deg;
         }
 #pragma unroll
-        for (int s = 0; s < SLOTS; s++) {
-            WinSlot& w = ws[s];
-            if (w.live && (w.i >= w.sn || w.j >= w.ln)) {
-                const uint32_t tot = wave_reduce_sum(w.c);
-                if (lane == 0) {
-                    if (tot && o.per_vertex) atomicAdd(o.per_vertex + w.credit, (unsigned long long)tot);
-                    acc += tot;
+        for (int j = 0; j < TC_IPT; j++) {
+            const int64_t n = c.seg[j] >= 0 ? (int64_t)deg[j] - (int64_t)c.k[j] * TC_G : 0;
+            const int32_t u = (int32_t)c.seg[j];
+            uint2 x[TC_G];
+#pragma unroll
+            for (int e = 0; e < TC_G; e++) x[e] = wc[e < n ? a[j][e] : 0];
+            uint32_t keep = 0, hubs = 0;
+#pragma unroll
+            for (int e = 0; e < TC_G; e++) {
+                const int32_t v = a[j][e];
+                const bool k = e < n && (!ORIENT || (uint32_t)deg[j] < x[e].x || ((uint32_t)deg[j] == x[e].x && u < v));
+                keep |= (uint32_t)k << e;
+                hubs |= (uint32_t)(k && !(x[e].y & TC_ID)) << e;
+                twice = twice || (e < n && v == (e ? a[j][e - 1] : prev[j]));
+            }
+            // both counts in one word: a wave holds at most 512 entries
+            const uint32_t cnt = (uint32_t)__popc(hubs) | (uint32_t)__popc(keep & ~hubs) << 16;
+            const uint32_t inc = wave_inclusive_scan(cnt);
+            const int32_t up = __shfl_up(u, 1, WAVE);
+            const uint64_t heads = __ballot(lane == 0 || u != up);
+            const int head = 63 - __clzll((long long)(heads & (lanemask_lt() | (1ull << lane))));
+            const uint64_t above = lane == WAVE - 1 ? 0ull : heads & (~0ull << (lane + 1));
+            const int tail = above ? __ffsll((unsigned long long)above) - 2 : WAVE - 1;
+            const uint32_t before = __shfl(inc - cnt, head, WAVE);
+            const uint32_t sum = __shfl(inc, tail, WAVE) - before;
+            unsigned long long at = 0;
+            if (lane == head && sum)
+                at = atomicAdd(reinterpret_cast<unsigned long long*>(&row[u].n16),
+                               (unsigned long long)(sum & 0xFFFFu) | (unsigned long long)(sum >> 16) << 32);
+            const uint32_t at16 = __shfl((uint32_t)at, head, WAVE), at32 = __shfl((uint32_t)(at >> 32), head, WAVE);
+            if (keep) {
+                const uint32_t mine = inc - cnt - before;
+                const int64_t base = (int64_t)row[u].base * TC_G;
+                uint16_t* o16 = codes + base + at16 + (mine & 0xFFFFu);
+                uint32_t* o32 = ids + base + at32 + (mine >> 16);
+#pragma unroll
+                for (int e = 0; e < TC_G; e++) {
+                    if ((hubs >> e) & 1u) *o16++ = (uint16_t)x[e].y;
+                    else if ((keep >> e) & 1u) *o32++ = (uint32_t)a[j][e];
                 }
-                fetch(w);
+            }
+        }
+        __syncthreads();
+    }
+    if (__ballot(twice) && lane == 0) ctl->repeats = 1u;   // every writer stores the same value
+}
+
+__global__ void tc_pad_kernel(int64_t nv, const TcRow* __restrict__ row, uint16_t* __restrict__ codes,
+                              uint32_t* __restrict__ ids) {
+    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= nv) return;
+    const TcRow r = row[v];
+    for (uint32_t i = r.n16; i & (TC_G - 1); i++) codes[(int64_t)r.base * TC_G + i] = (uint16_t)TC_PAD16;
+    for (uint32_t i = r.n32; i & (TC_G - 1); i++) ids[(int64_t)r.base * TC_G + i] = TC_PAD;
+}
+
+// entry i of a list, as a vertex
+__device__ __forceinline__ uint32_t tc_entry(const TcRow& r, uint32_t i, const uint16_t* __restrict__ codes,
+                                             const uint32_t* __restrict__ ids, const uint32_t* __restrict__ hub) {
+    return i < r.n16 ? hub[codes[(int64_t)r.base * TC_G + i]] : ids[(int64_t)r.base * TC_G + (i - r.n16)];
+}
+
+// ---- edges whose longer list is the destination's, grouped by it (where an
+// owner's edges cannot be read from its stored row), over the same partition
+// FILL = false: the edge's place in its group (TC_PAD: not grouped); FILL = true: the sources at their places
+template <bool FILL>
+__global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
+                                                         const uint32_t* __restrict__ P,
+                                                         const uint32_t* __restrict__ tile_lo, int sym,
+                                                         const TcCtl* __restrict__ ctl, const TcRow* __restrict__ row,
+                                                         const uint16_t* __restrict__ codes,
+                                                         const uint32_t* __restrict__ ids,
+                                                         const uint32_t* __restrict__ hub, uint32_t* __restrict__ gcnt,
+                                                         uint32_t* __restrict__ place, const uint32_t* __restrict__ goff,
+                                                         uint32_t* __restrict__ members) {
+    if (sym && !ctl->repeats) return;
+    __shared__ TcLb sh;
+    const uint32_t total = *ngroups;
+    const int64_t ntiles = ((int64_t)total + TC_TILE - 1) / TC_TILE;
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        uint32_t unused[TC_IPT];
+        const TcLoc c = tc_locate(P, nv, total, tile_lo, t, ntiles, sh, [&](int64_t) { return 0u; }, unused);
+#pragma unroll
+        for (int j = 0; j < TC_IPT; j++) {
+            if (c.seg[j] < 0) continue;
+            const uint32_t u = (uint32_t)c.seg[j];
+            const TcRow r = row[u];
+            const uint32_t lu = r.len();
+            if (lu < 2) continue;
+            // entries [8k, 8k + 8) of the list, which may end before its stored row
+            for (uint32_t i = c.k[j] * TC_G; i < min(lu, (c.k[j] + 1) * TC_G); i++) {
+                const uint32_t v = tc_entry(r, i, codes, ids, hub);
+                uint32_t* pl = place + (int64_t)r.base * TC_G + i;
+                if constexpr (FILL) {
+                    if (*pl != TC_PAD) members[(int64_t)goff[v] + *pl] = u;
+                } else {
+                    const uint32_t lv = row[v].len();
+                    *pl = lv > lu && lv > TC_SMALL && v != u ? atomicAdd(gcnt + v, 1u) : TC_PAD;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// ---- tasks: up to TC_CAND candidates of one owner
+struct TaskIn {
+    const TcRow* row;
+    const uint32_t* gcnt;
+    const hn_vrec* rec;
+    const TcCtl* ctl;
+    int sym;
+    __device__ __forceinline__ uint32_t operator()(int64_t v) const {
+        const TcRow r = row[v];
+        const uint32_t n = r.len();
+        if (n <= TC_SMALL) return 0u;
+        const uint32_t cand = sym && !ctl->repeats ? (uint32_t)rec[v].deg : n + gcnt[v];
+        return (cand + TC_CAND - 1) / TC_CAND;
+    }
+};
+struct TaskOut {
+    uint2* task;
+    __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t n) const {
+        for (uint32_t k = 0; k < n; k++) task[ex + k] = make_uint2((uint32_t)v, k);
+    }
+};
+
+struct OwnerShared {
+    uint32_t bits[(TC_HUBS + 1) / 32];
+    uint32_t hash[TC_HASH];
+    uint32_t y[TC_STEP], base[TC_STEP], n16[TC_STEP], n32[TC_STEP];   // the edges listed: vertex and rows of the shorter list
+    uint32_t cls[TC_ORDER];
+    uint32_t tail;
+    uint2 task;
+};
+static_assert(sizeof(OwnerShared) * 8 <= 160 * 1024, "eight workgroups fill a CU's LDS");
+
+__device__ __forceinline__ uint32_t tc_slot(uint32_t id) { return (id * 2654435761u) >> (32 - 9); }
+static_assert(TC_HASH == 1u << 9, "tc_slot yields nine bits");
+
+__device__ __forceinline__ uint32_t tc_test(const OwnerShared& sh, const uint4& x) {
+    const uint32_t q[4] = {x.x, x.y, x.z, x.w};
+    uint32_t k = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {   // two codes a word: bit (code & 31) of word code >> 5
+        const uint32_t lo = q[e], hi = q[e] >> 16;
+        k += (sh.bits[(lo >> 5) & 2047u] >> (lo & 31)) & 1u;
+        k += (sh.bits[hi >> 5] >> (hi & 31)) & 1u;
+    }
+    return k;
+}
+
+// The listed edges' shorter lists against the owner's set: a team of eight
+// lanes per list, eight codes per lane and group.  The lists are sorted by
+// length class, so that the teams of a wave stay together: TC_DEPTH groups of one
+// list in flight while lists are longer than a team's step, then TC_DEPTH lists.
+template <bool TAIL>
+__device__ __forceinline__ uint32_t tc_ids(const OwnerShared& sh, uint32_t it, int sub, const uint32_t* __restrict__ ids) {
+    uint32_t c = 0;
+    if constexpr (TAIL) {
+        const uint32_t* li = ids + (int64_t)sh.base[it] * TC_G;
+        const uint32_t n32 = sh.n32[it];
+        for (uint32_t i = sub; i < n32; i += TC_TEAM) {
+            const uint32_t q = li[i];
+            for (uint32_t s = tc_slot(q);; s = (s + 1) & (TC_HASH - 1)) {
+                const uint32_t z = sh.hash[s];
+                c += z == q ? 1u : 0u;
+                if (z == q || z == TC_PAD) break;
             }
         }
     }
-    if (lane == 0 && acc) atomicAdd(o.total, acc);
+    return c;
 }
-
-// ---- orientation of the symmetric storage
-constexpr int OR_IPT = 8;
-constexpr int OR_TILE = BLOCK * OR_IPT;
-
-__global__ __launch_bounds__(BLOCK) void orient_flags_kernel(int32_t nv, int64_t ne, const int64_t* __restrict__ eoff,
-                                                             const hn_vrec* __restrict__ rec,
-                                                             const int32_t* __restrict__ arena,
-                                                             int32_t* __restrict__ adj_tmp,
-                                                             uint8_t* __restrict__ keep) {
-    __shared__ LbShared<OR_IPT, int64_t> sh;
-    for (int64_t w0 = (int64_t)blockIdx.x * OR_TILE; w0 < ne; w0 += (int64_t)gridDim.x * OR_TILE) {
-        lb_tile<OR_IPT>(
-            eoff, (int64_t)nv, w0, ne, sh, [&](int64_t s) { return rec[s].off - eoff[s]; },
-            [&](int64_t s, int64_t w, int64_t base) {
-                const int32_t v = arena[base + w];
-                const int32_t u = (int32_t)s;
-                const int32_t du = (int32_t)(eoff[u + 1] - eoff[u]);
-                const int32_t dv = rec[v].deg;
-                adj_tmp[w] = v;
-                keep[w] = (du < dv || (du == dv && u < v)) ? 1 : 0;
-            });
+// the sums of eight lanes in lanes 7 and 15 of every row
+__device__ __forceinline__ uint32_t tc_team_sum(uint32_t c) {
+    c += dpp_move<0x111, 0xf>(c);
+    c += dpp_move<0x112, 0xf>(c);
+    c += dpp_move<0x114, 0xf>(c);
+    return c;
+}
+template <bool TAIL>
+__device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, uint32_t n,
+                                        const uint16_t* __restrict__ codes, const uint32_t* __restrict__ ids,
+                                        unsigned long long* __restrict__ per_vertex, uint64_t& acc) {
+    constexpr uint32_t TEAMS = BLOCK / TC_TEAM;
+    const int sub = threadIdx.x & (TC_TEAM - 1);
+    const uint4* rows = reinterpret_cast<const uint4*>(codes);
+    uint32_t it = threadIdx.x / TC_TEAM;
+    for (; it < nlong; it += TEAMS) {
+        const uint4* list = rows + sh.base[it];
+        const uint32_t ng = (sh.n16[it] + TC_G - 1) / TC_G;
+        uint32_t c = tc_ids<TAIL>(sh, it, sub, ids);
+        for (uint32_t g0 = sub; g0 < ng; g0 += TC_TEAM * TC_DEPTH) {
+            uint4 x[TC_DEPTH];
+#pragma unroll
+            for (int d = 0; d < TC_DEPTH; d++) {
+                const uint32_t g = g0 + d * TC_TEAM;
+                if (__ballot(g < ng) == 0) break;
+                x[d] = list[g < ng ? g : g0];
+            }
+#pragma unroll
+            for (int d = 0; d < TC_DEPTH; d++) {
+                const bool in = g0 + d * TC_TEAM < ng;
+                if (__ballot(in) == 0) break;
+                const uint32_t k = tc_test(sh, x[d]);
+                c += in ? k : 0u;
+            }
+        }
+        acc += c;
+        c = tc_team_sum(c);
+        if (sub == TC_TEAM - 1 && c && per_vertex) atomicAdd(per_vertex + sh.y[it], (unsigned long long)c);
+    }
+    for (; it < n; it += TEAMS * TC_DEPTH) {
+        uint4 x[TC_DEPTH];
+        bool in[TC_DEPTH];
+#pragma unroll
+        for (int d = 0; d < TC_DEPTH; d++) {
+            const uint32_t i = min(it + d * TEAMS, n - 1);
+            in[d] = it + d * TEAMS < n && (uint32_t)sub * TC_G < sh.n16[i];
+            x[d] = rows[(int64_t)sh.base[i] + (in[d] ? sub : 0)];
+        }
+#pragma unroll
+        for (int d = 0; d < TC_DEPTH; d++) {
+            const uint32_t i = it + d * TEAMS;
+            if (i >= n) break;
+            const uint32_t k = tc_test(sh, x[d]);
+            uint32_t c = (in[d] ? k : 0u) + tc_ids<TAIL>(sh, i, sub, ids);
+            acc += c;
+            c = tc_team_sum(c);
+            if (sub == TC_TEAM - 1 && c && per_vertex) atomicAdd(per_vertex + sh.y[i], (unsigned long long)c);
+        }
     }
 }
 
-__global__ void orient_compact_kernel(int64_t ne, const uint8_t* __restrict__ keep, const uint32_t* __restrict__ pos,
-                                      const int32_t* __restrict__ adj_tmp, int32_t* __restrict__ adjp) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < ne && keep[e]) adjp[pos[e]] = adj_tmp[e];
+// Bound by the sectors of the shorter lists that miss the L2: on R-MAT s22 360 M of
+// the 400 M that the walks touch, 7.4 ms at the 48 G/s that scattered sector reads
+// reach here; LDS and vector units are a third busy.
+__global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int sym, const hn_vrec* __restrict__ rec,
+                                                         const int32_t* __restrict__ arena,
+                                                         const uint2* __restrict__ wc, const uint2* __restrict__ task,
+                                                         const TcRow* __restrict__ row,
+                                                         const uint16_t* __restrict__ codes,
+                                                         const uint32_t* __restrict__ ids,
+                                                         const uint32_t* __restrict__ hub,
+                                                         const uint32_t* __restrict__ gcnt,
+                                                         const uint32_t* __restrict__ goff,
+                                                         const uint32_t* __restrict__ members, TcCtl* __restrict__ ctl,
+                                                         unsigned long long* __restrict__ per_vertex) {
+    __shared__ OwnerShared sh;
+    const uint32_t ntask = ctl->ntask;
+    const bool stored = sym && !ctl->repeats;
+    uint64_t acc = 0;
+    for (int i = threadIdx.x; i < (int)(TC_HUBS + 1) / 32; i += BLOCK) sh.bits[i] = 0;
+    // The next task is taken while this one runs.  Tickets are for `chunk` tasks, of
+    // one of TC_LANES interleaved shares; the others' once that one is used up.  (One
+    // ticket for each of R-MAT s22's 640 K tasks, from one counter, was what
+    // bounded the kernel: 10.1 ms, 7.6 ms so.)
+    const uint32_t chunk = min(max(ntask / (gridDim.x * 32u), 1u), 8u);
+    uint32_t cur = 0, end = 0, tried = 0;
+    auto next = [&]() {
+        while (cur >= end) {
+            if (tried == TC_LANES) return make_uint2(0u, TC_PAD);
+            const uint32_t share = (blockIdx.x + tried) % TC_LANES;
+            uint32_t* at = &ctl->ticket[share].v;
+            const uint32_t seen = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t first = ((uint64_t)seen * TC_LANES + share) * chunk;
+            uint64_t lo = first;
+            if (first < ntask) lo = ((uint64_t)atomicAdd(at, 1u) * TC_LANES + share) * chunk;
+            if (lo >= ntask) {
+                tried++;
+                continue;
+            }
+            cur = (uint32_t)lo;
+            end = (uint32_t)min(lo + chunk, (uint64_t)ntask);
+        }
+        return task[cur++];
+    };
+    uint2 ahead = make_uint2(0u, TC_PAD);
+    if (threadIdx.x == 0) sh.task = next();
+    __syncthreads();
+    for (;;) {
+        const uint2 tk = sh.task;
+        if (tk.y == TC_PAD) break;
+        if (threadIdx.x == 0) ahead = next();
+        const uint32_t x = tk.x;
+        const TcRow rx = row[x];
+        const hn_vrec sx = rec[x];
+        const uint32_t lx = rx.len(), cand = stored ? (uint32_t)sx.deg : lx + gcnt[x];
+        const uint32_t c0 = tk.y * TC_CAND, c1 = min(c0 + TC_CAND, cand);
+        const int64_t at = (int64_t)rx.base * TC_G;
+        const uint32_t passes = rx.n32 ? (rx.n32 + TC_TAIL - 1) / TC_TAIL : 1;
+        for (uint32_t p = 0; p < passes; p++) {
+            // the set: the hubs' bits in the first pass, TC_TAIL ids in each
+            if (p == 0)
+                for (uint32_t i = threadIdx.x; i < rx.n16; i += BLOCK) {
+                    const uint32_t q = codes[at + i];
+                    atomicOr(&sh.bits[q >> 5], 1u << (q & 31));
+                }
+            if (rx.n32) {
+                for (uint32_t i = threadIdx.x; i < TC_HASH; i += BLOCK) sh.hash[i] = TC_PAD;
+                __syncthreads();
+                for (uint32_t i = p * TC_TAIL + threadIdx.x; i < min(rx.n32, (p + 1) * TC_TAIL); i += BLOCK) {
+                    const uint32_t q = ids[at + i];
+                    for (uint32_t s = tc_slot(q);; s = (s + 1) & (TC_HASH - 1)) {
+                        const uint32_t z = atomicCAS(&sh.hash[s], TC_PAD, q);
+                        if (z == TC_PAD || z == q) break;
+                    }
+                }
+            }
+            for (uint32_t b = c0; b < c1; b += TC_STEP) {
+                if (threadIdx.x < TC_ORDER) sh.cls[threadIdx.x] = 0;
+                __syncthreads();   // (the set too)
+                uint32_t y[TC_STEP / BLOCK], cl[TC_STEP / BLOCK], pos[TC_STEP / BLOCK];
+                TcRow ry[TC_STEP / BLOCK];
+#pragma unroll
+                for (int j = 0; j < TC_STEP / BLOCK; j++) {
+                    const uint32_t i = b + j * BLOCK + threadIdx.x;
+                    y[j] = x;
+                    if (i < c1)
+                        y[j] = stored ? (uint32_t)arena[sx.off + i]
+                                      : i < lx ? tc_entry(rx, i, codes, ids, hub) : members[(int64_t)goff[x] + (i - lx)];
+                    ry[j] = row[y[j]];
+                }
+#pragma unroll
+                for (int j = 0; j < TC_STEP / BLOCK; j++) {
+                    const uint32_t ly = ry[j].len();
+                    // shorter lists, and lists as long of edges whose source x is
+                    bool take = y[j] != x && ly != 0 && ly <= lx;
+                    if (stored && take && ly == lx) {
+                        const uint32_t wx = wc[x].x, wy = wc[y[j]].x;
+                        take = wx < wy || (wx == wy && x < y[j]);
+                    }
+                    // classes by steps of a team, the longest first
+                    const uint32_t steps = (ry[j].n16 + TC_TEAM * TC_G - 1) / (TC_TEAM * TC_G);
+                    cl[j] = take ? TC_ORDER - 1 - min(steps, (uint32_t)TC_ORDER - 1) : TC_PAD;
+                    pos[j] = take ? atomicAdd(&sh.cls[cl[j]], 1u) : 0u;
+                }
+                __syncthreads();
+                uint32_t n = 0;
+                if (threadIdx.x < WAVE) {
+                    const uint32_t k = threadIdx.x < TC_ORDER ? sh.cls[threadIdx.x] : 0u;
+                    const uint32_t inc = wave_inclusive_scan(k);
+                    if (threadIdx.x < TC_ORDER) sh.cls[threadIdx.x] = inc - k;
+                    if (threadIdx.x == WAVE - 1) sh.tail = inc;
+                }
+                __syncthreads();
+                n = sh.tail;
+                const uint32_t nlong = sh.cls[TC_ORDER - 2];   // of the last two classes are one step or none
+#pragma unroll
+                for (int j = 0; j < TC_STEP / BLOCK; j++)
+                    if (cl[j] != TC_PAD) {
+                        const uint32_t k = sh.cls[cl[j]] + pos[j];
+                        sh.y[k] = y[j];
+                        sh.base[k] = ry[j].base;
+                        sh.n16[k] = p == 0 ? ry[j].n16 : 0u;   // later passes count only their ids
+                        sh.n32[k] = ry[j].n32;
+                    }
+                __syncthreads();
+                if (rx.n32) tc_walk<true>(sh, nlong, n, codes, ids, per_vertex, acc);
+                else tc_walk<false>(sh, nlong, n, codes, ids, per_vertex, acc);
+                __syncthreads();
+            }
+        }
+        for (uint32_t i = threadIdx.x; i < rx.n16; i += BLOCK) sh.bits[codes[at + i] >> 5] = 0;
+        if (threadIdx.x == 0) sh.task = ahead;
+        __syncthreads();
+    }
+    acc = wave_reduce_sum(acc);
+    if (__lane_id() == 0 && acc) atomicAdd(&ctl->total[(blockIdx.x + threadIdx.x / WAVE) % TC_SUMS].v, (unsigned long long)acc);
 }
 
-__global__ void orient_offsets_kernel(int32_t nv, const int64_t* __restrict__ eoff, const uint32_t* __restrict__ pos,
-                                      int64_t* __restrict__ offp) {
-    int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v <= nv) offp[v] = pos[eoff[v]];
+// The entries of list s that list l holds too, group by group; what pads l equals
+// no entry, and s is masked.
+__device__ __forceinline__ uint32_t tc_common(const TcRow& s, const TcRow& l, const uint16_t* __restrict__ codes,
+                                              const uint32_t* __restrict__ ids) {
+    uint32_t c = 0;
+    const uint4* c4 = reinterpret_cast<const uint4*>(codes);
+    for (uint32_t gs = 0; gs * TC_G < s.n16; gs++) {
+        const uint4 a = c4[(int64_t)s.base + gs];
+        const uint32_t x[4] = {a.x, a.y, a.z, a.w};
+        uint32_t m = 0;
+        for (uint32_t gl = 0; gl * TC_G < l.n16; gl++) {
+            const uint4 b = c4[(int64_t)l.base + gl];
+            const uint32_t y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int e = 0; e < TC_G; e++) {
+                const uint32_t q = x[e / 2] >> (16 * (e & 1)) & 0xFFFFu;
+                bool in = false;
+#pragma unroll
+                for (int f = 0; f < 4; f++) in = in || q == (y[f] & 0xFFFFu) || q == y[f] >> 16;
+                m |= (uint32_t)in << e;
+            }
+        }
+        c += (uint32_t)__popc(m & ((1u << min(s.n16 - gs * TC_G, (uint32_t)TC_G)) - 1u));
+    }
+    const uint4* i4 = reinterpret_cast<const uint4*>(ids);
+    for (uint32_t gs = 0; gs * 4 < s.n32; gs++) {
+        const uint4 a = i4[(int64_t)s.base * 2 + gs];
+        const uint32_t x[4] = {a.x, a.y, a.z, a.w};
+        uint32_t m = 0;
+        for (uint32_t gl = 0; gl * 4 < l.n32; gl++) {
+            const uint4 b = i4[(int64_t)l.base * 2 + gl];
+#pragma unroll
+            for (int e = 0; e < 4; e++) m |= (uint32_t)(x[e] == b.x || x[e] == b.y || x[e] == b.z || x[e] == b.w) << e;
+        }
+        c += (uint32_t)__popc(m & ((1u << min(s.n32 - gs * 4, 4u)) - 1u));
+    }
+    return c;
 }
 
-struct U8In {
-    const uint8_t* a;
-    __device__ __forceinline__ uint32_t operator()(int64_t i) const { return a[i]; }
-};
+// Edges between two lists of at most TC_SMALL entries: a lane per edge, TC_SMALL
+// lanes per source.  The chain source row, entry, hub, row, list is what bounds
+// it, so a lane starts four of them at once; a thread per source, one entry after
+// the other, took 330 us on a graph of a thousand vertices.
+constexpr int TC_SRC = 4;
+__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, const TcRow* __restrict__ row,
+                                                         const uint16_t* __restrict__ codes,
+                                                         const uint32_t* __restrict__ ids,
+                                                         const uint32_t* __restrict__ hub, TcCtl* __restrict__ ctl,
+                                                         unsigned long long* __restrict__ per_vertex) {
+    const int64_t u0 = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) / TC_SMALL * TC_SRC;
+    const uint32_t sub = threadIdx.x % TC_SMALL;
+    TcRow ru[TC_SRC], rv[TC_SRC];
+    uint32_t v[TC_SRC];
+#pragma unroll
+    for (int j = 0; j < TC_SRC; j++) ru[j] = u0 + j < nv ? row[u0 + j] : TcRow{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < TC_SRC; j++) {
+        const uint32_t n = ru[j].len();
+        v[j] = n >= 2 && n <= TC_SMALL && sub < n ? tc_entry(ru[j], sub, codes, ids, hub) : TC_PAD;
+    }
+#pragma unroll
+    for (int j = 0; j < TC_SRC; j++)
+        rv[j] = v[j] != TC_PAD && v[j] != (uint32_t)(u0 + j) ? row[v[j]] : TcRow{0u, 0u, 0u, 0u};
+    uint64_t acc = 0;
+#pragma unroll
+    for (int j = 0; j < TC_SRC; j++) {
+        if (rv[j].len() == 0 || rv[j].len() > TC_SMALL) continue;
+        const bool mine = ru[j].len() < rv[j].len();   // the source's list is the shorter one (ties: the destination's)
+        const uint32_t c = mine ? tc_common(ru[j], rv[j], codes, ids) : tc_common(rv[j], ru[j], codes, ids);
+        if (c && per_vertex) atomicAdd(per_vertex + (mine ? (uint32_t)(u0 + j) : v[j]), (unsigned long long)c);
+        acc += c;
+    }
+    acc = wave_reduce_sum(acc);
+    if (__lane_id() == 0 && acc) atomicAdd(&ctl->total[(blockIdx.x + threadIdx.x / WAVE) % TC_SUMS].v, (unsigned long long)acc);
+}
 
 }  // namespace
 
 // Resolves this file's code object (see preload_code_objects in graph.hip).
 void preload_tc_code() {
     hipFuncAttributes a;
-    if (hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&tc_light_kernel)) != hipSuccess) (void)hipGetLastError();
+    if (hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&tc_hist_kernel)) != hipSuccess) (void)hipGetLastError();
 }
 
-static int64_t al256(int64_t x) { return (x + 255) & ~int64_t(255); }
-
-// bytes of tc_core's buffers for ne stored edges
-static int64_t tc_core_bytes(int64_t ne) {
-    const int64_t ne1 = ne > 0 ? ne : 1;
-    return al256(512 + ne1 * 4) + al256(ne1 * 4) + al256(ne1 * 4);
-}
-
-// Triangle counting core over a device CSR (sorted adjacency); its buffers
-// start at `base` (tc_core_bytes(ne) bytes of the handle's TC scratch).
-static hn_status tc_core(hn_graph* g, int32_t nv, int64_t ne, const int64_t* off, const int32_t* adj,
-                         uint64_t* total_out, uint64_t* per_vertex, hipStream_t st, char* base) {
-    const int64_t ne1 = ne > 0 ? ne : 1;
-    int64_t o_tot = 0;
-    int64_t o_cnt = 256;
-    int64_t o_src = 512;
-    int64_t o_med = al256(o_src + ne1 * 4);
-    int64_t o_heavy = al256(o_med + ne1 * 4);
-    TcOut o;
-    o.total = reinterpret_cast<unsigned long long*>(base + o_tot);
-    o.cnt = reinterpret_cast<uint32_t*>(base + o_cnt);
-    o.src_of = reinterpret_cast<int32_t*>(base + o_src);
-    o.med_q = reinterpret_cast<uint32_t*>(base + o_med);
-    o.heavy_q = reinterpret_cast<uint32_t*>(base + o_heavy);
-    o.per_vertex = reinterpret_cast<unsigned long long*>(per_vertex);
-    HN_HIP(hipMemsetAsync(base, 0, 512, st));
+// Counts on the stored rows (orient: on their degree orientation).  Every buffer
+// is in the handle's grow-only scratch (s_tc).
+static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t* per_vertex, hipStream_t st) {
+    const int64_t nv = g->nv, ne = g->ne;
+    auto al = [](int64_t x) { return (x + 255) & ~int64_t(255); };
     if (per_vertex && nv > 0) HN_HIP(hipMemsetAsync(per_vertex, 0, sizeof(uint64_t) * (size_t)nv, st));
-    TcCsr c{off, adj};
-    const int64_t cap = (int64_t)num_cus() * 8;
-    if (ne > 0) {
-        int64_t grid = std::min<int64_t>(ceil_div(ne, TC_TILE), cap);
-        tc_light_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(nv, ne, c, o);
-        HN_CHECK_LAUNCH();
-        tc_group_kernel<MEDIUM_LANES><<<(unsigned)cap, BLOCK, 0, st>>>(c, o.med_q, o.cnt, o.src_of, o);
-        HN_CHECK_LAUNCH();
-        tc_window_kernel<<<(unsigned)cap, BLOCK, 0, st>>>(c, o.heavy_q, o.cnt + 1, o.src_of, o);
-        HN_CHECK_LAUNCH();
+    if (ne == 0 || nv == 0) {
+        HN_HIP(hipStreamSynchronize(st));
+        *total_out = 0;
+        return HN_OK;
     }
-    unsigned long long t = 0;
-    HN_TRY(read_back(g, o.total, 8, &t, st));
-    *total_out = t;
+    const int64_t groups = ne / TC_G + nv + 1;   // at most
+    const int64_t tiles = groups / TC_TILE + 2;
+    const int64_t tasks = nv + 2 * ne / TC_CAND + 1;
+    // what an owner's stored row says of its edges holds on symmetric storage only
+    const int sym = orient && graph_known_symmetric(g) ? 1 : 0;
+    int64_t o = 0;
+    auto take = [&](int64_t bytes) {
+        const int64_t at = o;
+        o = al(o + bytes);
+        return at;
+    };
+    const int64_t o_ctl = take(sizeof(TcCtl)), o_hist = take(TC_BINS * 4);
+    const int64_t o_gcnt = take(nv * 4), o_zero_end = o;   // cleared together
+    const int64_t o_weight = take(nv * 4), o_wc = take(nv * 8), o_hub = take((int64_t)(TC_HUBS + 1) * 4);
+    const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4);
+    const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
+    const int64_t o_goff = take((nv + 1) * 4), o_mem = take(ne * 4), o_task = take(tasks * 8);
+    const int64_t o_scan = take((int64_t)scan_temp_bytes(nv));
+    HN_TRY(g->s_tc.reserve((size_t)o));
+    char* base = g->s_tc.as<char>();
+    auto at = [&](int64_t off, auto* kind) { return reinterpret_cast<decltype(kind)>(base + off); };
+    TcCtl* ctl = at(o_ctl, (TcCtl*)nullptr);
+    uint32_t* hist = at(o_hist, (uint32_t*)nullptr);
+    uint32_t* gcnt = at(o_gcnt, (uint32_t*)nullptr);
+    uint32_t* weight = at(o_weight, (uint32_t*)nullptr);
+    uint2* wc = at(o_wc, (uint2*)nullptr);
+    uint32_t* hub = at(o_hub, (uint32_t*)nullptr);
+    TcRow* row = at(o_row, (TcRow*)nullptr);
+    uint32_t* P = at(o_P, (uint32_t*)nullptr);
+    uint32_t* tile_lo = at(o_tile, (uint32_t*)nullptr);
+    uint16_t* codes = at(o_codes, (uint16_t*)nullptr);
+    uint32_t* ids = at(o_ids, (uint32_t*)nullptr);
+    uint32_t* place = at(o_place, (uint32_t*)nullptr);
+    uint32_t* goff = at(o_goff, (uint32_t*)nullptr);
+    uint32_t* members = at(o_mem, (uint32_t*)nullptr);
+    uint2* task = at(o_task, (uint2*)nullptr);
+    void* tmp = base + o_scan;
+    unsigned long long* per = reinterpret_cast<unsigned long long*>(per_vertex);
+    const unsigned gv = (unsigned)ceil_div(nv, BLOCK);
+    const unsigned gt = (unsigned)std::min<int64_t>(tiles, (int64_t)num_cus() * 8);
+    const unsigned gw = (unsigned)std::min<int64_t>(gv, (int64_t)num_cus() * 2);
+
+    HN_HIP(hipMemsetAsync(base, 0, (size_t)o_zero_end, st));
+    // 1. hubs and codes
+    HN_TRY(exclusive_scan_fn<uint32_t>(StoredGroupsIn{g->rec}, StoredGroupsOut{row, P, tile_lo}, P + nv, nv, tmp, st));
+    if (nv <= (int64_t)TC_HUBS) {
+        tc_all_hubs_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, wc, hub);
+        HN_CHECK_LAUNCH();
+    } else {
+        if (orient) {
+            tc_weight_deg_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, weight);
+        } else {
+            HN_HIP(hipMemsetAsync(weight, 0, (size_t)nv * 4, st));
+            const int step = ne >= ((int64_t)1 << 22) ? 16 : 1;
+            tc_weight_freq_kernel<<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, step, weight);
+        }
+        HN_CHECK_LAUNCH();
+        tc_hist_kernel<<<gw, BLOCK, 0, st>>>(nv, weight, hist);
+        HN_CHECK_LAUNCH();
+        tc_cut_kernel<<<1, BLOCK, 0, st>>>(hist, ctl);
+        HN_CHECK_LAUNCH();
+        HN_TRY(exclusive_scan_fn<uint32_t>(HubIn{weight, ctl}, HubOut{weight, wc, hub}, &ctl->hubs, nv, tmp, st));
+    }
+    // 2. lists
+    if (orient)
+        tc_rows_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
+    else
+        tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
+    HN_CHECK_LAUNCH();
+    tc_pad_kernel<<<gv, BLOCK, 0, st>>>(nv, row, codes, ids);
+    HN_CHECK_LAUNCH();
+    // 3. edges owned by their destination
+    tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, place, nullptr, nullptr);
+    HN_CHECK_LAUNCH();
+    HN_TRY(exclusive_scan<uint32_t>(ArrayIn<uint32_t>{gcnt}, goff, nv, tmp, st));
+    tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, place, goff, members);
+    HN_CHECK_LAUNCH();
+    // 4. counts
+    HN_TRY(exclusive_scan_fn<uint32_t>(TaskIn{row, gcnt, g->rec, ctl, sym}, TaskOut{task}, &ctl->ntask, nv, tmp, st));
+    tc_owner_kernel<<<(unsigned)num_cus() * 8, BLOCK, 0, st>>>(sym, g->rec, g->arena, wc, task, row, codes, ids, hub,
+                                                               gcnt, goff, members, ctl, per);
+    HN_CHECK_LAUNCH();
+    tc_small_kernel<<<(unsigned)ceil_div(nv, TC_SRC * BLOCK / TC_SMALL), BLOCK, 0, st>>>(nv, row, codes, ids, hub, ctl, per);
+    HN_CHECK_LAUNCH();
+    TcSum sums[TC_SUMS];
+    HN_TRY(read_back(g, ctl->total, sizeof(sums), sums, st));
+    *total_out = 0;
+    for (const TcSum& x : sums) *total_out += x.v;
     return HN_OK;
 }
 
@@ -472,66 +862,16 @@ using namespace hn;
 
 extern "C" {
 
-// The TC entry points keep every buffer in the handle's grow-only scratch
-// (s_tc): the CSR they count on, then tc_core's buffers.
-
 hn_status hn_tc2_stored(hn_graph* g, uint64_t* total, uint64_t* per_vertex, void* stream) {
     HN_ARG(g && total, "null argument");
     HN_ARG(g->ne < (int64_t)0xFFFFFFFF, "edge count exceeds 32-bit queue ids");
-    hipStream_t st = as_stream(stream);
-    const int64_t nv = g->nv, ne = g->ne, ne1 = ne > 0 ? ne : 1;
-    const int64_t o_off = 0;
-    const int64_t o_adj = al256(o_off + (nv + 1) * 8);
-    const int64_t o_core = al256(o_adj + ne1 * 4);
-    HN_TRY(g->s_tc.reserve((size_t)(o_core + tc_core_bytes(ne))));
-    char* base = g->s_tc.as<char>();
-    int64_t* off = reinterpret_cast<int64_t*>(base + o_off);
-    int32_t* adj = reinterpret_cast<int32_t*>(base + o_adj);
-    HN_TRY(hn_graph_export_csr(g, off, adj, ne, stream));
-    return tc_core(g, g->nv, ne, off, adj, total, per_vertex, st, base + o_core);
+    return tc_run(g, false, total, per_vertex, as_stream(stream));
 }
 
 hn_status hn_tc_count(hn_graph* g, uint64_t* total, uint64_t* per_vertex, void* stream) {
     HN_ARG(g && total, "null argument");
     HN_ARG(g->ne < (int64_t)0xFFFFFFFF, "edge count exceeds the 32-bit scan");
-    hipStream_t st = as_stream(stream);
-    const int32_t nv = g->nv;
-    const int64_t ne = g->ne, ne1 = ne > 0 ? ne : 1;
-    // the oriented CSR holds at most half the entries of the symmetric one
-    // (a multigraph's repeated entries may all point up: size for ne)
-    const int64_t o_eoff = 0;
-    const int64_t o_offp = al256(o_eoff + ((int64_t)nv + 1) * 8);
-    const int64_t o_tmp = al256(o_offp + ((int64_t)nv + 1) * 8);
-    const int64_t o_adjp = al256(o_tmp + ne1 * 4);
-    const int64_t o_keep = al256(o_adjp + ne1 * 4);
-    const int64_t o_pos = al256(o_keep + ne1);
-    const int64_t o_scan = al256(o_pos + (ne1 + 1) * 4);
-    const int64_t o_core = al256(o_scan + (int64_t)scan_temp_bytes(ne1));
-    HN_TRY(g->s_tc.reserve((size_t)(o_core + tc_core_bytes(ne))));
-    char* base = g->s_tc.as<char>();
-    int64_t* eoff = reinterpret_cast<int64_t*>(base + o_eoff);
-    int64_t* offp = reinterpret_cast<int64_t*>(base + o_offp);
-    int32_t* adj_tmp = reinterpret_cast<int32_t*>(base + o_tmp);
-    int32_t* adjp = reinterpret_cast<int32_t*>(base + o_adjp);
-    uint8_t* keep = reinterpret_cast<uint8_t*>(base + o_keep);
-    uint32_t* pos = reinterpret_cast<uint32_t*>(base + o_pos);
-    void* tmp = base + o_scan;
-    HN_TRY(degree_prefix(g, eoff, st));
-    if (ne > 0) {
-        int64_t grid = std::min<int64_t>(ceil_div(ne, OR_TILE), (int64_t)num_cus() * 16);
-        orient_flags_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(nv, ne, eoff, g->rec, g->arena, adj_tmp, keep);
-        HN_CHECK_LAUNCH();
-    }
-    HN_TRY(exclusive_scan<uint32_t>(U8In{keep}, pos, ne, tmp, st));
-    if (ne > 0) {
-        orient_compact_kernel<<<(unsigned)ceil_div(ne, BLOCK), BLOCK, 0, st>>>(ne, keep, pos, adj_tmp, adjp);
-        HN_CHECK_LAUNCH();
-    }
-    orient_offsets_kernel<<<(unsigned)ceil_div((int64_t)nv + 1, BLOCK), BLOCK, 0, st>>>(nv, eoff, pos, offp);
-    HN_CHECK_LAUNCH();
-    uint32_t nep = 0;
-    HN_TRY(read_back(g, pos + ne, 4, &nep, st));
-    return tc_core(g, nv, (int64_t)nep, offp, adjp, total, per_vertex, st, base + o_core);
+    return tc_run(g, true, total, per_vertex, as_stream(stream));
 }
 
 }  // extern "C"
