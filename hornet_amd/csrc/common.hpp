@@ -56,6 +56,9 @@ inline hn_status dalloc(T** p, size_t count) {
     return dmalloc(reinterpret_cast<void**>(p), count * sizeof(T) + (count == 0 ? 16 : 0));
 }
 void dfree(void* p);
+// dfree for a block that no work queued on any stream uses any more: kept for reuse
+void dput(void* p);
+size_t didle();   // bytes of freed blocks kept for reuse: free memory that the driver does not count
 
 // grow-only device scratch buffer
 struct Scratch {
@@ -74,8 +77,8 @@ struct Scratch {
     }
     template <typename T>
     T* as() const { return reinterpret_cast<T*>(ptr); }
-    void release() {
-        dfree(ptr);
+    void release(void (*give)(void*) = dfree) {
+        give(ptr);
         ptr = nullptr;
         bytes = 0;
     }

@@ -11,8 +11,9 @@
 // is one load-balanced kernel.
 #include <algorithm>
 #include <cstring>
-#include <vector>
 #include <mutex>
+#include <unordered_map>
+#include <vector>
 
 #include "graph.hpp"
 #include "prims.hpp"
@@ -22,20 +23,186 @@ namespace hn {
 static thread_local std::string g_last_error;
 void set_error(const std::string& msg) { g_last_error = msg; }
 
+// ---- device memory
+// hipMalloc and hipFree of the buffers that live for one call cost more than the
+// call: a build of an R-MAT s21 graph, 5 ms of kernels with 3 GB of buffers, took
+// 8 ms when the driver had the memory at hand and 98 when it had not.  Freed
+// blocks up to POOL_BLOCK are therefore kept for the next request of their size
+// class (steps of an eighth, so that at most 12.5 % of a block lies idle), POOL_BYTES
+// of them at most, oldest out first.  They go back to the driver when they have not
+// been asked for during POOL_AGE frees, when an allocation here fails (it is then tried
+// again), and with the process.
+// Only dput keeps a block.  Its callers have waited for all work on it, as hipFree
+// does by itself, so that whichever stream or thread gets it next finds none.
+namespace {
+constexpr size_t POOL_BLOCK = size_t(2) << 30, POOL_BYTES = size_t(4) << 30;
+constexpr size_t POOL_COUNT = 256;
+constexpr uint64_t POOL_AGE = 512;
+
+struct BlockPool {
+    struct Block {
+        void* p;
+        size_t bytes;
+        int dev;
+        uint64_t stamp;   // `frees` when it came
+    };
+    std::mutex mu;
+    std::unordered_map<void*, Block> live;   // handed out, and may be kept once freed
+    std::vector<Block> idle;                 // oldest first
+    size_t idle_bytes = 0;
+    uint64_t frees = 0;
+
+    // the idle blocks beyond the limits (all: every one), taken out
+    std::vector<Block> surplus(bool all) {
+        size_t n = 0;
+        while (n < idle.size() && (all || idle_bytes > POOL_BYTES || idle.size() - n > POOL_COUNT ||
+                                   idle[n].stamp + POOL_AGE < frees)) {
+            idle_bytes -= idle[n].bytes;
+            n++;
+        }
+        std::vector<Block> out(idle.begin(), idle.begin() + (long)n);
+        idle.erase(idle.begin(), idle.begin() + (long)n);
+        return out;
+    }
+};
+// (never destroyed: handles may be freed while the process ends)
+BlockPool& block_pool() {
+    static BlockPool* const pool = new BlockPool;
+    return *pool;
+}
+size_t pool_class(size_t bytes) {
+    size_t step = 4096;
+    while (step * 16 <= bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+}  // namespace
+
+static void dtrim() {
+    BlockPool& pool = block_pool();
+    std::vector<BlockPool::Block> out;
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        out = pool.surplus(true);
+    }
+    for (const BlockPool::Block& b : out) (void)hipFree(b.p);
+}
+
+size_t didle() {
+    BlockPool& pool = block_pool();
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> lock(pool.mu);
+    size_t n = 0;
+    for (const BlockPool::Block& b : pool.idle) n += b.dev == dev ? b.bytes : 0;
+    return n;
+}
+
 hn_status dmalloc(void** p, size_t bytes) {
     *p = nullptr;
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    if (bytes == 0) bytes = 16;
+    int dev = 0;
+    const bool keep = bytes <= POOL_BLOCK && hipGetDevice(&dev) == hipSuccess;
+    BlockPool& pool = block_pool();
+    const size_t want = keep ? pool_class(bytes) : bytes;
+    if (keep) {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        for (size_t i = pool.idle.size(); i-- > 0;) {
+            const BlockPool::Block b = pool.idle[i];
+            if (b.bytes != want || b.dev != dev) continue;
+            pool.idle.erase(pool.idle.begin() + (long)i);
+            pool.idle_bytes -= b.bytes;
+            pool.live[b.p] = b;
+            *p = b.p;
+            return HN_OK;
+        }
+    }
+    hipError_t e = hipMalloc(p, want);
+    const bool kept = keep && e == hipSuccess;
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        dtrim();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;
         set_error(std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? HN_E_OOM : HN_E_HIP;
     }
+
+    if (kept) {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        pool.live[*p] = BlockPool::Block{*p, want, dev, 0};
+    }
     return HN_OK;
 }
+
 void dfree(void* p) {
-    if (p) (void)hipFree(p);
+    if (!p) return;
+    {
+        BlockPool& pool = block_pool();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        pool.live.erase(p);
+    }
+    (void)hipFree(p);
 }
+
+void dput(void* p) {
+    if (!p) return;
+    BlockPool& pool = block_pool();
+    std::vector<BlockPool::Block> out;
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        const auto it = pool.live.find(p);
+        if (it != pool.live.end()) {
+            BlockPool::Block b = it->second;
+            pool.live.erase(it);
+            b.stamp = ++pool.frees;
+            pool.idle.push_back(b);
+            pool.idle_bytes += b.bytes;
+            out = pool.surplus(false);
+        } else {
+            out.push_back(BlockPool::Block{p, 0, 0, 0});
+        }
+    }
+    for (const BlockPool::Block& x : out) (void)hipFree(x.p);
+}
+
+// The handles' page of pinned memory, kept alike (PINNED_PAGES at most).
+namespace {
+constexpr size_t PINNED_PAGES = 16;
+struct PagePool {
+    std::mutex mu;
+    std::vector<void*> idle;
+};
+PagePool& page_pool() {
+    static PagePool* const pool = new PagePool;
+    return *pool;
+}
+hipError_t page_take(void** p) {
+    PagePool& pool = page_pool();
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (!pool.idle.empty()) {
+            *p = pool.idle.back();
+            pool.idle.pop_back();
+            return hipSuccess;
+        }
+    }
+    return hipHostMalloc(p, 4096, 0);
+}
+void page_give(void* p) {
+    PagePool& pool = page_pool();
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (pool.idle.size() < PINNED_PAGES) {
+            pool.idle.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+}  // namespace
 
 int num_cus() {
     static int cus = 0;
@@ -477,24 +644,26 @@ hn_status read_back(hn_graph* g, const void* dptr, size_t bytes, void* host, hip
     return HN_OK;
 }
 
-static void destroy_graph(hn_graph* g) {
+// give: dput where the device is idle
+static void destroy_graph(hn_graph* g, void (*give)(void*) = dfree) {
     if (!g) return;
     if (g->ms && g->ms_release) g->ms_release(g->ms);
     g->ms = nullptr;
-    dfree(g->rec);
-    dfree(g->arena);
-    for (int f = 0; f < g->meta.n; f++) dfree(g->meta.p[f]);
-    dfree(g->alloc);
-    dfree(g->stacks);
-    dfree(g->stack_off);
-    g->s_bfs.release();
-    g->s_scan.release();
-    g->s_upd.release();
-    g->s_tc.release();
-    g->s_mstage.release();
-    g->s_stamp.release();
-    g->s_misc.release();
-    if (g->h_pinned) (void)hipHostFree(g->h_pinned);
+    give(g->rec);
+    give(g->arena);
+    for (int f = 0; f < g->meta.n; f++) give(g->meta.p[f]);
+    give(g->alloc);
+    give(g->stacks);
+    give(g->stack_off);
+    g->s_bfs.release(give);
+    g->s_scan.release(give);
+    g->s_upd.release(give);
+    g->s_tc.release(give);
+    g->s_mstage.release(give);
+    g->s_stamp.release(give);
+    g->s_misc.release(give);
+    if (g->h_pinned && give == dput) page_give(g->h_pinned);
+    else if (g->h_pinned) (void)hipHostFree(g->h_pinned);
     for (hipEvent_t& e : g->bfs_ev)
         if (e) (void)hipEventDestroy(e);
     delete g;
@@ -608,7 +777,7 @@ static hn_status new_graph(int32_t nv, hn_graph** out) {
     preload_code_objects();
     hn_graph* g = new hn_graph();
     g->nv = nv;
-    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&g->h_pinned), 4096, 0);
+    hipError_t e = page_take(reinterpret_cast<void**>(&g->h_pinned));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         g->h_pinned = nullptr;
@@ -683,11 +852,11 @@ static hn_status sort_rows_if_needed(int32_t nv, int64_t ne, const int64_t* d_of
     int32_t* res = nullptr;
     MetaSet om = meta_like(in_meta, nullptr);
     hn_status s = HN_OK;
-    auto cleanup = [&]() {
-        dfree(ka); dfree(kb); dfree(ia); dfree(ib); dfree(flag); dfree(tmp);
+    auto cleanup = [&](void (*give)(void*)) {
+        give(ka); give(kb); give(ia); give(ib); give(flag); give(tmp);
     };
     auto fail = [&](hn_status e) {
-        cleanup();
+        cleanup(dfree);
         dfree(res);
         for (int f = 0; f < om.n; f++) dfree(om.p[f]);
         return e;
@@ -700,7 +869,7 @@ static hn_status sort_rows_if_needed(int32_t nv, int64_t ne, const int64_t* d_of
     HN_HIP(hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, st));
     HN_HIP(hipStreamSynchronize(st));
     if (!h) {
-        cleanup();
+        cleanup(dput);
         return HN_OK;
     }
     if ((s = dalloc(&kb, (size_t)ne)) != HN_OK || (s = dmalloc(&tmp, sort_temp_bytes(ne))) != HN_OK ||
@@ -725,7 +894,7 @@ static hn_status sort_rows_if_needed(int32_t nv, int64_t ne, const int64_t* d_of
         set_error(std::string("row sort: ") + hipGetErrorString(e));
         return fail(HN_E_HIP);
     }
-    cleanup();
+    cleanup(dput);
     *out = res;
     *out_meta = om;
     return HN_OK;
@@ -763,8 +932,9 @@ hn_status graph_from_device_csr(int32_t nv, int64_t ne, const int64_t* d_off, co
                                                          d_meta);
     }
     hipError_t e = hipStreamSynchronize(st);
-    dfree(uoff);
-    dfree(tile_lo);
+    void (*const give)(void*) = e == hipSuccess ? dput : dfree;
+    give(uoff);
+    give(tile_lo);
     if (e != hipSuccess) {
         set_error(std::string("graph build: ") + hipGetErrorString(e));
         return fail(HN_E_HIP);
@@ -791,8 +961,8 @@ hn_status csr_from_device_coo(int32_t nv, int64_t m, const int32_t* src, const i
     int64_t* d_off = nullptr;
     int32_t* d_adj = nullptr;
     hn_status s = HN_OK;
-    auto cleanup = [&]() {
-        dfree(ka); dfree(kb); dfree(pos); dfree(bad); dfree(tmp);
+    auto cleanup = [&](void (*give)(void*) = dfree) {
+        give(ka); give(kb); give(pos); give(bad); give(tmp);
     };
     size_t tmpb = std::max(sort_temp_bytes(n), scan_temp_bytes(n));
     if ((s = dalloc(&ka, (size_t)n + 1)) != HN_OK || (s = dalloc(&kb, (size_t)n + 1)) != HN_OK ||
@@ -836,7 +1006,7 @@ hn_status csr_from_device_coo(int32_t nv, int64_t m, const int32_t* src, const i
     offsets_from_keys_kernel<<<(unsigned)ceil_div((int64_t)nv + 1, BLOCK), BLOCK, 0, st>>>(kb, u, sbits, nv, d_off);
     HN_CHECK_LAUNCH();
     hipError_t e = hipStreamSynchronize(st);
-    cleanup();
+    cleanup(e == hipSuccess ? dput : dfree);
     if (e != hipSuccess) {
         dfree(d_off); dfree(d_adj);
         set_error(std::string("coo->csr: ") + hipGetErrorString(e));
@@ -960,10 +1130,10 @@ hn_status hn_graph_create_csr_meta(int32_t nv, int64_t ne, const void* offsets, 
     int64_t* d_off = nullptr;
     int32_t* d_adj = nullptr;
     MetaSet up = meta_like(in_meta, nullptr);   // host meta-data copied to the device
-    auto release = [&]() {
-        dfree(d_off);
-        dfree(d_adj);
-        for (int f = 0; f < up.n; f++) dfree(up.p[f]);
+    auto release = [&](void (*give)(void*) = dfree) {
+        give(d_off);
+        give(d_adj);
+        for (int f = 0; f < up.n; f++) give(up.p[f]);
     };
     hn_status s;
     if ((s = dalloc(&d_off, (size_t)nv + 1)) != HN_OK) return s;
@@ -1001,10 +1171,11 @@ hn_status hn_graph_create_csr_meta(int32_t nv, int64_t ne, const void* offsets, 
     if (s == HN_OK)
         s = graph_from_device_csr(nv, ne, d_off, d_sorted ? d_sorted : adj_in, slack, st, out,
                                   d_sorted ? sorted_meta : dmeta);
-    release();
-    dfree(d_sorted);
+    void (*const give)(void*) = s == HN_OK ? dput : dfree;   // (a finished build has waited for its stream)
+    release(give);
+    give(d_sorted);
     if (d_sorted)
-        for (int f = 0; f < sorted_meta.n; f++) dfree(sorted_meta.p[f]);
+        for (int f = 0; f < sorted_meta.n; f++) give(sorted_meta.p[f]);
     return s;
 }
 
@@ -1030,15 +1201,15 @@ hn_status hn_graph_create_coo(int32_t nv, int64_t m, const int32_t* src, const i
     HN_TRY(csr_from_device_coo(nv, m, src, dst, flags, st, &d_off, &d_adj, &ne));
     hn_status s = graph_from_device_csr(nv, ne, d_off, d_adj, slack, st, out);
     if (s == HN_OK && (flags & HN_SYMMETRIZE)) (*out)->sym = 1;
-    dfree(d_off);
-    dfree(d_adj);
+    void (*const give)(void*) = s == HN_OK ? dput : dfree;
+    give(d_off);
+    give(d_adj);
     return s;
 }
 
 hn_status hn_graph_destroy(hn_graph* g) {
     if (g) {
-        (void)hipDeviceSynchronize();
-        destroy_graph(g);
+        destroy_graph(g, hipDeviceSynchronize() == hipSuccess ? dput : dfree);
     }
     return HN_OK;
 }
@@ -1151,9 +1322,10 @@ hn_status hn_graph_snapshot(hn_graph* g, double slack, void* stream, hn_graph** 
     if (s == HN_OK) s = flatten(g, nullptr, d_adj, d_off, st, tm);
     if (s == HN_OK)
         s = graph_from_device_csr(g->nv, g->ne, d_off, d_adj, slack < 1.0 ? 1.0 : slack, st, out, tm);
-    dfree(d_off);
-    dfree(d_adj);
-    for (int f = 0; f < tm.n; f++) dfree(tm.p[f]);
+    void (*const give)(void*) = s == HN_OK ? dput : dfree;
+    give(d_off);
+    give(d_adj);
+    for (int f = 0; f < tm.n; f++) give(tm.p[f]);
     if (s == HN_OK) {
         // the copy starts at version 0 with what is known of the source's symmetry
         const bool known = g->sym == 1 || (g->sym == -1 && g->sym_version == g->version);

@@ -581,7 +581,7 @@ hn_status hn_server_create(hn_graph* g, const hn_serve_config* cfg, hn_server** 
             (void)hipGetLastError();
             fr = (size_t)1 << 34;
         }
-        budget = (int64_t)(fr / 4);
+        budget = (int64_t)((fr + didle()) / 4);
     }
     int nslots = cfg->plain ? 1 : (int)std::min<int64_t>(cfg->slots, budget / s->slot_bytes);
     if (nslots < 1) {
