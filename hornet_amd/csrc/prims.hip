@@ -142,6 +142,102 @@ __global__ __launch_bounds__(BLOCK) void rs_scatter_kernel(const uint64_t* __res
     }
 }
 
+// Up to RS_SMALL keys are sorted by one workgroup in one launch: keys in registers,
+// LDS between the passes.  The batches of an edge stream are this short, and three
+// launches of 8 us (gaps included) per eight bits bounded them: 2,000 keys of 32 bits
+// 97 us, 11.5 so.  One CU ranks 8,192 keys of 49 bits in 23 us, about what the
+// launches' kernels alone take for as many; beyond that the whole device is faster.
+constexpr int RS_SMALL_BLOCK = 1024;
+constexpr int RS_SMALL_IPT = 8;
+constexpr int RS_SMALL = RS_SMALL_BLOCK * RS_SMALL_IPT;
+
+template <bool KV>
+__global__ __launch_bounds__(RS_SMALL_BLOCK) void rs_small_kernel(uint64_t* __restrict__ keys,
+                                                                  uint32_t* __restrict__ vals, int n, int key_bits) {
+    constexpr int WAVES = RS_SMALL_BLOCK / WAVE;
+    __shared__ uint64_t stage[RS_SMALL];
+    __shared__ uint32_t vstage[KV ? RS_SMALL : 1];
+    __shared__ uint32_t cnt[WAVES][RS_BUCKETS];   // a wave's digit counts, then the starts of its keys
+    __shared__ uint32_t wtot[RS_BUCKETS / WAVE];
+    const int w = threadIdx.x / WAVE;
+    const int l = __lane_id();
+    const int rows = (n + RS_SMALL_BLOCK - 1) / RS_SMALL_BLOCK;
+    const int base = w * rows * WAVE;
+    const uint64_t lt = lanemask_lt();
+    // past the end: the largest key, which a stable sort leaves there
+    uint64_t k[RS_SMALL_IPT];
+    uint32_t v[RS_SMALL_IPT], rank[RS_SMALL_IPT];
+#pragma unroll
+    for (int j = 0; j < RS_SMALL_IPT; j++) {
+        const int i = base + j * WAVE + l;
+        const bool in = j < rows && i < n;
+        k[j] = in ? keys[i] : ~0ull;
+        v[j] = KV && in ? vals[i] : 0u;
+    }
+    for (int shift = 0; shift < key_bits; shift += RS_BITS) {
+        for (int d = threadIdx.x; d < WAVES * RS_BUCKETS; d += RS_SMALL_BLOCK) (&cnt[0][0])[d] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < RS_SMALL_IPT; j++) {
+            if (j >= rows) break;
+            const uint32_t d = (uint32_t)(k[j] >> shift) & (RS_BUCKETS - 1);
+            uint64_t peers = ~0ull;
+#pragma unroll
+            for (int b = 0; b < RS_BITS; b++) {
+                const uint64_t bal = __ballot((d >> b) & 1u);
+                peers &= ((d >> b) & 1u) ? bal : ~bal;
+            }
+            const uint32_t before = (uint32_t)__popcll(peers & lt);
+            const uint32_t start = cnt[w][d];
+            rank[j] = start + before;
+            // the lowest peer lane publishes the new count after every peer has read it
+            if (before == 0) cnt[w][d] = start + (uint32_t)__popcll(peers);
+        }
+        __syncthreads();
+        uint32_t run = 0, inc = 0;
+        if (threadIdx.x < RS_BUCKETS) {
+#pragma unroll
+            for (int q = 0; q < WAVES; q++) run += cnt[q][threadIdx.x];
+            inc = wave_inclusive_scan(run);
+            if (l == WAVE - 1) wtot[w] = inc;
+        }
+        __syncthreads();
+        if (threadIdx.x < RS_BUCKETS) {
+            uint32_t at = inc - run;
+            for (int q = 0; q < w; q++) at += wtot[q];
+#pragma unroll
+            for (int q = 0; q < WAVES; q++) {
+                const uint32_t c = cnt[q][threadIdx.x];
+                cnt[q][threadIdx.x] = at;
+                at += c;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < RS_SMALL_IPT; j++) {
+            if (j >= rows) break;
+            const uint32_t p = cnt[w][(uint32_t)(k[j] >> shift) & (RS_BUCKETS - 1)] + rank[j];
+            stage[p] = k[j];
+            if constexpr (KV) vstage[p] = v[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < RS_SMALL_IPT; j++) {
+            if (j >= rows) break;
+            k[j] = stage[base + j * WAVE + l];
+            if constexpr (KV) v[j] = vstage[base + j * WAVE + l];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < RS_SMALL_IPT; j++) {
+        const int i = base + j * WAVE + l;
+        if (j < rows && i < n) {
+            keys[i] = k[j];
+            if constexpr (KV) vals[i] = v[j];
+        }
+    }
+}
+
 }  // namespace
 
 // Resolves this file's code object (see preload_code_objects in graph.hip).
@@ -159,6 +255,12 @@ size_t sort_temp_bytes(int64_t n) {
 static hn_status radix_sort_impl(uint64_t** keys, uint64_t** alt, uint32_t** vals, uint32_t** valt, int64_t n,
                                  int key_bits, void* tmp, hipStream_t st) {
     if (n <= 1) return HN_OK;
+    if (n <= RS_SMALL) {
+        if (vals) rs_small_kernel<true><<<1, RS_SMALL_BLOCK, 0, st>>>(*keys, *vals, (int)n, key_bits);
+        else rs_small_kernel<false><<<1, RS_SMALL_BLOCK, 0, st>>>(*keys, nullptr, (int)n, key_bits);
+        HN_CHECK_LAUNCH();
+        return HN_OK;
+    }
     int64_t tiles = ceil_div(n, RS_TILE);
     int64_t hn_ = tiles * RS_BUCKETS;
     HN_ARG(hn_ < (int64_t)0xFFFFFFFF && n < (int64_t)0xFFFFFFFF, "radix_sort_u64: too many keys");

@@ -234,6 +234,54 @@ __global__ __launch_bounds__(BLOCK) void scan_down_fn_kernel(InFn in, Cnt cnt, c
     }
 }
 
+// Up to SCAN_ONE values (batches of an edge stream, levels of small graphs) are
+// scanned by one workgroup in one launch: these scans are a launch and one chain
+// of loads each, and the second launch was as much again (2,000 values: 4 + 5.5 us
+// and the gap between them, 3 so).
+constexpr int SCAN_ONE_BLOCK = 1024;
+constexpr int SCAN_ONE_IPT = 8;
+constexpr int64_t SCAN_ONE = (int64_t)SCAN_ONE_BLOCK * SCAN_ONE_IPT;
+template <typename Out, typename InFn, typename OutFn, typename Cnt>
+__global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_one_kernel(InFn in, Cnt cnt, OutFn out, Out* __restrict__ total) {
+    constexpr int WAVES = SCAN_ONE_BLOCK / WAVE;
+    __shared__ Out wtot[WAVES];
+    const int64_t n = cnt.get();   // <= SCAN_ONE
+    const int w = threadIdx.x / WAVE;
+    const int l = __lane_id();
+    // a wave's rows of 64 are consecutive; as few rows as hold n
+    const int rows = (int)((n + SCAN_ONE_BLOCK - 1) / SCAN_ONE_BLOCK);
+    const int64_t base = (int64_t)w * rows * WAVE;
+    Out pre[SCAN_ONE_IPT], val[SCAN_ONE_IPT];
+    Out carry = 0;
+#pragma unroll
+    for (int j = 0; j < SCAN_ONE_IPT; j++) {
+        const int64_t i = base + (int64_t)j * WAVE + l;
+        val[j] = j < rows && i < n ? (Out)in(i) : (Out)0;
+    }
+#pragma unroll
+    for (int j = 0; j < SCAN_ONE_IPT; j++) {
+        if (j >= rows) break;
+        const Out inc = wave_inclusive_scan(val[j]);
+        pre[j] = carry + inc - val[j];
+        carry += __shfl(inc, WAVE - 1, WAVE);
+    }
+    if (l == 0) wtot[w] = carry;
+    __syncthreads();
+    Out off = 0, tot = 0;
+    for (int k = 0; k < WAVES; k++) {
+        const Out t = wtot[k];
+        off += k < w ? t : (Out)0;
+        tot += t;
+    }
+#pragma unroll
+    for (int j = 0; j < SCAN_ONE_IPT; j++) {
+        if (j >= rows) break;
+        const int64_t i = base + (int64_t)j * WAVE + l;
+        if (i < n) out(i, (Out)(off + pre[j]), val[j]);
+    }
+    if (threadIdx.x == 0) *total = tot;
+}
+
 template <typename Out>
 __global__ void scan_zero_kernel(Out* out) { *out = 0; }
 
@@ -257,6 +305,10 @@ hipError_t exclusive_scan_dev(InFn in, OutFn out, Out* total, int64_t n, void* t
         scan_zero_kernel<Out><<<1, 1, 0, st>>>(total);
         return hipGetLastError();
     }
+    if (n <= SCAN_ONE) {
+        scan_one_kernel<Out, InFn, OutFn, HostCount><<<1, SCAN_ONE_BLOCK, 0, st>>>(in, HostCount{n}, out, total);
+        return hipGetLastError();
+    }
     int64_t tiles = ceil_div(n, SCAN_TILE);
     Out* partial = reinterpret_cast<Out*>(tmp);
     scan_reduce_kernel<Out, InFn, HostCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, HostCount{n}, partial);
@@ -276,6 +328,10 @@ hipError_t exclusive_scan_dev(InFn in, OutFn out, Out* total, int64_t n, void* t
 template <typename Out, typename InFn, typename OutFn>
 hipError_t exclusive_scan_dev_count(InFn in, OutFn out, Out* total, const uint32_t* n_dev, int64_t max_n, void* tmp,
                                     hipStream_t st) {
+    if (max_n <= SCAN_ONE) {
+        scan_one_kernel<Out, InFn, OutFn, DevCount><<<1, SCAN_ONE_BLOCK, 0, st>>>(in, DevCount{n_dev}, out, total);
+        return hipGetLastError();
+    }
     const int64_t tiles = ceil_div(max_n > 0 ? max_n : 1, SCAN_TILE);
     Out* partial = reinterpret_cast<Out*>(tmp);
     scan_reduce_kernel<Out, InFn, DevCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, DevCount{n_dev}, partial);
