@@ -7,10 +7,9 @@
 // whose frontier touches it.
 //
 // One level step, captured once into a hipGraph and replayed until the
-// frontiers empty (the host reads a 4-byte "done" flag every few levels):
-//   decide   one workgroup reduces the previous collect's per-block counters
-//            and picks the direction: push while frontier degree * alpha <
-//            degree of the vertices still missing a source, else pull;
+// frontiers empty (the host reads the state every few levels):
+//   head     pull only: the first eight entries of every open vertex, a lane per
+//            vertex; most need no more;
 //   list     a scan of per-word popcounts of the frontier (push) or
 //            light-open (pull) bitset and an emit kernel turn the bitset
 //            into a compact work list carrying (vertex, degree, adjacency
@@ -30,14 +29,20 @@
 //                    vertex's bits with LDS atomics and stores them, with a
 //                    global atomicOr only for the two vertices it shares with
 //                    neighbouring tiles;
-//   heavy    pull only: open vertices of degree > T take one wave each and
-//            stop as soon as every missing bit is found (T is tuned);
+//   heavy    pull only, if a threshold T is set: open vertices of degree > T take
+//            one wave each and stop as soon as every missing bit is found;
+//   side     in a multi-version window only: pairs that storage does not hold;
 //   collect  one lane per vertex: new bits -> visited, frontier (masked by
-//            the per-source depth limits) and per-source distances (source
-//            major, int32, INT32_MAX unreached; written bit by bit so lanes
-//            store consecutive words), the three bitsets of the next level
-//            (frontier, light-open, heavy-open) from ballots, and per-block
-//            counters.  No atomics.
+//            the per-source depth limits) and the level's code in four bit
+//            planes (or, from level 15 on and for few sources, distances
+//            written bit by bit so lanes store consecutive words), the three
+//            bitsets of the next level (frontier, light-open, heavy-open) from
+//            ballots, and per-block counters.  No atomics;
+//   decide   one workgroup reduces the per-block counters: done, or the next
+//            level's direction: push while frontier degree * alpha < degree of
+//            the vertices still missing a source, else pull.
+// At the end the planes become distances (source major, int32, INT32_MAX
+// unreached), each written once.
 // Sources may carry a depth limit (the serving loop's 2-hop queries use 2).
 #include <algorithm>
 #include <cstring>
@@ -59,6 +64,22 @@ constexpr int MS_IPT_DEFAULT = 4;
 constexpr int MS_IPT_MIN = 2;                    // buffers are sized for the most tiles
 constexpr int MS_IPTS[] = {2, 4, 6};
 constexpr int MS_COLLECT_PER_CU = 8;             // collect workgroups per CU
+// Entries of an open vertex's row that a pull looks at first, a lane per vertex.
+// Rows ascend, and the hubs of the usual graphs have small ids: on R-MAT s22 most
+// vertices have every bit that is still to be found after eight of their entries.
+constexpr int MS_HEAD = 8;
+constexpr int MS_PLANES = 4;                     // bit planes of the level codes
+constexpr int MS_DIRECT = (1 << MS_PLANES) - 1;  // from this level on distances are written as they are found
+// Sources from which on the planes pay: they cost 72 bytes per vertex reached, level
+// by level, and 40 per vertex at the end, the other way 4 bytes per distance twice, in
+// runs that shrink with the level (R-MAT s22, planes and not: 8 sources 1351 and 1302 us,
+// 16 sources 2010 and 2100, 64 sources 2846 and 3802).
+constexpr int MS_PLANE_SOURCES = 16;
+// A pull over a frontier of fewer than one vertex in MS_SPARSE looks at the frontier's
+// bitset before it fetches a mask: the bitset stays in the L2, the masks (8 bytes a
+// vertex) do not, and most of them are empty (R-MAT s22, 64 sources, second level: 749
+// us without, 416 with; the third, whose frontier is most of the graph, would pay for both).
+constexpr unsigned MS_SPARSE = 8;
 constexpr int32_t MS_NO_HEAVY = 1 << 30;         // T: every open vertex goes through the edge-granular pull
 static_assert(UNIT_SLOTS % MS_G == 0, "groups must not straddle a block start");
 
@@ -79,6 +100,10 @@ struct MsState {
     uint64_t live;                  // bits with a non-empty frontier (OR over the frontier)
     unsigned long long push_levels;
     unsigned long long pull_levels;
+    int32_t sparse;                 // a small part of the vertices has a frontier (pulls look at its bitset first)
+    int32_t pad2;
+    int32_t* dist;                  // distances, or null: digests
+    uint64_t* planes;               // level codes, MS_PLANES words a vertex, or null: distances are written at once
 };
 
 struct MsParams {
@@ -88,6 +113,10 @@ struct MsParams {
     int32_t push_only;  // adjacency not symmetric: pulling over out-edges would be wrong
     int32_t digest;     // no distance matrix: per-source digests only
     int32_t depth_limit[64];
+};
+
+struct MsSources {
+    int32_t v[64];
 };
 
 __device__ __forceinline__ uint64_t wave_or64(uint64_t v) {
@@ -142,22 +171,27 @@ __global__ void ms_fill_dist_kernel(int64_t total, int32_t* __restrict__ dist) {
 }
 
 // one wave: lane b seeds source b; lane L builds the depth mask of level L
-__global__ __launch_bounds__(WAVE) void ms_seed_kernel(int32_t k, const int32_t* __restrict__ src, int64_t nv,
+__global__ __launch_bounds__(WAVE) void ms_seed_kernel(int32_t k, MsSources src, int64_t nv,
                                                        uint64_t* __restrict__ visited, uint64_t* __restrict__ frontier,
                                                        uint32_t* __restrict__ fbits, int32_t* __restrict__ dist,
+                                                       uint64_t* __restrict__ planes,
                                                        const hn_vrec* __restrict__ rec, MsState* S, MsParams P) {
     const int b = threadIdx.x;
     unsigned long long deg = 0, first = 0;
     if (b < k) {
-        const int32_t s = src[b];
+        const int32_t s = src.v[b];
         atomicOr(reinterpret_cast<unsigned long long*>(visited + s), 1ull << b);
         atomicOr(reinterpret_cast<unsigned long long*>(frontier + s), 1ull << b);
         atomicOr(fbits + (s >> 5), 1u << (s & 31));
-        if (dist) dist[(int64_t)b * nv + s] = 0;
+        if (planes)
+            for (int p = 0; p < MS_PLANES; p++)
+                atomicAnd(reinterpret_cast<unsigned long long*>(planes + (int64_t)s * MS_PLANES + p), ~(1ull << b));
+        else if (dist)
+            dist[(int64_t)b * nv + s] = 0;
         deg = (unsigned long long)rec[s].deg;
         first = 1;
         for (int c = 0; c < b; c++)
-            if (src[c] == s) first = 0;
+            if (src.v[c] == s) first = 0;
     }
     uint64_t m = 0;
     for (int c = 0; c < k; c++)
@@ -178,6 +212,8 @@ __global__ __launch_bounds__(WAVE) void ms_seed_kernel(int32_t k, const int32_t*
         S->tot = 0;
         S->edges = edges;
         S->push_levels = S->pull_levels = 0;
+        S->dist = dist;
+        S->planes = planes;
         S->active = act;
         S->active_deg = adeg;
         S->open_deg = ~0ull >> 1;   // the first expansion is always a push
@@ -185,7 +221,7 @@ __global__ __launch_bounds__(WAVE) void ms_seed_kernel(int32_t k, const int32_t*
 }
 
 // one workgroup: counters of the previous collect -> direction of this level
-__global__ __launch_bounds__(BLOCK) void ms_decide_kernel(MsState* S, MsParams P,
+__global__ __launch_bounds__(BLOCK) void ms_decide_kernel(MsState* S, MsParams P, int64_t nv,
                                                           const unsigned long long* __restrict__ part,
                                                           int32_t nparts) {
     // every thread reads the state before thread 0 changes it
@@ -231,6 +267,7 @@ __global__ __launch_bounds__(BLOCK) void ms_decide_kernel(MsState* S, MsParams P
         P.push_only || (unsigned long long)S->active_deg * (unsigned long long)P.alpha < S->open_deg;
     S->mode = push ? 0 : 1;
     if (push) S->push_levels++; else S->pull_levels++;
+    S->sparse = S->active * MS_SPARSE < (unsigned long long)nv ? 1 : 0;
 }
 
 // popcount of the word of this level's list bitset
@@ -244,6 +281,65 @@ struct ListWordIn {
     }
 };
 
+// pull: the first MS_HEAD entries of every light-open vertex, a lane per vertex.  It
+// stays on the list if it has more entries and misses a bit still, so that the lists
+// and tiles of the edge-granular pull hold only those (R-MAT s22, 64 sources: pulls, lists
+// and scans of a batch 2,720 us without, 2,420 with).  Bound by the rows' and masks'
+// scattered sectors.  Vertices with changed pairs in a window stay as they are.
+__global__ __launch_bounds__(BLOCK) void ms_head_kernel(int64_t nv, const MsState* S, uint32_t* __restrict__ obits,
+                                                        const hn_vrec* __restrict__ rec,
+                                                        const int32_t* __restrict__ arena,
+                                                        const uint32_t* __restrict__ fbits,
+                                                        const uint64_t* __restrict__ frontier,
+                                                        const uint64_t* __restrict__ visited,
+                                                        const uint8_t* __restrict__ dirty,
+                                                        const uint32_t* __restrict__ nchg, uint64_t* __restrict__ next) {
+    if (S->done || S->mode != 1) return;
+    typedef int32_t Vec __attribute__((ext_vector_type(MS_G)));
+    static_assert(MS_HEAD % MS_G == 0 && MS_HEAD <= UNIT_SLOTS, "whole groups of a row's first unit");
+    const uint64_t live = S->live;
+    const uint32_t nc = *nchg;
+    const bool sparse = S->sparse;
+    const int lane = __lane_id();
+    const int64_t pairs = (nv + 63) / 64;
+    uint64_t* open = reinterpret_cast<uint64_t*>(obits);
+    for (int64_t q = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) / WAVE; q < pairs; q += (int64_t)gridDim.x * NWAVES) {
+        const uint64_t word = open[q];
+        if (!word) continue;
+        const int64_t u = q * 64 + lane;
+        bool rest = (word >> lane) & 1ull;
+        if (rest && !(nc && dirty[u])) {
+            const hn_vrec r = rec[u];
+            const uint64_t miss = live & ~visited[u];
+            Vec nb[MS_HEAD / MS_G];
+#pragma unroll
+            for (int j = 0; j < MS_HEAD / MS_G; j++)
+                nb[j] = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(arena + r.off + j * MS_G));
+            uint64_t a = 0;
+            if (sparse) {
+                uint32_t f[MS_HEAD];
+#pragma unroll
+                for (int j = 0; j < MS_HEAD; j++) f[j] = fbits[j < r.deg ? nb[j / MS_G][j % MS_G] >> 5 : 0];
+#pragma unroll
+                for (int j = 0; j < MS_HEAD; j++)
+                    if (j < r.deg && (f[j] >> (nb[j / MS_G][j % MS_G] & 31) & 1u)) a |= frontier[nb[j / MS_G][j % MS_G]];
+            } else {
+#pragma unroll
+                for (int j = 0; j < MS_HEAD; j++) {
+                    const bool in = j < r.deg;
+                    const uint64_t x = frontier[in ? nb[j / MS_G][j % MS_G] : 0];
+                    a |= in ? x : 0ull;
+                }
+            }
+            a &= miss;
+            if (a) next[u] = a;
+            rest = a != miss && r.deg > MS_HEAD;
+        }
+        const uint64_t left = (uint64_t)__ballot(rest);
+        if (lane == 0 && left != word) open[q] = left;
+    }
+}
+
 // bitset -> work list (vertex, degree, offset, mask); lane per bitset word,
 // writes transposed so that consecutive lanes write consecutive entries
 __global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t words, const MsState* S,
@@ -254,10 +350,13 @@ __global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t words, const MsS
                                                         const uint64_t* __restrict__ visited,
                                                         const uint64_t* __restrict__ frontier,
                                                         const uint8_t* __restrict__ dirty,
+                                                        const uint32_t* __restrict__ nchg,
+                                                        const uint64_t* __restrict__ next,
                                                         int32_t* __restrict__ list, int32_t* __restrict__ qdeg,
                                                         int64_t* __restrict__ qoff, uint64_t* __restrict__ qmask) {
     if (S->done) return;
     const bool push = S->mode == 0;
+    const uint32_t nc = *nchg;
     const uint64_t live = S->live;
     const int64_t wi = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     const uint32_t found = wi < words ? (push ? fbits[wi] : obits[wi]) : 0u;
@@ -276,10 +375,12 @@ __global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t words, const MsS
             const int32_t v = (int32_t)((wbase + owner) * 32 + bit);
             const uint32_t pos = bo + (uint32_t)__popc(fw & below);
             const hn_vrec rv = rec[v];
-            const uint64_t m = push ? frontier[v] : (live & ~visited[v]);
+            // pull: what the first entries (ms_head_kernel) have left
+            const uint64_t m = push ? frontier[v] : (live & ~visited[v] & ~next[v]);
+            const int32_t skip = push || (nc && dirty[v]) ? 0 : MS_HEAD;
             list[pos] = v;
-            qdeg[pos] = m ? rv.deg : 0;
-            qoff[pos] = rv.off;
+            qdeg[pos] = m ? rv.deg - skip : 0;
+            qoff[pos] = rv.off + skip;
             qmask[pos] = m;
         }
     }
@@ -339,23 +440,23 @@ __device__ __forceinline__ uint64_t changed_range(const uint64_t* __restrict__ c
 
 // Edge-granular expansion of this level's work list (see the file comment).
 template <bool PULL, int IPT>
-__global__ __launch_bounds__(BLOCK) void ms_expand_kernel(const MsState* S, const uint32_t* __restrict__ P,
-                                                          const uint32_t* __restrict__ tile_lo,
-                                                          const int32_t* __restrict__ qdeg,
-                                                          const int64_t* __restrict__ qoff,
-                                                          const uint64_t* __restrict__ qmask,
-                                                          const int32_t* __restrict__ list,
-                                                          const int32_t* __restrict__ arena,
-                                                          const uint64_t* __restrict__ probe,
-                                                          unsigned long long* __restrict__ next,
-                                                          const uint8_t* __restrict__ dirty,
-                                                          const uint64_t* __restrict__ ckey,
-                                                          const uint64_t* __restrict__ cS,
-                                                          const uint32_t* __restrict__ nchg, int sbits) {
-    if (S->done || S->mode != (PULL ? 1 : 0)) return;
+__device__ __forceinline__ void ms_expand(MsShared<IPT>& sh, const MsState* S, const uint32_t* __restrict__ P,
+                                          const uint32_t* __restrict__ tile_lo,
+                                          const int32_t* __restrict__ qdeg,
+                                          const int64_t* __restrict__ qoff,
+                                          const uint64_t* __restrict__ qmask,
+                                          const int32_t* __restrict__ list,
+                                          const int32_t* __restrict__ arena,
+                                          const uint32_t* __restrict__ fbits,
+                                          const uint64_t* __restrict__ probe,
+                                          unsigned long long* __restrict__ next,
+                                          const uint8_t* __restrict__ dirty,
+                                          const uint64_t* __restrict__ ckey,
+                                          const uint64_t* __restrict__ cS,
+                                          const uint32_t* __restrict__ nchg, int sbits) {
     typedef int32_t Vec __attribute__((ext_vector_type(MS_G)));
-    __shared__ MsShared<IPT> sh;
     constexpr int TILE = BLOCK * IPT;
+    const bool sparse = PULL && S->sparse;
     const uint32_t nc = *nchg;
     const int64_t F = S->wn;
     const int64_t W = (uint32_t)S->tot;
@@ -423,10 +524,25 @@ __global__ __launch_bounds__(BLOCK) void ms_expand_kernel(const MsState* S, cons
             v[j] = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(arena + (nval[j] > 0 ? addr[j] : 0)));
         // phase 3: neighbour masks, all in flight (masked slots read probe[0])
         uint64_t pr[IPT][MS_G];
+        if (PULL && sparse) {
+            uint32_t f[IPT][MS_G];
 #pragma unroll
-        for (int j = 0; j < IPT; j++)
+            for (int j = 0; j < IPT; j++)
 #pragma unroll
-            for (int e = 0; e < MS_G; e++) pr[j][e] = probe[e < nval[j] ? v[j][e] : 0];
+                for (int e = 0; e < MS_G; e++) f[j][e] = fbits[e < nval[j] ? v[j][e] >> 5 : 0];
+#pragma unroll
+            for (int j = 0; j < IPT; j++)
+#pragma unroll
+                for (int e = 0; e < MS_G; e++) {
+                    pr[j][e] = 0;
+                    if (e < nval[j] && (f[j][e] >> (v[j][e] & 31) & 1u)) pr[j][e] = probe[v[j][e]];
+                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < IPT; j++)
+#pragma unroll
+                for (int e = 0; e < MS_G; e++) pr[j][e] = probe[e < nval[j] ? v[j][e] : 0];
+        }
         // window: a changed pair carries only the sources whose version holds
         // it (push: the others count as visited; pull: their bits are dropped)
 #pragma unroll
@@ -477,12 +593,37 @@ __global__ __launch_bounds__(BLOCK) void ms_expand_kernel(const MsState* S, cons
                     // the first and last vertex may share their groups with
                     // neighbouring tiles; the others belong to this tile only
                     if (i == 0 || i == (int)span - 1) atomicOr(next + u, a);
-                    else next[u] = a;
+                    else next[u] |= a;   // (its first entries' bits are there)
                 }
             }
         }
         __syncthreads();
     }
+}
+
+// one launch for both directions: which one is known on the device only
+template <int IPT>
+__global__ __launch_bounds__(BLOCK) void ms_expand_kernel(const MsState* S, const uint32_t* __restrict__ P,
+                                                          const uint32_t* __restrict__ tile_lo,
+                                                          const int32_t* __restrict__ qdeg,
+                                                          const int64_t* __restrict__ qoff,
+                                                          const uint64_t* __restrict__ qmask,
+                                                          const int32_t* __restrict__ list,
+                                                          const int32_t* __restrict__ arena,
+                                                          const uint32_t* __restrict__ fbits,
+                                                          const uint64_t* __restrict__ visited,
+                                                          const uint64_t* __restrict__ frontier,
+                                                          unsigned long long* __restrict__ next,
+                                                          const uint8_t* __restrict__ dirty,
+                                                          const uint64_t* __restrict__ ckey,
+                                                          const uint64_t* __restrict__ cS,
+                                                          const uint32_t* __restrict__ nchg, int sbits) {
+    __shared__ MsShared<IPT> sh;
+    if (S->done) return;
+    if (S->mode == 1)
+        ms_expand<true, IPT>(sh, S, P, tile_lo, qdeg, qoff, qmask, list, arena, fbits, frontier, next, dirty, ckey, cS, nchg, sbits);
+    else
+        ms_expand<false, IPT>(sh, S, P, tile_lo, qdeg, qoff, qmask, list, arena, fbits, visited, next, dirty, ckey, cS, nchg, sbits);
 }
 
 // pull, heavy open vertices (degree > T): one wave each, 256 slots per step,
@@ -536,7 +677,7 @@ __global__ __launch_bounds__(BLOCK) void ms_pull_heavy_kernel(int64_t words, con
 __global__ __launch_bounds__(BLOCK) void ms_collect_kernel(int64_t nv, const int32_t* __restrict__ degs,
                                                            uint64_t* __restrict__ visited,
                                                            uint64_t* __restrict__ frontier,
-                                                           uint64_t* __restrict__ next, int32_t* __restrict__ dist,
+                                                           uint64_t* __restrict__ next,
                                                            const MsState* S, int32_t T, const uint8_t* __restrict__ dirty,
                                                            uint32_t* __restrict__ fbits,
                                                            uint32_t* __restrict__ obits, uint32_t* __restrict__ hbits,
@@ -548,6 +689,10 @@ __global__ __launch_bounds__(BLOCK) void ms_collect_kernel(int64_t nv, const int
     __syncthreads();
     const int32_t level = S->level;
     const uint64_t dmn = S->depth_mask[level < 63 ? level : 63];
+    int32_t* const dist = S->dist;
+    uint64_t* const planes = S->planes;
+    const bool direct = !planes || level >= MS_DIRECT;
+    const int code = min(level, MS_DIRECT);
     // bits still expandable after this level: a superset of the next live set
     const uint64_t live = S->live & dmn;
     const int lane = __lane_id();
@@ -579,13 +724,24 @@ __global__ __launch_bounds__(BLOCK) void ms_collect_kernel(int64_t nv, const int
         odeg += miss ? (unsigned long long)deg : 0ull;
         edges += (unsigned long long)deg * (unsigned long long)__popcll(nb);
         fany |= f;
-        // distances, one source bit at a time so that lanes store consecutive
-        // words; in digest mode one count per source bit and wave
+        // distances: the level's code in the planes; else one source bit at a time
+        // so that lanes store consecutive words; in digest mode one count per
+        // source bit and wave
+        if (planes && nb) {
+            ulonglong2* pl = reinterpret_cast<ulonglong2*>(planes + u * MS_PLANES);
+            ulonglong2 x = pl[0], y = pl[1];
+            x.x = (x.x & ~nb) | (code & 1 ? nb : 0ull);
+            x.y = (x.y & ~nb) | (code & 2 ? nb : 0ull);
+            y.x = (y.x & ~nb) | (code & 4 ? nb : 0ull);
+            y.y = (y.y & ~nb) | (code & 8 ? nb : 0ull);
+            pl[0] = x;
+            pl[1] = y;
+        }
         if (digest) {
             // lane b counts the wave's vertices newly reached from source b
             const unsigned int c = (unsigned int)__popcll((unsigned long long)wave_transpose64(nb));
             if (c) atomicAdd(&dcnt[lane], c);
-        } else {
+        } else if (direct) {
             uint64_t M = wave_or64(nb);
             while (M) {
                 const int b = __ffsll((unsigned long long)M) - 1;
@@ -626,6 +782,58 @@ __global__ __launch_bounds__(BLOCK) void ms_collect_kernel(int64_t nv, const int
             p[0] += cnt;
             p[1] += (unsigned long long)cnt * (unsigned long long)level;
             p[2] = (unsigned long long)level;   // levels only grow
+        }
+    }
+}
+
+// Distances from the level codes: every one written once, in whole lines, where the
+// collects wrote them level by level over a fill of INT32_MAX (R-MAT s22, 64
+// sources: fill and collects 1,490 us; collects and this kernel 700, of which 262
+// here, 4.1 TB/s).  A lane has four vertices.  Bound by the stores.  Codes of
+// MS_DIRECT stand for distances that are there already.
+constexpr int MS_DIST_IPT = 4;
+typedef int32_t DistQuad __attribute__((ext_vector_type(4), aligned(4)));
+__global__ __launch_bounds__(BLOCK) void ms_dist_kernel(int64_t nv, int32_t k, const MsState* S,
+                                                        const uint64_t* __restrict__ visited) {
+    const uint64_t* __restrict__ planes = S->planes;
+    int32_t* __restrict__ dist = S->dist;
+    if (!S->done) return;   // (queued before the host knows)
+    const bool some_direct = S->level >= MS_DIRECT;
+    for (int64_t v = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) * MS_DIST_IPT; v < nv;
+         v += (int64_t)gridDim.x * BLOCK * MS_DIST_IPT) {
+        const int n = (int)min((int64_t)MS_DIST_IPT, nv - v);
+        uint64_t vis[MS_DIST_IPT], pl[MS_DIST_IPT][MS_PLANES];
+#pragma unroll
+        for (int i = 0; i < MS_DIST_IPT; i++) {
+            const int64_t u = i < n ? v + i : v;
+            const ulonglong2* q = reinterpret_cast<const ulonglong2*>(planes + u * MS_PLANES);
+            const ulonglong2 x = q[0], y = q[1];
+            vis[i] = visited[u];
+            pl[i][0] = x.x;
+            pl[i][1] = x.y;
+            pl[i][2] = y.x;
+            pl[i][3] = y.y;
+        }
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            for (int b = half * 32; b < min(k, half * 32 + 32); b++) {
+                DistQuad d;
+#pragma unroll
+                for (int i = 0; i < MS_DIST_IPT; i++) {
+                    uint32_t c = 0;
+#pragma unroll
+                    for (int p = 0; p < MS_PLANES; p++) c |= ((uint32_t)(pl[i][p] >> (32 * half)) >> (b & 31) & 1u) << p;
+                    d[i] = (uint32_t)(vis[i] >> (32 * half)) >> (b & 31) & 1u ? (int32_t)c : INF;
+                }
+                int32_t* at = dist + (int64_t)b * nv + v;
+                if (n == MS_DIST_IPT && !some_direct) {
+                    *reinterpret_cast<DistQuad*>(at) = d;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < MS_DIST_IPT; i++)
+                        if (i < n && d[i] != MS_DIRECT) at[i] = d[i];
+                }
+            }
         }
     }
 }
@@ -875,13 +1083,15 @@ struct MsEngine {
     uint64_t degs_version = ~0ull;
     void* scan_tmp = nullptr;
     MsState* S = nullptr;
-    int32_t* d_src = nullptr;
     int64_t nv = 0, tile_cap = 0, nparts = 0;
-    hipGraphExec_t exec = nullptr;
-    hipStream_t exec_stream = nullptr;
-    int32_t* exec_dist = nullptr;
-    const int32_t* exec_arena = nullptr;   // edge arena the captured level step reads (it moves when it grows)
-    MsParams exec_params{};
+    // the captured level step, without and with a window's side records
+    struct Step {
+        hipGraphExec_t exec = nullptr;
+        hipStream_t stream = nullptr;
+        const int32_t* arena = nullptr;   // the edge arena it reads (it moves when it grows)
+        MsParams params{};
+    } step[2];
+    Scratch planes;                   // level codes (batches with distances)
     MsParams params{};
     hipStream_t own = nullptr;        // non-blocking stream the level graph is captured on
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
@@ -905,9 +1115,15 @@ struct MsEngine {
                            &w_cE, &w_cS, &w_sflag})
             x->release();
     }
+    void drop_steps() {
+        for (Step& x : step) {
+            if (x.exec) (void)hipGraphExecDestroy(x.exec);
+            x.exec = nullptr;
+        }
+    }
     void release_mem() {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        exec = nullptr;
+        drop_steps();
+        planes.release();
         dfree(mem);
         mem = nullptr;
         mem_bytes = 0;
@@ -957,7 +1173,6 @@ size_t ms_layout(int64_t nv, int64_t tiles, int64_t nparts, MsEngine* e, char* b
     char* p_dd = take(64 * 3 * 8);
     char* p_st = take(std::max(scan_temp_bytes(n), scan_temp_bytes(words)));
     char* p_S = take(sizeof(MsState));
-    char* p_src = take(64 * 4);
     if (base) {
         e->visited = reinterpret_cast<uint64_t*>(p_vis);
         e->frontier = reinterpret_cast<uint64_t*>(p_fr);
@@ -982,7 +1197,6 @@ size_t ms_layout(int64_t nv, int64_t tiles, int64_t nparts, MsEngine* e, char* b
         e->digest = reinterpret_cast<unsigned long long*>(p_dd);
         e->scan_tmp = p_st;
         e->S = reinterpret_cast<MsState*>(p_S);
-        e->d_src = reinterpret_cast<int32_t*>(p_src);
     }
     return off;
 }
@@ -1076,19 +1290,22 @@ static hn_status ms_read(MsEngine* e, const void* dptr, size_t bytes, void* host
 }
 
 // record one level step on `st` (also used for capture); returns the first launch error
-static hipError_t ms_level(MsEngine* e, int32_t* dist, const MsParams& P, hipStream_t st) {
+static hipError_t ms_level(MsEngine* e, const MsParams& P, bool side, hipStream_t st) {
     hn_graph* g = e->g;
     const int64_t nv = g->nv;
     const int64_t words = ms_words(nv);
     const unsigned wgrid = (unsigned)((int64_t)num_cus() * 8);
     const unsigned xgrid = (unsigned)((int64_t)num_cus() * 16);
-    ms_decide_kernel<<<1, BLOCK, 0, st>>>(e->S, P, e->part, (int32_t)e->nparts);
+    if (!P.push_only)
+        ms_head_kernel<<<(unsigned)std::min<int64_t>(ceil_div(nv, BLOCK), wgrid), BLOCK, 0, st>>>(
+            nv, e->S, e->obits, g->rec, g->arena, e->fbits, e->frontier, e->visited, e->dirty, e->d_nchg, e->next);
     hipError_t err = exclusive_scan_dev(ListWordIn{e->S, e->fbits, e->obits}, ArrayOut<uint32_t>{e->wpre}, &e->S->wn,
                                         words, e->scan_tmp, st);
     if (err != hipSuccess) return err;
     ms_emit_kernel<<<(unsigned)ceil_div(words, BLOCK), BLOCK, 0, st>>>(words, e->S, e->fbits, e->obits, e->wpre,
                                                                        g->rec, e->visited, e->frontier, e->dirty,
-                                                                       e->list, e->qdeg, e->qoff, e->qmask);
+                                                                       e->d_nchg, e->next, e->list, e->qdeg, e->qoff,
+                                                                       e->qmask);
     err = exclusive_scan_dev_count<uint64_t>(GroupIn{e->qdeg}, GroupOut{e->P, e->tile_lo, (uint32_t)(BLOCK * P.ipt)},
                                              &e->S->tot, &e->S->wn, nv,
                                              e->scan_tmp, st);
@@ -1096,12 +1313,8 @@ static hipError_t ms_level(MsEngine* e, int32_t* dist, const MsParams& P, hipStr
     const int sbits = std::max(1, ceil_log2_host((int64_t)nv + 1));
     auto expand = [&](auto ipt_c) {
         constexpr int IPT = decltype(ipt_c)::value;
-        ms_expand_kernel<false, IPT><<<xgrid, BLOCK, 0, st>>>(
-            e->S, e->P, e->tile_lo, e->qdeg, e->qoff, e->qmask, e->list, g->arena, e->visited,
-            reinterpret_cast<unsigned long long*>(e->next), e->dirty, e->w_ckey.as<uint64_t>(), e->w_cS.as<uint64_t>(),
-            e->d_nchg, sbits);
-        ms_expand_kernel<true, IPT><<<xgrid, BLOCK, 0, st>>>(
-            e->S, e->P, e->tile_lo, e->qdeg, e->qoff, e->qmask, e->list, g->arena, e->frontier,
+        ms_expand_kernel<IPT><<<xgrid, BLOCK, 0, st>>>(
+            e->S, e->P, e->tile_lo, e->qdeg, e->qoff, e->qmask, e->list, g->arena, e->fbits, e->visited, e->frontier,
             reinterpret_cast<unsigned long long*>(e->next), e->dirty, e->w_ckey.as<uint64_t>(), e->w_cS.as<uint64_t>(),
             e->d_nchg, sbits);
     };
@@ -1110,13 +1323,16 @@ static hipError_t ms_level(MsEngine* e, int32_t* dist, const MsParams& P, hipStr
     else expand(std::integral_constant<int, 4>());
     e->exec_cS = e->w_cS.ptr;
     e->exec_ckey = e->w_ckey.ptr;
-    ms_pull_heavy_kernel<<<wgrid, BLOCK, 0, st>>>(words, e->S, e->hbits, g->rec, g->arena, e->frontier, e->visited,
-                                                  e->dirty, e->next);
-    ms_side_kernel<<<wgrid, BLOCK, 0, st>>>(e->S, e->d_nside, e->side_uw.as<int2>(), e->side_sm.as<uint64_t>(),
-                                            e->frontier, e->visited, reinterpret_cast<unsigned long long*>(e->next));
-    ms_collect_kernel<<<(unsigned)e->nparts, BLOCK, 0, st>>>(nv, e->degs, e->visited, e->frontier, e->next, dist, e->S,
-                                                             P.T, e->dirty, e->fbits, e->obits, e->hbits,
-                                                             e->part, P.digest, e->dg_part);
+    if (P.T != MS_NO_HEAVY)
+        ms_pull_heavy_kernel<<<wgrid, BLOCK, 0, st>>>(words, e->S, e->hbits, g->rec, g->arena, e->frontier, e->visited,
+                                                      e->dirty, e->next);
+    if (side)
+        ms_side_kernel<<<wgrid, BLOCK, 0, st>>>(e->S, e->d_nside, e->side_uw.as<int2>(), e->side_sm.as<uint64_t>(),
+                                                e->frontier, e->visited, reinterpret_cast<unsigned long long*>(e->next));
+    ms_collect_kernel<<<(unsigned)e->nparts, BLOCK, 0, st>>>(nv, e->degs, e->visited, e->frontier, e->next, e->S, P.T,
+                                                             e->dirty, e->fbits, e->obits, e->hbits, e->part, P.digest,
+                                                             e->dg_part);
+    ms_decide_kernel<<<1, BLOCK, 0, st>>>(e->S, P, nv, e->part, (int32_t)e->nparts);
     return hipGetLastError();
 }
 
@@ -1155,53 +1371,62 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
     for (int b = 0; b < 64; b++) P.depth_limit[b] = (depth_limit && b < k) ? depth_limit[b] : 0;
     const int64_t nv = g->nv;
     const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(nv, BLOCK), (int64_t)num_cus() * 8);
-    HN_HIP(hipMemcpyAsync(e->d_src, sources, sizeof(int32_t) * (size_t)k, hipMemcpyHostToDevice, st));
+    MsSources src{};
+    std::copy(sources, sources + k, src.v);
     if (e->degs_version != g->version) {   // degrees change with every applied update
         if (nv > 0) ms_degrees_kernel<<<(unsigned)ceil_div(nv, BLOCK), BLOCK, 0, st>>>(nv, g->rec, e->degs);
         e->degs_version = g->version;
     }
+    // (without memory for them distances are written as they are found)
+    uint64_t* planes = nullptr;
+    if (dist && k >= MS_PLANE_SOURCES && e->planes.reserve((size_t)nv * MS_PLANES * 8) == HN_OK)
+        planes = e->planes.as<uint64_t>();
     ms_init_kernel<<<grid, BLOCK, 0, st>>>(nv, e->visited, e->frontier, e->next, 3 * ms_bit_words(nv), e->fbits);
-    if (dist)
+    if (!dist)
+        HN_HIP(hipMemsetAsync(e->dg_part, 0, (size_t)e->nparts * 64 * 3 * 8, st));
+    else if (!planes)
         ms_fill_dist_kernel<<<(unsigned)std::min<int64_t>(ceil_div((int64_t)k * nv, 4 * BLOCK),
                                                           (int64_t)num_cus() * 16),
                               BLOCK, 0, st>>>((int64_t)k * nv, dist);
-    else
-        HN_HIP(hipMemsetAsync(e->dg_part, 0, (size_t)e->nparts * 64 * 3 * 8, st));
-    ms_seed_kernel<<<1, WAVE, 0, st>>>(k, e->d_src, nv, e->visited, e->frontier, e->fbits, dist, g->rec, e->S, P);
+    ms_seed_kernel<<<1, WAVE, 0, st>>>(k, src, nv, e->visited, e->frontier, e->fbits, dist, planes, g->rec, e->S, P);
     HN_CHECK_LAUNCH();
-    // capture the level step once per (stream, dist buffer, parameters, buffers)
-    const bool same = e->exec && e->exec_stream == st && e->exec_dist == dist && e->exec_arena == g->arena &&
-                      std::memcmp(&e->exec_params, &P, sizeof(P)) == 0;
+    ms_decide_kernel<<<1, BLOCK, 0, st>>>(e->S, P, nv, e->part, (int32_t)e->nparts);
+    HN_CHECK_LAUNCH();
+    // capture the level step once per (stream, parameters, buffers); what differs
+    // from batch to batch (sources, limits, distances) is in the device state
+    MsParams L = P;
+    std::fill(std::begin(L.depth_limit), std::end(L.depth_limit), 0);
+    MsEngine::Step& step = e->step[e->has_window ? 1 : 0];
+    const bool same = step.exec && step.stream == st && step.arena == g->arena &&
+                      std::memcmp(&step.params, &L, sizeof(L)) == 0;
     if (!same) {
-        if (e->exec) (void)hipGraphExecDestroy(e->exec);
-        e->exec = nullptr;
+        if (step.exec) (void)hipGraphExecDestroy(step.exec);
+        step.exec = nullptr;
         hipGraph_t graph = nullptr;
         HN_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        const hipError_t le = ms_level(e, dist, P, st);
+        const hipError_t le = ms_level(e, L, e->has_window, st);
         hipError_t ce = hipStreamEndCapture(st, &graph);
         if (le != hipSuccess || ce != hipSuccess) {
             if (graph) (void)hipGraphDestroy(graph);
             set_error(std::string("level-step capture: ") + hipGetErrorString(le != hipSuccess ? le : ce));
             return HN_E_HIP;
         }
-        hipError_t ie = hipGraphInstantiate(&e->exec, graph, nullptr, nullptr, 0);
+        hipError_t ie = hipGraphInstantiate(&step.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (ie != hipSuccess) {
-            e->exec = nullptr;
+            step.exec = nullptr;
             set_error(std::string("level-step instantiate: ") + hipGetErrorString(ie));
             return HN_E_HIP;
         }
-        e->exec_stream = st;
-        e->exec_dist = dist;
-        e->exec_arena = g->arena;
-        e->exec_params = P;
+        step.stream = st;
+        step.arena = g->arena;
+        step.params = L;
     }
-    // Replay.  The first poll of the done flag comes after as many steps as
-    // the last launch on this graph needed (a graph's depth barely changes
-    // between launches; depth-limited launches need at most limit + 2), the
-    // next ones after 1, 2, 4, 4, ... more steps: with a fixed poll every 4
-    // steps a launch ran up to 3 steps past its end, each one 11 kernels that
-    // return at once but still cost their launch gaps.
+    // Replay.  The first poll of the state comes after as many steps as the last
+    // launch on this graph needed (a graph's depth barely changes between launches;
+    // depth-limited launches need at most the limit: a step ends with the decision
+    // whether it was the last), the next ones after 1, 2, 4, 4, ... more steps: a step
+    // past the end returns at once but still costs its kernels' launch gaps.
     int32_t max_limit = 0;
     bool limited = k > 0;
     for (int b = 0; b < k; b++) {
@@ -1209,17 +1434,21 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
         max_limit = std::max(max_limit, P.depth_limit[b]);
     }
     int64_t next = e->last_steps > 0 ? e->last_steps : 4;
-    if (limited) next = std::min<int64_t>(next, max_limit + 2);
+    if (limited) next = std::min<int64_t>(next, max_limit);
     int64_t ramp = 1;
-    int32_t* host = e->pinned;   // [0] done, [1] level steps that did work
-    static_assert(offsetof(MsState, levels_run) == offsetof(MsState, done) + 4, "done, levels_run adjacent");
+    static_assert(sizeof(MsState) <= 4096, "state readback fits the pinned buffer");
+    MsState s;
     for (int64_t rep = 0; rep <= nv + 1;) {
-        for (int64_t c = 0; c < next; c++) HN_HIP(hipGraphLaunch(e->exec, st));
+        for (int64_t c = 0; c < next; c++) HN_HIP(hipGraphLaunch(step.exec, st));
         rep += next;
-        HN_HIP(hipMemcpyAsync(host, &e->S->done, 8, hipMemcpyDeviceToHost, st));
-        HN_HIP(hipStreamSynchronize(st));
-        if (host[0]) {
-            if (!limited) e->last_steps = host[1] + 1;
+        if (planes) {
+            ms_dist_kernel<<<(unsigned)std::min<int64_t>(ceil_div(nv, BLOCK * MS_DIST_IPT), (int64_t)num_cus() * 16), BLOCK,
+                             0, st>>>(nv, k, e->S, e->visited);
+            HN_CHECK_LAUNCH();
+        }
+        HN_TRY(ms_read(e, e->S, sizeof(MsState), &s, st));
+        if (s.done) {
+            if (!limited) e->last_steps = std::max(s.levels_run, 1);
             break;
         }
         next = ramp;
@@ -1230,9 +1459,6 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
         HN_CHECK_LAUNCH();
     }
     if (stats) {
-        MsState s;
-        static_assert(sizeof(MsState) <= 4096, "state readback fits the pinned buffer");
-        HN_TRY(ms_read(e, e->S, sizeof(MsState), &s, st));
         stats->levels = s.levels_run;
         stats->push_levels = (int32_t)s.push_levels;
         stats->pull_levels = (int32_t)s.pull_levels;
@@ -1334,8 +1560,7 @@ hn_status ms_window_end(MsEngine* e, int32_t m, uint64_t failed, const uint64_t*
     HN_TRY(e->side_sm.reserve((size_t)(nchg > 0 ? nchg : 1) * 8));
     if (e->side_uw.ptr != old_uw || e->side_sm.ptr != old_sm || e->w_cS.ptr != e->exec_cS ||
         e->w_ckey.ptr != e->exec_ckey) {   // the captured level step holds these pointers
-        if (e->exec) (void)hipGraphExecDestroy(e->exec);
-        e->exec = nullptr;
+        e->drop_steps();
     }
     set_u32_kernel<<<1, 1, 0, st>>>(e->d_nchg, nchg);
     HN_CHECK_LAUNCH();
