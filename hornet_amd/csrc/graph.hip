@@ -582,42 +582,100 @@ __global__ void pack_keys_kernel(PackArgs a, uint64_t* __restrict__ keys, unsign
     if (a.sym) keys[a.m + i] = self ? SENTINEL : (((uint64_t)d << a.sbits) | (uint64_t)s);
 }
 
-struct UniqueFlagIn {
-    const uint64_t* k;
-    uint64_t mask;   // sentinel pattern restricted to the sorted bits
-    __device__ __forceinline__ uint32_t operator()(int64_t i) const {
-        uint64_t x = k[i];
-        if (x == SENTINEL || (x & mask) == mask) return 0u;
-        return (i == 0 || k[i - 1] != x) ? 1u : 0u;
-    }
+// Sorted keys -> rows, each pair once.  A tile's keys are read twice, to count the
+// distinct ones and to write them; nothing but the adjacency and each row's start
+// and end is written (with positions and compacted keys in between, and a search for
+// every vertex's first key, this took 900 us for the 67 M keys of an R-MAT s21 build; 290 so, 120 and 140 of them in
+// the two readings, 4.5 TB/s).
+constexpr int UNIQ_IPT = 16;
+constexpr int UNIQ_TILE = BLOCK * UNIQ_IPT;
+
+// A wave's UNIQ_IPT rows of 64 keys: keys, the keys before them, and per row the
+// lanes whose key is the first of its pair.
+struct UniqRows {
+    uint64_t key[UNIQ_IPT];
+    uint64_t prev[UNIQ_IPT];    // (of the very first key: all ones)
+    uint64_t first[UNIQ_IPT];
+    int64_t base;
 };
-
-__global__ void unique_write_kernel(const uint64_t* __restrict__ k, int64_t n, uint64_t mask,
-                                    const uint32_t* __restrict__ pos, int sbits,
-                                    uint64_t* __restrict__ ukeys, int32_t* __restrict__ adj) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t x = k[i];
-    if (x == SENTINEL || (x & mask) == mask) return;
-    if (i > 0 && k[i - 1] == x) return;
-    uint32_t p = pos[i];
-    ukeys[p] = x;
-    adj[p] = (int32_t)(x & ((1ull << sbits) - 1));
-}
-
-__global__ void offsets_from_keys_kernel(const uint64_t* __restrict__ ukeys, int64_t u, int sbits,
-                                         int32_t nv, int64_t* __restrict__ off) {
-    int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v > nv) return;
-    // first compacted key with src >= v
-    uint64_t target = (uint64_t)v << sbits;
-    int64_t lo = 0, hi = u;
-    while (lo < hi) {
-        int64_t mid = (lo + hi) >> 1;
-        if (ukeys[mid] < target) lo = mid + 1; else hi = mid;
+__device__ __forceinline__ UniqRows uniq_rows(const uint64_t* __restrict__ k, int64_t n, uint64_t mask) {
+    UniqRows r;
+    const int lane = __lane_id();
+    r.base = (int64_t)blockIdx.x * UNIQ_TILE + (int64_t)(threadIdx.x / WAVE) * (WAVE * UNIQ_IPT);
+    const uint64_t before = r.base > 0 && r.base <= n ? k[r.base - 1] : SENTINEL;
+#pragma unroll
+    for (int j = 0; j < UNIQ_IPT; j++) {
+        const int64_t i = r.base + j * WAVE + lane;
+        r.key[j] = i < n ? k[i] : SENTINEL;
     }
-    off[v] = lo;
+#pragma unroll
+    for (int j = 0; j < UNIQ_IPT; j++) {
+        const uint64_t up = __shfl_up(r.key[j], 1, WAVE);
+        const uint64_t last = j ? __shfl(r.key[j - 1], WAVE - 1, WAVE) : before;
+        r.prev[j] = lane ? up : last;
+        const int64_t i = r.base + j * WAVE + lane;
+        const uint64_t x = r.key[j];
+        const bool valid = i < n && x != SENTINEL && (x & mask) != mask;
+        r.first[j] = __ballot(valid && (i == 0 || r.prev[j] != x));
+    }
+    return r;
 }
+
+__global__ __launch_bounds__(BLOCK) void unique_count_kernel(const uint64_t* __restrict__ k, int64_t n, uint64_t mask,
+                                                             uint32_t* __restrict__ count) {
+    __shared__ uint32_t sum;
+    if (threadIdx.x == 0) sum = 0;
+    __syncthreads();
+    const UniqRows r = uniq_rows(k, n, mask);
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < UNIQ_IPT; j++) c += (uint32_t)__popcll(r.first[j]);
+    if (__lane_id() == 0) atomicAdd(&sum, c);
+    __syncthreads();
+    if (threadIdx.x == 0) count[blockIdx.x] = sum;
+}
+
+// row_start / row_end of a vertex with entries (the others keep their zeros): the
+// first key of a row starts it and ends the row before; the last key of all ends its own
+__global__ __launch_bounds__(BLOCK) void unique_rows_kernel(const uint64_t* __restrict__ k, int64_t n, uint64_t mask,
+                                                            const uint32_t* __restrict__ tile_first, uint32_t total,
+                                                            int sbits, int32_t* __restrict__ adj,
+                                                            uint32_t* __restrict__ row_start,
+                                                            uint32_t* __restrict__ row_end) {
+    __shared__ uint32_t wsum[NWAVES];
+    const UniqRows r = uniq_rows(k, n, mask);
+    const int w = threadIdx.x / WAVE;
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < UNIQ_IPT; j++) c += (uint32_t)__popcll(r.first[j]);
+    if (__lane_id() == 0) wsum[w] = c;
+    __syncthreads();
+    uint32_t at = tile_first[blockIdx.x];
+    for (int q = 0; q < w; q++) at += wsum[q];
+    const uint64_t lt = lanemask_lt();
+    const uint64_t low = (1ull << sbits) - 1;
+#pragma unroll
+    for (int j = 0; j < UNIQ_IPT; j++) {
+        if ((r.first[j] >> __lane_id()) & 1ull) {
+            const uint64_t x = r.key[j];
+            const uint32_t p = at + (uint32_t)__popcll(r.first[j] & lt);
+            adj[p] = (int32_t)(x & low);
+            const bool very_first = r.base + j * WAVE + __lane_id() == 0;
+            if (very_first || (r.prev[j] >> sbits) != (x >> sbits)) {
+                row_start[x >> sbits] = p;
+                if (!very_first) row_end[r.prev[j] >> sbits] = p;
+            }
+            if (p == total - 1) row_end[x >> sbits] = total;
+        }
+        at += (uint32_t)__popcll(r.first[j]);
+    }
+}
+
+struct RowLenIn {
+    const uint32_t* start;
+    const uint32_t* end;
+    __device__ __forceinline__ int64_t operator()(int64_t v) const { return (int64_t)(end[v] - start[v]); }
+};
 
 }  // namespace
 
@@ -955,18 +1013,20 @@ hn_status csr_from_device_coo(int32_t nv, int64_t m, const int32_t* src, const i
     const uint64_t mask = key_bits >= 64 ? ~0ull : ((1ull << key_bits) - 1);
     uint64_t* ka = nullptr;
     uint64_t* kb = nullptr;
-    uint32_t* pos = nullptr;
+    uint32_t* count = nullptr;   // distinct keys per tile, then the rows' starts and ends
     unsigned* bad = nullptr;
     void* tmp = nullptr;
     int64_t* d_off = nullptr;
     int32_t* d_adj = nullptr;
     hn_status s = HN_OK;
     auto cleanup = [&](void (*give)(void*) = dfree) {
-        give(ka); give(kb); give(pos); give(bad); give(tmp);
+        give(ka); give(kb); give(count); give(bad); give(tmp);
     };
-    size_t tmpb = std::max(sort_temp_bytes(n), scan_temp_bytes(n));
+    const int64_t tiles = ceil_div(n, UNIQ_TILE);
+    const size_t counts = ((size_t)tiles + 1 + 63) & ~size_t(63);
+    size_t tmpb = std::max(sort_temp_bytes(n), scan_temp_bytes(std::max<int64_t>(tiles, nv)));
     if ((s = dalloc(&ka, (size_t)n + 1)) != HN_OK || (s = dalloc(&kb, (size_t)n + 1)) != HN_OK ||
-        (s = dalloc(&pos, (size_t)n + 1)) != HN_OK || (s = dalloc(&bad, 1)) != HN_OK ||
+        (s = dalloc(&count, counts + 2 * (size_t)(nv > 0 ? nv : 1))) != HN_OK || (s = dalloc(&bad, 1)) != HN_OK ||
         (s = dmalloc(&tmp, tmpb)) != HN_OK) {
         cleanup();
         return s;
@@ -978,13 +1038,20 @@ hn_status csr_from_device_coo(int32_t nv, int64_t m, const int32_t* src, const i
         HN_CHECK_LAUNCH();
     }
     if ((s = radix_sort_u64(&ka, &kb, n, key_bits, tmp, st)) != HN_OK) { cleanup(); return s; }
-    if ((s = exclusive_scan<uint32_t>(UniqueFlagIn{ka, mask}, pos, n, tmp, st)) != HN_OK) {
+    uint32_t* row_start = count + counts;
+    uint32_t* row_end = row_start + (nv > 0 ? nv : 1);
+    HN_HIP(hipMemsetAsync(row_start, 0, 2 * sizeof(uint32_t) * (size_t)(nv > 0 ? nv : 1), st));
+    if (n > 0) {
+        unique_count_kernel<<<(unsigned)tiles, BLOCK, 0, st>>>(ka, n, mask, count);
+        HN_CHECK_LAUNCH();
+    }
+    if ((s = exclusive_scan<uint32_t>(ArrayIn<uint32_t>{count}, count, tiles, tmp, st)) != HN_OK) {
         cleanup();
         return s;
     }
     uint32_t u32 = 0;
     unsigned hbad = 0;
-    HN_HIP(hipMemcpyAsync(&u32, pos + n, 4, hipMemcpyDeviceToHost, st));
+    HN_HIP(hipMemcpyAsync(&u32, count + tiles, 4, hipMemcpyDeviceToHost, st));
     HN_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, st));
     HN_HIP(hipStreamSynchronize(st));
     if (hbad) {
@@ -998,13 +1065,15 @@ hn_status csr_from_device_coo(int32_t nv, int64_t m, const int32_t* src, const i
         cleanup();
         return s;
     }
-    // compacted keys reuse kb
-    if (n > 0) {
-        unique_write_kernel<<<(unsigned)ceil_div(n, BLOCK), BLOCK, 0, st>>>(ka, n, mask, pos, sbits, kb, d_adj);
+    if (u > 0) {
+        unique_rows_kernel<<<(unsigned)tiles, BLOCK, 0, st>>>(ka, n, mask, count, u32, sbits, d_adj, row_start, row_end);
         HN_CHECK_LAUNCH();
     }
-    offsets_from_keys_kernel<<<(unsigned)ceil_div((int64_t)nv + 1, BLOCK), BLOCK, 0, st>>>(kb, u, sbits, nv, d_off);
-    HN_CHECK_LAUNCH();
+    if ((s = exclusive_scan<int64_t>(RowLenIn{row_start, row_end}, d_off, nv, tmp, st)) != HN_OK) {
+        dfree(d_off); dfree(d_adj);
+        cleanup();
+        return s;
+    }
     hipError_t e = hipStreamSynchronize(st);
     cleanup(e == hipSuccess ? dput : dfree);
     if (e != hipSuccess) {
