@@ -97,6 +97,23 @@ inline int ceil_log2_host(int64_t x) {
 size_t sort_temp_bytes(int64_t n);
 hn_status radix_sort_u64(uint64_t** keys, uint64_t** alt, int64_t n, int key_bits, void* tmp,
                          hipStream_t st);
+// Up to sort_small_max() keys, made of pairs, are packed and sorted by one launch into
+// keys (and, if given, their positions into idx).  It clears `words` words at `state`
+// first, and then ORs `bad` into *err for a pair with an end outside [0, nv), whose key
+// is 0.
+struct SortPairs {
+    const int32_t* src;
+    const int32_t* dst;
+    int32_t nv;
+    int sbits;
+    uint32_t* state;
+    int words;
+    uint32_t* err;
+    uint32_t bad;
+};
+int64_t sort_small_max(bool values);
+hn_status radix_sort_small_pairs(const SortPairs& pairs, uint64_t* keys, uint32_t* idx, int64_t n, int key_bits,
+                                 hipStream_t st);
 // The same sort carrying a 32-bit value per key (vals / valt swap with the
 // keys): the values of equal keys keep their input order.
 hn_status radix_sort_u64_kv(uint64_t** keys, uint64_t** alt, uint32_t** vals, uint32_t** valt, int64_t n,

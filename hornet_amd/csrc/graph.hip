@@ -521,6 +521,17 @@ struct DegIn {
     __device__ __forceinline__ int64_t operator()(int64_t v) const { return rec[v].deg; }
 };
 
+// the degree prefix, and the segment that holds each copy tile's first entry
+struct DegOut {
+    int64_t* P;
+    uint32_t* tile_lo;
+    __device__ __forceinline__ void operator()(int64_t v, int64_t ex, int64_t deg) const {
+        P[v] = ex;
+        if (deg)
+            for (int64_t t = (ex + COPY_TILE - 1) / COPY_TILE; t * COPY_TILE < ex + deg; t++) tile_lo[t] = (uint32_t)v;
+    }
+};
+
 __global__ void degrees_kernel(int32_t nv, const hn_vrec* __restrict__ rec, int32_t* __restrict__ deg) {
     int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v < nv) deg[v] = rec[v].deg;
@@ -1321,10 +1332,9 @@ static hn_status flatten(hn_graph* g, int32_t* src, int32_t* dst, int64_t* eoff_
     HN_TRY(g->s_misc.reserve(eoff_bytes + sizeof(uint32_t) * (size_t)(tiles + 1)));
     int64_t* eoff = eoff_out ? eoff_out : g->s_misc.as<int64_t>();
     uint32_t* tile_lo = reinterpret_cast<uint32_t*>(g->s_misc.as<char>() + eoff_bytes);
-    HN_TRY(degree_prefix(g, eoff, st));
+    HN_TRY(g->s_scan.reserve(scan_temp_bytes(g->nv)));
+    HN_TRY(exclusive_scan_fn<int64_t>(DegIn{g->rec}, DegOut{eoff, tile_lo}, eoff + g->nv, g->nv, g->s_scan.ptr, st));
     if (g->ne > 0) {
-        tile_starts_kernel<<<(unsigned)ceil_div(tiles, BLOCK), BLOCK, 0, st>>>(tiles, eoff, g->nv, tile_lo);
-        HN_CHECK_LAUNCH();
         int64_t grid = std::min<int64_t>(tiles, (int64_t)num_cus() * 8);
         flatten_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(g->nv, g->ne, eoff, tile_lo, g->rec, g->arena, src, dst,
                                                          out, g->meta);

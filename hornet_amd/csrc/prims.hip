@@ -206,9 +206,34 @@ __global__ __launch_bounds__(THREADS) void rs_scatter_kernel(const uint64_t* __r
 constexpr int RS_SMALL_BLOCK = 1024;
 constexpr int64_t RS_SMALL = RS_SMALL_BLOCK * 16, RS_SMALL_KV = RS_SMALL_BLOCK * 8;   // what 160 KB of LDS hold
 
-template <bool KV, int IPT>
-__global__ __launch_bounds__(RS_SMALL_BLOCK) void rs_small_kernel(uint64_t* __restrict__ keys,
-                                                                  uint32_t* __restrict__ vals, int n, int key_bits) {
+// what it sorts: keys (and values) in place, or pairs, packed as they are loaded
+struct SmallKeys {
+    const uint64_t* k;
+    const uint32_t* v;
+    __device__ __forceinline__ void begin() const {}
+    __device__ __forceinline__ uint64_t key(int i) const { return k[i]; }
+    __device__ __forceinline__ uint32_t val(int i) const { return v[i]; }
+};
+struct SmallPairs {
+    SortPairs p;
+    __device__ __forceinline__ void begin() const {
+        if ((int)threadIdx.x < p.words) p.state[threadIdx.x] = 0;
+        __syncthreads();   // before any error is noted
+    }
+    __device__ __forceinline__ uint64_t key(int i) const {
+        const int32_t s = p.src[i], d = p.dst[i];
+        if (s < 0 || s >= p.nv || d < 0 || d >= p.nv) {
+            atomicOr(p.err, p.bad);
+            return 0;
+        }
+        return ((uint64_t)s << p.sbits) | (uint64_t)d;
+    }
+    __device__ __forceinline__ uint32_t val(int i) const { return (uint32_t)i; }
+};
+
+template <bool KV, int IPT, typename Src>
+__global__ __launch_bounds__(RS_SMALL_BLOCK) void rs_small_kernel(Src in, uint64_t* keys, uint32_t* vals, int n,
+                                                                  int key_bits) {
     constexpr int WAVES = RS_SMALL_BLOCK / WAVE;
     __shared__ uint64_t stage[RS_SMALL_BLOCK * IPT];
     __shared__ uint32_t vstage[KV ? RS_SMALL_BLOCK * IPT : 1];
@@ -219,15 +244,16 @@ __global__ __launch_bounds__(RS_SMALL_BLOCK) void rs_small_kernel(uint64_t* __re
     const int rows = (n + RS_SMALL_BLOCK - 1) / RS_SMALL_BLOCK;
     const int base = w * rows * WAVE;
     const uint64_t lt = lanemask_lt();
+    in.begin();
     // past the end: the largest key, which a stable sort leaves there
     uint64_t k[IPT];
     uint32_t v[IPT], rank[IPT];
 #pragma unroll
     for (int j = 0; j < IPT; j++) {
         const int i = base + j * WAVE + l;
-        const bool in = j < rows && i < n;
-        k[j] = in ? keys[i] : ~0ull;
-        v[j] = KV && in ? vals[i] : 0u;
+        const bool any = j < rows && i < n;
+        k[j] = any ? in.key(i) : ~0ull;
+        v[j] = KV && any ? in.val(i) : 0u;
     }
     for (int shift = 0; shift < key_bits; shift += RS_BITS) {
         for (int d = threadIdx.x; d < WAVES * RS_BUCKETS; d += RS_SMALL_BLOCK) (&cnt[0][0])[d] = 0;
@@ -332,16 +358,27 @@ static hn_status rs_pass(const uint64_t* in, uint64_t* out, const uint32_t* vin,
     return HN_OK;
 }
 
+int64_t sort_small_max(bool values) { return values ? RS_SMALL_KV : RS_SMALL; }
+
+template <typename Src>
+static hn_status rs_small(Src in, uint64_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t st) {
+    if (vals) rs_small_kernel<true, 8><<<1, RS_SMALL_BLOCK, 0, st>>>(in, keys, vals, (int)n, key_bits);
+    else if (n <= RS_SMALL_BLOCK * 8) rs_small_kernel<false, 8><<<1, RS_SMALL_BLOCK, 0, st>>>(in, keys, vals, (int)n, key_bits);
+    else rs_small_kernel<false, 16><<<1, RS_SMALL_BLOCK, 0, st>>>(in, keys, vals, (int)n, key_bits);
+    HN_CHECK_LAUNCH();
+    return HN_OK;
+}
+
+hn_status radix_sort_small_pairs(const SortPairs& pairs, uint64_t* keys, uint32_t* idx, int64_t n, int key_bits,
+                                 hipStream_t st) {
+    return rs_small(SmallPairs{pairs}, keys, idx, n, key_bits, st);
+}
+
 static hn_status radix_sort_impl(uint64_t** keys, uint64_t** alt, uint32_t** vals, uint32_t** valt, int64_t n,
                                  int key_bits, void* tmp, hipStream_t st) {
     if (n <= 1) return HN_OK;
-    if (n <= (vals ? RS_SMALL_KV : RS_SMALL)) {
-        if (vals) rs_small_kernel<true, 8><<<1, RS_SMALL_BLOCK, 0, st>>>(*keys, *vals, (int)n, key_bits);
-        else if (n <= RS_SMALL_BLOCK * 8) rs_small_kernel<false, 8><<<1, RS_SMALL_BLOCK, 0, st>>>(*keys, nullptr, (int)n, key_bits);
-        else rs_small_kernel<false, 16><<<1, RS_SMALL_BLOCK, 0, st>>>(*keys, nullptr, (int)n, key_bits);
-        HN_CHECK_LAUNCH();
-        return HN_OK;
-    }
+    if (n <= sort_small_max(vals != nullptr))
+        return rs_small(SmallKeys{*keys, vals ? *vals : nullptr}, *keys, vals ? *vals : nullptr, n, key_bits, st);
     const int64_t tile = rs_tile_keys(n);
     const int64_t hn_ = ceil_div(n, tile) * RS_BUCKETS;
     HN_ARG(hn_ < (int64_t)0xFFFFFFFF && n < (int64_t)0xFFFFFFFF, "radix_sort_u64: too many keys");

@@ -140,18 +140,27 @@ struct FirstKeepIn {
     }
 };
 
-// kept keys (and, when given, the values of one or two parallel arrays)
-__global__ void compact_keys_kernel(int64_t n, const uint64_t* __restrict__ in, const uint32_t* __restrict__ pos,
-                                    uint64_t* __restrict__ out, const uint32_t* __restrict__ iin,
-                                    uint32_t* __restrict__ iout, const uint32_t* __restrict__ jin,
-                                    uint32_t* __restrict__ jout) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && pos[i + 1] != pos[i]) {
-        out[pos[i]] = in[i];
-        if (iin) iout[pos[i]] = iin[i];
-        if (jin) jout[pos[i]] = jin[i];
+// The steps over a batch are scans whose output is written where the prefix is
+// known: a launch each, where compaction and segments were launches of their own
+// that read the prefixes back (a batch of 1,000 pairs is bounded by its launches, 5 us
+// each).
+
+// scan output of the keep flags: the kept keys (and, when given, the values of one
+// or two parallel arrays) in their new places
+struct CompactOut {
+    const uint64_t* in;
+    uint64_t* out;
+    const uint32_t* iin;
+    uint32_t* iout;
+    const uint32_t* jin;
+    uint32_t* jout;
+    __device__ __forceinline__ void operator()(int64_t i, uint32_t ex, uint32_t keep) const {
+        if (!keep) return;
+        out[ex] = in[i];
+        if (iin) iout[ex] = iin[i];
+        if (jin) jout[ex] = jin[i];
     }
-}
+};
 
 // segment starts over the first `*cnt` keys: key i starts a segment when its
 // group (given by `shift`: the source, or the whole key) differs from key i-1
@@ -166,21 +175,23 @@ struct SegStartIn {
     }
 };
 
-__global__ void seg_write_kernel(int64_t n, const uint64_t* __restrict__ k, const uint32_t* __restrict__ cnt,
-                                 const uint32_t* __restrict__ spos, uint32_t* __restrict__ seg_start,
-                                 uint64_t* __restrict__ seg_key) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t m = *cnt;
-    if (i > m || i >= n + 1) return;
-    if (i == m) {
-        seg_start[spos[n]] = (uint32_t)m;
-        return;
+// and its output: every segment's start and first key, and the end of the last one
+struct SegOut {
+    const uint64_t* k;
+    const uint32_t* cnt;
+    uint32_t* spos;
+    uint32_t* seg_start;
+    uint64_t* seg_key;
+    __device__ __forceinline__ void operator()(int64_t i, uint32_t ex, uint32_t is) const {
+        const int64_t m = *cnt;
+        spos[i] = ex;
+        if (is) {
+            seg_start[ex] = (uint32_t)i;
+            seg_key[ex] = k[i];
+        }
+        if (i + 1 == m || (i == 0 && m == 0)) seg_start[ex + is] = (uint32_t)m;
     }
-    if (spos[i + 1] != spos[i]) {
-        seg_start[spos[i]] = (uint32_t)i;
-        seg_key[spos[i]] = k[i];
-    }
-}
+};
 
 // Per touched vertex.  A vertex is either updated in place (its block still
 // fits: insert new_deg <= capacity, the reference's `new_degree > limit`
@@ -318,10 +329,11 @@ __global__ __launch_bounds__(ALLOC_BLOCK) void commit_kernel(const uint32_t* __r
                                                              const TouchInfo* __restrict__ ti,
                                                              const uint8_t* __restrict__ skip,
                                                              hn_vrec* __restrict__ rec, AllocView A,
-                                                             const UpdScal* sc) {
+                                                             const uint32_t* __restrict__ changed, UpdScal* sc) {
     __shared__ AllocShared ash;
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = j < (int64_t)*ucnt && !sc->err;   // every thread reaches the release below
+    if (j == 0 && !sc->err) sc->changed = *changed;
     bool rel = false;
     TouchInfo t{};
     if (active) {
@@ -393,6 +405,29 @@ struct DLenIn {
     const uint32_t* dlen;
     const uint32_t* dcnt;
     __device__ __forceinline__ uint32_t operator()(int64_t i) const { return i < (int64_t)*dcnt ? dlen[i] : 0u; }
+};
+
+// the deletions in the low and the segments in the high half (neither sum exceeds
+// the 2^32 - 1 stored entries)
+struct DelGroupIn {
+    DLenIn len;
+    SegStartIn seg;
+    __device__ __forceinline__ uint64_t operator()(int64_t i) const {
+        return (uint64_t)len(i) | (uint64_t)seg(i) << 32;
+    }
+};
+struct DelGroupOut {
+    SegOut seg;
+    uint32_t* dlp;   // n + 1; seg.spos too
+    int64_t n;
+    __device__ __forceinline__ void operator()(int64_t i, uint64_t ex, uint64_t x) const {
+        dlp[i] = (uint32_t)ex;
+        seg(i, (uint32_t)(ex >> 32), (uint32_t)(x >> 32));
+        if (i == n - 1) {
+            dlp[n] = (uint32_t)(ex + x);
+            seg.spos[n] = (uint32_t)((ex + x) >> 32);
+        }
+    }
 };
 
 // per touched source u (segments of the distinct keys): deletions; in place
@@ -530,46 +565,39 @@ struct GapLenIn {
 // deleted before them in that vertex; measured at 1-2 % of the moved entries
 // on R-MAT graphs, where the staged alternative copies every moved entry
 // twice.
-__global__ void erase_defer_kernel(int64_t ntile_max, int64_t nruns, const int64_t* __restrict__ P,
-                                   const uint32_t* __restrict__ tile_lo, const int64_t* __restrict__ src,
-                                   const int64_t* __restrict__ dst, const uint32_t* __restrict__ rtail,
-                                   uint32_t* __restrict__ tcnt, const UpdScal* sc) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntile_max) return;
-    const int64_t W = P[nruns];
-    const int64_t ntiles = (W + ERASE_TILE - 1) / ERASE_TILE;
-    int64_t c = 0;
-    if (!sc->err && t > 0 && t < ntiles) {
+struct EraseDeferIn {
+    int64_t nruns;
+    const int64_t* P;
+    const uint32_t* tile_lo;
+    const int64_t* src;
+    const int64_t* dst;
+    const uint32_t* rtail;
+    const UpdScal* sc;
+    __device__ __forceinline__ int64_t operator()(int64_t t) const {
+        const int64_t ntiles = (P[nruns] + ERASE_TILE - 1) / ERASE_TILE;
+        if (sc->err || t == 0 || t >= ntiles) return 0;
         const int64_t i0 = t * ERASE_TILE;
         const int64_t r = tile_lo[t];                                   // holds i0
         const int64_t rp = upper_bound_m1<int64_t>(P, 0, r + 1, i0 - 1);  // holds i0 - 1
-        if ((src[r] & RUN_INPLACE) && rtail[r] == rtail[rp]) {
-            const int64_t d0 = dst[r] - P[r] + i0;
-            const int64_t sprev = (src[rp] & ~RUN_INPLACE) - P[rp] + (i0 - 1);
-            if (sprev >= d0) {
-                c = sprev - d0 + 1;
-                const int64_t vend = P[rtail[r] + 1];   // end of the vertex's items
-                c = c < vend - i0 ? c : vend - i0;
-                c = c < (int64_t)ERASE_TILE ? c : (int64_t)ERASE_TILE;
-            }
-        }
+        if (!(src[r] & RUN_INPLACE) || rtail[r] != rtail[rp]) return 0;
+        const int64_t d0 = dst[r] - P[r] + i0;
+        const int64_t sprev = (src[rp] & ~RUN_INPLACE) - P[rp] + (i0 - 1);
+        if (sprev < d0) return 0;
+        const int64_t vend = P[rtail[r] + 1];   // end of the vertex's items
+        return min(min(sprev - d0 + 1, vend - i0), (int64_t)ERASE_TILE);
     }
-    tcnt[t] = (uint32_t)c;
-}
-
-struct TileCountIn {
-    const uint32_t* c;
-    __device__ __forceinline__ int64_t operator()(int64_t t) const { return (int64_t)c[t]; }
 };
 
-// scan output of the deferred counts: each tile's offset in the side buffer;
-// the last tile also records the total in the batch's status word, read back
-// with it
+// scan output of the deferred counts: each tile's count and offset in the side
+// buffer; the last tile also records the total in the batch's status word, read
+// back with it
 struct SideOut {
+    uint32_t* tcnt;
     int64_t* P;
     int64_t last;
     UpdScal* sc;
     __device__ __forceinline__ void operator()(int64_t i, int64_t ex, int64_t x) const {
+        tcnt[i] = (uint32_t)x;
         P[i] = ex;
         if (i == last) sc->side = ex + x;
     }
@@ -702,31 +730,30 @@ __device__ __forceinline__ int64_t count_below(const uint64_t* __restrict__ B, i
 // whose destination reaches source(i1) are deferred: at most
 // c = #(B < A[r_last]) of them, since r + #(B < A[r]) > r_last needs
 // r > r_last - c.  They are placed once every tile has read.
-__global__ void insert_defer_kernel(int64_t ntile_max, int64_t nseg, const int64_t* __restrict__ aP,
-                                    const uint32_t* __restrict__ tile_lo, const TouchInfo* __restrict__ ti,
-                                    const uint32_t* __restrict__ seg_start, const uint64_t* __restrict__ keys,
-                                    KeyFmt f, const int32_t* __restrict__ arena, uint32_t* __restrict__ tcnt,
-                                    const UpdScal* sc) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntile_max) return;
-    const int64_t W = aP[nseg];
-    const int64_t ntiles = (W + COPY_TILE - 1) / COPY_TILE;
-    int64_t c = 0;
-    if (!sc->err && t + 1 < ntiles) {
+struct InsertDeferIn {
+    int64_t nseg;
+    const int64_t* aP;
+    const uint32_t* tile_lo;
+    const TouchInfo* ti;
+    const uint32_t* seg_start;
+    const uint64_t* keys;
+    KeyFmt f;
+    const int32_t* arena;
+    const UpdScal* sc;
+    __device__ __forceinline__ int64_t operator()(int64_t t) const {
+        const int64_t ntiles = (aP[nseg] + COPY_TILE - 1) / COPY_TILE;
+        if (sc->err || t + 1 >= ntiles) return 0;
         const int64_t i1 = (t + 1) * COPY_TILE;
         const int64_t j = tile_lo[t + 1];   // holds i1
-        if (aP[j] < i1) {                   // and i1 - 1, the tile's last item
-            const TouchInfo tj = ti[j];
-            if (tj.inplace) {
-                const int64_t r_last = tj.p + (i1 - 1 - aP[j]);
-                c = count_below(keys + seg_start[j], tj.new_deg - tj.old_deg, f, arena[tj.old_off + r_last]);
-                const int64_t first = aP[j] > t * COPY_TILE ? aP[j] : t * COPY_TILE;
-                c = c < i1 - first ? c : i1 - first;
-            }
-        }
+        if (aP[j] >= i1) return 0;          // else it holds i1 - 1 too, the tile's last item
+        const TouchInfo tj = ti[j];
+        if (!tj.inplace) return 0;
+        const int64_t r_last = tj.p + (i1 - 1 - aP[j]);
+        const int64_t c = count_below(keys + seg_start[j], tj.new_deg - tj.old_deg, f, arena[tj.old_off + r_last]);
+        const int64_t first = aP[j] > t * COPY_TILE ? aP[j] : t * COPY_TILE;
+        return min(c, i1 - first);
     }
-    tcnt[t] = (uint32_t)c;
-}
+};
 
 struct MoveShared {
     LbShared<COPY_CAP_IPT, int64_t> lb;   // pref = aP[j], base = old_off + p - aP[j]
@@ -879,7 +906,7 @@ void preload_update_code() {
 struct UpdBufs {
     uint64_t* ka;
     uint64_t* kb;
-    uint32_t* pos;       // n+1
+    uint32_t* nkeep;     // entries kept
     uint32_t* spos;      // n+1
     uint32_t* seg_start; // n+1
     uint64_t* seg_key;   // n+1
@@ -916,7 +943,7 @@ static hn_status upd_buffers(hn_graph* g, int64_t n, UpdBufs* b) {
     int64_t o = 0;
     int64_t o_ka = o; o = al(o + n1 * 8);
     int64_t o_kb = o; o = al(o + n1 * 8);
-    int64_t o_pos = o; o = al(o + n1 * 4);
+    int64_t o_nkeep = o; o = al(o + 4);
     int64_t o_spos = o; o = al(o + n1 * 4);
     int64_t o_ss = o; o = al(o + n1 * 4);
     int64_t o_sk = o; o = al(o + n1 * 8);
@@ -951,7 +978,7 @@ static hn_status upd_buffers(hn_graph* g, int64_t n, UpdBufs* b) {
     char* base = g->s_upd.as<char>();
     b->ka = reinterpret_cast<uint64_t*>(base + o_ka);
     b->kb = reinterpret_cast<uint64_t*>(base + o_kb);
-    b->pos = reinterpret_cast<uint32_t*>(base + o_pos);
+    b->nkeep = reinterpret_cast<uint32_t*>(base + o_nkeep);
     b->spos = reinterpret_cast<uint32_t*>(base + o_spos);
     b->seg_start = reinterpret_cast<uint32_t*>(base + o_ss);
     b->seg_key = reinterpret_cast<uint64_t*>(base + o_sk);
@@ -983,6 +1010,29 @@ static hn_status upd_buffers(hn_graph* g, int64_t n, UpdBufs* b) {
     return HN_OK;
 }
 
+template <typename Defer>
+__global__ void defer_kernel(int64_t ntiles, Defer in, uint32_t* __restrict__ tcnt) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < ntiles) tcnt[t] = (uint32_t)in(t);
+}
+
+struct TileCountIn {
+    const uint32_t* c;
+    __device__ __forceinline__ int64_t operator()(int64_t t) const { return (int64_t)c[t]; }
+};
+
+// Deferred counts of the copy tiles and their prefix.  One workgroup's scan counts as
+// it goes; the two readings of a larger one would count twice, sixteen tiles to a
+// lane (500 K tiles of an R-MAT s24 erase: 290 us, 25 with the counts on their own).
+template <typename Defer>
+static hn_status defer_offsets(Defer in, UpdBufs& b, int64_t ntiles, hipStream_t st) {
+    const SideOut out{b.tcnt, b.doff, ntiles - 1, b.sc};
+    if (ntiles <= SCAN_ONE) return exclusive_scan_fn<int64_t>(in, out, b.doff + ntiles, ntiles, b.tmp, st);
+    defer_kernel<<<(unsigned)ceil_div(ntiles, BLOCK), BLOCK, 0, st>>>(ntiles, in, b.tcnt);
+    HN_CHECK_LAUNCH();
+    return exclusive_scan_fn<int64_t>(TileCountIn{b.tcnt}, out, b.doff + ntiles, ntiles, b.tmp, st);
+}
+
 // copy a host or device batch into the key buffer (packed, validated) and sort it
 static hn_status load_and_sort(hn_graph* g, const int32_t* src, const int32_t* dst, int64_t n, uint32_t flags,
                                UpdBufs& b, KeyFmt f, hipStream_t st, uint64_t** sorted) {
@@ -996,13 +1046,23 @@ static hn_status load_and_sort(hn_graph* g, const int32_t* src, const int32_t* d
         ds = staged;
         dd = staged + n;
     }
-    HN_HIP(hipMemsetAsync(b.sc, 0, sizeof(UpdScal), st));
-    pack_batch_kernel<<<(unsigned)ceil_div(n, BLOCK), BLOCK, 0, st>>>(n, ds, dd, g->nv, f.sbits, b.ka, b.ia, b.sc);
-    HN_CHECK_LAUNCH();
+    // a batch that one workgroup sorts is packed (and the status cleared) by the same launch
+    const bool small = n <= sort_small_max(b.ia != nullptr);
+    if (small) {
+        const SortPairs pairs{ds, dd, g->nv, f.sbits, reinterpret_cast<uint32_t*>(b.sc), (int)(sizeof(UpdScal) / 4),
+                              &b.sc->err, ERR_BAD_ID};
+        HN_TRY(radix_sort_small_pairs(pairs, b.ka, b.ia, n, 2 * f.sbits, st));
+    } else {
+        HN_HIP(hipMemsetAsync(b.sc, 0, sizeof(UpdScal), st));
+        pack_batch_kernel<<<(unsigned)ceil_div(n, BLOCK), BLOCK, 0, st>>>(n, ds, dd, g->nv, f.sbits, b.ka, b.ia, b.sc);
+        HN_CHECK_LAUNCH();
+    }
     if (staged) {
         HN_HIP(hipStreamSynchronize(st));
-        dfree(staged);
+        dput(staged);
     }
+    *sorted = b.ka;
+    if (small) return HN_OK;
     uint64_t* keys = b.ka;
     uint64_t* alt = b.kb;
     uint32_t* vals = b.ia;
@@ -1029,10 +1089,6 @@ static hn_status check_scal(hn_graph* g, UpdBufs& b, hipStream_t st, UpdScal* h)
         return HN_E_ARENA_FULL;   // the entry point grows the arena and runs the batch again
     }
     return HN_OK;
-}
-
-__global__ void store_changed_kernel(const uint32_t* __restrict__ total, UpdScal* sc) {
-    if (!sc->err) sc->changed = *total;
 }
 
 // After a batch applied to a symmetric graph: pairs outside the batch kept
@@ -1266,15 +1322,13 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
         n, keys, f, (flags & HN_DEDUP_BATCH) ? 1 : 0, (flags & HN_DEDUP_GRAPH) ? 1 : 0, g->rec, g->arena, b.dpos,
         b.dlen, b.sc);
     HN_CHECK_LAUNCH();
-    HN_TRY(exclusive_scan<uint32_t>(ArrayIn<uint32_t>{b.dpos}, b.pos, n, b.tmp, st));
     uint32_t* ubk = b.dlp;
-    compact_keys_kernel<<<gridn, BLOCK, 0, st>>>(n, keys, b.pos, b.kb, b.ia, b.ib, b.dlen, ubk);
-    HN_CHECK_LAUNCH();
-    uint32_t* nb = b.pos + n;   // entries kept
+    uint32_t* nb = b.nkeep;   // entries kept
+    HN_TRY(exclusive_scan_fn<uint32_t>(ArrayIn<uint32_t>{b.dpos}, CompactOut{keys, b.kb, b.ia, b.ib, b.dlen, ubk}, nb,
+                                       n, b.tmp, st));
     // 2. segments by source
-    HN_TRY(exclusive_scan<uint32_t>(SegStartIn{b.kb, nb, f.sbits}, b.spos, n, b.tmp, st));
-    seg_write_kernel<<<gridn, BLOCK, 0, st>>>(n, b.kb, nb, b.spos, b.seg_start, b.seg_key);
-    HN_CHECK_LAUNCH();
+    HN_TRY(exclusive_scan_fn<uint32_t>(SegStartIn{b.kb, nb, f.sbits}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key},
+                                       b.spos + n, n, b.tmp, st));
     uint32_t* ucnt = b.spos + n;
     // 3. in place or new blocks
     uint32_t* stamp = nullptr;
@@ -1303,11 +1357,7 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
     HN_UNDO_TRY(exclusive_scan_fn<int64_t>(MoveLenIn{b.ti, ucnt, b.sc}, RunOut{b.wpos, b.tile_lo}, b.wpos + n, n,
                                            b.tmp, st));
     const int64_t nt = b.ntile_max;
-    insert_defer_kernel<<<(unsigned)ceil_div(nt, BLOCK), BLOCK, 0, st>>>(nt, n, b.wpos, b.tile_lo, b.ti, b.seg_start,
-                                                                        b.kb, f, g->arena, b.tcnt, b.sc);
-    HN_UNDO_LAUNCH();
-    HN_UNDO_TRY(exclusive_scan_fn<int64_t>(TileCountIn{b.tcnt}, SideOut{b.doff, nt - 1, b.sc}, b.doff + nt, nt,
-                                           b.tmp, st));
+    HN_UNDO_TRY(defer_offsets(InsertDeferIn{n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, g->arena, b.sc}, b, nt, st));
     int64_t ndefer = 0;
     int32_t* side = nullptr;
     int64_t* side_dst = nullptr;
@@ -1327,9 +1377,7 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
 #undef HN_UNDO_LAUNCH
 #undef HN_UNDO_TRY
     // 5. publish
-    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg_key, f, b.ti, nullptr, g->rec, g->alloc_view(), b.sc);
-    HN_CHECK_LAUNCH();
-    store_changed_kernel<<<1, 1, 0, st>>>(nb, b.sc);
+    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg_key, f, b.ti, nullptr, g->rec, g->alloc_view(), nb, b.sc);
     HN_CHECK_LAUNCH();
     const bool was_sym = g->sym == 1;
     if (was_sym) {
@@ -1362,24 +1410,22 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
     HN_TRY(load_and_sort(g, src, dst, n, flags, b, f, st, &keys));
     const unsigned gridn = (unsigned)ceil_div(n + 1, BLOCK);
     // 1. optional in-batch dedup -> kb
-    HN_TRY(exclusive_scan<uint32_t>(FirstKeepIn{keys, (flags & HN_DEDUP_BATCH) ? 1 : 0}, b.pos, n, b.tmp, st));
-    compact_keys_kernel<<<gridn, BLOCK, 0, st>>>(n, keys, b.pos, b.kb, nullptr, nullptr, nullptr, nullptr);
-    HN_CHECK_LAUNCH();
-    uint32_t* nb = b.pos + n;
+    uint32_t* nb = b.nkeep;
+    HN_TRY(exclusive_scan_fn<uint32_t>(FirstKeepIn{keys, (flags & HN_DEDUP_BATCH) ? 1 : 0},
+                                       CompactOut{keys, b.kb, nullptr, nullptr, nullptr, nullptr}, nb, n, b.tmp, st));
     // 2. distinct keys with multiplicities
-    HN_TRY(exclusive_scan<uint32_t>(SegStartIn{b.kb, nb, 64}, b.spos, n, b.tmp, st));
-    seg_write_kernel<<<gridn, BLOCK, 0, st>>>(n, b.kb, nb, b.spos, b.seg_start, b.seg_key);
-    HN_CHECK_LAUNCH();
+    HN_TRY(exclusive_scan_fn<uint32_t>(SegStartIn{b.kb, nb, 64}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key},
+                                       b.spos + n, n, b.tmp, st));
     uint32_t* dcnt = b.spos + n;
     // 3. stored ranges and deletion counts per distinct key
     erase_locate_kernel<<<gridn, BLOCK, 0, st>>>(dcnt, b.seg_start, b.seg_key, f, g->rec, g->arena, b.dpos, b.dlen,
                                                  b.live, b.sc);
     HN_CHECK_LAUNCH();
-    HN_TRY(exclusive_scan<uint32_t>(DLenIn{b.dlen, dcnt}, b.dlp, n, b.tmp, st));
-    // 4. group the distinct keys by source
-    HN_TRY(exclusive_scan<uint32_t>(SegStartIn{b.seg_key, dcnt, f.sbits}, b.tpos, n, b.tmp, st));
-    seg_write_kernel<<<gridn, BLOCK, 0, st>>>(n, b.seg_key, dcnt, b.tpos, b.seg2_start, b.seg2_key);
-    HN_CHECK_LAUNCH();
+    // 4. deletions before each distinct key, and the keys grouped by source: both
+    // counts in one scan
+    HN_TRY(exclusive_scan_fn<uint64_t>(DelGroupIn{DLenIn{b.dlen, dcnt}, SegStartIn{b.seg_key, dcnt, f.sbits}},
+                                       DelGroupOut{SegOut{b.seg_key, dcnt, b.tpos, b.seg2_start, b.seg2_key}, b.dlp, n},
+                                       reinterpret_cast<uint64_t*>(b.wpos), n, b.tmp, st));
     uint32_t* ucnt = b.tpos + n;
     // 5. in place, smaller block, or no block
     uint32_t* stamp = nullptr;
@@ -1411,11 +1457,7 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
     // 7. in-place compaction in one pass; the few entries that would overwrite
     // a source of an earlier tile go through a side buffer
     const int64_t nt = b.ntile_max;
-    erase_defer_kernel<<<(unsigned)ceil_div(nt, BLOCK), BLOCK, 0, st>>>(nt, 2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst,
-                                                                       b.rtail, b.tcnt, b.sc);
-    HN_UNDO_LAUNCH();
-    HN_UNDO_TRY(exclusive_scan_fn<int64_t>(TileCountIn{b.tcnt}, SideOut{b.doff, nt - 1, b.sc}, b.doff + nt, nt,
-                                           b.tmp, st));
+    HN_UNDO_TRY(defer_offsets(EraseDeferIn{2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.rtail, b.sc}, b, nt, st));
     int64_t ndefer = 0;
     int32_t* side = nullptr;
     int64_t* side_dst = nullptr;
@@ -1438,9 +1480,7 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
 #undef HN_UNDO_LAUNCH
 #undef HN_UNDO_TRY
     // 8. publish
-    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg2_key, f, b.ti, b.skip, g->rec, g->alloc_view(), b.sc);
-    HN_CHECK_LAUNCH();
-    store_changed_kernel<<<1, 1, 0, st>>>(b.dlp + n, b.sc);
+    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg2_key, f, b.ti, b.skip, g->rec, g->alloc_view(), b.dlp + n, b.sc);
     HN_CHECK_LAUNCH();
     const bool was_sym = g->sym == 1;
     if (was_sym) {

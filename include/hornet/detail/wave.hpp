@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace hn {
 
 constexpr int WAVE = 64;          // CDNA wavefront width
@@ -115,16 +117,23 @@ __device__ __forceinline__ int64_t upper_bound_m1(const P* a, int64_t lo, int64_
 }
 
 // ------------------------------------------------------------------ scan
-constexpr int SCAN_IPT = 16;                   // values per lane per tile
+// Values per lane per tile.  Up to SCAN_FINE values a scan takes tiles a quarter as
+// large: with few tiles it is one lane's chain, above all where the output functor
+// loads and stores (batch keys compacted: 200 K 18 us with 16, 7 with 4; 2 M 24 and
+// 17).  Beyond, the sums that each tile makes of the totals before it would grow.
+constexpr int SCAN_IPT = 16, SCAN_FINE_IPT = 4;
 constexpr int SCAN_TILE = BLOCK * SCAN_IPT;    // 4096
-constexpr int SCAN_WAVE_CHUNK = WAVE * SCAN_IPT;
 
 // up to this many tiles a down-sweep tile sums the totals before it itself
 // (at most SCAN_SELF_TILES loads each) instead of a separate partials launch
 constexpr int64_t SCAN_SELF_TILES = 1024;
 
+constexpr int64_t SCAN_FINE = 4 * SCAN_SELF_TILES * BLOCK * SCAN_FINE_IPT;   // 4 M
+
 inline size_t scan_temp_bytes(int64_t n) {
-    int64_t tiles = ceil_div(n > 0 ? n : 1, SCAN_TILE);
+    // (of any smaller count too)
+    int64_t tiles = std::max(ceil_div(std::min(n > 0 ? n : 1, SCAN_FINE), BLOCK * SCAN_FINE_IPT),
+                             ceil_div(n > 0 ? n : 1, SCAN_TILE));
     return (size_t)(tiles + 1) * 8 + 256;
 }
 
@@ -141,15 +150,15 @@ struct DevCount {
     __device__ __forceinline__ int64_t get() const { return (int64_t)*p; }
 };
 
-template <typename Out, typename InFn, typename Cnt>
+template <typename Out, int IPT, typename InFn, typename Cnt>
 __global__ __launch_bounds__(BLOCK) void scan_reduce_kernel(InFn in, Cnt cnt, Out* __restrict__ partial) {
     __shared__ Out lds[NWAVES];
     const int64_t n = cnt.get();
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
+    const int64_t base = (int64_t)blockIdx.x * (BLOCK * IPT);
     if (base >= n && blockIdx.x > 0) return;
     Out acc = 0;
 #pragma unroll
-    for (int j = 0; j < SCAN_IPT; j++) {
+    for (int j = 0; j < IPT; j++) {
         int64_t i = base + (int64_t)j * BLOCK + threadIdx.x;
         if (i < n) acc += (Out)in(i);
     }
@@ -186,16 +195,17 @@ __global__ __launch_bounds__(BLOCK) void scan_partials_kernel(Out* __restrict__ 
 // SELF the tile adds up the totals of the tiles before it itself (used when
 // there are few tiles, saving the partials launch), and the last tile writes
 // the grand total.
-template <typename Out, typename InFn, typename OutFn, typename Cnt, bool SELF = false>
+template <typename Out, int IPT, typename InFn, typename OutFn, typename Cnt, bool SELF = false>
 __global__ __launch_bounds__(BLOCK) void scan_down_fn_kernel(InFn in, Cnt cnt, const Out* __restrict__ partial,
                                                              OutFn out, Out* __restrict__ total = nullptr) {
+    constexpr int TILE = BLOCK * IPT;
     __shared__ Out wtot[NWAVES];
     const int64_t n = cnt.get();
     const int w = threadIdx.x / WAVE;
     const int l = __lane_id();
     Out toff = 0;   // prefix of the tile totals before this tile
     if constexpr (SELF) {
-        const int64_t last = n > 0 ? (n - 1) / SCAN_TILE : 0;
+        const int64_t last = n > 0 ? (n - 1) / TILE : 0;
         if ((int64_t)blockIdx.x > last) return;
         Out s = 0;
         for (int64_t k = threadIdx.x; k < (int64_t)blockIdx.x; k += BLOCK) s += partial[k];
@@ -208,14 +218,14 @@ __global__ __launch_bounds__(BLOCK) void scan_down_fn_kernel(InFn in, Cnt cnt, c
         __syncthreads();   // wtot is reused below
         if (n <= 0) return;
     } else {
-        if ((int64_t)blockIdx.x * SCAN_TILE >= n) return;
+        if ((int64_t)blockIdx.x * TILE >= n) return;
     }
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)w * SCAN_WAVE_CHUNK;
-    Out pre[SCAN_IPT];
-    Out val[SCAN_IPT];
+    const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)w * (WAVE * IPT);
+    Out pre[IPT];
+    Out val[IPT];
     Out carry = 0;
 #pragma unroll
-    for (int j = 0; j < SCAN_IPT; j++) {
+    for (int j = 0; j < IPT; j++) {
         int64_t i = base + (int64_t)j * WAVE + l;
         Out v = i < n ? (Out)in(i) : (Out)0;
         Out inc = wave_inclusive_scan(v);
@@ -228,7 +238,7 @@ __global__ __launch_bounds__(BLOCK) void scan_down_fn_kernel(InFn in, Cnt cnt, c
     Out off = SELF ? toff : partial[blockIdx.x];
     for (int k = 0; k < w; k++) off += wtot[k];
 #pragma unroll
-    for (int j = 0; j < SCAN_IPT; j++) {
+    for (int j = 0; j < IPT; j++) {
         int64_t i = base + (int64_t)j * WAVE + l;
         if (i < n) out(i, (Out)(off + pre[j]), val[j]);
     }
@@ -297,6 +307,29 @@ struct ArrayIn {
     __device__ __forceinline__ T operator()(int64_t i) const { return a[i]; }
 };
 
+// the launches of a scan of up to max_n > 0 values
+template <typename Out, typename InFn, typename OutFn, typename Cnt>
+hipError_t scan_tiles(InFn in, Cnt cnt, OutFn out, Out* total, int64_t max_n, void* tmp, hipStream_t st) {
+    Out* partial = reinterpret_cast<Out*>(tmp);
+    if (max_n <= SCAN_FINE) {
+        const unsigned tiles = (unsigned)ceil_div(max_n, BLOCK * SCAN_FINE_IPT);
+        scan_reduce_kernel<Out, SCAN_FINE_IPT, InFn, Cnt><<<tiles, BLOCK, 0, st>>>(in, cnt, partial);
+        scan_down_fn_kernel<Out, SCAN_FINE_IPT, InFn, OutFn, Cnt, true><<<tiles, BLOCK, 0, st>>>(in, cnt, partial, out,
+                                                                                                 total);
+        return hipGetLastError();
+    }
+    const int64_t tiles = ceil_div(max_n, SCAN_TILE);
+    scan_reduce_kernel<Out, SCAN_IPT, InFn, Cnt><<<(unsigned)tiles, BLOCK, 0, st>>>(in, cnt, partial);
+    if (tiles <= SCAN_SELF_TILES) {
+        scan_down_fn_kernel<Out, SCAN_IPT, InFn, OutFn, Cnt, true><<<(unsigned)tiles, BLOCK, 0, st>>>(in, cnt, partial,
+                                                                                                      out, total);
+        return hipGetLastError();
+    }
+    scan_partials_kernel<Out, Cnt><<<1, BLOCK, 0, st>>>(partial, cnt, total);
+    scan_down_fn_kernel<Out, SCAN_IPT, InFn, OutFn, Cnt><<<(unsigned)tiles, BLOCK, 0, st>>>(in, cnt, partial, out);
+    return hipGetLastError();
+}
+
 // Exclusive scan of in(0..n) delivered to out(i, prefix, value); *total = sum.
 // tmp: scan_temp_bytes(n) bytes of device memory.
 template <typename Out, typename InFn, typename OutFn>
@@ -309,18 +342,7 @@ hipError_t exclusive_scan_dev(InFn in, OutFn out, Out* total, int64_t n, void* t
         scan_one_kernel<Out, InFn, OutFn, HostCount><<<1, SCAN_ONE_BLOCK, 0, st>>>(in, HostCount{n}, out, total);
         return hipGetLastError();
     }
-    int64_t tiles = ceil_div(n, SCAN_TILE);
-    Out* partial = reinterpret_cast<Out*>(tmp);
-    scan_reduce_kernel<Out, InFn, HostCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, HostCount{n}, partial);
-    if (tiles <= SCAN_SELF_TILES) {
-        scan_down_fn_kernel<Out, InFn, OutFn, HostCount, true><<<(unsigned)tiles, BLOCK, 0, st>>>(
-            in, HostCount{n}, partial, out, total);
-        return hipGetLastError();
-    }
-    scan_partials_kernel<Out, HostCount><<<1, BLOCK, 0, st>>>(partial, HostCount{n}, total);
-    scan_down_fn_kernel<Out, InFn, OutFn, HostCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, HostCount{n}, partial,
-                                                                                        out);
-    return hipGetLastError();
+    return scan_tiles<Out>(in, HostCount{n}, out, total, n, tmp, st);
 }
 
 // Same, with the count read on the device (*n_dev <= max_n); a zero count
@@ -332,18 +354,7 @@ hipError_t exclusive_scan_dev_count(InFn in, OutFn out, Out* total, const uint32
         scan_one_kernel<Out, InFn, OutFn, DevCount><<<1, SCAN_ONE_BLOCK, 0, st>>>(in, DevCount{n_dev}, out, total);
         return hipGetLastError();
     }
-    const int64_t tiles = ceil_div(max_n > 0 ? max_n : 1, SCAN_TILE);
-    Out* partial = reinterpret_cast<Out*>(tmp);
-    scan_reduce_kernel<Out, InFn, DevCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, DevCount{n_dev}, partial);
-    if (tiles <= SCAN_SELF_TILES) {
-        scan_down_fn_kernel<Out, InFn, OutFn, DevCount, true><<<(unsigned)tiles, BLOCK, 0, st>>>(
-            in, DevCount{n_dev}, partial, out, total);
-        return hipGetLastError();
-    }
-    scan_partials_kernel<Out, DevCount><<<1, BLOCK, 0, st>>>(partial, DevCount{n_dev}, total);
-    scan_down_fn_kernel<Out, InFn, OutFn, DevCount><<<(unsigned)tiles, BLOCK, 0, st>>>(in, DevCount{n_dev}, partial,
-                                                                                       out);
-    return hipGetLastError();
+    return scan_tiles<Out>(in, DevCount{n_dev}, out, total, max_n, tmp, st);
 }
 
 // ------------------------------------------------------------ load balancing
