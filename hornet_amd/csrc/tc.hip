@@ -162,8 +162,9 @@ __global__ void tc_weight_deg_kernel(int64_t nv, const hn_vrec* __restrict__ rec
 // ids.  One launch in place of six (weights, histogram, cut and codes), 110 us of
 // the 590 that a stored graph of 6 K vertices and 100 K entries took.
 __global__ void tc_all_hubs_kernel(int64_t nv, const hn_vrec* __restrict__ rec, uint2* __restrict__ wc,
-                                   uint32_t* __restrict__ hub) {
+                                   uint32_t* __restrict__ hub, TcCtl* __restrict__ ctl) {
     const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v == 0) ctl->hubs = (uint32_t)nv;
     if (v >= nv) return;
     wc[v] = make_uint2((uint32_t)rec[v].deg, (uint32_t)v);
     hub[v] = (uint32_t)v;
@@ -238,7 +239,9 @@ __device__ __forceinline__ TcLoc tc_locate(const uint32_t* __restrict__ P, int64
 }
 
 // How often a vertex is an entry, from every `step`-th tile of the stored rows
-// (any choice of hubs gives the same counts).
+// (any choice of hubs gives the same counts).  Bound by the atomics on the most
+// frequent one, 10 ns each: a quarter of a million to a million entries are looked
+// at (all 2.8 M of an R-MAT s18 orientation took 660 us, 73 so).
 __global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
                                                                const uint32_t* __restrict__ P,
                                                                const uint32_t* __restrict__ tile_lo,
@@ -364,6 +367,8 @@ __device__ __forceinline__ uint32_t tc_entry(const TcRow& r, uint32_t i, const u
 // ---- edges whose longer list is the destination's, grouped by it (where an
 // owner's edges cannot be read from its stored row), over the same partition
 // FILL = false: the edge's place in its group (TC_PAD: not grouped); FILL = true: the sources at their places
+// A hub's group is counted in TC_LANES parts (by workgroup, the same in both passes),
+// as atomics on one counter take 10 ns each: R-MAT s18 oriented, 319 us in one part, 118 so.
 template <bool FILL>
 __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
                                                          const uint32_t* __restrict__ P,
@@ -372,9 +377,11 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
                                                          const uint16_t* __restrict__ codes,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, uint32_t* __restrict__ gcnt,
+                                                         uint32_t* __restrict__ part, int64_t nhub,
                                                          uint32_t* __restrict__ place, const uint32_t* __restrict__ goff,
                                                          uint32_t* __restrict__ members) {
     if (sym && !ctl->repeats) return;
+    uint32_t* const mine = part + (blockIdx.x % TC_LANES) * nhub;
     __shared__ TcLb sh;
     const uint32_t total = *ngroups;
     const int64_t ntiles = ((int64_t)total + TC_TILE - 1) / TC_TILE;
@@ -390,18 +397,36 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
             if (lu < 2) continue;
             // entries [8k, 8k + 8) of the list, which may end before its stored row
             for (uint32_t i = c.k[j] * TC_G; i < min(lu, (c.k[j] + 1) * TC_G); i++) {
-                const uint32_t v = tc_entry(r, i, codes, ids, hub);
+                const bool is_hub = i < r.n16;
+                const uint32_t q = is_hub ? codes[(int64_t)r.base * TC_G + i] : 0u;
+                const uint32_t v = is_hub ? hub[q] : ids[(int64_t)r.base * TC_G + (i - r.n16)];
                 uint32_t* pl = place + (int64_t)r.base * TC_G + i;
                 if constexpr (FILL) {
-                    if (*pl != TC_PAD) members[(int64_t)goff[v] + *pl] = u;
+                    if (*pl != TC_PAD) members[(int64_t)goff[v] + (is_hub ? mine[q] : 0u) + *pl] = u;
                 } else {
                     const uint32_t lv = row[v].len();
-                    *pl = lv > lu && lv > TC_SMALL && v != u ? atomicAdd(gcnt + v, 1u) : TC_PAD;
+                    *pl = lv > lu && lv > TC_SMALL && v != u ? atomicAdd(is_hub ? mine + q : gcnt + v, 1u) : TC_PAD;
                 }
             }
         }
         __syncthreads();
     }
+}
+
+// a hub's parts: their starts within its group, and the group's size
+__global__ __launch_bounds__(BLOCK) void tc_parts_kernel(int sym, const TcCtl* __restrict__ ctl, int64_t nhub,
+                                                         const uint32_t* __restrict__ hub, uint32_t* __restrict__ part,
+                                                         uint32_t* __restrict__ gcnt) {
+    if (sym && !ctl->repeats) return;
+    const int64_t q = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (q >= nhub || q >= (int64_t)ctl->hubs) return;
+    uint32_t at = 0;
+    for (int p = 0; p < TC_LANES; p++) {
+        const uint32_t c = part[p * nhub + q];
+        part[p * nhub + q] = at;
+        at += c;
+    }
+    gcnt[hub[q]] = at;
 }
 
 // ---- tasks: up to TC_CAND candidates of one owner
@@ -777,7 +802,8 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
         return at;
     };
     const int64_t o_ctl = take(sizeof(TcCtl)), o_hist = take(TC_BINS * 4);
-    const int64_t o_gcnt = take(nv * 4), o_zero_end = o;   // cleared together
+    const int64_t nhub = std::min<int64_t>(nv, TC_HUBS + 1);
+    const int64_t o_gcnt = take(nv * 4), o_part = take(nhub * TC_LANES * 4), o_zero_end = o;   // cleared together
     const int64_t o_weight = take(nv * 4), o_wc = take(nv * 8), o_hub = take((int64_t)(TC_HUBS + 1) * 4);
     const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4);
     const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
@@ -789,6 +815,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     TcCtl* ctl = at(o_ctl, (TcCtl*)nullptr);
     uint32_t* hist = at(o_hist, (uint32_t*)nullptr);
     uint32_t* gcnt = at(o_gcnt, (uint32_t*)nullptr);
+    uint32_t* part = at(o_part, (uint32_t*)nullptr);
     uint32_t* weight = at(o_weight, (uint32_t*)nullptr);
     uint2* wc = at(o_wc, (uint2*)nullptr);
     uint32_t* hub = at(o_hub, (uint32_t*)nullptr);
@@ -811,14 +838,14 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     // 1. hubs and codes
     HN_TRY(exclusive_scan_fn<uint32_t>(StoredGroupsIn{g->rec}, StoredGroupsOut{row, P, tile_lo}, P + nv, nv, tmp, st));
     if (nv <= (int64_t)TC_HUBS) {
-        tc_all_hubs_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, wc, hub);
+        tc_all_hubs_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, wc, hub, ctl);
         HN_CHECK_LAUNCH();
     } else {
         if (orient) {
             tc_weight_deg_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, weight);
         } else {
             HN_HIP(hipMemsetAsync(weight, 0, (size_t)nv * 4, st));
-            const int step = ne >= ((int64_t)1 << 22) ? 16 : 1;
+            const int step = (int)std::clamp<int64_t>(ne >> 18, 1, 64);
             tc_weight_freq_kernel<<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, step, weight);
         }
         HN_CHECK_LAUNCH();
@@ -837,10 +864,14 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     tc_pad_kernel<<<gv, BLOCK, 0, st>>>(nv, row, codes, ids);
     HN_CHECK_LAUNCH();
     // 3. edges owned by their destination
-    tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, place, nullptr, nullptr);
+    tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, part, nhub,
+                                                 place, nullptr, nullptr);
+    HN_CHECK_LAUNCH();
+    tc_parts_kernel<<<(unsigned)ceil_div(nhub, BLOCK), BLOCK, 0, st>>>(sym, ctl, nhub, hub, part, gcnt);
     HN_CHECK_LAUNCH();
     HN_TRY(exclusive_scan<uint32_t>(ArrayIn<uint32_t>{gcnt}, goff, nv, tmp, st));
-    tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, place, goff, members);
+    tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, part, nhub,
+                                                place, goff, members);
     HN_CHECK_LAUNCH();
     // 4. counts
     HN_TRY(exclusive_scan_fn<uint32_t>(TaskIn{row, gcnt, g->rec, ctl, sym}, TaskOut{task}, &ctl->ntask, nv, tmp, st));
