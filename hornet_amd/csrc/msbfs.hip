@@ -13,8 +13,7 @@
 //   list     a scan of per-word popcounts of the frontier (push) or
 //            light-open (pull) bitset and an emit kernel turn the bitset
 //            into a compact work list carrying (vertex, degree, adjacency
-//            offset, mask) -- writes transposed so lanes write consecutive
-//            entries;
+//            offset, mask);
 //   scan     a scan of the list's 16-byte adjacency groups whose element
 //            count is read on the device (so it stays inside the graph),
 //            writing the group prefix and the tile partition;
@@ -340,9 +339,10 @@ __global__ __launch_bounds__(BLOCK) void ms_head_kernel(int64_t nv, const MsStat
     }
 }
 
-// bitset -> work list (vertex, degree, offset, mask); lane per bitset word,
-// writes transposed so that consecutive lanes write consecutive entries
-__global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t words, const MsState* S,
+// bitset -> work list (vertex, degree, offset, mask), a lane per vertex: the lanes of
+// a wave write consecutive entries.  (A lane per word, its vertices in turn, was a
+// chain of 32 loads: 19 us on a graph of 4 K vertices, 3 so.)
+__global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t nv, const MsState* S,
                                                         const uint32_t* __restrict__ fbits,
                                                         const uint32_t* __restrict__ obits,
                                                         const uint32_t* __restrict__ wpre,
@@ -358,32 +358,20 @@ __global__ __launch_bounds__(BLOCK) void ms_emit_kernel(int64_t words, const MsS
     const bool push = S->mode == 0;
     const uint32_t nc = *nchg;
     const uint64_t live = S->live;
-    const int64_t wi = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const uint32_t found = wi < words ? (push ? fbits[wi] : obits[wi]) : 0u;
-    if (__ballot(found != 0) == 0) return;
-    const uint32_t b = wi < words ? wpre[wi] : 0u;
-    const int lane = __lane_id();
-    const int64_t wbase = wi - lane;
-    const int bit = lane & 31;
-    const uint32_t below = (1u << bit) - 1u;
-    for (int r = 0; r < WAVE / 2; r++) {
-        const int owner = 2 * r + (lane >> 5);
-        const uint32_t fw = __shfl(found, owner, WAVE);
-        if (__ballot(fw != 0) == 0) continue;
-        const uint32_t bo = __shfl(b, owner, WAVE);
-        if ((fw >> bit) & 1u) {
-            const int32_t v = (int32_t)((wbase + owner) * 32 + bit);
-            const uint32_t pos = bo + (uint32_t)__popc(fw & below);
-            const hn_vrec rv = rec[v];
-            // pull: what the first entries (ms_head_kernel) have left
-            const uint64_t m = push ? frontier[v] : (live & ~visited[v] & ~next[v]);
-            const int32_t skip = push || (nc && dirty[v]) ? 0 : MS_HEAD;
-            list[pos] = v;
-            qdeg[pos] = m ? rv.deg - skip : 0;
-            qoff[pos] = rv.off + skip;
-            qmask[pos] = m;
-        }
-    }
+    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= nv) return;
+    const uint32_t word = push ? fbits[v >> 5] : obits[v >> 5];
+    const int bit = (int)(v & 31);
+    if (!((word >> bit) & 1u)) return;
+    const uint32_t pos = wpre[v >> 5] + (uint32_t)__popc(word & ((1u << bit) - 1u));
+    const hn_vrec rv = rec[v];
+    // pull: what the first entries (ms_head_kernel) have left
+    const uint64_t m = push ? frontier[v] : (live & ~visited[v] & ~next[v]);
+    const int32_t skip = push || (nc && dirty[v]) ? 0 : MS_HEAD;
+    list[pos] = (int32_t)v;
+    qdeg[pos] = m ? rv.deg - skip : 0;
+    qoff[pos] = rv.off + skip;
+    qmask[pos] = m;
 }
 
 struct GroupIn {
@@ -1302,7 +1290,7 @@ static hipError_t ms_level(MsEngine* e, const MsParams& P, bool side, hipStream_
     hipError_t err = exclusive_scan_dev(ListWordIn{e->S, e->fbits, e->obits}, ArrayOut<uint32_t>{e->wpre}, &e->S->wn,
                                         words, e->scan_tmp, st);
     if (err != hipSuccess) return err;
-    ms_emit_kernel<<<(unsigned)ceil_div(words, BLOCK), BLOCK, 0, st>>>(words, e->S, e->fbits, e->obits, e->wpre,
+    ms_emit_kernel<<<(unsigned)ceil_div(nv, BLOCK), BLOCK, 0, st>>>(nv, e->S, e->fbits, e->obits, e->wpre,
                                                                        g->rec, e->visited, e->frontier, e->dirty,
                                                                        e->d_nchg, e->next, e->list, e->qdeg, e->qoff,
                                                                        e->qmask);
