@@ -251,9 +251,13 @@ constexpr int COPY_TILE = BLOCK * COPY_IPT;
 // reads for four of them, where a search per item took eleven dependent ones each.
 // A lane holds four consecutive items and moves them at once if they lie in one
 // segment (element-aligned 16-byte accesses: neither side of a row is aligned).
-// Export of 520 M entries of an R-MAT s24 graph: 2.09 ms with searches, 1.26 so
-// (3.5 TB/s); both sides are read and written once, past the caches (1.30 through them).
+// Export of 520 M entries of an R-MAT s24 graph: 2.09 ms with searches, 1.05 so
+// (4.2 TB/s); both sides are read and written once, past the caches (3 % slower through
+// them).
 constexpr int COPY_LANE = 4;
+// Workgroups per CU.  Six run at once; with eight the last two ran on their own (1.27
+// ms instead of 1.05; six: 1.07, twelve: 1.11).
+constexpr int COPY_GRID = 64;
 constexpr int64_t COPY_SPAN = 4 * COPY_TILE;   // segments staged at most (empty ones included): searched otherwise
 typedef int32_t Quad __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -996,7 +1000,7 @@ hn_status graph_from_device_csr(int32_t nv, int64_t ne, const int64_t* d_off, co
         const int64_t tiles = ceil_div(ne, COPY_TILE);
         if ((s = dalloc(&tile_lo, (size_t)tiles)) != HN_OK) { dfree(uoff); return fail(s); }
         tile_starts_kernel<<<(unsigned)ceil_div(tiles, BLOCK), BLOCK, 0, st>>>(tiles, d_off, nv, tile_lo);
-        const int64_t grid = std::min<int64_t>(tiles, (int64_t)num_cus() * 8);
+        const int64_t grid = std::min<int64_t>(tiles, (int64_t)num_cus() * COPY_GRID);
         copy_in_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(nv, ne, d_off, tile_lo, d_adj, g->rec, g->arena, g->meta,
                                                          d_meta);
     }
@@ -1335,7 +1339,7 @@ static hn_status flatten(hn_graph* g, int32_t* src, int32_t* dst, int64_t* eoff_
     HN_TRY(g->s_scan.reserve(scan_temp_bytes(g->nv)));
     HN_TRY(exclusive_scan_fn<int64_t>(DegIn{g->rec}, DegOut{eoff, tile_lo}, eoff + g->nv, g->nv, g->s_scan.ptr, st));
     if (g->ne > 0) {
-        int64_t grid = std::min<int64_t>(tiles, (int64_t)num_cus() * 8);
+        const int64_t grid = std::min<int64_t>(tiles, (int64_t)num_cus() * COPY_GRID);
         flatten_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(g->nv, g->ne, eoff, tile_lo, g->rec, g->arena, src, dst,
                                                          out, g->meta);
         HN_CHECK_LAUNCH();

@@ -54,7 +54,10 @@ constexpr int COPY_CAP_IPT = 1;
 // fastest at 4 (0.97 ms, 1.04 at 8).
 constexpr int ERASE_IPT = 8;
 constexpr int ERASE_TILE = BLOCK * ERASE_IPT;
-constexpr int COPY_GRID_PER_CU = 8;
+// the copies' workgroups per CU: more than run at once (8, or 4 with fields), so that the
+// last ones even out (a million pairs on R-MAT s24: insert 151 us with 8, 117 with 32;
+// erase 199 and 148; 64 the same)
+constexpr int COPY_GRID_PER_CU = 32;
 
 // bits per endpoint of a packed (src, dst) key: ids are below nv, and no key
 // needs a sentinel, so 2^24 vertices pack into 48 bits (6 radix passes)
