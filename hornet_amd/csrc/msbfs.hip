@@ -8,7 +8,7 @@
 //
 // One level step, captured once into a hipGraph and replayed until the
 // frontiers empty (the host reads the state every few levels):
-//   head     pull only: the first eight entries of every open vertex, a lane per
+//   head     pull only: the first four entries of every open vertex, a lane per
 //            vertex; most need no more;
 //   list     a scan of per-word popcounts of the frontier (push) or
 //            light-open (pull) bitset and an emit kernel turn the bitset
@@ -64,9 +64,10 @@ constexpr int MS_IPT_MIN = 2;                    // buffers are sized for the mo
 constexpr int MS_IPTS[] = {2, 4, 6};
 constexpr int MS_COLLECT_PER_CU = 8;             // collect workgroups per CU
 // Entries of an open vertex's row that a pull looks at first, a lane per vertex.
-// Rows ascend, and the hubs of the usual graphs have small ids: on R-MAT s22 most
-// vertices have every bit that is still to be found after eight of their entries.
-constexpr int MS_HEAD = 8;
+// Rows ascend, and the hubs of the usual graphs have small ids: from the fourth level of
+// an R-MAT s22 batch on, nearly all that is still to be found is (64 sources, whole
+// batch: 2,727 us with 4 entries, 2,890 with 8, 3,080 with 16).
+constexpr int MS_HEAD = 4;
 constexpr int MS_PLANES = 4;                     // bit planes of the level codes
 constexpr int MS_DIRECT = (1 << MS_PLANES) - 1;  // from this level on distances are written as they are found
 // Sources from which on the planes pay: they cost 72 bytes per vertex reached, level
@@ -283,7 +284,7 @@ struct ListWordIn {
 // pull: the first MS_HEAD entries of every light-open vertex, a lane per vertex.  It
 // stays on the list if it has more entries and misses a bit still, so that the lists
 // and tiles of the edge-granular pull hold only those (R-MAT s22, 64 sources: pulls, lists
-// and scans of a batch 2,720 us without, 2,420 with).  Bound by the rows' and masks'
+// and scans of a batch 2,720 us without, 2,450 with eight entries).  Bound by the rows' and masks'
 // scattered sectors.  Vertices with changed pairs in a window stay as they are.
 __global__ __launch_bounds__(BLOCK) void ms_head_kernel(int64_t nv, const MsState* S, uint32_t* __restrict__ obits,
                                                         const hn_vrec* __restrict__ rec,

@@ -38,7 +38,7 @@ def test_paths(hn, n, k):
         assert np.array_equal(ms.run(srcs).cpu().numpy(), expected(off, adj, srcs))
 
 
-@pytest.mark.parametrize("deg", [1, 4, 7, 8, 9, 12, 33])
+@pytest.mark.parametrize("deg", [1, 3, 4, 5, 7, 8, 9, 12, 33])
 @pytest.mark.parametrize("alpha", [1, 1 << 20])
 def test_row_lengths(hn, deg, alpha):
     print("case msbfs rows", deg, alpha, flush=True)
