@@ -138,8 +138,9 @@ static void worker_loop(hn_server* s, ServeSlot* slot) {
         }
         // Up to SERVE_SINGLE_MAX BFS or 2-hop queries run the single-source
         // TopDown one after the other over the slot's own buffers (a 2-hop
-        // query stops after two levels; 6.2 ms per BFS on R-MAT s25 against
-        // 12.6 ms for a batched launch of one or two sources), each finishing
+        // query stops after two levels; 0.7 ms per BFS on R-MAT s24 against
+        // 3.7 ms for a batched launch of two sources, 0.15 against 0.5 on s20),
+        // each finishing
         // when its own traversal does; a window's queries need the batched
         // engine's version masks.
         BfsBufs bb;

@@ -93,7 +93,7 @@ typedef struct hn_bfs_stats {
     int64_t visited;         /* reached vertices, source included             */
     int64_t edges_scanned;   /* sum of degrees of reached vertices (m_C)      */
     int64_t expand_ns;       /* out: summed expansion-kernel time (HIP events) */
-    int32_t expand_launches; /* out: expansion-kernel launches                */
+    int32_t expand_launches; /* out: levels                                   */
     int32_t pad_;
 } hn_bfs_stats;
 
@@ -233,8 +233,9 @@ hn_status hn_graph_update_stats(hn_graph* g, hn_update_stats* out, void* stream)
 /* --------------------------------------------------------- algorithms */
 /* BfsTopDown{set_parameters(source); run()} --
  * hornetsnest/src/Static/BreadthFirstSearch/TopDown.cu:88-106.
- * dist: device int32[nv]; source gets 0, unreached INT32_MAX.  Level loop on
- * the host with one 4-byte readback per level.  stats may be NULL. */
+ * dist: device int32[nv]; source gets 0, unreached INT32_MAX.  The host queues
+ * as many rounds as the last traversal took before it reads the state back;
+ * on return the distances are complete.  stats may be NULL. */
 hn_status hn_bfs_topdown(hn_graph* g, int32_t source, int32_t* dist, hn_bfs_stats* stats,
                          void* stream);
 /* hn_bfs_topdown without any device allocation.  No counterpart in the
