@@ -93,7 +93,8 @@ inline int ceil_log2_host(int64_t x) {
 }
 
 // Stable LSD radix sort of 64-bit keys over bits [0, key_bits).  The result
-// ends in *keys (the two buffers may be swapped).  tmp from sort_temp_bytes().
+// ends in *keys (the two buffers may be swapped).  tmp from sort_temp_bytes() of as
+// many keys or more.
 size_t sort_temp_bytes(int64_t n);
 hn_status radix_sort_u64(uint64_t** keys, uint64_t** alt, int64_t n, int key_bits, void* tmp,
                          hipStream_t st);

@@ -10,6 +10,7 @@
 // come out as per-bucket runs.
 #include "prims.hpp"
 
+#include <algorithm>
 #include <utility>
 
 namespace hn {
@@ -331,12 +332,19 @@ void preload_prims_code() {
 // keys, per pass: 10.6 us with 1,024, 12.5 with 2,048, 16.5 with 4,096; 2 M keys:
 // 27, 24 and 26); many where they are many, as runs are then longer and there are
 // fewer counts (67 M keys: 690, 484 and 393; 8,192 in workgroups of 512 lanes: 403).
-static int64_t rs_tile_keys(int64_t n) {
-    return n < ((int64_t)1 << 20) ? 256 * 4 : n < ((int64_t)1 << 23) ? 256 * 8 : 256 * 16;
+constexpr int64_t RS_FINE = (int64_t)1 << 20, RS_MIDDLE = (int64_t)1 << 23;
+static int64_t rs_tile_keys(int64_t n) { return n < RS_FINE ? 256 * 4 : n < RS_MIDDLE ? 256 * 8 : 256 * 16; }
+
+// tiles of the largest sort of up to n keys (fewer keys may take more of them)
+static int64_t rs_max_tiles(int64_t n) {
+    int64_t t = ceil_div(n, rs_tile_keys(n));
+    for (const int64_t edge : {RS_FINE - 1, RS_MIDDLE - 1})
+        if (n > edge) t = std::max(t, ceil_div(edge, rs_tile_keys(edge)));
+    return t;
 }
 
 size_t sort_temp_bytes(int64_t n) {
-    const int64_t hn_ = ceil_div(n > 0 ? n : 1, rs_tile_keys(n)) * RS_BUCKETS;
+    const int64_t hn_ = rs_max_tiles(n > 0 ? n : 1) * RS_BUCKETS;
     return (size_t)(hn_ + 1) * 4 * 2 + RS_BUCKETS * 4 + 512;
 }
 

@@ -38,3 +38,19 @@ def test_rows_with_a_field(m):
     gs, gd, meta = h.getCOO(meta=True)
     assert np.array_equal(gs.cpu().numpy(), s[order]) and np.array_equal(gd.cpu().numpy(), d[order])
     assert np.array_equal(meta[0].cpu().numpy(), f[order])
+
+
+@pytest.mark.parametrize("m", [(1 << 20) - 1, 1 << 20, (1 << 23) - 1])
+def test_batches(m):
+    """An update lays its scratch out for one key more than it sorts."""
+    print("case sort tiles batch", m, flush=True)
+    n = 4099
+    rng = np.random.default_rng(m)
+    s, d = rng.integers(0, n, m).astype(np.int32), rng.integers(0, n, m).astype(np.int32)
+    h = Hornet(HornetInit(n, 0, np.zeros(n + 1, np.int32), np.zeros(0, np.int32)))
+    from hornet_amd.graph import BatchUpdate
+    key = np.unique(s.astype(np.int64) * n + d)
+    assert h.insert(BatchUpdate(s, d), True, True) == key.size
+    gs, gd = h.getCOO()
+    assert np.array_equal(gs.cpu().numpy().astype(np.int64) * n + gd.cpu().numpy(), key)
+    assert h.erase(BatchUpdate(s, d), True) == key.size and h.nE() == 0
