@@ -41,6 +41,7 @@ namespace {
 
 constexpr uint32_t ERR_BAD_ID = 1u;
 constexpr uint32_t ERR_OOM = 2u;     // AllocState::error bit 0 is mirrored here
+constexpr uint32_t ERR_SIDE = 4u;    // more deferred entries than the side buffer holds: nothing moved yet
 // Segmented copies: 4 items per lane, at most BLOCK + 1 runs staged in LDS
 // per tile (a tile with more runs searches them in global memory), 8
 // workgroups per CU striding over the tiles.  A one-entry-per-item LDS stage
@@ -592,19 +593,24 @@ struct EraseDeferIn {
 };
 
 // scan output of the deferred counts: each tile's count and offset in the side
-// buffer; the last tile also records the total in the batch's status word, read
-// back with it
+// buffer; the last tile also records the total, and stops the batch if that is
+// more than the side buffer holds (no count is made after it: see defer_offsets)
 struct SideOut {
     uint32_t* tcnt;
     int64_t* P;
     int64_t last;
+    int64_t cap;
     UpdScal* sc;
     __device__ __forceinline__ void operator()(int64_t i, int64_t ex, int64_t x) const {
         tcnt[i] = (uint32_t)x;
         P[i] = ex;
-        if (i == last) sc->side = ex + x;
+        if (i == last) {
+            sc->side = ex + x;
+            if (ex + x > cap) sc->err |= ERR_SIDE;
+        }
     }
 };
+__global__ void side_fits_kernel(UpdScal* sc) { sc->err &= ~ERR_SIDE; }
 
 // s_waitcnt vmcnt(0): every vector memory load of the wave has returned
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -872,13 +878,17 @@ __global__ __launch_bounds__(BLOCK) void insert_move_kernel(int64_t nseg, const 
 
 // the deferred entries of either in-place pass (and their fields) to their
 // destinations, once every copy tile has read its sources
-__global__ void place_side_kernel(int64_t m, const int32_t* __restrict__ side, const int64_t* __restrict__ side_dst,
-                                    int32_t* __restrict__ arena, MetaSet am, MetaSet sm) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    const int64_t d = side_dst[k];
-    arena[d] = side[k];
-    if (am.any()) meta_put(am, d, sm, k);
+__global__ __launch_bounds__(BLOCK) void place_side_kernel(const int32_t* __restrict__ side,
+                                                           const int64_t* __restrict__ side_dst,
+                                                           int32_t* __restrict__ arena, const UpdScal* sc, MetaSet am,
+                                                           MetaSet sm) {
+    if (sc->err) return;
+    const int64_t m = sc->side;
+    for (int64_t k = (int64_t)blockIdx.x * BLOCK + threadIdx.x; k < m; k += (int64_t)gridDim.x * BLOCK) {
+        const int64_t d = side_dst[k];
+        arena[d] = side[k];
+        if (am.any()) meta_put(am, d, sm, k);
+    }
 }
 
 // kept batch entry i (the q-th of its source segment j) to slot
@@ -1028,8 +1038,8 @@ struct TileCountIn {
 // it goes; the two readings of a larger one would count twice, sixteen tiles to a
 // lane (500 K tiles of an R-MAT s24 erase: 290 us, 25 with the counts on their own).
 template <typename Defer>
-static hn_status defer_offsets(Defer in, UpdBufs& b, int64_t ntiles, hipStream_t st) {
-    const SideOut out{b.tcnt, b.doff, ntiles - 1, b.sc};
+static hn_status defer_offsets(Defer in, UpdBufs& b, int64_t ntiles, int64_t cap, hipStream_t st) {
+    const SideOut out{b.tcnt, b.doff, ntiles - 1, cap, b.sc};
     if (ntiles <= SCAN_ONE) return exclusive_scan_fn<int64_t>(in, out, b.doff + ntiles, ntiles, b.tmp, st);
     defer_kernel<<<(unsigned)ceil_div(ntiles, BLOCK), BLOCK, 0, st>>>(ntiles, in, b.tcnt);
     HN_CHECK_LAUNCH();
@@ -1180,13 +1190,18 @@ static void note_symmetry(hn_graph* g, bool was_sym, const UpdScal& h) {
     g->sym_version = g->version;
 }
 
-// the side buffer for the batch's deferred entries (their count is read back
-// with the error word, which is checked first), one per meta-data field in
-// b.sm, and when asked one 64-bit destination per entry
-static hn_status reserve_side(hn_graph* g, UpdBufs& b, hipStream_t st, int64_t* total, int32_t** stage,
-                              int64_t** dst = nullptr) {
-    UpdScal h;
-    HN_TRY(check_scal(g, b, st, &h));
+// The side buffer of the batch's deferred entries: entries, destinations and one
+// array per meta-data field (b.sm), as many as the handle's scratch holds, at least
+// `want`.  A batch goes on with what is there before the host knows how many it
+// defers, and is stopped on the device (ERR_SIDE) if that is too little; the host
+// then makes room and launches the copies again.  Waiting for the count cost every
+// batch a readback, 25 to 40 us with the device idle.
+struct SideBuf {
+    int32_t* entry;
+    int64_t* dst;
+    int64_t cap;
+};
+static hn_status side_buffer(hn_graph* g, UpdBufs& b, int64_t want, SideBuf* out) {
     // test hook: HORNET_HIP_FAIL_SIDE_RESERVE=1 makes this reservation fail as
     // a device allocation would, after the batch's blocks were allocated
     if (const char* e = std::getenv("HORNET_HIP_FAIL_SIDE_RESERVE"))
@@ -1194,25 +1209,30 @@ static hn_status reserve_side(hn_graph* g, UpdBufs& b, hipStream_t st, int64_t* 
             set_error("side buffer: allocation failure forced by HORNET_HIP_FAIL_SIDE_RESERVE");
             return HN_E_OOM;
         }
-    *total = (int64_t)h.side;
-    const size_t cnt = (size_t)(*total > 0 ? *total : 1);
-    // entries, then (when asked for) one 64-bit destination per entry
-    const size_t vbytes = (sizeof(int32_t) * cnt + 255) & ~size_t(255);
-    HN_TRY(g->s_misc.reserve(vbytes + (dst ? sizeof(int64_t) * cnt : 0)));
-    *stage = g->s_misc.as<int32_t>();
-    if (dst) *dst = reinterpret_cast<int64_t*>(g->s_misc.as<char>() + vbytes);
+    want = std::max<int64_t>(want, 1 << 14);
+    constexpr size_t EACH = sizeof(int32_t) + sizeof(int64_t), ALIGN = 256;
+    HN_TRY(g->s_misc.reserve((size_t)want * EACH + ALIGN));
+    int64_t cap = (int64_t)((g->s_misc.bytes - ALIGN) / EACH);
     if (g->meta.any()) {
-        // one side array per meta-data field, 256-byte aligned, in s_mstage
-        size_t bytes = 0;
-        for (int f = 0; f < g->meta.n; f++) bytes += (cnt * g->meta.bytes[f] + 255) & ~size_t(255);
-        HN_TRY(g->s_mstage.reserve(bytes));
+        size_t each = 0;
+        for (int f = 0; f < g->meta.n; f++) each += (size_t)g->meta.bytes[f];
+        const size_t pad = ALIGN * (size_t)g->meta.n;
+        HN_TRY(g->s_mstage.reserve((size_t)want * each + pad));
+        cap = std::min(cap, (int64_t)((g->s_mstage.bytes - pad) / each));
         size_t at = 0;
         for (int f = 0; f < g->meta.n; f++) {
             b.sm.p[f] = g->s_mstage.as<char>() + at;
-            at += (cnt * g->meta.bytes[f] + 255) & ~size_t(255);
+            at += ((size_t)cap * (size_t)g->meta.bytes[f] + ALIGN - 1) & ~(ALIGN - 1);
         }
     }
+    out->entry = g->s_misc.as<int32_t>();
+    out->dst = reinterpret_cast<int64_t*>(g->s_misc.as<char>() + (((size_t)cap * sizeof(int32_t) + ALIGN - 1) & ~(ALIGN - 1)));
+    out->cap = cap;
     return HN_OK;
+}
+
+static unsigned side_grid(int64_t cap) {
+    return (unsigned)std::min<int64_t>(ceil_div(cap, BLOCK), (int64_t)num_cus() * 4);
 }
 
 static void record_last(hn_graph* g, int32_t kind, int64_t submitted, int64_t applied, const TouchInfo* ti,
@@ -1360,35 +1380,47 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
     HN_UNDO_TRY(exclusive_scan_fn<int64_t>(MoveLenIn{b.ti, ucnt, b.sc}, RunOut{b.wpos, b.tile_lo}, b.wpos + n, n,
                                            b.tmp, st));
     const int64_t nt = b.ntile_max;
-    HN_UNDO_TRY(defer_offsets(InsertDeferIn{n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, g->arena, b.sc}, b, nt, st));
-    int64_t ndefer = 0;
-    int32_t* side = nullptr;
-    int64_t* side_dst = nullptr;
-    HN_UNDO_TRY(reserve_side(g, b, st, &ndefer, &side, &side_dst));
-    const int64_t grid = (int64_t)num_cus() * COPY_GRID_PER_CU;
-    insert_move_kernel<<<(unsigned)grid, BLOCK, 0, st>>>(n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, b.tcnt,
-                                                         b.doff, g->arena, side, side_dst, b.sc, g->meta, b.sm);
-    HN_UNDO_LAUNCH();
-    if (ndefer > 0) {
-        place_side_kernel<<<(unsigned)ceil_div(ndefer, BLOCK), BLOCK, 0, st>>>(ndefer, side, side_dst, g->arena,
-                                                                                 g->meta, b.sm);
-        HN_UNDO_LAUNCH();
-    }
-    insert_batch_kernel<<<gridn, BLOCK, 0, st>>>(nb, b.kb, b.spos, b.seg_start, ubk, b.ti, f, g->arena, b.sc, g->meta,
-                                                 bm.m, b.ib);
-    HN_UNDO_LAUNCH();
-#undef HN_UNDO_LAUNCH
-#undef HN_UNDO_TRY
-    // 5. publish
-    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg_key, f, b.ti, nullptr, g->rec, g->alloc_view(), nb, b.sc);
-    HN_CHECK_LAUNCH();
-    const bool was_sym = g->sym == 1;
-    if (was_sym) {
-        insert_symmetry_kernel<<<gridn, BLOCK, 0, st>>>(nb, b.kb, f, stamp, g->rec, g->arena, b.sc);
+    SideBuf side;
+    HN_UNDO_TRY(side_buffer(g, b, 0, &side));
+    HN_UNDO_TRY(defer_offsets(InsertDeferIn{n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, g->arena, b.sc}, b, nt,
+                              side.cap, st));
+    auto rewrite = [&]() -> hn_status {
+        insert_move_kernel<<<(unsigned)num_cus() * COPY_GRID_PER_CU, BLOCK, 0, st>>>(
+            n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, b.tcnt, b.doff, g->arena, side.entry, side.dst, b.sc,
+            g->meta, b.sm);
         HN_CHECK_LAUNCH();
-    }
+        place_side_kernel<<<side_grid(side.cap), BLOCK, 0, st>>>(side.entry, side.dst, g->arena, b.sc, g->meta, b.sm);
+        HN_CHECK_LAUNCH();
+        insert_batch_kernel<<<gridn, BLOCK, 0, st>>>(nb, b.kb, b.spos, b.seg_start, ubk, b.ti, f, g->arena, b.sc,
+                                                     g->meta, bm.m, b.ib);
+        HN_CHECK_LAUNCH();
+        return HN_OK;
+    };
+    // 5. publish
+    const bool was_sym = g->sym == 1;
+    auto publish = [&]() -> hn_status {
+        commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(
+            ucnt, b.seg_key, f, b.ti, nullptr, g->rec, g->alloc_view(), nb, b.sc);
+        HN_CHECK_LAUNCH();
+        if (was_sym) {
+            insert_symmetry_kernel<<<gridn, BLOCK, 0, st>>>(nb, b.kb, f, stamp, g->rec, g->arena, b.sc);
+            HN_CHECK_LAUNCH();
+        }
+        return HN_OK;
+    };
+    HN_UNDO_TRY(rewrite());
+    HN_TRY(publish());
     UpdScal h;
     HN_TRY(check_scal(g, b, st, &h));
+    if (h.err & ERR_SIDE) {   // nothing has moved: with room, again
+        side_fits_kernel<<<1, 1, 0, st>>>(b.sc);
+        HN_UNDO_TRY(side_buffer(g, b, h.side, &side));
+        HN_UNDO_TRY(rewrite());
+        HN_TRY(publish());
+        HN_TRY(check_scal(g, b, st, &h));
+    }
+#undef HN_UNDO_LAUNCH
+#undef HN_UNDO_TRY
     g->ne += (int64_t)h.changed;
     g->version++;
     note_symmetry(g, was_sym, h);
@@ -1460,38 +1492,47 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
     // 7. in-place compaction in one pass; the few entries that would overwrite
     // a source of an earlier tile go through a side buffer
     const int64_t nt = b.ntile_max;
-    HN_UNDO_TRY(defer_offsets(EraseDeferIn{2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.rtail, b.sc}, b, nt, st));
-    int64_t ndefer = 0;
-    int32_t* side = nullptr;
-    int64_t* side_dst = nullptr;
-    HN_UNDO_TRY(reserve_side(g, b, st, &ndefer, &side, &side_dst));
-    const int64_t grid = (int64_t)num_cus() * COPY_GRID_PER_CU;
-    if (g->meta.n > 0)
-        erase_copy_kernel<true><<<(unsigned)grid, BLOCK, 0, st>>>(2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.tcnt,
-                                                                  b.doff, g->arena, side, side_dst, b.sc, g->meta,
-                                                                  b.sm);
-    else
-        erase_copy_kernel<false><<<(unsigned)grid, BLOCK, 0, st>>>(2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.tcnt,
-                                                                   b.doff, g->arena, side, side_dst, b.sc, g->meta,
-                                                                   b.sm);
-    HN_UNDO_LAUNCH();
-    if (ndefer > 0) {
-        place_side_kernel<<<(unsigned)ceil_div(ndefer, BLOCK), BLOCK, 0, st>>>(ndefer, side, side_dst, g->arena,
-                                                                               g->meta, b.sm);
-        HN_UNDO_LAUNCH();
+    SideBuf side;
+    HN_UNDO_TRY(side_buffer(g, b, 0, &side));
+    HN_UNDO_TRY(defer_offsets(EraseDeferIn{2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.rtail, b.sc}, b, nt, side.cap, st));
+    auto rewrite = [&]() -> hn_status {
+        auto copy = [&](auto kernel) {
+            kernel<<<(unsigned)num_cus() * COPY_GRID_PER_CU, BLOCK, 0, st>>>(2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst,
+                                                                             b.tcnt, b.doff, g->arena, side.entry,
+                                                                             side.dst, b.sc, g->meta, b.sm);
+        };
+        if (g->meta.n > 0) copy(erase_copy_kernel<true>);
+        else copy(erase_copy_kernel<false>);
+        HN_CHECK_LAUNCH();
+        place_side_kernel<<<side_grid(side.cap), BLOCK, 0, st>>>(side.entry, side.dst, g->arena, b.sc, g->meta, b.sm);
+        HN_CHECK_LAUNCH();
+        return HN_OK;
+    };
+    // 8. publish
+    const bool was_sym = g->sym == 1;
+    auto publish = [&]() -> hn_status {
+        commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(
+            ucnt, b.seg2_key, f, b.ti, b.skip, g->rec, g->alloc_view(), b.dlp + n, b.sc);
+        HN_CHECK_LAUNCH();
+        if (was_sym) {
+            erase_symmetry_kernel<<<gridn, BLOCK, 0, st>>>(dcnt, b.seg_key, f, b.dlen, b.live, stamp, b.sc);
+            HN_CHECK_LAUNCH();
+        }
+        return HN_OK;
+    };
+    HN_UNDO_TRY(rewrite());
+    HN_TRY(publish());
+    UpdScal h;
+    HN_TRY(check_scal(g, b, st, &h));
+    if (h.err & ERR_SIDE) {   // nothing has moved: with room, again
+        side_fits_kernel<<<1, 1, 0, st>>>(b.sc);
+        HN_UNDO_TRY(side_buffer(g, b, h.side, &side));
+        HN_UNDO_TRY(rewrite());
+        HN_TRY(publish());
+        HN_TRY(check_scal(g, b, st, &h));
     }
 #undef HN_UNDO_LAUNCH
 #undef HN_UNDO_TRY
-    // 8. publish
-    commit_kernel<<<(unsigned)ceil_div(n + 1, ALLOC_BLOCK), ALLOC_BLOCK, 0, st>>>(ucnt, b.seg2_key, f, b.ti, b.skip, g->rec, g->alloc_view(), b.dlp + n, b.sc);
-    HN_CHECK_LAUNCH();
-    const bool was_sym = g->sym == 1;
-    if (was_sym) {
-        erase_symmetry_kernel<<<gridn, BLOCK, 0, st>>>(dcnt, b.seg_key, f, b.dlen, b.live, stamp, b.sc);
-        HN_CHECK_LAUNCH();
-    }
-    UpdScal h;
-    HN_TRY(check_scal(g, b, st, &h));
     g->ne -= (int64_t)h.changed;
     g->version++;
     note_symmetry(g, was_sym, h);
