@@ -55,6 +55,15 @@ constexpr uint32_t TC_CAND = 1024;             // candidates per task
 constexpr int TC_STEP = 2 * BLOCK;             // ... listed at a time
 constexpr uint32_t TC_TAIL = 256;              // ids hashed at a time
 constexpr uint32_t TC_HASH = 2 * TC_TAIL;
+constexpr uint32_t TC_WIDE_HASH = (TC_HUBS + 1) / 32, TC_WIDE_TAIL = TC_WIDE_HASH / 2;   // ... in the bits' place
+// Stored rows with more ids are searched, as they are sorted, and not hashed: hashing
+// them goes over all candidates once per table, which is quadratic (all stored entries of
+// R-MAT s20: 930 ms, a star of four million leaves: 1 s; so: 56 and 0.8 ms.  R-MAT s18 and
+// s20, searched from one table less on: 6.7 and 57 ms, from two more on: 8.1 and 64).  The
+// lists of an orientation are not whole rows, and long ones of ids take more than 65,535
+// vertices of a like degree: they are hashed, one table of 1,024 after the other (cliques
+// of 700, in tables of 256: 18.3 ms, 6.4 so; of 5,000: 1.6 s).
+constexpr uint32_t TC_SEARCH = TC_TAIL + 2 * TC_WIDE_TAIL;
 constexpr int TC_TEAM = 8;                     // lanes per shorter list
 constexpr int TC_DEPTH = 4;                    // groups per lane in flight (2 and 8: 3 and 2 % slower on R-MAT s22)
 constexpr int TC_ORDER = 32;                   // classes of list lengths that a step is sorted by
@@ -102,9 +111,17 @@ __global__ __launch_bounds__(BLOCK) void tc_hist_kernel(int64_t nv, const uint32
     __shared__ uint32_t h[TC_BINS];
     for (int i = threadIdx.x; i < TC_BINS; i += BLOCK) h[i] = 0;
     __syncthreads();
-    for (int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x; v < nv; v += (int64_t)gridDim.x * BLOCK) {
-        const uint32_t w = weight[v];
-        if (w > 1) atomicAdd(&h[tc_bin(w)], 1u);
+    constexpr int K = 8;   // loads in flight (one: 45 us for 16 M vertices, 22 so)
+    for (int64_t b = (int64_t)blockIdx.x * (K * BLOCK); b < nv; b += (int64_t)gridDim.x * (K * BLOCK)) {
+        uint32_t w[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int64_t v = b + k * BLOCK + threadIdx.x;
+            w[k] = v < nv ? weight[v] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (w[k] > 1) atomicAdd(&h[tc_bin(w[k])], 1u);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < TC_BINS; i += BLOCK)
@@ -153,11 +170,6 @@ struct HubOut {
     }
 };
 
-__global__ void tc_weight_deg_kernel(int64_t nv, const hn_vrec* __restrict__ rec, uint32_t* __restrict__ weight) {
-    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if (v < nv) weight[v] = (uint32_t)rec[v].deg;
-}
-
 // Where every vertex can have a bit there is nothing to choose: codes are the
 // ids.  One launch in place of six (weights, histogram, cut and codes), 110 us of
 // the 590 that a stored graph of 6 K vertices and 100 K entries took.
@@ -182,11 +194,15 @@ __device__ __forceinline__ void tc_tiles(uint32_t* __restrict__ tile_lo, int64_t
         for (uint32_t t = (ex + TC_TILE - 1) / TC_TILE; (uint64_t)t * TC_TILE < (uint64_t)ex + x; t++)
             tile_lo[t] = (uint32_t)v;
 }
+// weight, where given: the degrees, from records that were just read
 struct StoredGroupsOut {
+    const hn_vrec* rec;
     TcRow* row;
     uint32_t* P;
     uint32_t* tile_lo;
+    uint32_t* weight;
     __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t x) const {
+        if (weight) weight[v] = (uint32_t)rec[v].deg;
         row[v] = TcRow{ex, 0u, 0u, 0u};
         P[v] = ex;
         tc_tiles(tile_lo, v, ex, x);
@@ -241,7 +257,9 @@ __device__ __forceinline__ TcLoc tc_locate(const uint32_t* __restrict__ P, int64
 // How often a vertex is an entry, from every `step`-th tile of the stored rows
 // (any choice of hubs gives the same counts).  Bound by the atomics on the most
 // frequent one, 10 ns each: a quarter of a million to a million entries are looked
-// at (all 2.8 M of an R-MAT s18 orientation took 660 us, 73 so).
+// at (all 2.8 M of an R-MAT s18 orientation took 660 us, 73 so), and a wave adds the
+// entries equal to its first one together (a star of four million leaves: 1538 us without,
+// 34 so).
 __global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
                                                                const uint32_t* __restrict__ P,
                                                                const uint32_t* __restrict__ tile_lo,
@@ -257,10 +275,17 @@ __global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const
                                   [&](int64_t s) { return (uint32_t)(rec[s].off / UNIT_SLOTS); }, unit);
 #pragma unroll
         for (int j = 0; j < TC_IPT; j++) {
-            if (c.seg[j] < 0) continue;
             const int64_t at = (int64_t)unit[j] * UNIT_SLOTS + (int64_t)c.k[j] * TC_G;
-            const int64_t n = min((int64_t)TC_G, (int64_t)rec[c.seg[j]].deg - (int64_t)c.k[j] * TC_G);
-            for (int64_t e = 0; e < n; e++) atomicAdd(weight + arena[at + e], 1u);
+            const int64_t n = c.seg[j] < 0 ? 0 : (int64_t)rec[c.seg[j]].deg - (int64_t)c.k[j] * TC_G;
+            for (int e = 0; e < TC_G; e++) {
+                const bool in = e < n;
+                const uint64_t some = __ballot(in);
+                if (some == 0) break;
+                const int first = __ffsll((unsigned long long)some) - 1;
+                const int32_t v = in ? arena[at + e] : -1, lead = __shfl(v, first, WAVE);
+                const uint32_t same = (uint32_t)__popcll(__ballot(v == lead));
+                if (in && (v != lead || (int)__lane_id() == first)) atomicAdd(weight + v, v == lead ? same : 1u);
+            }
         }
         __syncthreads();
     }
@@ -268,7 +293,9 @@ __global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const
 
 // Stored rows -> lists (ORIENT: only the entries up the degree order).  A lane
 // holds eight entries of one row; the lanes of a wave that hold the same row
-// claim its next places, in both of its rows, with one atomic.
+// claim its next places, in both of its rows, with one atomic, or none if they hold
+// all of it (four million rows of four entries: 461 us with one for each, 440 so;
+// of one entry: 457, 274).
 typedef int32_t TcVec __attribute__((ext_vector_type(4)));
 template <bool ORIENT>
 __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
@@ -328,13 +355,16 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
             const uint32_t before = __shfl(inc - cnt, head, WAVE);
             const uint32_t sum = __shfl(inc, tail, WAVE) - before;
             unsigned long long at = 0;
-            if (lane == head && sum)
-                at = atomicAdd(reinterpret_cast<unsigned long long*>(&row[u].n16),
-                               (unsigned long long)(sum & 0xFFFFu) | (unsigned long long)(sum >> 16) << 32);
+            if (lane == head && sum) {
+                unsigned long long* cur = reinterpret_cast<unsigned long long*>(&row[u].n16);
+                const unsigned long long n2 = (unsigned long long)(sum & 0xFFFFu) | (unsigned long long)(sum >> 16) << 32;
+                if (c.k[j] == 0 && (tail - head + 1) * TC_G >= deg[j]) *cur = n2;
+                else at = atomicAdd(cur, n2);
+            }
             const uint32_t at16 = __shfl((uint32_t)at, head, WAVE), at32 = __shfl((uint32_t)(at >> 32), head, WAVE);
             if (keep) {
                 const uint32_t mine = inc - cnt - before;
-                const int64_t base = (int64_t)row[u].base * TC_G;
+                const int64_t base = (t * TC_TILE + (int64_t)j * BLOCK + threadIdx.x - c.k[j]) * TC_G;   // (as row[u].base)
                 uint16_t* o16 = codes + base + at16 + (mine & 0xFFFFu);
                 uint32_t* o32 = ids + base + at32 + (mine >> 16);
 #pragma unroll
@@ -349,11 +379,14 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
     if (__ballot(twice) && lane == 0) ctl->repeats = 1u;   // every writer stores the same value
 }
 
-__global__ void tc_pad_kernel(int64_t nv, const TcRow* __restrict__ row, uint16_t* __restrict__ codes,
-                              uint32_t* __restrict__ ids) {
+// The lists' padding, and a bit per vertex whose list is long enough for it to be an owner.
+__global__ __launch_bounds__(BLOCK) void tc_pad_kernel(int64_t nv, const TcRow* __restrict__ row,
+                                                       uint16_t* __restrict__ codes, uint32_t* __restrict__ ids,
+                                                       uint64_t* __restrict__ owner) {
     const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if (v >= nv) return;
-    const TcRow r = row[v];
+    const TcRow r = v < nv ? row[v] : TcRow{0u, 0u, 0u, 0u};
+    const uint64_t big = __ballot(r.len() > TC_SMALL);
+    if (__lane_id() == 0 && v < nv) owner[v / WAVE] = big;
     for (uint32_t i = r.n16; i & (TC_G - 1); i++) codes[(int64_t)r.base * TC_G + i] = (uint16_t)TC_PAD16;
     for (uint32_t i = r.n32; i & (TC_G - 1); i++) ids[(int64_t)r.base * TC_G + i] = TC_PAD;
 }
@@ -369,11 +402,14 @@ __device__ __forceinline__ uint32_t tc_entry(const TcRow& r, uint32_t i, const u
 // FILL = false: the edge's place in its group (TC_PAD: not grouped); FILL = true: the sources at their places
 // A hub's group is counted in TC_LANES parts (by workgroup, the same in both passes),
 // as atomics on one counter take 10 ns each: R-MAT s18 oriented, 319 us in one part, 118 so.
+// Otherwise bound by the lookups of the entries' lists: only owners' are looked up, by a
+// bit that the L2 holds (four million vertices of four entries: 525 us without, 217 so).
 template <bool FILL>
 __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
                                                          const uint32_t* __restrict__ P,
                                                          const uint32_t* __restrict__ tile_lo, int sym,
                                                          const TcCtl* __restrict__ ctl, const TcRow* __restrict__ row,
+                                                         const uint64_t* __restrict__ owner,
                                                          const uint16_t* __restrict__ codes,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, uint32_t* __restrict__ gcnt,
@@ -396,17 +432,36 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
             const uint32_t lu = r.len();
             if (lu < 2) continue;
             // entries [8k, 8k + 8) of the list, which may end before its stored row
-            for (uint32_t i = c.k[j] * TC_G; i < min(lu, (c.k[j] + 1) * TC_G); i++) {
-                const bool is_hub = i < r.n16;
-                const uint32_t q = is_hub ? codes[(int64_t)r.base * TC_G + i] : 0u;
-                const uint32_t v = is_hub ? hub[q] : ids[(int64_t)r.base * TC_G + (i - r.n16)];
-                uint32_t* pl = place + (int64_t)r.base * TC_G + i;
-                if constexpr (FILL) {
-                    if (*pl != TC_PAD) members[(int64_t)goff[v] + (is_hub ? mine[q] : 0u) + *pl] = u;
-                } else {
-                    const uint32_t lv = row[v].len();
-                    *pl = lv > lu && lv > TC_SMALL && v != u ? atomicAdd(is_hub ? mine + q : gcnt + v, 1u) : TC_PAD;
+            const int64_t at = (int64_t)r.base * TC_G;
+            const uint32_t i0 = c.k[j] * TC_G;
+            if (i0 >= lu) continue;
+            uint32_t q[TC_G], v[TC_G];
+#pragma unroll
+            for (int e = 0; e < TC_G; e++) {
+                const uint32_t i = i0 + e;
+                q[e] = i < r.n16 ? codes[at + i] : TC_PAD;
+                v[e] = i >= r.n16 && i < lu ? ids[at + (i - r.n16)] : u;
+            }
+#pragma unroll
+            for (int e = 0; e < TC_G; e++)
+                if (q[e] != TC_PAD) v[e] = hub[q[e]];
+            if constexpr (FILL) {
+#pragma unroll
+                for (int e = 0; e < TC_G; e++) {
+                    const uint32_t pl = i0 + e < lu ? place[at + i0 + e] : TC_PAD;
+                    if (pl != TC_PAD) members[(int64_t)goff[v[e]] + (q[e] != TC_PAD ? mine[q[e]] : 0u) + pl] = u;
                 }
+            } else {
+                uint64_t big[TC_G];
+                uint32_t lv[TC_G];
+#pragma unroll
+                for (int e = 0; e < TC_G; e++) big[e] = owner[v[e] / WAVE];
+#pragma unroll
+                for (int e = 0; e < TC_G; e++) lv[e] = v[e] != u && (big[e] >> (v[e] % WAVE) & 1u) ? row[v[e]].len() : 0u;
+#pragma unroll
+                for (int e = 0; e < TC_G; e++)
+                    if (i0 + e < lu)
+                        place[at + i0 + e] = lv[e] > lu ? atomicAdd(q[e] != TC_PAD ? mine + q[e] : gcnt + v[e], 1u) : TC_PAD;
             }
         }
         __syncthreads();
@@ -430,17 +485,17 @@ __global__ __launch_bounds__(BLOCK) void tc_parts_kernel(int sym, const TcCtl* _
 }
 
 // ---- tasks: up to TC_CAND candidates of one owner
+// (the owners' bits spare the pass the others' lists: 16 M vertices, 117 us without, 38 so)
 struct TaskIn {
+    const uint64_t* owner;
     const TcRow* row;
     const uint32_t* gcnt;
     const hn_vrec* rec;
     const TcCtl* ctl;
     int sym;
     __device__ __forceinline__ uint32_t operator()(int64_t v) const {
-        const TcRow r = row[v];
-        const uint32_t n = r.len();
-        if (n <= TC_SMALL) return 0u;
-        const uint32_t cand = sym && !ctl->repeats ? (uint32_t)rec[v].deg : n + gcnt[v];
+        if (!(owner[v / WAVE] >> (v % WAVE) & 1u)) return 0u;
+        const uint32_t cand = sym && !ctl->repeats ? (uint32_t)rec[v].deg : row[v].len() + gcnt[v];
         return (cand + TC_CAND - 1) / TC_CAND;
     }
 };
@@ -461,8 +516,28 @@ struct OwnerShared {
 };
 static_assert(sizeof(OwnerShared) * 8 <= 160 * 1024, "eight workgroups fill a CU's LDS");
 
-__device__ __forceinline__ uint32_t tc_slot(uint32_t id) { return (id * 2654435761u) >> (32 - 9); }
-static_assert(TC_HASH == 1u << 9, "tc_slot yields nine bits");
+// Two sizes of table: beside the hubs' bits, or, where these are done with, in their place.
+template <uint32_t SLOTS>
+__device__ __forceinline__ uint32_t tc_slot(uint32_t id) { return (id * 2654435761u) >> (__builtin_clz(SLOTS) + 1); }
+template <uint32_t SLOTS>
+__device__ __forceinline__ void tc_fill(uint32_t* table, const uint32_t* __restrict__ ids, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < SLOTS; i += BLOCK) table[i] = TC_PAD;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += BLOCK) {
+        const uint32_t q = ids[i];
+        for (uint32_t s = tc_slot<SLOTS>(q);; s = (s + 1) & (SLOTS - 1)) {
+            const uint32_t z = atomicCAS(table + s, TC_PAD, q);
+            if (z == TC_PAD || z == q) break;
+        }
+    }
+}
+template <uint32_t SLOTS>
+__device__ __forceinline__ bool tc_holds(const uint32_t* table, uint32_t q) {
+    for (uint32_t s = tc_slot<SLOTS>(q);; s = (s + 1) & (SLOTS - 1)) {
+        const uint32_t z = table[s];
+        if (z == q || z == TC_PAD) return z == q;
+    }
+}
 
 __device__ __forceinline__ uint32_t tc_test(const OwnerShared& sh, const uint4& x) {
     const uint32_t q[4] = {x.x, x.y, x.z, x.w};
@@ -480,19 +555,31 @@ __device__ __forceinline__ uint32_t tc_test(const OwnerShared& sh, const uint4& 
 // lanes per list, eight codes per lane and group.  The lists are sorted by
 // length class, so that the teams of a wave stay together: TC_DEPTH groups of one
 // list in flight while lists are longer than a team's step, then TC_DEPTH lists.
-template <bool TAIL>
-__device__ __forceinline__ uint32_t tc_ids(const OwnerShared& sh, uint32_t it, int sub, const uint32_t* __restrict__ ids) {
+enum TcTail { TC_NONE, TC_HASHED, TC_HASHED_WIDE, TC_SORTED };
+struct TcSorted {   // an owner's stored row
+    const int32_t* entry;
+    int32_t deg;
+    __device__ __forceinline__ bool has(uint32_t q) const {
+        int32_t lo = 0, hi = deg;
+        while (lo < hi) {
+            const int32_t mid = (lo + hi) >> 1;
+            if ((uint32_t)entry[mid] < q) lo = mid + 1; else hi = mid;
+        }
+        return lo < deg && (uint32_t)entry[lo] == q;
+    }
+};
+template <TcTail TAIL>
+__device__ __forceinline__ uint32_t tc_ids(const OwnerShared& sh, uint32_t it, int sub, const uint32_t* __restrict__ ids,
+                                           const TcSorted& sorted) {
     uint32_t c = 0;
-    if constexpr (TAIL) {
+    if constexpr (TAIL != TC_NONE) {
         const uint32_t* li = ids + (int64_t)sh.base[it] * TC_G;
         const uint32_t n32 = sh.n32[it];
         for (uint32_t i = sub; i < n32; i += TC_TEAM) {
             const uint32_t q = li[i];
-            for (uint32_t s = tc_slot(q);; s = (s + 1) & (TC_HASH - 1)) {
-                const uint32_t z = sh.hash[s];
-                c += z == q ? 1u : 0u;
-                if (z == q || z == TC_PAD) break;
-            }
+            if constexpr (TAIL == TC_HASHED) c += tc_holds<TC_HASH>(sh.hash, q) ? 1u : 0u;
+            if constexpr (TAIL == TC_HASHED_WIDE) c += tc_holds<TC_WIDE_HASH>(sh.bits, q) ? 1u : 0u;
+            if constexpr (TAIL == TC_SORTED) c += sorted.has(q) ? 1u : 0u;
         }
     }
     return c;
@@ -504,9 +591,10 @@ __device__ __forceinline__ uint32_t tc_team_sum(uint32_t c) {
     c += dpp_move<0x114, 0xf>(c);
     return c;
 }
-template <bool TAIL>
+template <TcTail TAIL>
 __device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, uint32_t n,
                                         const uint16_t* __restrict__ codes, const uint32_t* __restrict__ ids,
+                                        const TcSorted& sorted,
                                         unsigned long long* __restrict__ per_vertex, uint64_t& acc) {
     constexpr uint32_t TEAMS = BLOCK / TC_TEAM;
     const int sub = threadIdx.x & (TC_TEAM - 1);
@@ -515,7 +603,7 @@ __device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, u
     for (; it < nlong; it += TEAMS) {
         const uint4* list = rows + sh.base[it];
         const uint32_t ng = (sh.n16[it] + TC_G - 1) / TC_G;
-        uint32_t c = tc_ids<TAIL>(sh, it, sub, ids);
+        uint32_t c = tc_ids<TAIL>(sh, it, sub, ids, sorted);
         for (uint32_t g0 = sub; g0 < ng; g0 += TC_TEAM * TC_DEPTH) {
             uint4 x[TC_DEPTH];
 #pragma unroll
@@ -550,7 +638,7 @@ __device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, u
             const uint32_t i = it + d * TEAMS;
             if (i >= n) break;
             const uint32_t k = tc_test(sh, x[d]);
-            uint32_t c = (in[d] ? k : 0u) + tc_ids<TAIL>(sh, i, sub, ids);
+            uint32_t c = (in[d] ? k : 0u) + tc_ids<TAIL>(sh, i, sub, ids, sorted);
             acc += c;
             c = tc_team_sum(c);
             if (sub == TC_TEAM - 1 && c && per_vertex) atomicAdd(per_vertex + sh.y[i], (unsigned long long)c);
@@ -561,7 +649,7 @@ __device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, u
 // Bound by the sectors of the shorter lists that miss the L2: on R-MAT s22 360 M of
 // the 400 M that the walks touch, 7.4 ms at the 48 G/s that scattered sector reads
 // reach here; LDS and vector units are a third busy.
-__global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int sym, const hn_vrec* __restrict__ rec,
+__global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, const hn_vrec* __restrict__ rec,
                                                          const int32_t* __restrict__ arena,
                                                          const uint2* __restrict__ wc, const uint2* __restrict__ task,
                                                          const TcRow* __restrict__ row,
@@ -614,24 +702,24 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int sym, const hn_vrec*
         const uint32_t lx = rx.len(), cand = stored ? (uint32_t)sx.deg : lx + gcnt[x];
         const uint32_t c0 = tk.y * TC_CAND, c1 = min(c0 + TC_CAND, cand);
         const int64_t at = (int64_t)rx.base * TC_G;
-        const uint32_t passes = rx.n32 ? (rx.n32 + TC_TAIL - 1) / TC_TAIL : 1;
+        const bool search = !orient && rx.n32 > TC_SEARCH;
+        const TcSorted sorted = {arena + sx.off, sx.deg};
+        // the set: the hubs' bits and the first ids, then the other ids in tables that
+        // take the bits' place (alone where no hub is listed)
+        const bool narrow = rx.n16 || search || rx.n32 <= TC_TAIL;
+        const uint32_t near = narrow ? min(rx.n32, TC_TAIL) : 0u;
+        const uint32_t passes = search ? 1u : (narrow ? 1u : 0u) + (rx.n32 - near + TC_WIDE_TAIL - 1) / TC_WIDE_TAIL;
         for (uint32_t p = 0; p < passes; p++) {
-            // the set: the hubs' bits in the first pass, TC_TAIL ids in each
-            if (p == 0)
+            const bool wide = !narrow || p > 0;
+            if (wide) {
+                const uint32_t from = near + (narrow ? p - 1 : p) * TC_WIDE_TAIL;
+                tc_fill<TC_WIDE_HASH>(sh.bits, ids + at + from, min(rx.n32 - from, TC_WIDE_TAIL));
+            } else {
                 for (uint32_t i = threadIdx.x; i < rx.n16; i += BLOCK) {
                     const uint32_t q = codes[at + i];
                     atomicOr(&sh.bits[q >> 5], 1u << (q & 31));
                 }
-            if (rx.n32) {
-                for (uint32_t i = threadIdx.x; i < TC_HASH; i += BLOCK) sh.hash[i] = TC_PAD;
-                __syncthreads();
-                for (uint32_t i = p * TC_TAIL + threadIdx.x; i < min(rx.n32, (p + 1) * TC_TAIL); i += BLOCK) {
-                    const uint32_t q = ids[at + i];
-                    for (uint32_t s = tc_slot(q);; s = (s + 1) & (TC_HASH - 1)) {
-                        const uint32_t z = atomicCAS(&sh.hash[s], TC_PAD, q);
-                        if (z == TC_PAD || z == q) break;
-                    }
-                }
+                if (near && !search) tc_fill<TC_HASH>(sh.hash, ids + at, near);
             }
             for (uint32_t b = c0; b < c1; b += TC_STEP) {
                 if (threadIdx.x < TC_ORDER) sh.cls[threadIdx.x] = 0;
@@ -678,16 +766,21 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int sym, const hn_vrec*
                         const uint32_t k = sh.cls[cl[j]] + pos[j];
                         sh.y[k] = y[j];
                         sh.base[k] = ry[j].base;
-                        sh.n16[k] = p == 0 ? ry[j].n16 : 0u;   // later passes count only their ids
+                        sh.n16[k] = wide ? 0u : ry[j].n16;   // (no bits then)
                         sh.n32[k] = ry[j].n32;
                     }
                 __syncthreads();
-                if (rx.n32) tc_walk<true>(sh, nlong, n, codes, ids, per_vertex, acc);
-                else tc_walk<false>(sh, nlong, n, codes, ids, per_vertex, acc);
+                if (rx.n32 == 0) tc_walk<TC_NONE>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
+                else if (search) tc_walk<TC_SORTED>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
+                else if (wide) tc_walk<TC_HASHED_WIDE>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
+                else tc_walk<TC_HASHED>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
                 __syncthreads();
             }
         }
-        for (uint32_t i = threadIdx.x; i < rx.n16; i += BLOCK) sh.bits[codes[at + i] >> 5] = 0;
+        if (passes > 1 || !narrow)
+            for (uint32_t i = threadIdx.x; i < TC_WIDE_HASH; i += BLOCK) sh.bits[i] = 0;
+        else
+            for (uint32_t i = threadIdx.x; i < rx.n16; i += BLOCK) sh.bits[codes[at + i] >> 5] = 0;
         if (threadIdx.x == 0) sh.task = ahead;
         __syncthreads();
     }
@@ -738,34 +831,51 @@ __device__ __forceinline__ uint32_t tc_common(const TcRow& s, const TcRow& l, co
 // lanes per source.  The chain source row, entry, hub, row, list is what bounds
 // it, so a lane starts four of them at once; a thread per source, one entry after
 // the other, took 330 us on a graph of a thousand vertices.
+// A wave's sources are those of `per` vertices, its lanes' own rows: 16, one step at
+// most, or 64 where there are waves enough all the same (16 M vertices with
+// a thousand edges: 186 us with every lane reading its source's row, 51 so; four million of
+// four entries: 975, 690; R-MAT s12 is 20 % slower with 64, 16 M vertices are so with 16).
 constexpr int TC_SRC = 4;
-__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, const TcRow* __restrict__ row,
+constexpr int64_t TC_WIDE = 1 << 20;
+__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, const TcRow* __restrict__ row,
                                                          const uint16_t* __restrict__ codes,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, TcCtl* __restrict__ ctl,
                                                          unsigned long long* __restrict__ per_vertex) {
-    const int64_t u0 = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) / TC_SMALL * TC_SRC;
-    const uint32_t sub = threadIdx.x % TC_SMALL;
-    TcRow ru[TC_SRC], rv[TC_SRC];
-    uint32_t v[TC_SRC];
-#pragma unroll
-    for (int j = 0; j < TC_SRC; j++) ru[j] = u0 + j < nv ? row[u0 + j] : TcRow{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int j = 0; j < TC_SRC; j++) {
-        const uint32_t n = ru[j].len();
-        v[j] = n >= 2 && n <= TC_SMALL && sub < n ? tc_entry(ru[j], sub, codes, ids, hub) : TC_PAD;
-    }
-#pragma unroll
-    for (int j = 0; j < TC_SRC; j++)
-        rv[j] = v[j] != TC_PAD && v[j] != (uint32_t)(u0 + j) ? row[v[j]] : TcRow{0u, 0u, 0u, 0u};
+    const int lane = __lane_id(), sub = lane % TC_SMALL, team = lane / TC_SMALL;
+    const int64_t w0 = ((int64_t)blockIdx.x * NWAVES + threadIdx.x / WAVE) * per;
+    if (w0 >= nv) return;
+    const TcRow own = lane < per && w0 + lane < nv ? row[w0 + lane] : TcRow{0u, 0u, 0u, 0u};
+    const bool has = own.len() >= 2 && own.len() <= TC_SMALL;
+    const uint64_t m = __ballot(has);
+    const int nsrc = __popcll(m);
+    // lane k gets the k-th source's lane (the others fill up behind)
+    const int to = has ? __popcll(m & lanemask_lt()) : nsrc + __popcll(~m & lanemask_lt());
+    const int from = __builtin_amdgcn_ds_permute(to * 4, lane);
     uint64_t acc = 0;
+    for (int k0 = 0; k0 < nsrc; k0 += TC_SRC * (WAVE / TC_SMALL)) {
+        TcRow ru[TC_SRC], rv[TC_SRC];
+        uint32_t u[TC_SRC], v[TC_SRC];
 #pragma unroll
-    for (int j = 0; j < TC_SRC; j++) {
-        if (rv[j].len() == 0 || rv[j].len() > TC_SMALL) continue;
-        const bool mine = ru[j].len() < rv[j].len();   // the source's list is the shorter one (ties: the destination's)
-        const uint32_t c = mine ? tc_common(ru[j], rv[j], codes, ids) : tc_common(rv[j], ru[j], codes, ids);
-        if (c && per_vertex) atomicAdd(per_vertex + (mine ? (uint32_t)(u0 + j) : v[j]), (unsigned long long)c);
-        acc += c;
+        for (int j = 0; j < TC_SRC; j++) {
+            const int k = k0 + j * (WAVE / TC_SMALL) + team, l = __shfl(from, min(k, WAVE - 1), WAVE);
+            ru[j] = TcRow{(uint32_t)__shfl(own.base, l, WAVE), 0u, (uint32_t)__shfl(own.n16, l, WAVE),
+                          (uint32_t)__shfl(own.n32, l, WAVE)};
+            u[j] = (uint32_t)(w0 + l);
+            v[j] = k < nsrc && sub < (int)ru[j].len() ? tc_entry(ru[j], sub, codes, ids, hub) : TC_PAD;
+        }
+#pragma unroll
+        for (int j = 0; j < TC_SRC; j++) rv[j] = v[j] != TC_PAD && v[j] != u[j] ? row[v[j]] : TcRow{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < TC_SRC; j++) {
+            if (rv[j].len() == 0 || rv[j].len() > TC_SMALL) continue;
+            const bool mine = ru[j].len() < rv[j].len();   // the source's list is the shorter one (ties: the destination's)
+            const TcRow a = {mine ? ru[j].base : rv[j].base, 0u, mine ? ru[j].n16 : rv[j].n16, mine ? ru[j].n32 : rv[j].n32};
+            const TcRow b = {mine ? rv[j].base : ru[j].base, 0u, mine ? rv[j].n16 : ru[j].n16, mine ? rv[j].n32 : ru[j].n32};
+            const uint32_t c = tc_common(a, b, codes, ids);
+            if (c && per_vertex) atomicAdd(per_vertex + (mine ? u[j] : v[j]), (unsigned long long)c);
+            acc += c;
+        }
     }
     acc = wave_reduce_sum(acc);
     if (__lane_id() == 0 && acc) atomicAdd(&ctl->total[(blockIdx.x + threadIdx.x / WAVE) % TC_SUMS].v, (unsigned long long)acc);
@@ -808,6 +918,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4);
     const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
     const int64_t o_goff = take((nv + 1) * 4), o_mem = take(ne * 4), o_task = take(tasks * 8);
+    const int64_t o_owner = take((nv + WAVE - 1) / WAVE * 8);
     const int64_t o_scan = take((int64_t)scan_temp_bytes(nv));
     HN_TRY(g->s_tc.reserve((size_t)o));
     char* base = g->s_tc.as<char>();
@@ -828,6 +939,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     uint32_t* goff = at(o_goff, (uint32_t*)nullptr);
     uint32_t* members = at(o_mem, (uint32_t*)nullptr);
     uint2* task = at(o_task, (uint2*)nullptr);
+    uint64_t* owner = at(o_owner, (uint64_t*)nullptr);
     void* tmp = base + o_scan;
     unsigned long long* per = reinterpret_cast<unsigned long long*>(per_vertex);
     const unsigned gv = (unsigned)ceil_div(nv, BLOCK);
@@ -836,19 +948,20 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
 
     HN_HIP(hipMemsetAsync(base, 0, (size_t)o_zero_end, st));
     // 1. hubs and codes
-    HN_TRY(exclusive_scan_fn<uint32_t>(StoredGroupsIn{g->rec}, StoredGroupsOut{row, P, tile_lo}, P + nv, nv, tmp, st));
-    if (nv <= (int64_t)TC_HUBS) {
+    const bool all_hubs = nv <= (int64_t)TC_HUBS;
+    HN_TRY(exclusive_scan_fn<uint32_t>(StoredGroupsIn{g->rec},
+                                       StoredGroupsOut{g->rec, row, P, tile_lo, orient && !all_hubs ? weight : nullptr},
+                                       P + nv, nv, tmp, st));
+    if (all_hubs) {
         tc_all_hubs_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, wc, hub, ctl);
         HN_CHECK_LAUNCH();
     } else {
-        if (orient) {
-            tc_weight_deg_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, weight);
-        } else {
+        if (!orient) {
             HN_HIP(hipMemsetAsync(weight, 0, (size_t)nv * 4, st));
             const int step = (int)std::clamp<int64_t>(ne >> 18, 1, 64);
             tc_weight_freq_kernel<<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, step, weight);
+            HN_CHECK_LAUNCH();
         }
-        HN_CHECK_LAUNCH();
         tc_hist_kernel<<<gw, BLOCK, 0, st>>>(nv, weight, hist);
         HN_CHECK_LAUNCH();
         tc_cut_kernel<<<1, BLOCK, 0, st>>>(hist, ctl);
@@ -861,24 +974,25 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     else
         tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
     HN_CHECK_LAUNCH();
-    tc_pad_kernel<<<gv, BLOCK, 0, st>>>(nv, row, codes, ids);
+    tc_pad_kernel<<<gv, BLOCK, 0, st>>>(nv, row, codes, ids, owner);
     HN_CHECK_LAUNCH();
     // 3. edges owned by their destination
-    tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, part, nhub,
+    tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, owner, codes, ids, hub, gcnt, part, nhub,
                                                  place, nullptr, nullptr);
     HN_CHECK_LAUNCH();
     tc_parts_kernel<<<(unsigned)ceil_div(nhub, BLOCK), BLOCK, 0, st>>>(sym, ctl, nhub, hub, part, gcnt);
     HN_CHECK_LAUNCH();
     HN_TRY(exclusive_scan<uint32_t>(ArrayIn<uint32_t>{gcnt}, goff, nv, tmp, st));
-    tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, codes, ids, hub, gcnt, part, nhub,
+    tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, owner, codes, ids, hub, gcnt, part, nhub,
                                                 place, goff, members);
     HN_CHECK_LAUNCH();
     // 4. counts
-    HN_TRY(exclusive_scan_fn<uint32_t>(TaskIn{row, gcnt, g->rec, ctl, sym}, TaskOut{task}, &ctl->ntask, nv, tmp, st));
-    tc_owner_kernel<<<(unsigned)num_cus() * 8, BLOCK, 0, st>>>(sym, g->rec, g->arena, wc, task, row, codes, ids, hub,
-                                                               gcnt, goff, members, ctl, per);
+    HN_TRY(exclusive_scan_fn<uint32_t>(TaskIn{owner, row, gcnt, g->rec, ctl, sym}, TaskOut{task}, &ctl->ntask, nv, tmp, st));
+    tc_owner_kernel<<<(unsigned)num_cus() * 8, BLOCK, 0, st>>>(orient ? 1 : 0, sym, g->rec, g->arena, wc, task, row, codes, ids,
+                                                               hub, gcnt, goff, members, ctl, per);
     HN_CHECK_LAUNCH();
-    tc_small_kernel<<<(unsigned)ceil_div(nv, TC_SRC * BLOCK / TC_SMALL), BLOCK, 0, st>>>(nv, row, codes, ids, hub, ctl, per);
+    const int small_per = nv > TC_WIDE ? WAVE : TC_SRC * (WAVE / TC_SMALL);
+    tc_small_kernel<<<(unsigned)ceil_div(nv, (int64_t)small_per * NWAVES), BLOCK, 0, st>>>(nv, small_per, row, codes, ids, hub, ctl, per);
     HN_CHECK_LAUNCH();
     TcSum sums[TC_SUMS];
     HN_TRY(read_back(g, ctl->total, sizeof(sums), sums, st));

@@ -109,3 +109,69 @@ def test_star_of_cliques_many_tasks(hn):
     total, per = run(hn, h, False)
     do, da = O.directed_by_degree(off, adj)
     assert total == O.triangles(off, adj) and np.array_equal(per, O.tc2_per_vertex(do, da))
+
+
+@pytest.mark.parametrize("both", [True, False])
+def test_long_lists_of_ids(hn, both):
+    """Stars of 510 to 514 leaves and one of 5,000, the leaves of each in a ring
+    with its second neighbours: 70,000 vertices of one frequency, too many to be
+    hubs, so that rows on both sides of 512 hold ids only.  The leaves name
+    their centre or not."""
+    print(f"case tc long id lists both={both}", flush=True)
+    sizes = [510 + i % 5 for i in range(128)] + [5000]
+    src, dst, n = [], [], 0
+    for k in sizes:
+        leaf = n + 1 + np.arange(k)
+        src.append(np.full(k, n)), dst.append(leaf)
+        if both:
+            src.append(leaf), dst.append(np.full(k, n))
+        for d in (1, 2, k - 1, k - 2):
+            src.append(leaf), dst.append(n + 1 + (np.arange(k) + d) % k)
+        n += k + 1
+    off, adj = O.coo_to_csr(n, np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32))
+    h = hn.Hornet.from_csr(off, adj)
+    total, per = run(hn, h, True)
+    exp = O.tc2_per_vertex(off, adj)
+    assert total == int(exp.sum()) and np.array_equal(per, exp)
+
+
+def test_oriented_lists_of_ids(hn):
+    """66 cliques of 1,000 and one of 1,100: 67,100 vertices with too many of a
+    degree to be hubs, whose oriented lists lie on both sides of 512."""
+    import torch
+    print("case tc oriented id lists", flush=True)
+    src, dst, n = [], [], 0
+    for k in [1000] * 66 + [1100]:
+        i, j = np.triu_indices(k, 1)
+        src.append((i + n).astype(np.int32)), dst.append((j + n).astype(np.int32))
+        n += k
+    h = hn.Hornet.from_coo_device(n, torch.from_numpy(np.concatenate(src)).cuda(),
+                                  torch.from_numpy(np.concatenate(dst)).cuda())
+    total, per = run(hn, h, False)
+    exp = []
+    for k in (1000, 1100):
+        off, adj = complete(k)
+        exp.append(O.tc2_per_vertex(*O.directed_by_degree(off, adj)))
+    assert total == 66 * comb(1000, 3) + comb(1100, 3)
+    assert np.array_equal(per[:66000].reshape(66, 1000), np.broadcast_to(exp[0], (66, 1000)))
+    assert np.array_equal(per[66000:], exp[1])
+
+
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 37])
+def test_short_lists_of_many_vertices(hn, n):
+    """Both sides of where a wave takes 64 vertices instead of 16: a strip of
+    triangles with gaps, so that sources are few, many or none among a wave's."""
+    print(f"case tc short lists n={n}", flush=True)
+    i = np.arange(n - 2, dtype=np.int32)
+    i = i[(i // 300) % 3 != 1]
+    i = np.concatenate([i[: i.size // 2], i[i.size // 2 :][::7], [n - 3]]).astype(np.int32)
+    s, d = np.concatenate([i, i, i + 1]), np.concatenate([i + 1, i + 2, i + 2])
+    off, adj = O.coo_to_csr(n, s, d, symmetrize=True, dedup=True)
+    h = hn.Hornet.from_csr(off, adj)
+    total, per = run(hn, h, False)
+    do, da = O.directed_by_degree(off, adj)
+    exp = O.tc2_per_vertex(do, da)
+    assert total == int(exp.sum()) and np.array_equal(per, exp)
+    total, per = run(hn, h, True)
+    exp = O.tc2_per_vertex(off, adj)
+    assert total == int(exp.sum()) and np.array_equal(per, exp)
