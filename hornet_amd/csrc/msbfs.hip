@@ -778,10 +778,15 @@ __global__ __launch_bounds__(BLOCK) void ms_collect_kernel(int64_t nv, const int
 // Distances from the level codes: every one written once, in whole lines, where the
 // collects wrote them level by level over a fill of INT32_MAX (R-MAT s22, 64
 // sources: fill and collects 1,490 us; collects and this kernel 700, of which 262
-// here, 4.1 TB/s).  A lane has four vertices.  Bound by the stores.  Codes of
-// MS_DIRECT stand for distances that are there already.
+// here, 4.1 TB/s).  A lane has four vertices.  Bound by the stores, and where graphs
+// do not fit the L2, by the codes' bytes: those of vertices that no source reaches are
+// not read then (16 M vertices, few of them reached, 64 sources: 1,380 -> 1,220 us for
+// the traversal; smaller graphs 2 % slower so).  Codes of MS_DIRECT stand for distances
+// that are there already.
 constexpr int MS_DIST_IPT = 4;
+constexpr int64_t MS_DIST_LATE = 1 << 20;
 typedef int32_t DistQuad __attribute__((ext_vector_type(4), aligned(4)));
+template <bool LATE>
 __global__ __launch_bounds__(BLOCK) void ms_dist_kernel(int64_t nv, int32_t k, const MsState* S,
                                                         const uint64_t* __restrict__ visited) {
     const uint64_t* __restrict__ planes = S->planes;
@@ -794,10 +799,14 @@ __global__ __launch_bounds__(BLOCK) void ms_dist_kernel(int64_t nv, int32_t k, c
         uint64_t vis[MS_DIST_IPT], pl[MS_DIST_IPT][MS_PLANES];
 #pragma unroll
         for (int i = 0; i < MS_DIST_IPT; i++) {
-            const int64_t u = i < n ? v + i : v;
-            const ulonglong2* q = reinterpret_cast<const ulonglong2*>(planes + u * MS_PLANES);
+            vis[i] = visited[i < n ? v + i : v];
+            pl[i][0] = pl[i][1] = pl[i][2] = pl[i][3] = 0;
+        }
+#pragma unroll
+        for (int i = 0; i < MS_DIST_IPT; i++) {
+            if (LATE && !vis[i]) continue;
+            const ulonglong2* q = reinterpret_cast<const ulonglong2*>(planes + (i < n ? v + i : v) * MS_PLANES);
             const ulonglong2 x = q[0], y = q[1];
-            vis[i] = visited[u];
             pl[i][0] = x.x;
             pl[i][1] = x.y;
             pl[i][2] = y.x;
@@ -1431,8 +1440,9 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
         for (int64_t c = 0; c < next; c++) HN_HIP(hipGraphLaunch(step.exec, st));
         rep += next;
         if (planes) {
-            ms_dist_kernel<<<(unsigned)std::min<int64_t>(ceil_div(nv, BLOCK * MS_DIST_IPT), (int64_t)num_cus() * 16), BLOCK,
-                             0, st>>>(nv, k, e->S, e->visited);
+            const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(nv, BLOCK * MS_DIST_IPT), (int64_t)num_cus() * 16);
+            if (nv > MS_DIST_LATE) ms_dist_kernel<true><<<blocks, BLOCK, 0, st>>>(nv, k, e->S, e->visited);
+            else ms_dist_kernel<false><<<blocks, BLOCK, 0, st>>>(nv, k, e->S, e->visited);
             HN_CHECK_LAUNCH();
         }
         HN_TRY(ms_read(e, e->S, sizeof(MsState), &s, st));

@@ -69,3 +69,18 @@ def test_depth_limits(hn, limit):
         limits = limits.astype(np.int32)
         got = ms.run(srcs, depth_limits=limits).cpu().numpy()
         assert np.array_equal(got, expected(off, adj, srcs, limits))
+
+
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 3])
+def test_few_reached_of_many(hn, n):
+    """Both sides of where the codes of unreached vertices are not read."""
+    print("case msbfs few reached", n, flush=True)
+    rng = np.random.default_rng(n)
+    s, d = rng.integers(0, n, 3000).astype(np.int32), rng.integers(0, n, 3000).astype(np.int32)
+    v = np.arange(n - 40, n - 1, dtype=np.int32)   # a path that ends in the last vertex
+    off, adj = O.coo_to_csr(n, np.concatenate([s, v]), np.concatenate([d, v + 1]))
+    h = hn.Hornet.from_csr(off, adj)
+    srcs = np.concatenate([s[:15], v[:1], v[-1:]]).astype(np.int32)
+    ms = hn.BfsMulti(h)
+    for _ in range(2):
+        assert np.array_equal(ms.run(srcs).cpu().numpy(), expected(off, adj, srcs))
