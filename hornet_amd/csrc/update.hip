@@ -594,7 +594,8 @@ struct EraseDeferIn {
 
 // scan output of the deferred counts: each tile's count and offset in the side
 // buffer; the last tile also records the total, and stops the batch if that is
-// more than the side buffer holds (no count is made after it: see defer_offsets)
+// more than the side buffer holds (no count is made after it: see
+// item_and_defer_offsets)
 struct SideOut {
     uint32_t* tcnt;
     int64_t* P;
@@ -1034,13 +1035,16 @@ struct TileCountIn {
     __device__ __forceinline__ int64_t operator()(int64_t t) const { return (int64_t)c[t]; }
 };
 
-// Deferred counts of the copy tiles and their prefix.  One workgroup's scan counts as
-// it goes; the two readings of a larger one would count twice, sixteen tiles to a
-// lane (500 K tiles of an R-MAT s24 erase: 290 us, 25 with the counts on their own).
-template <typename Defer>
-static hn_status defer_offsets(Defer in, UpdBufs& b, int64_t ntiles, int64_t cap, hipStream_t st) {
+// The copies' items (scan `items`), then the deferred counts of their tiles and these
+// counts' prefix.  One workgroup's scan counts as it goes, in the launch of the items'
+// where that is one workgroup's too; the two readings of a larger one would count twice, sixteen
+// tiles to a lane (500 K tiles of an R-MAT s24 erase: 290 us, 25 with the counts on their own).
+template <typename Items, typename Defer>
+static hn_status item_and_defer_offsets(const Items& items, Defer in, UpdBufs& b, int64_t ntiles, int64_t cap,
+                                        hipStream_t st) {
     const SideOut out{b.tcnt, b.doff, ntiles - 1, cap, b.sc};
-    if (ntiles <= SCAN_ONE) return exclusive_scan_fn<int64_t>(in, out, b.doff + ntiles, ntiles, b.tmp, st);
+    if (ntiles <= SCAN_ONE) return exclusive_scan_two(items, scan_of<int64_t>(in, out, b.doff + ntiles, ntiles), b.tmp, st);
+    HN_TRY(exclusive_scan_fn<int64_t>(items.in, items.out, items.total, items.n, b.tmp, st));
     defer_kernel<<<(unsigned)ceil_div(ntiles, BLOCK), BLOCK, 0, st>>>(ntiles, in, b.tcnt);
     HN_CHECK_LAUNCH();
     return exclusive_scan_fn<int64_t>(TileCountIn{b.tcnt}, out, b.doff + ntiles, ntiles, b.tmp, st);
@@ -1347,11 +1351,11 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
     HN_CHECK_LAUNCH();
     uint32_t* ubk = b.dlp;
     uint32_t* nb = b.nkeep;   // entries kept
-    HN_TRY(exclusive_scan_fn<uint32_t>(ArrayIn<uint32_t>{b.dpos}, CompactOut{keys, b.kb, b.ia, b.ib, b.dlen, ubk}, nb,
-                                       n, b.tmp, st));
     // 2. segments by source
-    HN_TRY(exclusive_scan_fn<uint32_t>(SegStartIn{b.kb, nb, f.sbits}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key},
-                                       b.spos + n, n, b.tmp, st));
+    HN_TRY(exclusive_scan_two(
+        scan_of<uint32_t>(ArrayIn<uint32_t>{b.dpos}, CompactOut{keys, b.kb, b.ia, b.ib, b.dlen, ubk}, nb, n),
+        scan_of<uint32_t>(SegStartIn{b.kb, nb, f.sbits}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key}, b.spos + n, n),
+        b.tmp, st));
     uint32_t* ucnt = b.spos + n;
     // 3. in place or new blocks
     uint32_t* stamp = nullptr;
@@ -1377,13 +1381,12 @@ static hn_status insert_once(hn_graph* g, const int32_t* src, const int32_t* dst
     // 4. the old entries that move, in place in one pass (the few that could
     // overwrite a slot a later copy tile has not read go through a side
     // buffer), then the batch entries into the slots left between them
-    HN_UNDO_TRY(exclusive_scan_fn<int64_t>(MoveLenIn{b.ti, ucnt, b.sc}, RunOut{b.wpos, b.tile_lo}, b.wpos + n, n,
-                                           b.tmp, st));
     const int64_t nt = b.ntile_max;
     SideBuf side;
     HN_UNDO_TRY(side_buffer(g, b, 0, &side));
-    HN_UNDO_TRY(defer_offsets(InsertDeferIn{n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, g->arena, b.sc}, b, nt,
-                              side.cap, st));
+    HN_UNDO_TRY(item_and_defer_offsets(
+        scan_of<int64_t>(MoveLenIn{b.ti, ucnt, b.sc}, RunOut{b.wpos, b.tile_lo}, b.wpos + n, n),
+        InsertDeferIn{n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, g->arena, b.sc}, b, nt, side.cap, st));
     auto rewrite = [&]() -> hn_status {
         insert_move_kernel<<<(unsigned)num_cus() * COPY_GRID_PER_CU, BLOCK, 0, st>>>(
             n, b.wpos, b.tile_lo, b.ti, b.seg_start, b.kb, f, b.tcnt, b.doff, g->arena, side.entry, side.dst, b.sc,
@@ -1446,11 +1449,12 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
     const unsigned gridn = (unsigned)ceil_div(n + 1, BLOCK);
     // 1. optional in-batch dedup -> kb
     uint32_t* nb = b.nkeep;
-    HN_TRY(exclusive_scan_fn<uint32_t>(FirstKeepIn{keys, (flags & HN_DEDUP_BATCH) ? 1 : 0},
-                                       CompactOut{keys, b.kb, nullptr, nullptr, nullptr, nullptr}, nb, n, b.tmp, st));
     // 2. distinct keys with multiplicities
-    HN_TRY(exclusive_scan_fn<uint32_t>(SegStartIn{b.kb, nb, 64}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key},
-                                       b.spos + n, n, b.tmp, st));
+    HN_TRY(exclusive_scan_two(
+        scan_of<uint32_t>(FirstKeepIn{keys, (flags & HN_DEDUP_BATCH) ? 1 : 0},
+                          CompactOut{keys, b.kb, nullptr, nullptr, nullptr, nullptr}, nb, n),
+        scan_of<uint32_t>(SegStartIn{b.kb, nb, 64}, SegOut{b.kb, nb, b.spos, b.seg_start, b.seg_key}, b.spos + n, n),
+        b.tmp, st));
     uint32_t* dcnt = b.spos + n;
     // 3. stored ranges and deletion counts per distinct key
     erase_locate_kernel<<<gridn, BLOCK, 0, st>>>(dcnt, b.seg_start, b.seg_key, f, g->rec, g->arena, b.dpos, b.dlen,
@@ -1487,14 +1491,14 @@ static hn_status erase_once(hn_graph* g, const int32_t* src, const int32_t* dst,
     erase_gaps_kernel<<<gridn, BLOCK, 0, st>>>(dcnt, ucnt, b.seg2_start, b.tpos, b.dpos, b.dlen, b.dlp, b.ti, b.skip,
                                                b.glen, b.gsrc, b.gdst, b.rtail, b.sc);
     HN_UNDO_LAUNCH();
-    HN_UNDO_TRY(exclusive_scan_fn<int64_t>(GapLenIn{b.glen, dcnt, ucnt}, RunOutT<ERASE_TILE>{b.gP, b.tile_lo},
-                                           b.gP + 2 * n, 2 * n, b.tmp, st));
     // 7. in-place compaction in one pass; the few entries that would overwrite
     // a source of an earlier tile go through a side buffer
     const int64_t nt = b.ntile_max;
     SideBuf side;
     HN_UNDO_TRY(side_buffer(g, b, 0, &side));
-    HN_UNDO_TRY(defer_offsets(EraseDeferIn{2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.rtail, b.sc}, b, nt, side.cap, st));
+    HN_UNDO_TRY(item_and_defer_offsets(
+        scan_of<int64_t>(GapLenIn{b.glen, dcnt, ucnt}, RunOutT<ERASE_TILE>{b.gP, b.tile_lo}, b.gP + 2 * n, 2 * n),
+        EraseDeferIn{2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst, b.rtail, b.sc}, b, nt, side.cap, st));
     auto rewrite = [&]() -> hn_status {
         auto copy = [&](auto kernel) {
             kernel<<<(unsigned)num_cus() * COPY_GRID_PER_CU, BLOCK, 0, st>>>(2 * n, b.gP, b.tile_lo, b.gsrc, b.gdst,

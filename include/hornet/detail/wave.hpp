@@ -251,11 +251,9 @@ __global__ __launch_bounds__(BLOCK) void scan_down_fn_kernel(InFn in, Cnt cnt, c
 constexpr int SCAN_ONE_BLOCK = 1024;
 constexpr int SCAN_ONE_IPT = 8;
 constexpr int64_t SCAN_ONE = (int64_t)SCAN_ONE_BLOCK * SCAN_ONE_IPT;
-template <typename Out, typename InFn, typename OutFn, typename Cnt>
-__global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_one_kernel(InFn in, Cnt cnt, OutFn out, Out* __restrict__ total) {
-    constexpr int WAVES = SCAN_ONE_BLOCK / WAVE;
-    __shared__ Out wtot[WAVES];
-    const int64_t n = cnt.get();   // <= SCAN_ONE
+constexpr int SCAN_ONE_WAVES = SCAN_ONE_BLOCK / WAVE;
+template <typename Out, typename InFn, typename OutFn>
+__device__ __forceinline__ void scan_one(InFn in, int64_t n, OutFn out, Out* total, Out* wtot) {
     const int w = threadIdx.x / WAVE;
     const int l = __lane_id();
     // a wave's rows of 64 are consecutive; as few rows as hold n
@@ -278,7 +276,7 @@ __global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_one_kernel(InFn in, Cnt c
     if (l == 0) wtot[w] = carry;
     __syncthreads();
     Out off = 0, tot = 0;
-    for (int k = 0; k < WAVES; k++) {
+    for (int k = 0; k < SCAN_ONE_WAVES; k++) {
         const Out t = wtot[k];
         off += k < w ? t : (Out)0;
         tot += t;
@@ -290,6 +288,31 @@ __global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_one_kernel(InFn in, Cnt c
         if (i < n) out(i, (Out)(off + pre[j]), val[j]);
     }
     if (threadIdx.x == 0) *total = tot;
+}
+template <typename Out, typename InFn, typename OutFn, typename Cnt>
+__global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_one_kernel(InFn in, Cnt cnt, OutFn out, Out* __restrict__ total) {
+    __shared__ Out wtot[SCAN_ONE_WAVES];
+    scan_one<Out>(in, cnt.get(), out, total, wtot);   // cnt.get() <= SCAN_ONE
+}
+
+// Two of them, the second over what the first wrote, in one launch (the stream's
+// batches are chains of such launches of 4 to 5 us each: 1,000 pairs each way into an
+// R-MAT s16 and out of it, 249 us with four such pairs as eight launches, 237 so).
+template <typename T, typename InFn, typename OutFn>
+struct ScanOf {
+    using Out = T;
+    InFn in;
+    OutFn out;
+    T* total;
+    int64_t n;   // <= SCAN_ONE
+};
+template <typename A, typename B>
+__global__ __launch_bounds__(SCAN_ONE_BLOCK) void scan_two_kernel(A a, B b) {
+    __shared__ typename A::Out wa[SCAN_ONE_WAVES];
+    __shared__ typename B::Out wb[SCAN_ONE_WAVES];
+    scan_one<typename A::Out>(a.in, a.n, a.out, a.total, wa);
+    __syncthreads();
+    scan_one<typename B::Out>(b.in, b.n, b.out, b.total, wb);
 }
 
 template <typename Out>

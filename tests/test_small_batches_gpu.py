@@ -57,3 +57,28 @@ def test_fields_keep_the_order_of_equal_pairs(hn, n):
     order = np.lexsort((f, bd, bs))
     assert np.array_equal(s.cpu().numpy(), bs[order]) and np.array_equal(d.cpu().numpy(), bd[order])
     assert np.array_equal(m[0].cpu().numpy(), f[order])
+
+
+@pytest.mark.parametrize("scale", [10, 19])
+@pytest.mark.parametrize("n", [100, 4095, 4096])
+def test_there_and_back(hn, scale, n):
+    """Gaps of an erase on both sides of one workgroup's scan, and copy tiles
+    (s19: 15 M entries) that are too many for one where the batch is not."""
+    import torch
+    print("case small batch there and back", scale, n, flush=True)
+    h = hn.Hornet.rmat(scale, 3, edge_factor=16)
+    off, adj = (x.clone() for x in h.getCSR())
+    rng = np.random.default_rng(n)
+    v = 1 << scale
+    s = torch.from_numpy(rng.integers(0, v, n).astype(np.int32)).cuda()
+    d = torch.from_numpy(rng.integers(0, v, n).astype(np.int32)).cuda()
+    src = torch.repeat_interleave(torch.arange(v, device="cuda"), off[1:] - off[:-1])
+    old = src * v + adj
+    new = torch.unique(s.long() * v + d)
+    both = torch.unique(torch.cat([old, new]))
+    h.insert(hn.BatchUpdate(s, d), True, True)
+    cs, cd = h.getCOO()
+    assert torch.equal(cs.long() * v + cd, both)
+    h.erase(hn.BatchUpdate(s, d), True)
+    cs, cd = h.getCOO()
+    assert torch.equal(cs.long() * v + cd, old[~torch.isin(old, new)])
