@@ -559,13 +559,18 @@ enum TcTail { TC_NONE, TC_HASHED, TC_HASHED_WIDE, TC_SORTED };
 struct TcSorted {   // an owner's stored row
     const int32_t* entry;
     int32_t deg;
+    const uint2* wc;    // where only the entries up the degree order are in its list, else null
+    uint32_t owner;
     __device__ __forceinline__ bool has(uint32_t q) const {
         int32_t lo = 0, hi = deg;
         while (lo < hi) {
             const int32_t mid = (lo + hi) >> 1;
             if ((uint32_t)entry[mid] < q) lo = mid + 1; else hi = mid;
         }
-        return lo < deg && (uint32_t)entry[lo] == q;
+        if (lo == deg || (uint32_t)entry[lo] != q) return false;
+        if (!wc) return true;
+        const uint32_t w = wc[q].x;
+        return (uint32_t)deg < w || ((uint32_t)deg == w && owner < q);
     }
 };
 template <TcTail TAIL>
@@ -662,7 +667,8 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, co
                                                          unsigned long long* __restrict__ per_vertex) {
     __shared__ OwnerShared sh;
     const uint32_t ntask = ctl->ntask;
-    const bool stored = sym && !ctl->repeats;
+    const bool repeats = ctl->repeats != 0;
+    const bool stored = sym && !repeats;
     uint64_t acc = 0;
     for (int i = threadIdx.x; i < (int)(TC_HUBS + 1) / 32; i += BLOCK) sh.bits[i] = 0;
     // The next task is taken while this one runs.  Tickets are for `chunk` tasks, of
@@ -702,8 +708,10 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, co
         const uint32_t lx = rx.len(), cand = stored ? (uint32_t)sx.deg : lx + gcnt[x];
         const uint32_t c0 = tk.y * TC_CAND, c1 = min(c0 + TC_CAND, cand);
         const int64_t at = (int64_t)rx.base * TC_G;
-        const bool search = !orient && rx.n32 > TC_SEARCH;
-        const TcSorted sorted = {arena + sx.off, sx.deg};
+        // An entry that is stored twice must not lie in two tables, or it counts twice:
+        // with repeats, what does not fit one table is searched.
+        const bool search = repeats ? rx.n32 > (rx.n16 ? TC_TAIL : TC_WIDE_TAIL) : !orient && rx.n32 > TC_SEARCH;
+        const TcSorted sorted = {arena + sx.off, sx.deg, orient ? wc : nullptr, x};
         // the set: the hubs' bits and the first ids, then the other ids in tables that
         // take the bits' place (alone where no hub is listed)
         const bool narrow = rx.n16 || search || rx.n32 <= TC_TAIL;
