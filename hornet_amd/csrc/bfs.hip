@@ -67,6 +67,7 @@
 #include <hip/hip_ext.h>
 
 #include "bfs.hpp"
+#include "bfs_pulls.hpp"
 #include "prims.hpp"
 
 namespace hn {
@@ -107,16 +108,12 @@ inline int any_shift_for(int64_t nv) { return nv <= (1 << 24) ? 7 : nv <= (1 << 
 static_assert(UNIT_SLOTS % EXP_G == 0, "groups must not straddle a block start");
 typedef int32_t AdjVec __attribute__((ext_vector_type(EXP_G)));
 
-// ---- one workgroup, many levels (bfs_small_kernel)
-#ifndef BFS_SMALL_W
-#define BFS_SMALL_W 4096         // groups of a frontier that one workgroup expands
-#endif
+// ---- one workgroup, many levels (bfs_small_kernel): up to SM_W groups
 #ifndef BFS_SMALL_DENSE_W
-#define BFS_SMALL_DENSE_W 1024   // ... where they average more than two groups a vertex
+#define BFS_SMALL_DENSE_W 1024   // ... and this many where they average more than two groups a vertex
 #endif
 constexpr int SM_BLOCK = 1024;
 constexpr int SM_IPT = 4;                      // groups per lane in flight
-constexpr uint32_t SM_W = BFS_SMALL_W;
 constexpr uint32_t SM_DENSE_W = BFS_SMALL_DENSE_W;
 constexpr int SM_CAP = 4096;                   // frontier entries held in LDS (two levels' worth, 64 KB)
 constexpr int64_t SM_NE = 0xFFFF0000;          // group prefixes are kept in 30 bits
@@ -221,27 +218,10 @@ __device__ __forceinline__ uint8_t probe_u8(__amdgpu_buffer_rsrc_t r, uint32_t o
     return (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(r, (int)off, 0, 0);
 }
 
-// Whether a round pulls (every unreached vertex looks for a reached neighbour)
-// instead of pushing (every frontier vertex marks its neighbours).  Every
-// kernel that asks passes the same counters of the control block, so they
-// agree.  Estimated device time in ps: a push takes about 7 per frontier entry
-// and 20 per discovery, whose frontier entry the collect writes (R-MAT s24: 45 M
-// entries, 4.4 M discoveries, 320 + 100 us); a pull reads every record (4 per
-// vertex) and the first line of every unreached vertex with edges (25; about
-// half of an R-MAT's vertices have none, which the first pull finds out, so 16
-// per vertex not reached), and ne / (frontier entries) slots of each on average
-// before it meets the frontier, fewer in skewed graphs, whose rows begin with
-// the hubs (0.5 per slot).  Pulling follows the stored entries backwards, so
-// only adjacency known to be symmetric pulls.
+// Pulling follows the stored entries backwards, so only adjacency known to be
+// symmetric pulls (sym).
 __device__ __forceinline__ bool bfs_pulls(const BfsRound& rd, int64_t nv, int64_t ne, int32_t sym) {
-    const uint32_t W = (uint32_t)rd.fc;
-    if (!sym || W <= SM_W) return false;
-    const float mf = 4.0f * (float)W;
-    const float mu = fmaxf((float)ne - (float)rd.scan - mf, 0.0f);
-    const float nu = (float)(nv - (int64_t)rd.vis - (int64_t)(rd.fc >> 32));
-    const float touch = fminf(nu, mu);
-    const float slots = fminf(mu, touch * ((float)ne / mf));
-    return 4.0f * (float)nv + 16.0f * touch + 0.5f * slots < 7.0f * mf + 20.0f * fminf(mf, touch);
+    return sym && hn::bfs_pulls(rd.fc >> 32, (uint32_t)rd.fc, rd.scan, rd.vis, nv, ne);
 }
 
 // the frontier slice of a tile: group prefix, adjacency offset in 128-byte
