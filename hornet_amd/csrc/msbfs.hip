@@ -1086,8 +1086,8 @@ struct MsEngine {
     struct Step {
         hipGraphExec_t exec = nullptr;
         hipStream_t stream = nullptr;
-        const int32_t* arena = nullptr;   // the edge arena it reads (it moves when it grows)
         MsParams params{};
+        const void* buf[5] = {};          // what it names that may move
     } step[2];
     Scratch planes;                   // level codes (batches with distances)
     MsParams params{};
@@ -1103,8 +1103,6 @@ struct MsEngine {
     unsigned long long* digest = nullptr;    // digest mode: per source {reached, sum, max}
     Scratch side_uw, side_sm;         // side records (u, w) and source masks
     Scratch w_keys, w_alt, w_tmp, w_seg, w_e0, w_E, w_chg, w_ckey, w_cE, w_cS, w_sflag;
-    void* exec_cS = nullptr;          // window buffers the captured level step was built with
-    void* exec_ckey = nullptr;
     int64_t w_n = 0;                  // entries of the open window
     uint64_t* w_sorted = nullptr;     // its sorted keys (in w_keys or w_alt)
     bool has_window = false;
@@ -1319,8 +1317,6 @@ static hipError_t ms_level(MsEngine* e, const MsParams& P, bool side, hipStream_
     if (P.ipt == 2) expand(std::integral_constant<int, 2>());
     else if (P.ipt == 6) expand(std::integral_constant<int, 6>());
     else expand(std::integral_constant<int, 4>());
-    e->exec_cS = e->w_cS.ptr;
-    e->exec_ckey = e->w_ckey.ptr;
     if (P.T != MS_NO_HEAVY)
         ms_pull_heavy_kernel<<<wgrid, BLOCK, 0, st>>>(words, e->S, e->hbits, g->rec, g->arena, e->frontier, e->visited,
                                                       e->dirty, e->next);
@@ -1395,7 +1391,10 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
     MsParams L = P;
     std::fill(std::begin(L.depth_limit), std::end(L.depth_limit), 0);
     MsEngine::Step& step = e->step[e->has_window ? 1 : 0];
-    const bool same = step.exec && step.stream == st && step.arena == g->arena &&
+    // (the edge arena and a window's buffers move when they grow)
+    const void* const buf[] = {g->arena, e->w_ckey.ptr, e->w_cS.ptr, e->side_uw.ptr, e->side_sm.ptr};
+    static_assert(sizeof(buf) == sizeof(step.buf), "one entry each");
+    const bool same = step.exec && step.stream == st && std::memcmp(step.buf, buf, sizeof(buf)) == 0 &&
                       std::memcmp(&step.params, &L, sizeof(L)) == 0;
     if (!same) {
         if (step.exec) (void)hipGraphExecDestroy(step.exec);
@@ -1417,7 +1416,7 @@ static hn_status ms_run_on(MsEngine* e, const int32_t* sources, int32_t k, const
             return HN_E_HIP;
         }
         step.stream = st;
-        step.arena = g->arena;
+        std::copy(std::begin(buf), std::end(buf), step.buf);
         step.params = L;
     }
     // Replay.  The first poll of the state comes after as many steps as the last
@@ -1553,14 +1552,8 @@ hn_status ms_window_end(MsEngine* e, int32_t m, uint64_t failed, const uint64_t*
     // sources per changed pair; the pairs absent from storage become side records
     HN_TRY(e->w_cS.reserve((size_t)(nchg > 0 ? nchg : 1) * 8));
     HN_TRY(e->w_sflag.reserve((size_t)(2 * (int64_t)nchg + 2) * 4 + 256));
-    void* old_uw = e->side_uw.ptr;
-    void* old_sm = e->side_sm.ptr;
     HN_TRY(e->side_uw.reserve((size_t)(nchg > 0 ? nchg : 1) * 8));
     HN_TRY(e->side_sm.reserve((size_t)(nchg > 0 ? nchg : 1) * 8));
-    if (e->side_uw.ptr != old_uw || e->side_sm.ptr != old_sm || e->w_cS.ptr != e->exec_cS ||
-        e->w_ckey.ptr != e->exec_ckey) {   // the captured level step holds these pointers
-        e->drop_steps();
-    }
     set_u32_kernel<<<1, 1, 0, st>>>(e->d_nchg, nchg);
     HN_CHECK_LAUNCH();
     if (nchg > 0) {
