@@ -717,6 +717,14 @@ hn_status read_back(hn_graph* g, const void* dptr, size_t bytes, void* host, hip
     return HN_OK;
 }
 
+// waits for all work on `dev`, whichever device is current
+static bool wait_device(int dev) {
+    int cur = 0;
+    if (hipGetDevice(&cur) != hipSuccess || (cur != dev && hipSetDevice(dev) != hipSuccess)) return false;
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    return (cur == dev || hipSetDevice(cur) == hipSuccess) && idle;
+}
+
 // give: dput where the device is idle
 static void destroy_graph(hn_graph* g, void (*give)(void*) = dfree) {
     if (!g) return;
@@ -850,7 +858,8 @@ static hn_status new_graph(int32_t nv, hn_graph** out) {
     preload_code_objects();
     hn_graph* g = new hn_graph();
     g->nv = nv;
-    hipError_t e = page_take(reinterpret_cast<void**>(&g->h_pinned));
+    hipError_t e = hipGetDevice(&g->dev);
+    if (e == hipSuccess) e = page_take(reinterpret_cast<void**>(&g->h_pinned));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         g->h_pinned = nullptr;
@@ -1293,7 +1302,7 @@ hn_status hn_graph_create_coo(int32_t nv, int64_t m, const int32_t* src, const i
 
 hn_status hn_graph_destroy(hn_graph* g) {
     if (g) {
-        destroy_graph(g, hipDeviceSynchronize() == hipSuccess ? dput : dfree);
+        destroy_graph(g, wait_device(g->dev) ? dput : dfree);
     }
     return HN_OK;
 }

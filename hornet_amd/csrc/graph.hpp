@@ -182,6 +182,7 @@ struct hn_graph {
     hn::Scratch s_mstage;             // staging of edge meta-data during updates
     hn::Scratch s_stamp;              // per vertex: its source segment in the current batch (unchecked)
     uint64_t* h_pinned = nullptr;     // small pinned readback area
+    int dev = 0;                      // the device it lives on
     // whole-device rounds of the last single-source BFS (-1: none yet): how many
     // the next one queues at first (serving slots run BFS concurrently, hence atomic)
     std::atomic<int> bfs_last_rounds{-1};

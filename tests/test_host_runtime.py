@@ -86,3 +86,20 @@ for k in range(8):                    # one reservation further each time
     assert window(10) == 0
     assert fake.fake_stale() == 0, (k, fake.fake_stale())
 """)
+
+
+@pytest.mark.parametrize("current", [0, 1])
+def test_destroy_waits_for_the_graphs_device(fake, current):
+    """Freed blocks are kept for reuse: the wait before that is for the device that they
+    are on, whichever is current."""
+    program(fake, f"current = {current}" + r"""
+fake.hipSetDevice(1)
+g = graph()
+fake.hipSetDevice(current)
+fake.fake_clear_trace()
+ok(lib.hn_graph_destroy(g))
+assert fake.fake_trace() == b"wait@1 ", fake.fake_trace()   # and nothing went back to the driver
+d = c_int32(-1)
+fake.hipGetDevice(byref(d))
+assert d.value == current
+""")
