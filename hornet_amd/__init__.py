@@ -12,7 +12,7 @@ def __getattr__(name):
     # torch is imported lazily so that the ABI can be inspected without it
     if name in ("Hornet", "HornetInit", "BatchUpdate", "BatchUpdatePtr", "BfsTopDown", "BfsMulti",
                 "TriangleCounting2", "StaticAlgorithm", "rmat_pairs_device", "chung_lu_pairs_device",
-                "uniform_pairs_device", "INF"):
+                "uniform_pairs_device", "trim_memory", "INF"):
         from . import graph
         return getattr(graph, name)
     raise AttributeError(name)

@@ -117,6 +117,7 @@ SIGNATURES = {
     "hn_graph_export_coo_meta": [P, P, P, P, I64, PI64, P],
     "hn_graph_insert_meta": [P, P, P, P, I64, U32, PI64, P],
     "hn_graph_destroy": [P],
+    "hn_memory_trim": [],
     "hn_graph_nv": [P, PI32],
     "hn_graph_ne": [P, PI64],
     "hn_graph_device_view": [P, ctypes.POINTER(HnDview)],

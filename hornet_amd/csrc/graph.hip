@@ -31,7 +31,7 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 // class (steps of an eighth, so that at most 12.5 % of a block lies idle), POOL_BYTES
 // of them at most, oldest out first.  They go back to the driver when they have not
 // been asked for during POOL_AGE frees, when an allocation here fails (it is then tried
-// again), and with the process.
+// again), with hn_memory_trim, and with the process.
 // Only dput keeps a block.  Its callers have waited for all work on it, as hipFree
 // does by itself, so that whichever stream or thread gets it next finds none.
 namespace {
@@ -1304,6 +1304,11 @@ hn_status hn_graph_destroy(hn_graph* g) {
     if (g) {
         destroy_graph(g, wait_device(g->dev) ? dput : dfree);
     }
+    return HN_OK;
+}
+
+hn_status hn_memory_trim(void) {
+    dtrim();
     return HN_OK;
 }
 

@@ -35,6 +35,19 @@ def _dev() -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def trim_memory() -> None:
+    """Gives the device memory that the library keeps of released graphs back to the driver."""
+    call("hn_memory_trim")
+
+
+def _empty(n: int, dtype=torch.int32) -> torch.Tensor:
+    try:
+        return torch.empty(n, dtype=dtype, device=_dev())
+    except torch.OutOfMemoryError:   # once more without what the library keeps
+        trim_memory()
+        return torch.empty(n, dtype=dtype, device=_dev())
+
+
 def _stream(stream=None):
     s = stream if stream is not None else torch.cuda.current_stream()
     return ctypes.c_void_p(s.cuda_stream)
@@ -364,7 +377,7 @@ class Hornet:
         return d.value
 
     def degrees(self) -> torch.Tensor:
-        out = torch.empty(max(self.nV(), 1), dtype=torch.int32, device=_dev())
+        out = _empty(max(self.nV(), 1))
         call("hn_graph_degrees", self._h, _ptr(out), _stream())
         return out[: self.nV()]
 
@@ -379,13 +392,13 @@ class Hornet:
         with meta=True also a list of the meta-data fields (int32 / int64 tensors
         holding the fields' bits)."""
         ne = self.nE()
-        src = torch.empty(max(ne, 1), dtype=torch.int32, device=_dev())
-        dst = torch.empty(max(ne, 1), dtype=torch.int32, device=_dev())
+        src = _empty(max(ne, 1))
+        dst = _empty(max(ne, 1))
         n = ctypes.c_int64()
         if not meta:
             call("hn_graph_export_coo", self._h, _ptr(src), _ptr(dst), ne, ctypes.byref(n), _stream())
             return src[:ne], dst[:ne]
-        fields = [torch.empty(max(ne, 1), dtype=torch.int64 if b == 8 else torch.int32, device=_dev())
+        fields = [_empty(max(ne, 1), torch.int64 if b == 8 else torch.int32)
                   for b in self.edge_meta_bytes()]
         ptrs = _ptr_array([t.data_ptr() for t in fields])
         call("hn_graph_export_coo_meta", self._h, _ptr(src), _ptr(dst), ptrs, ne, ctypes.byref(n), _stream())
@@ -393,8 +406,8 @@ class Hornet:
 
     def getCSR(self):
         nv, ne = self.nV(), self.nE()
-        off = torch.empty(nv + 1, dtype=torch.int64, device=_dev())
-        adj = torch.empty(max(ne, 1), dtype=torch.int32, device=_dev())
+        off = _empty(nv + 1, torch.int64)
+        adj = _empty(max(ne, 1))
         call("hn_graph_export_csr", self._h, _ptr(off), _ptr(adj), ne, _stream())
         return off, adj[:ne]
 
@@ -495,7 +508,7 @@ class BfsTopDown(StaticAlgorithm):
 
     def __init__(self, hornet: Hornet):
         super().__init__(hornet)
-        self.d_distances = torch.empty(max(hornet.nV(), 1), dtype=torch.int32, device=_dev())
+        self.d_distances = _empty(max(hornet.nV(), 1))
         self.bfs_source = 0
         self.stats = _lib.HnBfsStats()
 
@@ -533,7 +546,7 @@ class TriangleCounting2(StaticAlgorithm):
         self.total = 0
 
     def init(self):
-        self.triPerVertex = torch.zeros(max(self.hornet.nV(), 1), dtype=torch.int64, device=_dev())
+        self.triPerVertex = _empty(max(self.hornet.nV(), 1), torch.int64).zero_()
 
     def reset(self):
         if self.triPerVertex is not None:
@@ -581,7 +594,7 @@ class BfsMulti:
     def _buf(self, k: int) -> torch.Tensor:
         n = k * max(self.hornet.nV(), 1)
         if self._dist is None or self._dist.numel() < n:
-            self._dist = torch.empty(n, dtype=torch.int32, device=_dev())
+            self._dist = _empty(n)
         return self._dist[:n]
 
     def run(self, sources, depth_limits=None, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -626,8 +639,8 @@ def rmat_pairs_device(scale: int, seed: int, edge_factor: int = 16, first: int =
     m = edge_factor << scale
     if count is None:
         count = m - first
-    src = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
-    dst = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
+    src = _empty(max(count, 1))
+    dst = _empty(max(count, 1))
     call("hn_gen_rmat_pairs", int(scale), int(first), int(count), int(seed), _ptr(src), _ptr(dst),
          _stream())
     return src[:count], dst[:count]
@@ -713,14 +726,14 @@ class Server:
 
 
 def chung_lu_pairs_device(n: int, count: int, seed: int, gamma: float = 2.1):
-    src = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
-    dst = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
+    src = _empty(max(count, 1))
+    dst = _empty(max(count, 1))
     call("hn_gen_chung_lu_pairs", int(n), float(gamma), 0, int(count), int(seed), _ptr(src), _ptr(dst), _stream())
     return src[:count], dst[:count]
 
 
 def uniform_pairs_device(n: int, count: int, seed: int):
-    src = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
-    dst = torch.empty(max(count, 1), dtype=torch.int32, device=_dev())
+    src = _empty(max(count, 1))
+    dst = _empty(max(count, 1))
     call("hn_gen_uniform_pairs", int(n), int(count), int(seed), _ptr(src), _ptr(dst), _stream())
     return src[:count], dst[:count]

@@ -145,6 +145,23 @@ private:
     const void* _meta[HN_MAX_EDGE_META] = {};
 };
 
+namespace detail {
+// hipMalloc, and once more when the memory that the library keeps has been given back
+inline hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        (void)hn_memory_trim();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+template <typename T>
+void allocate(T*& p, size_t bytes, const char* where) {
+    check(device_malloc(reinterpret_cast<void**>(&p), bytes) == hipSuccess ? HN_OK : HN_E_OOM, where);
+}
+}  // namespace detail
+
 // Flat (src, dst, meta...) edge list; device storage owned by the object
 template <DeviceType device = DeviceType::DEVICE, typename VID = vid_t, typename EMeta = EMPTY,
           typename DEG = degree_t>
@@ -155,12 +172,12 @@ public:
     COO() = default;
     explicit COO(int64_t n) : _n(n) {
         if (n > 0) {
-            check(hipMalloc(&_src, sizeof(VID) * (size_t)n) == hipSuccess ? HN_OK : HN_E_OOM, "COO");
-            check(hipMalloc(&_dst, sizeof(VID) * (size_t)n) == hipSuccess ? HN_OK : HN_E_OOM, "COO");
+            detail::allocate(_src, sizeof(VID) * (size_t)n, "COO");
+            detail::allocate(_dst, sizeof(VID) * (size_t)n, "COO");
             hn_edge_meta m;
             detail::MetaTraits<EMeta>::layout(m);
             for (int f = 0; f < NM; f++)
-                check(hipMalloc(&_meta[f], (size_t)m.bytes[f] * (size_t)n) == hipSuccess ? HN_OK : HN_E_OOM, "COO");
+                detail::allocate(_meta[f], (size_t)m.bytes[f] * (size_t)n, "COO");
         }
     }
     COO(const COO&) = delete;
@@ -229,8 +246,8 @@ class CSR {
 public:
     CSR() = default;
     CSR(int64_t nv, int64_t ne) : _nv(nv), _ne(ne), _index(ne) {
-        check(hipMalloc(&_off64, sizeof(int64_t) * (size_t)(nv + 1)) == hipSuccess ? HN_OK : HN_E_OOM, "CSR");
-        check(hipMalloc(&_off, sizeof(DEG) * (size_t)(nv + 1)) == hipSuccess ? HN_OK : HN_E_OOM, "CSR");
+        detail::allocate(_off64, sizeof(int64_t) * (size_t)(nv + 1), "CSR");
+        detail::allocate(_off, sizeof(DEG) * (size_t)(nv + 1), "CSR");
     }
     CSR(const CSR&) = delete;
     CSR& operator=(const CSR&) = delete;

@@ -52,7 +52,8 @@ namespace gpu {
 template <typename T>
 void allocate(T*& ptr, size_t num_items) {
     ptr = nullptr;
-    hip_check(hipMalloc(reinterpret_cast<void**>(&ptr), sizeof(T) * (num_items ? num_items : 1)), "gpu::allocate");
+    hip_check(hornet::detail::device_malloc(reinterpret_cast<void**>(&ptr), sizeof(T) * (num_items ? num_items : 1)),
+              "gpu::allocate");
 }
 template <typename T>
 void free(T* ptr) {
@@ -449,7 +450,7 @@ private:
         if (items <= _cap) return;
         release();
         gpu::allocate(_work, items + 1);
-        hip_check(hipMalloc(&_tmp, hn::scan_temp_bytes((int64_t)items)), "BinarySearch");
+        hip_check(hornet::detail::device_malloc(&_tmp, hn::scan_temp_bytes((int64_t)items)), "BinarySearch");
         _cap = items;
     }
     void release() {
@@ -613,7 +614,7 @@ void adj_unions_run(HornetClass& hornet, Pairs pairs, int64_t n, const Operator&
     int64_t* P = nullptr;
     void* tmp = nullptr;
     gpu::allocate(P, (size_t)n + 1);
-    hip_check(hipMalloc(&tmp, hn::scan_temp_bytes(n)), "forAllAdjUnions");
+    hip_check(hornet::detail::device_malloc(&tmp, hn::scan_temp_bytes(n)), "forAllAdjUnions");
     hip_check(hn::exclusive_scan_dev<int64_t>(AdjUnionThreadsIn<Pairs>{h, pairs, work_factor},
                                               hn::ArrayOut<int64_t>{P}, P + n, n, tmp, st),
               "forAllAdjUnions (scan)");

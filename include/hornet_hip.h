@@ -143,6 +143,11 @@ hn_status hn_graph_create_coo(int32_t nv, int64_t m, const int32_t* src, const i
                               uint32_t flags, double arena_slack, void* stream, hn_graph** out);
 /* ~Hornet() */
 hn_status hn_graph_destroy(hn_graph* g);
+/* Device memory of destroyed graphs and finished builds is kept for the next ones, 4 GiB
+ * at most; the library gives it back when an allocation of its own fails.  This gives it
+ * back for others' allocations (the C++ headers and the Python package call it when
+ * theirs fail).  No counterpart in the reference. */
+hn_status hn_memory_trim(void);
 /* Hornet::nV() / nE() -- Hornet.cuh:113-117 */
 hn_status hn_graph_nv(const hn_graph* g, int32_t* nv);
 hn_status hn_graph_ne(const hn_graph* g, int64_t* ne);

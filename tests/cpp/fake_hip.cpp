@@ -28,7 +28,10 @@ using Launches = std::vector<Launch>;
 
 std::recursive_mutex mu;
 std::map<char*, Block> live;
-std::map<const void*, std::string> kernels;
+std::map<const void*, std::string>& kernels() {   // (needed before this file's globals are there)
+    static auto* const m = new std::map<const void*, std::string>;
+    return *m;
+}
 Launches* capturing = nullptr;
 int device = 0;
 long device_total = 0;          // bytes that may be allocated (0: no limit)
@@ -52,7 +55,7 @@ int pointer_args(const std::string& name) {
 hipError_t launch(const void* f, void** args) {
     std::lock_guard<std::recursive_mutex> lock(mu);
     if (!capturing) return hipSuccess;
-    Launch l{kernels[f], {}};
+    Launch l{kernels()[f], {}};
     for (int i = 0; i < pointer_args(l.kernel); i++) l.ptr.push_back(*static_cast<void**>(args[i]));
     capturing->push_back(l);
     return hipSuccess;
@@ -73,7 +76,7 @@ void fake_clear_trace() { trace.clear(); }
 // ---- the runtime
 void __hipRegisterFunction(void** modules, const void* host, char* dev, const char* name, unsigned limit, void* tid,
                            void* bid, void* block, void* grid, int* size) {
-    kernels[host] = name;
+    kernels()[host] = name;
     using F = void (*)(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*);
     static const F real = reinterpret_cast<F>(dlsym(RTLD_NEXT, "__hipRegisterFunction"));
     if (real) real(modules, host, dev, name, limit, tid, bid, block, grid, size);

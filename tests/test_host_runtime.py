@@ -103,3 +103,67 @@ d = c_int32(-1)
 fake.hipGetDevice(byref(d))
 assert d.value == current
 """)
+
+
+def test_memory_of_destroyed_graphs_is_given_back(fake):
+    program(fake, r"""
+base = fake.fake_used()
+ok(lib.hn_graph_destroy(graph()))
+assert fake.fake_used() > base            # kept for the next graph
+ok(lib.hn_memory_trim())
+assert fake.fake_used() == base
+""")
+
+
+def test_headers_allocate_what_the_library_keeps(fake, tmp_path):
+    """The C++ headers' own allocations, on a device filled by a destroyed graph."""
+    (tmp_path / "main.cpp").write_text(r"""
+#include "hornet/operators.hpp"
+extern "C" void fake_device_total(long);
+extern "C" long fake_used();
+static void keep() {   // the device is full of it
+    hn_graph* g = nullptr;
+    int64_t off[1001] = {};
+    fake_device_total(0);
+    (void)hn_memory_trim();
+    if (hn_graph_create_csr(1000, 0, off, nullptr, 0, 0.0, nullptr, &g) != HN_OK) throw 1;
+    (void)hn_graph_destroy(g);
+    fake_device_total(fake_used());
+}
+int main() {
+    keep();
+    hornet::COO<> coo(1000);
+    keep();
+    hornet::CSR<> csr(100, 1000);
+    keep();
+    int* p = nullptr;
+    hornets_nest::gpu::allocate(p, 1000);
+    return 0;
+}
+""")
+    lib = os.path.join(ROOT, "hornet_amd")
+    exe = str(tmp_path / "main")
+    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{ROOT}/include",
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", str(tmp_path / "main.cpp"), "-x", "none",
+                    fake, f"{lib}/libhornet_hip.so", "-o", exe, f"-Wl,-rpath,{lib}", f"-Wl,-rpath,{os.path.dirname(fake)}"],
+                   check=True, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_package_allocates_what_the_library_keeps(monkeypatch):
+    import torch
+
+    import hornet_amd.graph as G
+    calls = []
+
+    def empty(n, dtype, device):
+        calls.append(n)
+        if len(calls) == 1:
+            raise torch.OutOfMemoryError("no memory")
+        return torch.zeros(n, dtype=dtype)
+
+    monkeypatch.setattr(G, "_dev", lambda: "cpu")
+    monkeypatch.setattr(G, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(G.torch, "empty", empty)
+    assert G._empty(7).shape == (7,) and calls == [7, "hn_memory_trim", 7]
