@@ -950,10 +950,11 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int CAP, int BMW>
+template <int CAP, int BMW, int ANYW>
 struct SmallShared {
     uint2 ent[2][CAP];       // x: group prefix << 2 | deg % 4, y: adjacency offset in 128-byte units
     uint32_t bm[BMW];
+    uint32_t any[ANYW];      // the summary, where the bitmap is in memory
     uint32_t bm0[BMW > TINY_NV / 32 ? 1 : BMW];   // one-launch pulls: the level's start
     unsigned long long cnt[3];   // per level % 3: size << 32 | groups
     uint32_t multi[3];           // some vertex of the level has other than one group
@@ -1066,8 +1067,9 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
                                                              int64_t words, int32_t* __restrict__ qdeg, uint32_t* __restrict__ qbase,
                                                              uint32_t* __restrict__ P, uint32_t* __restrict__ tile_lo,
                                                              const uint64_t* __restrict__ part, int64_t nparts,
-                                                             BfsCtl* __restrict__ ctl, BfsCtl* __restrict__ host) {
-    __shared__ SmallShared<CAP, BMW> sh;
+                                                             BfsCtl* __restrict__ ctl, BfsCtl* __restrict__ host,
+                                                             int first) {
+    __shared__ SmallShared<CAP, BMW, LDSBM ? 1 : ANY_WORDS> sh;
     const int tid = threadIdx.x, lane = __lane_id();
     BfsRound rd{};
     uint64_t visited = 0, scanned = 0, dsum = 0, deg = 0;
@@ -1104,8 +1106,14 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
             const int F = (int)(fc >> 32);
             for (int i = tid; i < F; i += SM_BLOCK)
                 sh.ent[L & 1][i] = make_uint2((P[i] << 2) | ((uint32_t)qdeg[i] & 3u), qbase[i]);
-            if constexpr (LDSBM)
-                for (int i = tid; i < (int)words; i += SM_BLOCK) sh.bm[i] = bitmap[i];
+            if constexpr (LDSBM) {
+                for (int i = tid; i < (int)words; i += SM_BLOCK) sh.bm[i] = first ? 0u : bitmap[i];
+                if (first && tid == (source >> 5) % SM_BLOCK) sh.bm[source >> 5] = 1u << (source & 31);
+            } else if (any_shift > 0) {
+                const uint32_t ab = (uint32_t)source >> any_shift;
+                for (int i = tid; i < ANY_WORDS; i += SM_BLOCK)
+                    sh.any[i] = !first ? any[i] : i == (int)(ab >> 5) ? 1u << (ab & 31) : 0u;
+            }
         }
         if (tid < 3) {
             sh.cnt[tid] = 0;
@@ -1131,10 +1139,9 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
             if (dist) dist[v] = (int32_t)L;
             if constexpr (!LDSBM) {   // (else from the bitmap at the end)
                 state[v] = (uint8_t)STATE_DIRECT;
+                // (in LDS: neighbouring ids share a word, and atomics on one word in memory take 10 ns each)
                 const uint32_t ab = (uint32_t)v >> any_shift;
-                if (any_shift > 0)
-                    __hip_atomic_fetch_or(any + (ab >> 5), 1u << (ab & 31), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (any_shift > 0) atomicOr(&sh.any[ab >> 5], 1u << (ab & 31));
             }
         };
         auto found = [&](int32_t v, const hn_vrec& rv, uint32_t slot, uint32_t gb) {
@@ -1195,11 +1202,13 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
                 // claim: the one lane that sets a vertex's bit owns the discovery
-                // (a lane without a slot sets no bit of word 0)
+                // (a lane without a slot sets no bit of word 0, in LDS; in memory that
+                // many atomics on one word took 10 ns each: a binary tree of a million
+                // vertices 540 us with them, 360 so)
                 word[j] = bit[j] ? (uint32_t)t[j] >> 5 : 0u;
                 bit[j] <<= t[j] & 31;
                 if constexpr (LDSBM) old[j] = atomicOr(&sh.bm[word[j]], bit[j]);
-                else old[j] = __hip_atomic_fetch_or(bitmap + word[j], bit[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                else old[j] = bit[j] ? __hip_atomic_fetch_or(bitmap + word[j], bit[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
             }
             bool won[NJ];
             hn_vrec rv[NJ];
@@ -1342,9 +1351,29 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
         }
     }
     __syncthreads();
-    if (work) {
-        if constexpr (!INIT) {
-            // hand the frontier and the bitmap over
+    const bool over = (fc >> 32) == 0 || (max_levels > 0 && (int64_t)L > max_levels);
+    if constexpr (!INIT && LDSBM)
+        if (work && (dist || !over)) {
+            // the state bytes of the vertices claimed here, and their bits
+            for (int i = tid; i < (int)words; i += SM_BLOCK) {
+                const uint32_t was = first ? (i == (source >> 5) ? 1u << (source & 31) : 0u) : bitmap[i];
+                const uint32_t now = sh.bm[i], won = now & ~was;
+                if (!won) continue;
+                uint4* q = reinterpret_cast<uint4*>(state + (int64_t)i * 32);
+                uint4 a = q[0], b = q[1];
+                // four bits of a word to the low bits of four bytes
+                auto bytes = [&](int k) { return ((((won >> (4 * k)) & 15u) * 0x00204081u) & 0x01010101u) * STATE_DIRECT; };
+                a.x |= bytes(0), a.y |= bytes(1), a.z |= bytes(2), a.w |= bytes(3);
+                b.x |= bytes(4), b.y |= bytes(5), b.z |= bytes(6), b.w |= bytes(7);
+                q[0] = a;
+                q[1] = b;
+                bitmap[i] = now;
+            }
+        }
+    // A round takes over: the frontier and the summary.  (A traversal that is over needs
+    // neither: from a vertex without edges, R-MAT s16 39 us with them, 30 so.)
+    if constexpr (!INIT)
+        if (work && !over) {
             const uint32_t F = (uint32_t)(fc >> 32), W = (uint32_t)fc;
             const uint32_t n = min(F, (uint32_t)CAP);
             const uint2* cur = sh.ent[L & 1];
@@ -1358,35 +1387,24 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
                 for (uint64_t t = (g0 + EXP_TILE - 1) / EXP_TILE; t * EXP_TILE < g1; t++) tile_lo[t] = i;
             }
             if constexpr (LDSBM) {
-                // the state bytes of the vertices claimed here
-                for (int i = tid; i < (int)words; i += SM_BLOCK) {
-                    const uint32_t now = sh.bm[i], won = now & ~bitmap[i];
-                    if (!won) continue;
-                    uint4* q = reinterpret_cast<uint4*>(state + (int64_t)i * 32);
-                    uint4 a = q[0], b = q[1];
-                    // four bits of a word to the low bits of four bytes
-                    auto bytes = [&](int k) { return ((((won >> (4 * k)) & 15u) * 0x00204081u) & 0x01010101u) * STATE_DIRECT; };
-                    a.x |= bytes(0), a.y |= bytes(1), a.z |= bytes(2), a.w |= bytes(3);
-                    b.x |= bytes(4), b.y |= bytes(5), b.z |= bytes(6), b.w |= bytes(7);
-                    q[0] = a;
-                    q[1] = b;
-                    bitmap[i] = now;
-                }
-                // (a vertex without edges may set a summary bit: nothing probes it)
-                for (int i = tid; i < (int)((words + 127) / 128); i += SM_BLOCK) {
+                // a lane per bit, of four words (any_shift is 7 here)
+                // (a vertex without edges may set one: nothing probes it)
+                for (int b0 = tid - lane; b0 * 4 < (int)words; b0 += SM_BLOCK) {
                     uint32_t x = 0;
-                    for (int k = 0; k < 128; k++) {   // any_shift is 7 here: four words a bit
-                        const int w = i * 128 + ((k + 4 * tid) & 127);
-                        x |= (uint32_t)(w < (int)words && sh.bm[w < (int)words ? w : 0] != 0) << ((w & 127) >> 2);
+                    for (int k = 0; k < 4; k++) {
+                        const int w = (b0 + lane) * 4 + k;
+                        x |= w < (int)words ? sh.bm[w] : 0u;
                     }
-                    any[i] = x;
+                    const uint64_t bits = __ballot(x != 0);
+                    if (lane == 0) any[b0 / 32] = (uint32_t)bits;
+                    if (lane == 1) any[b0 / 32 + 1] = (uint32_t)(bits >> 32);
                 }
+            } else if (any_shift > 0) {
+                for (int i = tid; i < ANY_WORDS; i += SM_BLOCK) any[i] = sh.any[i];
             }
         }
-    }
     // the degree sums (and, when the traversal is over after whole-device
     // rounds, those of their discoveries)
-    const bool over = (fc >> 32) == 0 || (max_levels > 0 && (int64_t)L > max_levels);
     uint64_t x = 0;
     if (!INIT && over && work && rounds)
         for (int64_t i = tid; i < nparts; i += SM_BLOCK) x += part[i];
@@ -1462,8 +1480,8 @@ int64_t bfs_layout(int64_t nv_in, int64_t ne, char* base, BfsBufs* b) {
 // The level loop over laid-out buffers.  A tiny graph is one launch.  Otherwise
 // the host queues the one-workgroup kernel, then as many whole-device rounds as
 // the last traversal of this graph took (three before the first), then the
-// one-workgroup kernel again, which takes the tail and writes the control block
-// to the host's pinned memory; if the traversal is not over by then, 1, 2, 4,
+// one-workgroup kernel again (if there was a round), which takes the tail and writes
+// the control block to the host's pinned memory; if the traversal is not over by then, 1, 2, 4,
 // ... rounds more, each time followed by the one-workgroup kernel.  Rounds
 // queued past the end change nothing.  Nothing here allocates (kernel timing,
 // which creates its events, only with `may_time`).
@@ -1509,19 +1527,19 @@ hn_status bfs_run(hn_graph* g, int32_t source, int32_t* dist, hn_bfs_stats* stat
                                            std::max(ceil_div(ne / EXP_G + nv, EXP_TILE), ceil_div(words, PULL_SPAN_SMALL * EXP_WAVES)));
     uint32_t r = 0;   // rounds launched
     const bool tiny = nv <= TINY_NV && ne <= TINY_NE;
-    auto small = [&]() {
+    auto small = [&](int first) {
         if (tiny)
             BFS_LAUNCH((bfs_small_kernel<TINY_CAP, TINY_NV / 32, true, true>), 1, SM_BLOCK, r, max_levels, sym, nv, ne,
                        source, g->rec, g->arena, dist, b.state, b.bitmap, b.any, any_shift, words, b.qdeg, b.qbase, b.P, b.tile_lo,
-                       b.part, nparts, b.ctl, hctl);
+                       b.part, nparts, b.ctl, hctl, first);
         else if (words <= SM_BM_WORDS)
             BFS_LAUNCH((bfs_small_kernel<SM_CAP, SM_BM_WORDS, true, false>), 1, SM_BLOCK, r, max_levels, sym, nv, ne,
                        source, g->rec, g->arena, dist, b.state, b.bitmap, b.any, any_shift, words, b.qdeg, b.qbase, b.P, b.tile_lo,
-                       b.part, nparts, b.ctl, hctl);
+                       b.part, nparts, b.ctl, hctl, first);
         else
             BFS_LAUNCH((bfs_small_kernel<SM_CAP, 1, false, false>), 1, SM_BLOCK, r, max_levels, sym, nv, ne, source,
                        g->rec, g->arena, dist, b.state, b.bitmap, b.any, any_shift, words, b.qdeg, b.qbase, b.P, b.tile_lo, b.part,
-                       nparts, b.ctl, hctl);
+                       nparts, b.ctl, hctl, first);
     };
     if (!tiny) {
         // kernels only (no memset node), so a captured copy of this sequence replays correctly
@@ -1529,7 +1547,7 @@ hn_status bfs_run(hn_graph* g, int32_t source, int32_t* dist, hn_bfs_stats* stat
             g->nv, g->rec, b.bitmap, b.full, b.any, any_shift, reinterpret_cast<uint32_t*>(b.state), source, b.qdeg, b.qbase, b.P,
             b.tile_lo, b.part, b.ctl);
         HN_CHECK_LAUNCH();
-        small();
+        small(1);
         if (e != hipSuccess) {
             set_error(std::string("bfs launch: ") + hipGetErrorString(e));
             return HN_E_HIP;
@@ -1557,7 +1575,8 @@ hn_status bfs_run(hn_graph* g, int32_t source, int32_t* dist, hn_bfs_stats* stat
             e = hipGetLastError();
             r++;
         }
-        if (e == hipSuccess) small();
+        // (without rounds since the last one it would find nothing to do)
+        if (e == hipSuccess && (next > 0 || tiny)) small(0);
         if (e == hipSuccess && dist && !tiny) {
             bfs_dist_kernel<<<(unsigned)std::min<int64_t>(ceil_div(nv, BLOCK * 8), 4096), BLOCK, 0, st>>>(
                 r, max_levels, nv, b.state, b.ctl, dist);

@@ -66,3 +66,25 @@ def test_more_than_2_25_vertices(hn, path):
     print(f"case bfs big path={path}", flush=True)
     sizes = [1] * path + [1000, 3001, 1 << 20, 1 << 25, 70000, 3, 1]
     check(hn, *layered(hn, sizes, 2, False, lone=77))
+
+
+# bitmap in LDS and in memory; a bit of the summary stands for 128 vertices up to 2^24, then for 256
+@pytest.mark.parametrize("rest", [600000, 1 << 20, (1 << 24) - 52000, (1 << 24) + 77, 20000003])
+def test_summary_of_visited_vertices(hn, rest):
+    """Levels by one workgroup, then a pull that asks the summary they have written: few
+    vertices are visited and their rows hold most entries."""
+    print(f"case bfs summary rest={rest}", flush=True)
+    check(hn, *layered(hn, [1, 1, 1, 200, 900, 50000, rest, 3, 1], 2, False))
+
+
+# the frontier doubles on ids that share words of the bitmap and of the summary
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("n", [3000, 700001, (1 << 20) - 1, 2000003])
+def test_binary_trees(hn, n, directed):
+    import torch
+    print(f"case bfs tree n={n} directed={directed}", flush=True)
+    v = torch.arange(1, n, dtype=torch.int32, device="cuda")
+    h = hn.Hornet.from_coo_device(n + 3, (v - 1) // 2, v, symmetrize=not directed)
+    dist = torch.full((n + 3,), INF, dtype=torch.int32, device="cuda")
+    dist[:n] = torch.from_numpy(np.frexp(np.arange(1, n + 1))[1] - 1).to(dist)
+    check(hn, h, 0, dist)
