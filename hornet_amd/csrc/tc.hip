@@ -189,10 +189,26 @@ struct StoredGroupsIn {
     const hn_vrec* rec;
     __device__ __forceinline__ uint32_t operator()(int64_t v) const { return ((uint32_t)rec[v].deg + TC_G - 1) / TC_G; }
 };
+// body(v, first, k) for every k of a lane's [first, last): one lane's long range by all
+// lanes that are here (a star of four million leaves: its 4,096 tasks by one lane 128 us).
+template <typename Body>
+__device__ __forceinline__ void tc_spread(uint32_t v, uint32_t first, uint32_t last, Body body) {
+    constexpr uint32_t OWN = 16;
+    const uint32_t n = last > first ? last - first : 0u;
+    if (n <= OWN)
+        for (uint32_t k = 0; k < n; k++) body(v, first, first + k);
+    uint64_t more = __ballot(n > OWN);
+    const uint64_t here = __ballot(true);
+    const uint32_t lanes = (uint32_t)__popcll(here), rank = (uint32_t)__popcll(here & lanemask_lt());
+    for (; more; more &= more - 1) {
+        const int from = __ffsll((unsigned long long)more) - 1;
+        const uint32_t w = __shfl(v, from, WAVE), a = __shfl(first, from, WAVE), b = __shfl(last, from, WAVE);
+        for (uint32_t k = a + rank; k < b; k += lanes) body(w, a, k);
+    }
+}
 __device__ __forceinline__ void tc_tiles(uint32_t* __restrict__ tile_lo, int64_t v, uint32_t ex, uint32_t x) {
-    if (x)
-        for (uint32_t t = (ex + TC_TILE - 1) / TC_TILE; (uint64_t)t * TC_TILE < (uint64_t)ex + x; t++)
-            tile_lo[t] = (uint32_t)v;
+    auto tile = [](uint64_t g) { return (uint32_t)((g + TC_TILE - 1) / TC_TILE); };   // the first that starts at g or later
+    tc_spread((uint32_t)v, tile(ex), tile((uint64_t)ex + x), [&](uint32_t w, uint32_t, uint32_t t) { tile_lo[t] = w; });
 }
 // weight, where given: the degrees, from records that were just read
 struct StoredGroupsOut {
@@ -502,7 +518,7 @@ struct TaskIn {
 struct TaskOut {
     uint2* task;
     __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t n) const {
-        for (uint32_t k = 0; k < n; k++) task[ex + k] = make_uint2((uint32_t)v, k);
+        tc_spread((uint32_t)v, ex, ex + n, [&](uint32_t w, uint32_t a, uint32_t k) { task[k] = make_uint2(w, k - a); });
     }
 };
 
