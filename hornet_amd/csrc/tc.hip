@@ -924,9 +924,11 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
         *total_out = 0;
         return HN_OK;
     }
-    const int64_t groups = ne / TC_G + nv + 1;   // at most
+    // at most: a vertex without entries has no group, and one with a list of TC_SMALL
+    // entries or fewer no task (two billion vertices with few entries need 40 bytes each)
+    const int64_t groups = ne / TC_G + std::min(nv, ne) + 1;
     const int64_t tiles = groups / TC_TILE + 2;
-    const int64_t tasks = nv + 2 * ne / TC_CAND + 1;
+    const int64_t tasks = std::min(nv, ne / TC_SMALL) + 2 * ne / TC_CAND + 1;
     // what an owner's stored row says of its edges holds on symmetric storage only
     const int sym = orient && graph_known_symmetric(g) ? 1 : 0;
     int64_t o = 0;

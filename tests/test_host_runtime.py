@@ -115,6 +115,23 @@ assert fake.fake_used() == base
 """)
 
 
+def test_triangle_scratch_of_sparse_graphs(fake):
+    """What a count reserves for vertices without entries: 40 bytes each, and a quarter
+    more in a scratch buffer, in blocks that are rounded up by an eighth at most."""
+    program(fake, r"""
+nv = 1 << 20
+off = (c_int64 * (nv + 1))(*([0, 1] + [2] * (nv - 1)))
+h = c_void_p()
+ok(lib.hn_graph_create_csr(nv, 2, off, (c_int32 * 2)(1, 0), 1, 0.0, None, byref(h)))
+used, total = fake.fake_used(), c_uint64()
+for count in lib.hn_tc2_stored, lib.hn_tc_count:
+    count.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p]
+    ok(count(h, byref(total), None, None))
+scratch = fake.fake_used() - used
+assert 0 < scratch < 1.25 * 1.125 * (40 * nv + (4 << 20)), scratch / nv
+""")
+
+
 def test_headers_allocate_what_the_library_keeps(fake, tmp_path):
     """The C++ headers' own allocations, on a device filled by a destroyed graph."""
     (tmp_path / "main.cpp").write_text(r"""
