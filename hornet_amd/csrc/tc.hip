@@ -91,8 +91,8 @@ struct alignas(128) TcTicket {
 struct TcCtl {
     TcSum total[TC_SUMS];
     TcTicket ticket[TC_LANES];
+    uint64_t owned;      // grouped edges, and the number of tasks << 32
     uint32_t cut;        // bins from this one on are hubs
-    uint32_t ntask;
     uint32_t hubs;
     uint32_t repeats;    // some row stores an entry twice
 };
@@ -190,7 +190,7 @@ struct StoredGroupsIn {
     __device__ __forceinline__ uint32_t operator()(int64_t v) const { return ((uint32_t)rec[v].deg + TC_G - 1) / TC_G; }
 };
 // body(v, first, k) for every k of a lane's [first, last): one lane's long range by all
-// lanes that are here (a star of four million leaves: its 4,096 tasks by one lane 128 us).
+// lanes that are here, those without a range too (a star of four million leaves: its 4,096 tasks by one lane 128 us).
 template <typename Body>
 __device__ __forceinline__ void tc_spread(uint32_t v, uint32_t first, uint32_t last, Body body) {
     constexpr uint32_t OWN = 16;
@@ -211,13 +211,17 @@ __device__ __forceinline__ void tc_tiles(uint32_t* __restrict__ tile_lo, int64_t
     tc_spread((uint32_t)v, tile(ex), tile((uint64_t)ex + x), [&](uint32_t w, uint32_t, uint32_t t) { tile_lo[t] = w; });
 }
 // weight, where given: the degrees, from records that were just read
+// (a wave has the 64 vertices of one word of `some`)
 struct StoredGroupsOut {
     const hn_vrec* rec;
     TcRow* row;
     uint32_t* P;
     uint32_t* tile_lo;
     uint32_t* weight;
+    uint64_t* some;
     __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t x) const {
+        const uint64_t any = __ballot(x != 0);
+        if (v % WAVE == 0) some[v / WAVE] = any;
         if (weight) weight[v] = (uint32_t)rec[v].deg;
         row[v] = TcRow{ex, 0u, 0u, 0u};
         P[v] = ex;
@@ -395,16 +399,36 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
     if (__ballot(twice) && lane == 0) ctl->repeats = 1u;   // every writer stores the same value
 }
 
-// The lists' padding, and a bit per vertex whose list is long enough for it to be an owner.
-__global__ __launch_bounds__(BLOCK) void tc_pad_kernel(int64_t nv, const TcRow* __restrict__ row,
-                                                       uint16_t* __restrict__ codes, uint32_t* __restrict__ ids,
-                                                       uint64_t* __restrict__ owner) {
-    const int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const TcRow r = v < nv ? row[v] : TcRow{0u, 0u, 0u, 0u};
-    const uint64_t big = __ballot(r.len() > TC_SMALL);
-    if (__lane_id() == 0 && v < nv) owner[v / WAVE] = big;
-    for (uint32_t i = r.n16; i & (TC_G - 1); i++) codes[(int64_t)r.base * TC_G + i] = (uint16_t)TC_PAD16;
-    for (uint32_t i = r.n32; i & (TC_G - 1); i++) ids[(int64_t)r.base * TC_G + i] = TC_PAD;
+// The lists' padding, and two bits per vertex: its list is long enough for it to be an
+// owner (whose counter of grouped edges starts at 0), or one that tc_small_kernel takes.
+// Vertices without entries, all but a few of some graphs, cost this pass and the
+// later ones their bits only (16 M vertices with a thousand edges, where it was
+// their 16-byte rows and counters: 72 -> 28 us here, 52 -> 22 there, 129 -> 58 in the
+// scans; stored 663 -> 535 in all, oriented 646 -> 540).
+constexpr int TC_PAD_WORDS = 4;   // of 64 vertices to a wave
+__global__ __launch_bounds__(BLOCK) void tc_pad_kernel(int64_t nv, const uint64_t* __restrict__ some,
+                                                       const TcRow* __restrict__ row, uint16_t* __restrict__ codes,
+                                                       uint32_t* __restrict__ ids, uint64_t* __restrict__ owner,
+                                                       uint64_t* __restrict__ small, uint32_t* __restrict__ gcnt) {
+    const int64_t w0 = ((int64_t)blockIdx.x * NWAVES + threadIdx.x / WAVE) * TC_PAD_WORDS, words = (nv + WAVE - 1) / WAVE;
+    const int lane = __lane_id();
+    TcRow r[TC_PAD_WORDS];
+#pragma unroll
+    for (int j = 0; j < TC_PAD_WORDS; j++) {
+        const bool any = w0 + j < words && (some[w0 + j] >> lane & 1u);
+        r[j] = any ? row[(w0 + j) * WAVE + lane] : TcRow{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int j = 0; j < TC_PAD_WORDS; j++) {
+        const uint64_t big = __ballot(r[j].len() > TC_SMALL), few = __ballot(r[j].len() >= 2 && r[j].len() <= TC_SMALL);
+        if (lane == 0 && w0 + j < words) {
+            owner[w0 + j] = big;
+            small[w0 + j] = few;
+        }
+        if (r[j].len() > TC_SMALL) gcnt[(w0 + j) * WAVE + lane] = 0;
+        for (uint32_t i = r[j].n16; i & (TC_G - 1); i++) codes[(int64_t)r[j].base * TC_G + i] = (uint16_t)TC_PAD16;
+        for (uint32_t i = r[j].n32; i & (TC_G - 1); i++) ids[(int64_t)r[j].base * TC_G + i] = TC_PAD;
+    }
 }
 
 // entry i of a list, as a vertex
@@ -500,25 +524,29 @@ __global__ __launch_bounds__(BLOCK) void tc_parts_kernel(int sym, const TcCtl* _
     gcnt[hub[q]] = at;
 }
 
-// ---- tasks: up to TC_CAND candidates of one owner
-// (the owners' bits spare the pass the others' lists: 16 M vertices, 117 us without, 38 so)
-struct TaskIn {
+// ---- owners: where their grouped edges start, and tasks of up to TC_CAND candidates
+// (low and high half of one scan, which looks at owners only)
+struct OwnerIn {
     const uint64_t* owner;
     const TcRow* row;
     const uint32_t* gcnt;
     const hn_vrec* rec;
     const TcCtl* ctl;
     int sym;
-    __device__ __forceinline__ uint32_t operator()(int64_t v) const {
+    __device__ __forceinline__ uint64_t operator()(int64_t v) const {
         if (!(owner[v / WAVE] >> (v % WAVE) & 1u)) return 0u;
-        const uint32_t cand = sym && !ctl->repeats ? (uint32_t)rec[v].deg : row[v].len() + gcnt[v];
-        return (cand + TC_CAND - 1) / TC_CAND;
+        const uint32_t n = gcnt[v];
+        const uint32_t cand = sym && !ctl->repeats ? (uint32_t)rec[v].deg : row[v].len() + n;
+        return (uint64_t)n | (uint64_t)((cand + TC_CAND - 1) / TC_CAND) << 32;
     }
 };
-struct TaskOut {
+struct OwnerOut {
+    uint32_t* goff;
     uint2* task;
-    __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t n) const {
-        tc_spread((uint32_t)v, ex, ex + n, [&](uint32_t w, uint32_t a, uint32_t k) { task[k] = make_uint2(w, k - a); });
+    __device__ __forceinline__ void operator()(int64_t v, uint64_t ex, uint64_t x) const {
+        if (x) goff[v] = (uint32_t)ex;
+        const uint32_t first = (uint32_t)(ex >> 32);
+        tc_spread((uint32_t)v, first, first + (uint32_t)(x >> 32), [&](uint32_t w, uint32_t a, uint32_t k) { task[k] = make_uint2(w, k - a); });
     }
 };
 
@@ -682,7 +710,7 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, co
                                                          const uint32_t* __restrict__ members, TcCtl* __restrict__ ctl,
                                                          unsigned long long* __restrict__ per_vertex) {
     __shared__ OwnerShared sh;
-    const uint32_t ntask = ctl->ntask;
+    const uint32_t ntask = (uint32_t)(ctl->owned >> 32);
     const bool repeats = ctl->repeats != 0;
     const bool stored = sym && !repeats;
     uint64_t acc = 0;
@@ -861,7 +889,8 @@ __device__ __forceinline__ uint32_t tc_common(const TcRow& s, const TcRow& l, co
 // four entries: 975, 690; R-MAT s12 is 20 % slower with 64, 16 M vertices are so with 16).
 constexpr int TC_SRC = 4;
 constexpr int64_t TC_WIDE = 1 << 20;
-__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, const TcRow* __restrict__ row,
+__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, const uint64_t* __restrict__ small,
+                                                         const TcRow* __restrict__ row,
                                                          const uint16_t* __restrict__ codes,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, TcCtl* __restrict__ ctl,
@@ -869,9 +898,10 @@ __global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, co
     const int lane = __lane_id(), sub = lane % TC_SMALL, team = lane / TC_SMALL;
     const int64_t w0 = ((int64_t)blockIdx.x * NWAVES + threadIdx.x / WAVE) * per;
     if (w0 >= nv) return;
-    const TcRow own = lane < per && w0 + lane < nv ? row[w0 + lane] : TcRow{0u, 0u, 0u, 0u};
-    const bool has = own.len() >= 2 && own.len() <= TC_SMALL;
+    const bool has = lane < per && (small[w0 / WAVE] >> (w0 % WAVE) >> lane & 1u);   // (no bits from nv on)
     const uint64_t m = __ballot(has);
+    if (m == 0) return;
+    const TcRow own = has ? row[w0 + lane] : TcRow{0u, 0u, 0u, 0u};
     const int nsrc = __popcll(m);
     // lane k gets the k-th source's lane (the others fill up behind)
     const int to = has ? __popcll(m & lanemask_lt()) : nsrc + __popcll(~m & lanemask_lt());
@@ -939,12 +969,12 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     };
     const int64_t o_ctl = take(sizeof(TcCtl)), o_hist = take(TC_BINS * 4);
     const int64_t nhub = std::min<int64_t>(nv, TC_HUBS + 1);
-    const int64_t o_gcnt = take(nv * 4), o_part = take(nhub * TC_LANES * 4), o_zero_end = o;   // cleared together
-    const int64_t o_weight = take(nv * 4), o_wc = take(nv * 8), o_hub = take((int64_t)(TC_HUBS + 1) * 4);
+    const int64_t o_part = take(nhub * TC_LANES * 4), o_zero_end = o;   // cleared together
+    const int64_t o_gcnt = take(nv * 4), o_weight = take(nv * 4), o_wc = take(nv * 8), o_hub = take((int64_t)(TC_HUBS + 1) * 4);
     const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4);
     const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
     const int64_t o_goff = take((nv + 1) * 4), o_mem = take(ne * 4), o_task = take(tasks * 8);
-    const int64_t o_owner = take((nv + WAVE - 1) / WAVE * 8);
+    const int64_t bits = (nv + WAVE - 1) / WAVE * 8, o_some = take(bits), o_owner = take(bits), o_small = take(bits);
     const int64_t o_scan = take((int64_t)scan_temp_bytes(nv));
     HN_TRY(g->s_tc.reserve((size_t)o));
     char* base = g->s_tc.as<char>();
@@ -965,7 +995,9 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     uint32_t* goff = at(o_goff, (uint32_t*)nullptr);
     uint32_t* members = at(o_mem, (uint32_t*)nullptr);
     uint2* task = at(o_task, (uint2*)nullptr);
+    uint64_t* some = at(o_some, (uint64_t*)nullptr);
     uint64_t* owner = at(o_owner, (uint64_t*)nullptr);
+    uint64_t* small = at(o_small, (uint64_t*)nullptr);
     void* tmp = base + o_scan;
     unsigned long long* per = reinterpret_cast<unsigned long long*>(per_vertex);
     const unsigned gv = (unsigned)ceil_div(nv, BLOCK);
@@ -976,7 +1008,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     // 1. hubs and codes
     const bool all_hubs = nv <= (int64_t)TC_HUBS;
     HN_TRY(exclusive_scan_fn<uint32_t>(StoredGroupsIn{g->rec},
-                                       StoredGroupsOut{g->rec, row, P, tile_lo, orient && !all_hubs ? weight : nullptr},
+                                       StoredGroupsOut{g->rec, row, P, tile_lo, orient && !all_hubs ? weight : nullptr, some},
                                        P + nv, nv, tmp, st));
     if (all_hubs) {
         tc_all_hubs_kernel<<<gv, BLOCK, 0, st>>>(nv, g->rec, wc, hub, ctl);
@@ -1000,7 +1032,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     else
         tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
     HN_CHECK_LAUNCH();
-    tc_pad_kernel<<<gv, BLOCK, 0, st>>>(nv, row, codes, ids, owner);
+    tc_pad_kernel<<<(unsigned)ceil_div(nv, BLOCK * TC_PAD_WORDS), BLOCK, 0, st>>>(nv, some, row, codes, ids, owner, small, gcnt);
     HN_CHECK_LAUNCH();
     // 3. edges owned by their destination
     tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, owner, codes, ids, hub, gcnt, part, nhub,
@@ -1008,17 +1040,17 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     HN_CHECK_LAUNCH();
     tc_parts_kernel<<<(unsigned)ceil_div(nhub, BLOCK), BLOCK, 0, st>>>(sym, ctl, nhub, hub, part, gcnt);
     HN_CHECK_LAUNCH();
-    HN_TRY(exclusive_scan<uint32_t>(ArrayIn<uint32_t>{gcnt}, goff, nv, tmp, st));
+    HN_TRY(exclusive_scan_fn<uint64_t>(OwnerIn{owner, row, gcnt, g->rec, ctl, sym}, OwnerOut{goff, task}, &ctl->owned, nv, tmp, st));
     tc_group_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, owner, codes, ids, hub, gcnt, part, nhub,
                                                 place, goff, members);
     HN_CHECK_LAUNCH();
     // 4. counts
-    HN_TRY(exclusive_scan_fn<uint32_t>(TaskIn{owner, row, gcnt, g->rec, ctl, sym}, TaskOut{task}, &ctl->ntask, nv, tmp, st));
     tc_owner_kernel<<<(unsigned)num_cus() * 8, BLOCK, 0, st>>>(orient ? 1 : 0, sym, g->rec, g->arena, wc, task, row, codes, ids,
                                                                hub, gcnt, goff, members, ctl, per);
     HN_CHECK_LAUNCH();
     const int small_per = nv > TC_WIDE ? WAVE : TC_SRC * (WAVE / TC_SMALL);
-    tc_small_kernel<<<(unsigned)ceil_div(nv, (int64_t)small_per * NWAVES), BLOCK, 0, st>>>(nv, small_per, row, codes, ids, hub, ctl, per);
+    tc_small_kernel<<<(unsigned)ceil_div(nv, (int64_t)small_per * NWAVES), BLOCK, 0, st>>>(nv, small_per, small, row, codes, ids,
+                                                                                           hub, ctl, per);
     HN_CHECK_LAUNCH();
     TcSum sums[TC_SUMS];
     HN_TRY(read_back(g, ctl->total, sizeof(sums), sums, st));

@@ -1,0 +1,31 @@
+"""Triangle counts of graphs whose vertices have almost all no entries: the passes over
+vertices go by bits, 64 to a word and four words to a wave, and lists of 2 to 16
+entries and of more have bits of their own."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nv", [63, 64, 65, 257, 65535, 70001, (1 << 20) - 255, (1 << 20) + 1])
+@pytest.mark.parametrize("stored", [False, True])
+def test_few_entries(nv, stored):
+    """Cliques with lists of 1 to 17 entries (oriented; 2, 16 and 17 as stored) at the
+    first vertices, the last, and across a word and four of them."""
+    import torch
+
+    import hornet_amd.graph as G
+    print(f"case tc sparse nv={nv} stored={stored}", flush=True)
+    at = [(0, 3), (3, 17), (nv - 18, 18)] + ([(64 * k - 9, 18) for k in (2, 3, nv // 128)] if nv > 256 else [])
+    src, dst = (torch.from_numpy(np.concatenate([v + np.triu_indices(n, 1)[e] for v, n in at]).astype(np.int32)).cuda()
+                for e in (0, 1))
+    h = G.Hornet.from_coo_device(nv, src, dst)
+    off, adj = (x.cpu().numpy() for x in h.getCSR())
+    tc = G.TriangleCounting2(h)
+    tc.init()
+    want = O.tc2_per_vertex(*((off, adj) if stored else O.directed_by_degree(off, adj)))
+    for _ in range(2):   # the second one on dirty scratch
+        (tc.run if stored else tc.run_undirected)()
+        assert tc.countTriangles() == int(want.sum()) and np.array_equal(tc.copyTCToHost(), want)
