@@ -29,3 +29,31 @@ def test_few_entries(nv, stored):
     for _ in range(2):   # the second one on dirty scratch
         (tc.run if stored else tc.run_undirected)()
         assert tc.countTriangles() == int(want.sum()) and np.array_equal(tc.copyTCToHost(), want)
+
+
+@pytest.mark.parametrize("length", [16, 17, 600])
+def test_edges_grouped_in_some_tiles(length):
+    """Stored rows of four entries, of which those of every sixteenth thousand vertices
+    also go to one of three long lists: most tiles of rows hold no edge that its
+    destination owns."""
+    import torch
+
+    import hornet_amd.graph as G
+    print(f"case tc grouped tiles length={length}", flush=True)
+    nv, rng = 100_003, np.random.default_rng(length)
+    src = np.repeat(np.arange(nv), 4)
+    dst = rng.integers(0, 2000, src.size)
+    some = np.flatnonzero(np.arange(nv) // 1000 % 16 == 3)
+    long = np.array([5, 50_000, nv - 1])
+    src = np.concatenate([src, np.repeat(some, 3), np.repeat(long, length - 4)])
+    dst = np.concatenate([dst, np.tile(long, some.size), rng.integers(0, 2000, 3 * (length - 4))])
+    k = np.unique(src * nv + dst)
+    src, dst = (torch.from_numpy(x.astype(np.int32)).cuda() for x in (k // nv, k % nv))
+    h = G.Hornet.from_coo_device(nv, src, dst, symmetrize=False, drop_self_loops=False)
+    want = O.tc2_per_vertex(*(x.cpu().numpy() for x in h.getCSR()))
+    assert want.any()
+    tc = G.TriangleCounting2(h)
+    tc.init()
+    for _ in range(2):
+        tc.run()
+        assert tc.countTriangles() == int(want.sum()) and np.array_equal(tc.copyTCToHost(), want)
