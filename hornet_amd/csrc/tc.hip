@@ -62,7 +62,7 @@ constexpr uint32_t TC_WIDE_HASH = (TC_HUBS + 1) / 32, TC_WIDE_TAIL = TC_WIDE_HAS
 // s20, searched from one table less on: 6.7 and 57 ms, from two more on: 8.1 and 64).  The
 // lists of an orientation are not whole rows, and long ones of ids take more than 65,535
 // vertices of a like degree: they are hashed, one table of 1,024 after the other (cliques
-// of 700, in tables of 256: 18.3 ms, 6.4 so; of 5,000: 1.6 s).
+// of 700, in tables of 256: 18.3 ms, 3.3 so; of 5,000: 0.89 s).
 constexpr uint32_t TC_SEARCH = TC_TAIL + 2 * TC_WIDE_TAIL;
 constexpr int TC_TEAM = 8;                     // lanes per shorter list
 constexpr int TC_DEPTH = 4;                    // groups per lane in flight (2 and 8: 3 and 2 % slower on R-MAT s22)
@@ -577,6 +577,7 @@ struct OwnerShared {
     uint32_t cls[TC_ORDER];
     uint32_t tail;
     uint2 task;
+    uint32_t cur, end, tried;        // the first lane's tickets (in LDS: it has no registers to spare)
 };
 static_assert(sizeof(OwnerShared) * 8 <= 160 * 1024, "eight workgroups fill a CU's LDS");
 
@@ -619,7 +620,7 @@ __device__ __forceinline__ uint32_t tc_test(const OwnerShared& sh, const uint4& 
 // lanes per list, eight codes per lane and group.  The lists are sorted by
 // length class, so that the teams of a wave stay together: TC_DEPTH groups of one
 // list in flight while lists are longer than a team's step, then TC_DEPTH lists.
-enum TcTail { TC_NONE, TC_HASHED, TC_HASHED_WIDE, TC_SORTED };
+enum TcTail { TC_NONE, TC_HASHED, TC_SORTED };
 struct TcSorted {   // an owner's stored row
     const int32_t* entry;
     int32_t deg;
@@ -647,7 +648,6 @@ __device__ __forceinline__ uint32_t tc_ids(const OwnerShared& sh, uint32_t it, i
         for (uint32_t i = sub; i < n32; i += TC_TEAM) {
             const uint32_t q = li[i];
             if constexpr (TAIL == TC_HASHED) c += tc_holds<TC_HASH>(sh.hash, q) ? 1u : 0u;
-            if constexpr (TAIL == TC_HASHED_WIDE) c += tc_holds<TC_WIDE_HASH>(sh.bits, q) ? 1u : 0u;
             if constexpr (TAIL == TC_SORTED) c += sorted.has(q) ? 1u : 0u;
         }
     }
@@ -715,6 +715,38 @@ __device__ __forceinline__ void tc_walk(const OwnerShared& sh, uint32_t nlong, u
     }
 }
 
+// The same against a table in the bits' place: ids only.  An owner with that many has
+// neighbours with lists like its own, so a lane has eight ids on their way (14 cliques of
+// 5,000: 1.60 s with one, 0.89 so; in tc_walk they would cost registers that the walks of
+// codes need: R-MAT s22 2 % slower).
+__device__ __forceinline__ void tc_walk_wide(const OwnerShared& sh, uint32_t n, const uint32_t* __restrict__ ids,
+                                             unsigned long long* __restrict__ per_vertex, uint64_t& acc) {
+    constexpr uint32_t STEP = TC_TEAM * 4, DEPTH = 2;
+    const uint32_t sub = threadIdx.x & (TC_TEAM - 1);
+    for (uint32_t it = threadIdx.x / TC_TEAM; it < n; it += BLOCK / TC_TEAM) {
+        const uint32_t* li = ids + (int64_t)sh.base[it] * TC_G;
+        const uint32_t n32 = sh.n32[it];
+        uint32_t c = 0, i0 = 0;
+        auto test = [&](uint32_t q) { c += tc_holds<TC_WIDE_HASH>(sh.bits, q) ? 1u : 0u; };
+        for (; i0 + STEP * DEPTH <= n32; i0 += STEP * DEPTH) {
+            uint4 x[DEPTH];
+#pragma unroll
+            for (int d = 0; d < (int)DEPTH; d++) x[d] = *reinterpret_cast<const uint4*>(li + i0 + d * STEP + sub * 4);
+#pragma unroll
+            for (int d = 0; d < (int)DEPTH; d++) {
+                test(x[d].x);
+                test(x[d].y);
+                test(x[d].z);
+                test(x[d].w);
+            }
+        }
+        for (uint32_t i = i0 + sub; i < n32; i += TC_TEAM) test(li[i]);
+        acc += c;
+        c = tc_team_sum(c);
+        if (sub == TC_TEAM - 1 && c && per_vertex) atomicAdd(per_vertex + sh.y[it], (unsigned long long)c);
+    }
+}
+
 // Bound by the sectors of the shorter lists that miss the L2: on R-MAT s22 360 M of
 // the 400 M that the walks touch, 7.4 ms at the 48 G/s that scattered sector reads
 // reach here; LDS and vector units are a third busy.
@@ -740,24 +772,24 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, co
     // ticket for each of R-MAT s22's 640 K tasks, from one counter, was what
     // bounded the kernel: 10.1 ms, 7.6 ms so.)
     const uint32_t chunk = min(max(ntask / (gridDim.x * 32u), 1u), 8u);
-    uint32_t cur = 0, end = 0, tried = 0;
+    if (threadIdx.x == 0) sh.cur = sh.end = sh.tried = 0;
     auto next = [&]() {
-        while (cur >= end) {
-            if (tried == TC_LANES) return make_uint2(0u, TC_PAD);
-            const uint32_t share = (blockIdx.x + tried) % TC_LANES;
+        while (sh.cur >= sh.end) {
+            if (sh.tried == TC_LANES) return make_uint2(0u, TC_PAD);
+            const uint32_t share = (blockIdx.x + sh.tried) % TC_LANES;
             uint32_t* at = &ctl->ticket[share].v;
             const uint32_t seen = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const uint64_t first = ((uint64_t)seen * TC_LANES + share) * chunk;
             uint64_t lo = first;
             if (first < ntask) lo = ((uint64_t)atomicAdd(at, 1u) * TC_LANES + share) * chunk;
             if (lo >= ntask) {
-                tried++;
+                sh.tried++;
                 continue;
             }
-            cur = (uint32_t)lo;
-            end = (uint32_t)min(lo + chunk, (uint64_t)ntask);
+            sh.cur = (uint32_t)lo;
+            sh.end = (uint32_t)min(lo + chunk, (uint64_t)ntask);
         }
-        return task[cur++];
+        return task[sh.cur++];
     };
     uint2 ahead = make_uint2(0u, TC_PAD);
     if (threadIdx.x == 0) sh.task = next();
@@ -838,13 +870,13 @@ __global__ __launch_bounds__(BLOCK) void tc_owner_kernel(int orient, int sym, co
                         const uint32_t k = sh.cls[cl[j]] + pos[j];
                         sh.y[k] = y[j];
                         sh.base[k] = ry[j].base;
-                        sh.n16[k] = wide ? 0u : ry[j].n16;   // (no bits then)
+                        sh.n16[k] = ry[j].n16;
                         sh.n32[k] = ry[j].n32;
                     }
                 __syncthreads();
                 if (rx.n32 == 0) tc_walk<TC_NONE>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
                 else if (search) tc_walk<TC_SORTED>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
-                else if (wide) tc_walk<TC_HASHED_WIDE>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
+                else if (wide) tc_walk_wide(sh, n, ids, per_vertex, acc);
                 else tc_walk<TC_HASHED>(sh, nlong, n, codes, ids, sorted, per_vertex, acc);
                 __syncthreads();
             }
