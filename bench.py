@@ -8,8 +8,8 @@ Workload (one "step" = one pass of the hot path over one batch of input):
   adjacency entries scanned (sum of degrees of reached vertices, m_C) per
   second; Graph500's convention (m_C / 2) is reported beside it.
 
-Printed: ONE JSON line with the metric, the roofline of the dominant kernel
-(bfs_expand_kernel, HIP events around every launch in the timed region) and
+Printed: ONE JSON line with the metric, the roofline of the expansions of its
+levels (HIP events around every such launch in the timed region) and
 a CPU baseline (the oracle's sequential host BFS, restated from
 xlib/src/Graph/BFS.cpp:54-76, on a bounded sample of the same sources).
 """
@@ -96,8 +96,46 @@ def update_bytes(st):
             + 8 * st["relocated_deg"] + 16 * st["relocated"])
 
 
+def bfs_roofline(args, entries: int, vertices: int, ns: int, levels: int):
+    """The expansions of `levels` levels in `ns` nanoseconds: whole-device rounds
+    (bfs_expand_kernel), and the launches of bfs_small_kernel, which take several
+    levels each.  A pull round skips most entries of its level, so the bytes moved
+    are those that the counters saw per level of this workload (committed
+    summaries, None for another one); what a traversal that reads every entry
+    cannot do without (4 B per entry, 16 B record + 4 B queue read per frontier
+    vertex, 4 B distance + 4 B queue write per discovery) is given beside them."""
+    same = (args.scale, args.edge_factor, args.seed) == (24, 16, 24)
+    traffic = load_traffic("bfs_expand_traffic.json") if same else None
+    l2req = load_traffic("bfs_expand_l2req.json") if same else None
+    level_s = ns * 1e-9 / max(levels, 1)
+    moved = (traffic or {}).get("bytes_per_level")
+    achieved = round(moved / level_s / 1e9, 1) if moved and level_s > 0 else None
+    roofline = {
+        "kernel": "bfs_expand_kernel, bfs_small_kernel",
+        "bound": "hbm",
+        "achieved": achieved,
+        "peak": HBM_PEAK_GBS,
+        "unit": "GB/s",
+        "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
+        "traffic": moved,
+        "topdown_bytes_per_level": round((4 * entries + 28 * vertices) / max(levels, 1)),
+        "avg_level_us": round(level_s * 1e6, 2),
+        "levels": levels,
+        "entries_per_level": round(entries / max(levels, 1)),
+    }
+    if l2req and l2req.get("read_req_per_level") and level_s > 0:
+        # L1 -> L2 read requests (TCP_TCC_READ_REQ, likewise per level)
+        rate = l2req["read_req_per_level"] / level_s / 1e9
+        roofline["l2_requests"] = {
+            "bound": "l2 request rate", "unit": "G req/s", "peak": L2_PEAK_GREQS,
+            "achieved": round(rate, 1), "frac": round(rate / L2_PEAK_GREQS, 4),
+            "req_per_level": l2req["read_req_per_level"],
+        }
+    return roofline
+
+
 def load_traffic(name: str):
-    """HBM bytes per launch measured by rocprofv3 FETCH_SIZE/WRITE_SIZE for the
+    """HBM bytes measured by rocprofv3 FETCH_SIZE/WRITE_SIZE for the
     same workload (committed summary), or None."""
     path = os.path.join(ROOT, "profiles", name)
     try:
@@ -658,7 +696,7 @@ def main() -> int:
     bfs = BfsTopDown(h)
 
     def step(timed: bool):
-        tot_m = tot_n = kns = launches = 0
+        tot_m = tot_n = kns = levels = 0
         for s in sources:
             bfs.set_parameters(int(s))
             bfs.stats.time_kernels = 1 if timed else 0
@@ -666,8 +704,8 @@ def main() -> int:
             tot_m += bfs.stats.edges_scanned
             tot_n += bfs.stats.visited
             kns += bfs.stats.expand_ns
-            launches += bfs.stats.expand_launches
-        return tot_m, tot_n, kns, launches
+            levels += bfs.stats.levels
+        return tot_m, tot_n, kns, levels
 
     for _ in range(args.warmup):
         step(False)
@@ -685,38 +723,7 @@ def main() -> int:
     print(f"# timed {args.steps} steps in {elapsed:.3f}s", file=sys.stderr, flush=True)
 
     gteps = agg_m / elapsed / 1e9
-    # bfs_expand_kernel algorithmic bytes: 4 B per adjacency entry scanned,
-    # 16 B vertex record + 4 B queue read per frontier vertex, 4 B distance +
-    # 4 B queue write per discovered vertex -> 4 m_C + 28 n_C
-    alg_bytes = 4 * agg_m + 28 * agg_n
-    kernel_s = agg_ns * 1e-9
-    achieved = alg_bytes / kernel_s / 1e9 if kernel_s > 0 else 0.0
-    traffic = load_traffic("bfs_expand_traffic.json")
-    l2req = load_traffic("bfs_expand_l2req.json")
-    roofline = {
-        "kernel": "bfs_expand_kernel",
-        "bound": "hbm",
-        "achieved": round(achieved, 1),
-        "peak": HBM_PEAK_GBS,
-        "unit": "GB/s",
-        "frac": round(achieved / HBM_PEAK_GBS, 4),
-        "traffic": (traffic or {}).get("bytes_per_launch"),
-        "alg_bytes_per_launch": round(alg_bytes / max(agg_l, 1)),
-        "avg_launch_us": round(agg_ns / max(agg_l, 1) / 1e3, 2),
-        "launches": agg_l,
-        "entries_per_launch": round(agg_m / max(agg_l, 1)),
-    }
-    if l2req and l2req.get("read_req_per_entry"):
-        # the bound the random visited probes meet: L1 -> L2 read requests
-        # (TCP_TCC_READ_REQ per scanned entry, from the committed counter
-        # pass on the same workload) over the live kernel time
-        reqs = l2req["read_req_per_entry"] * agg_m
-        roofline["l2_requests"] = {
-            "bound": "l2 request rate", "unit": "G req/s", "peak": L2_PEAK_GREQS,
-            "achieved": round(reqs / kernel_s / 1e9, 1) if kernel_s > 0 else 0.0,
-            "frac": round(reqs / kernel_s / 1e9 / L2_PEAK_GREQS, 4) if kernel_s > 0 else 0.0,
-            "req_per_entry": l2req["read_req_per_entry"],
-        }
+    roofline = bfs_roofline(args, agg_m, agg_n, agg_ns, agg_l)
 
     updates = tc_info = ms_info = snap_info = meta_info = None
     if args.snapshot:

@@ -89,11 +89,12 @@ typedef struct hn_dview {
 /* BFS statistics for one traversal. */
 typedef struct hn_bfs_stats {
     int32_t levels;          /* number of non-empty frontiers                 */
-    int32_t time_kernels;    /* in: nonzero -> time the expansion kernel      */
+    int32_t time_kernels;    /* in: nonzero -> time the expansions            */
     int64_t visited;         /* reached vertices, source included             */
     int64_t edges_scanned;   /* sum of degrees of reached vertices (m_C)      */
-    int64_t expand_ns;       /* out: summed expansion-kernel time (HIP events) */
-    int32_t expand_launches; /* out: levels                                   */
+    int64_t expand_ns;       /* out: device time of the launches that expand levels (HIP events) */
+    int32_t expand_launches; /* out: levels, as above; one launch may expand several, and some
+                              * none: expand_ns / expand_launches is a level's time, not a launch's */
     int32_t pad_;
 } hn_bfs_stats;
 
