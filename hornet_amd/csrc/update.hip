@@ -1207,9 +1207,10 @@ struct SideBuf {
 };
 static hn_status side_buffer(hn_graph* g, UpdBufs& b, int64_t want, SideBuf* out) {
     // test hook: HORNET_HIP_FAIL_SIDE_RESERVE=1 makes this reservation fail as
-    // a device allocation would, after the batch's blocks were allocated
+    // a device allocation would, after the batch's blocks were allocated; 2, only
+    // one for the entries that a batch was stopped with
     if (const char* e = std::getenv("HORNET_HIP_FAIL_SIDE_RESERVE"))
-        if (e[0] == '1') {
+        if (e[0] == '1' || (e[0] == '2' && want > 0)) {
             set_error("side buffer: allocation failure forced by HORNET_HIP_FAIL_SIDE_RESERVE");
             return HN_E_OOM;
         }
