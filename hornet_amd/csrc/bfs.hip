@@ -57,7 +57,7 @@
 // next frontier current.  The distances are written at the end, from the state
 // bytes (bfs_dist_kernel).
 // R-MAT s24, one traversal: 2.3 ms with push rounds alone, 0.67 ms; s20: 0.25 ms,
-// 0.14 ms; s12: 0.11 ms, 0.033 ms; a 733 x 1021 lattice: 28 ms, 5.4 ms.
+// 0.14 ms; s12: 0.11 ms, 0.033 ms; a 733 x 1021 lattice from its corner: 36 ms, 4.1 ms.
 // Distances: source 0, its neighbours 1, unreached INT32_MAX (TopDown.cu:42,81).
 #include <algorithm>
 #include <cstddef>
@@ -936,9 +936,10 @@ __global__ __launch_bounds__(CB) void bfs_collect_kernel(uint32_t r, int32_t max
 // else runs on it).  A level is a chain of two loads, the adjacency group and
 // the record of each newly claimed neighbour, and one barrier, where a round
 // of two whole-device launches takes over 10 us however small the frontier.
-// 733 x 1021 lattice, about 1190 levels of up to 1500 vertices: 28 ms with one
-// round per level, 5.4 ms, 3.4 us a level: two loads from memory.  It stops where the frontier outgrows it, and leaves
-// everything as a round would: state bytes, bitmap, frontier arrays, counters.
+// 733 x 1021 lattice, from its corner 1,753 levels of up to 733 vertices: 36 ms with
+// one round per level, 4.1 ms so, 2.3 us a level: two loads from memory; from its middle
+// 877 levels of up to 1,466: 21 ms, 3.9 ms.  It stops where the frontier outgrows it,
+// and leaves everything as a round would: state bytes, bitmap, frontier arrays, counters.
 // INIT: the whole traversal of a graph with at most TINY_NV vertices and
 // TINY_NE entries (frontiers of any size fit), in this launch alone.
 // A workgroup barrier that orders LDS only: __syncthreads also waits until the

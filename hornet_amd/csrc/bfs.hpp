@@ -49,7 +49,8 @@ struct BfsBufs {
     uint32_t* qbase;
     uint32_t* P;
     uint32_t* tile_lo;
-    uint8_t* state;     // one byte per vertex, padded to whole bitmap words: 1 reached, 2 no edges
+    uint8_t* state;     // one byte per vertex, padded to whole bitmap words: 0 not reached, 1 .. 126 distance + 1,
+                        // 127 reached, its distance is in the caller's array, 128 no edges
     uint64_t* part;     // per collect workgroup: the degrees of discoveries so far
     BfsCtl* ctl;
     uint32_t* any;      // bit b: some vertex of the b-th 2^shift is visited (BFS_ANY_BYTES)

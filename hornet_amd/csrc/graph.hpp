@@ -186,7 +186,7 @@ struct hn_graph {
     // whole-device rounds of the last single-source BFS (-1: none yet): how many
     // the next one queues at first (serving slots run BFS concurrently, hence atomic)
     std::atomic<int> bfs_last_rounds{-1};
-    // timing events of the BFS expansion (one pair per queued level), created
+    // timing events of the BFS expansions (one pair per launch that expands), created
     // on the first timed traversal
     static constexpr int BFS_EVENTS = 64;
     hipEvent_t bfs_ev[BFS_EVENTS] = {};

@@ -43,8 +43,8 @@ constexpr uint32_t ERR_BAD_ID = 1u;
 constexpr uint32_t ERR_OOM = 2u;     // AllocState::error bit 0 is mirrored here
 constexpr uint32_t ERR_SIDE = 4u;    // more deferred entries than the side buffer holds: nothing moved yet
 // Segmented copies: 4 items per lane, at most BLOCK + 1 runs staged in LDS
-// per tile (a tile with more runs searches them in global memory), 8
-// workgroups per CU striding over the tiles.  A one-entry-per-item LDS stage
+// per tile (a tile with more runs searches them in global memory), the
+// workgroups striding over the tiles.  A one-entry-per-item LDS stage
 // (49 KB at 8 items per lane) left three workgroups per CU and halved the
 // copy rate; measured on a 2 M-entry erase at R-MAT s24, 5.0 -> 3.6 ms.
 constexpr int COPY_IPT = 4;
