@@ -218,10 +218,22 @@ __device__ __forceinline__ uint8_t probe_u8(__amdgpu_buffer_rsrc_t r, uint32_t o
     return (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(r, (int)off, 0, 0);
 }
 
+// A round's record, known to be the same for all lanes: the rules over it run in scalar
+// registers, every workgroup's first instructions.
+__device__ __forceinline__ BfsRound bfs_round(const BfsRound* p) {
+    BfsRound rd = *p;
+    uint32_t w[sizeof(BfsRound) / 4];
+    __builtin_memcpy(w, &rd, sizeof rd);
+#pragma unroll
+    for (uint32_t& x : w) x = (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+    __builtin_memcpy(&rd, w, sizeof rd);
+    return rd;
+}
+
 // Pulling follows the stored entries backwards, so only adjacency known to be
 // symmetric pulls (sym).
 __device__ __forceinline__ bool bfs_pulls(const BfsRound& rd, int64_t nv, int64_t ne, int32_t sym) {
-    return sym && hn::bfs_pulls(rd.fc >> 32, (uint32_t)rd.fc, rd.scan, rd.vis, nv, ne);
+    return sym && hn::bfs_pulls(rd.fc >> 32, (uint32_t)rd.fc, rd.scan, rd.vis, nv, ne, rd.prev);
 }
 
 // the frontier slice of a tile: group prefix, adjacency offset in 128-byte
@@ -242,7 +254,11 @@ struct ExpShared {
 constexpr int PULL_J = BFS_PULL_J;        // open vertices per lane and batch
 constexpr int PULL_BATCH = WAVE * PULL_J;
 constexpr int PULL_SPAN_WORDS = 32;       // bitmap words (32 vertices each) a wave takes at a time
-constexpr int PULL_SPAN_SMALL = 8;        // ... on graphs too small to give every wave that many
+constexpr int PULL_SPAN_SMALL = 8;        // ... on graphs too small to give every wave that many,
+// and on few words: a wave's rows that do not settle are a chain of steps (20 layers of
+// 2,000 vertices with 64 edges each to the next, 510 us with 8, 400 so; R-MAT s18, whose rows do, 108 and 124 us)
+constexpr int PULL_SPAN_TINY = 2;
+constexpr int64_t PULL_TINY_WORDS = 2048;
 constexpr int PULL_FLUSH = 112;           // rows left that make the second step run
 constexpr int PULL_ROWS = PULL_FLUSH + PULL_BATCH;
 constexpr int TEAM = 8;                   // lanes that scan one row: 8 x 16 bytes, a 128-byte line
@@ -453,7 +469,8 @@ __device__ __forceinline__ void bfs_pull(PullShared& sh, uint32_t L, int64_t nv,
     };
     // small graphs: shorter spans, so that every wave has one
     const int64_t nwaves = (int64_t)gridDim.x * EXP_WAVES;
-    const int sw = words >= nwaves * PULL_SPAN_WORDS / 2 ? PULL_SPAN_WORDS : PULL_SPAN_SMALL;
+    const int sw = words >= nwaves * PULL_SPAN_WORDS / 2 ? PULL_SPAN_WORDS
+                   : words > PULL_TINY_WORDS ? PULL_SPAN_SMALL : PULL_SPAN_TINY;
     for (int64_t c = (int64_t)blockIdx.x * EXP_WAVES + wv; c * sw < words; c += nwaves) {
         const int64_t w0 = c * sw, v0 = w0 * 32;
         uint32_t bits = 0;
@@ -571,7 +588,7 @@ __global__ __launch_bounds__(EXP_BLOCK, 6) void bfs_expand_kernel(uint32_t r, in
     ExpShared& sh = ssh.push;
     const __amdgpu_buffer_rsrc_t rbm = probe_rsrc(bitmap, (uint32_t)(words * 4));
     const __amdgpu_buffer_rsrc_t rst = probe_rsrc(state, (uint32_t)(words * 32));
-    const BfsRound rd = ctl->rd[r % 3];
+    const BfsRound rd = bfs_round(&ctl->rd[r % 3]);
     const uint32_t L = rd.lev;
     const int64_t F = (int64_t)(rd.fc >> 32);
     const bool over = F == 0 || (max_levels > 0 && (int64_t)L > max_levels);
@@ -601,6 +618,7 @@ __global__ __launch_bounds__(EXP_BLOCK, 6) void bfs_expand_kernel(uint32_t r, in
                 ctl->rd[(r + 1) % 3].scan = t;
                 ctl->rd[(r + 1) % 3].vis = rd.vis + (uint64_t)F;
                 ctl->rd[(r + 1) % 3].lev = L + 1;
+                ctl->rd[(r + 1) % 3].prev = (uint32_t)rd.fc;
                 ctl->claim = 0;
                 ctl->scanned = t;
                 ctl->levels = L;
@@ -611,7 +629,9 @@ __global__ __launch_bounds__(EXP_BLOCK, 6) void bfs_expand_kernel(uint32_t r, in
         }
     }
     if (over) return;
-    if (bfs_pulls(rd, nv, ne, sym)) {
+    const bool pull = bfs_pulls(rd, nv, ne, sym);
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->pulled = pull ? 1u : 0u;
+    if (pull) {
         PullSum s;
         // (a visited vertex sets at most one of the summary's bits)
         if (any_shift > 0 && rd.vis + (uint64_t)F < (uint64_t)ANY_WORDS * 32)
@@ -783,14 +803,14 @@ __global__ __launch_bounds__(CB) void bfs_collect_kernel(uint32_t r, int32_t max
                                                             int32_t* __restrict__ qdeg, uint32_t* __restrict__ qbase,
                                                             uint32_t* __restrict__ P, uint32_t* __restrict__ tile_lo,
                                                             uint64_t* __restrict__ part, BfsCtl* __restrict__ ctl) {
-    const BfsRound rd = ctl->rd[r % 3];
+    const BfsRound rd = bfs_round(&ctl->rd[r % 3]);
     if ((rd.fc >> 32) == 0) return;   // a round launched after the traversal ended
     if (max_levels > 0 && (int64_t)rd.lev > max_levels) return;
     const int32_t level = (int32_t)rd.lev;
     // after a pull the discoveries are counted; their frontier is written only if
     // the next round pushes it
-    const bool pulled = bfs_pulls(rd, nv, ne, sym);
-    const bool want_list = !pulled || !bfs_pulls(ctl->rd[(r + 1) % 3], nv, ne, sym);
+    const bool pulled = __builtin_amdgcn_readfirstlane((int)ctl->pulled) != 0;
+    const bool want_list = !pulled || !bfs_pulls(bfs_round(&ctl->rd[(r + 1) % 3]), nv, ne, sym);
     const int64_t wi = (int64_t)blockIdx.x * CB + threadIdx.x;
     uint32_t found = 0;
     bool wfull = false, wany = false;
@@ -1134,6 +1154,8 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
         dsum += (uint64_t)F * (L - 1);
         rd.scan += 4ull * W;
         rd.vis += F;
+        const uint32_t prev = rd.prev;
+        rd.prev = W;
         const int top = 31 - __clz((int)F | 1);   // F < 2^(top + 1)
         // a claimed vertex's distance, and its frontier entry
         auto mark = [&](int32_t v) {
@@ -1176,8 +1198,12 @@ __global__ __launch_bounds__(SM_BLOCK) void bfs_small_kernel(uint32_t r, int32_t
                 sh.multi[(L + 1) % 3] = 1;
             }
         };
-        // (every unreached vertex costs a pull at least one group)
-        const bool pull = INIT && sym && W > SM_DENSE_W && 2 * (uint64_t)W > (uint64_t)nv - visited;
+        // every unreached vertex costs a pull at least one group, and one that it does not
+        // reach (see bfs_pulls) all of its row: 20 layers of 300 vertices with 16 edges each
+        // to the next, 380 us without, 130 so
+        const uint64_t open = (uint64_t)nv - visited, mu = (uint64_t)ne > rd.scan ? (uint64_t)ne - rd.scan : 0;
+        const bool pull = INIT && sym && W > SM_DENSE_W && 2 * (uint64_t)W > open &&
+                          (2 * (uint64_t)W > open + mu / EXP_G || 2 * (uint64_t)W > open + bfs_wasted(F, W, prev, open, mu) / EXP_G);
         if constexpr (INIT)
             if (pull) {
                 for (int i = tid; i < (int)words; i += SM_BLOCK) sh.bm0[i] = sh.bm[i];
@@ -1525,7 +1551,7 @@ hn_status bfs_run(hn_graph* g, int32_t source, int32_t* dist, hn_bfs_stats* stat
         e = hipGetLastError();                                                                           \
     } while (0)
     const int64_t grid = std::min<int64_t>((int64_t)num_cus() * BFS_GRID_PER_CU * BLOCK / EXP_BLOCK,
-                                           std::max(ceil_div(ne / EXP_G + nv, EXP_TILE), ceil_div(words, PULL_SPAN_SMALL * EXP_WAVES)));
+                                           std::max(ceil_div(ne / EXP_G + nv, EXP_TILE), ceil_div(words, (words > PULL_TINY_WORDS ? PULL_SPAN_SMALL : PULL_SPAN_TINY) * EXP_WAVES)));
     uint32_t r = 0;   // rounds launched
     const bool tiny = nv <= TINY_NV && ne <= TINY_NE;
     auto small = [&](int first) {

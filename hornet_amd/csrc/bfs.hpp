@@ -16,7 +16,7 @@ struct BfsRound {
                        // bfs_small_kernel: 4 per group)
     uint64_t vis;      // sum of their sizes
     uint32_t lev;      // its level (its vertices lie at distance lev - 1)
-    uint32_t pad_;
+    uint32_t prev;     // groups of the frontier before it (0: there was none)
 };
 struct BfsCtl {
     // round r reads rd[r % 3], adds its discoveries to rd[(r + 1) % 3].fc and
@@ -24,6 +24,8 @@ struct BfsCtl {
     // written in it
     BfsRound rd[3];
     uint64_t claim;    // frontier slots claimed by the collect of a pull round, as in fc
+    uint32_t pulled;   // whether the last round's expansion pulled, for its collect
+    uint32_t pad_;
     uint32_t levels;   // last non-empty level = number of non-empty frontiers
     uint32_t rounds;   // rounds that expanded a frontier
     uint64_t visited;  // sum of the frontier sizes expanded
