@@ -444,9 +444,10 @@ __device__ __forceinline__ uint32_t tc_entry(const TcRow& r, uint32_t i, const u
 // as atomics on one counter take 10 ns each: R-MAT s18 oriented, 319 us in one part, 118 so.
 // Otherwise bound by the lookups of the entries' lists: only owners' are looked up, by a
 // bit that the L2 holds (four million vertices of four entries: 525 us without, 217 so).
-// Eight entries without a grouped edge have a bit (`placed`) and no places, and a tile
-// without any is not read again (the same vertices, of which few are owners: 213 and
-// 119 us, 138 and 11 so).
+// 512 entries without a grouped edge (a wave's) have that noted (`placed`) and no places, and
+// a tile without any is not read again (the same vertices, of which few are owners: 213
+// and 119 us, 122 and 5 so; by eight entries, places would be parts of lines, and 256 K
+// vertices of 64 entries take 35 us more to read them).
 template <bool FILL>
 __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
                                                          const uint32_t* __restrict__ P,
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, uint32_t* __restrict__ gcnt,
                                                          uint32_t* __restrict__ part, int64_t nhub,
-                                                         uint32_t* __restrict__ place, uint64_t* __restrict__ placed,
+                                                         uint32_t* __restrict__ place, uint8_t* __restrict__ placed,
                                                          const uint32_t* __restrict__ goff, uint32_t* __restrict__ members) {
     if (sym && !ctl->repeats) return;
     uint32_t* const mine = part + (blockIdx.x % TC_LANES) * nhub;
@@ -465,27 +466,27 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
     const uint32_t total = *ngroups;
     const int64_t ntiles = ((int64_t)total + TC_TILE - 1) / TC_TILE;
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        uint64_t* const bits = placed + t * (TC_TILE / WAVE);   // a word per wave and step
+        uint8_t* const some = placed + t * (TC_TILE / WAVE);   // of a wave's 64 groups
+        bool fill[TC_IPT] = {};
         if constexpr (FILL) {
-            uint64_t any = 0;
 #pragma unroll
-            for (int k = 0; k < TC_TILE / WAVE; k++) any |= bits[k];
-            if (!any) continue;
+            for (int j = 0; j < TC_IPT; j++) fill[j] = some[j * NWAVES + threadIdx.x / WAVE] != 0;
+            static_assert(TC_TILE / WAVE == 8, "one word has all");
+            if (*reinterpret_cast<const uint64_t*>(some) == 0) continue;
         }
         uint32_t unused[TC_IPT];
         const TcLoc c = tc_locate(P, nv, total, tile_lo, t, ntiles, sh, [&](int64_t) { return 0u; }, unused);
 #pragma unroll
         for (int j = 0; j < TC_IPT; j++) {
-            uint64_t* const word = bits + j * NWAVES + threadIdx.x / WAVE;
-            bool some = FILL ? (*word >> __lane_id() & 1u) != 0 : c.seg[j] >= 0;
             // entries [8k, 8k + 8) of a list, which may end before its stored row
-            const uint32_t u = some ? (uint32_t)c.seg[j] : 0u, i0 = c.k[j] * TC_G;
-            const TcRow r = some ? row[u] : TcRow{0u, 0u, 0u, 0u};
+            bool in = (FILL ? fill[j] : true) && c.seg[j] >= 0;
+            const uint32_t u = in ? (uint32_t)c.seg[j] : 0u, i0 = c.k[j] * TC_G;
+            const TcRow r = in ? row[u] : TcRow{0u, 0u, 0u, 0u};
             const uint32_t lu = r.len();
-            some = some && lu >= 2 && i0 < lu;
-            if (some) {
-                const int64_t at = (int64_t)r.base * TC_G;
-                uint32_t q[TC_G], v[TC_G];
+            const int64_t at = (int64_t)r.base * TC_G;
+            in = in && lu >= 2 && i0 < lu;
+            uint32_t q[TC_G], v[TC_G], lv[TC_G];
+            if (in) {
 #pragma unroll
                 for (int e = 0; e < TC_G; e++) {
                     const uint32_t i = i0 + e;
@@ -495,32 +496,32 @@ __global__ __launch_bounds__(BLOCK) void tc_group_kernel(int64_t nv, const uint3
 #pragma unroll
                 for (int e = 0; e < TC_G; e++)
                     if (q[e] != TC_PAD) v[e] = hub[q[e]];
-                if constexpr (FILL) {
+            }
+            if constexpr (FILL) {
+                if (!in) continue;
 #pragma unroll
-                    for (int e = 0; e < TC_G; e++) {
-                        const uint32_t pl = i0 + e < lu ? place[at + i0 + e] : TC_PAD;
-                        if (pl != TC_PAD) members[(int64_t)goff[v[e]] + (q[e] != TC_PAD ? mine[q[e]] : 0u) + pl] = u;
-                    }
-                } else {
+                for (int e = 0; e < TC_G; e++) {
+                    const uint32_t pl = i0 + e < lu ? place[at + i0 + e] : TC_PAD;
+                    if (pl != TC_PAD) members[(int64_t)goff[v[e]] + (q[e] != TC_PAD ? mine[q[e]] : 0u) + pl] = u;
+                }
+            } else {
+                bool any = false;
+                if (in) {
                     uint64_t big[TC_G];
-                    uint32_t lv[TC_G];
 #pragma unroll
                     for (int e = 0; e < TC_G; e++) big[e] = owner[v[e] / WAVE];
 #pragma unroll
                     for (int e = 0; e < TC_G; e++) lv[e] = v[e] != u && (big[e] >> (v[e] % WAVE) & 1u) ? row[v[e]].len() : 0u;
-                    some = false;
 #pragma unroll
-                    for (int e = 0; e < TC_G; e++) some = some || (i0 + e < lu && lv[e] > lu);
-                    if (some)
-#pragma unroll
-                        for (int e = 0; e < TC_G; e++)
-                            if (i0 + e < lu)
-                                place[at + i0 + e] = lv[e] > lu ? atomicAdd(q[e] != TC_PAD ? mine + q[e] : gcnt + v[e], 1u) : TC_PAD;
+                    for (int e = 0; e < TC_G; e++) any = any || (i0 + e < lu && lv[e] > lu);
                 }
-            }
-            if constexpr (!FILL) {
-                const uint64_t mask = __ballot(some);
-                if (__lane_id() == 0) *word = mask;
+                const bool write = __ballot(any) != 0;
+                if (write && in)
+#pragma unroll
+                    for (int e = 0; e < TC_G; e++)
+                        if (i0 + e < lu)
+                            place[at + i0 + e] = lv[e] > lu ? atomicAdd(q[e] != TC_PAD ? mine + q[e] : gcnt + v[e], 1u) : TC_PAD;
+                if (__lane_id() == 0) some[j * NWAVES + threadIdx.x / WAVE] = write ? 1 : 0;
             }
         }
         __syncthreads();
@@ -1022,7 +1023,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     const int64_t nhub = std::min<int64_t>(nv, TC_HUBS + 1);
     const int64_t o_part = take(nhub * TC_LANES * 4), o_zero_end = o;   // cleared together
     const int64_t o_gcnt = take(nv * 4), o_weight = take(nv * 4), o_wc = take(nv * 8), o_hub = take((int64_t)(TC_HUBS + 1) * 4);
-    const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4), o_placed = take(tiles * (TC_TILE / WAVE) * 8);
+    const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4), o_placed = take(tiles * (TC_TILE / WAVE));
     const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
     const int64_t o_goff = take((nv + 1) * 4), o_mem = take(ne * 4), o_task = take(tasks * 8);
     const int64_t bits = (nv + WAVE - 1) / WAVE * 8, o_some = take(bits), o_owner = take(bits), o_small = take(bits);
@@ -1043,7 +1044,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     uint16_t* codes = at(o_codes, (uint16_t*)nullptr);
     uint32_t* ids = at(o_ids, (uint32_t*)nullptr);
     uint32_t* place = at(o_place, (uint32_t*)nullptr);
-    uint64_t* placed = at(o_placed, (uint64_t*)nullptr);
+    uint8_t* placed = at(o_placed, (uint8_t*)nullptr);
     uint32_t* goff = at(o_goff, (uint32_t*)nullptr);
     uint32_t* members = at(o_mem, (uint32_t*)nullptr);
     uint2* task = at(o_task, (uint2*)nullptr);
