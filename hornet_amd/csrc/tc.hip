@@ -50,7 +50,8 @@ constexpr uint32_t TC_PAD16 = 0xFFFF;          // fills the last group of a row 
 constexpr uint32_t TC_PAD = 0xFFFFFFFFu;       // ... of a row of ids
 constexpr uint32_t TC_ID = 0x80000000u;        // (in a vertex's code) no hub: TC_ID | id
 constexpr int TC_BINS = 4096;
-constexpr uint32_t TC_SMALL = 16;              // lists up to this long are compared in registers
+constexpr uint32_t TC_SMALL = 16;              // lists up to this long are compared in registers,
+constexpr uint32_t TC_SMALL_GROUPED = 32;      // up to this where there are many and owners' edges are grouped
 constexpr uint32_t TC_CAND = 1024;             // candidates per task
 constexpr int TC_STEP = 2 * BLOCK;             // ... listed at a time
 constexpr uint32_t TC_TAIL = 256;              // ids hashed at a time
@@ -408,8 +409,9 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
 constexpr int TC_PAD_WORDS = 4;   // of 64 vertices to a wave
 __global__ __launch_bounds__(BLOCK) void tc_pad_kernel(int64_t nv, const uint64_t* __restrict__ some,
                                                        const TcRow* __restrict__ row, uint16_t* __restrict__ codes,
-                                                       uint32_t* __restrict__ ids, uint64_t* __restrict__ owner,
-                                                       uint64_t* __restrict__ small, uint32_t* __restrict__ gcnt) {
+                                                       uint32_t* __restrict__ ids, uint32_t most,
+                                                       uint64_t* __restrict__ owner, uint64_t* __restrict__ small,
+                                                       uint32_t* __restrict__ gcnt) {
     const int64_t w0 = ((int64_t)blockIdx.x * NWAVES + threadIdx.x / WAVE) * TC_PAD_WORDS, words = (nv + WAVE - 1) / WAVE;
     const int lane = __lane_id();
     TcRow r[TC_PAD_WORDS];
@@ -420,12 +422,12 @@ __global__ __launch_bounds__(BLOCK) void tc_pad_kernel(int64_t nv, const uint64_
     }
 #pragma unroll
     for (int j = 0; j < TC_PAD_WORDS; j++) {
-        const uint64_t big = __ballot(r[j].len() > TC_SMALL), few = __ballot(r[j].len() >= 2 && r[j].len() <= TC_SMALL);
+        const uint64_t big = __ballot(r[j].len() > most), few = __ballot(r[j].len() >= 2 && r[j].len() <= most);
         if (lane == 0 && w0 + j < words) {
             owner[w0 + j] = big;
             small[w0 + j] = few;
         }
-        if (r[j].len() > TC_SMALL) gcnt[(w0 + j) * WAVE + lane] = 0;
+        if (r[j].len() > most) gcnt[(w0 + j) * WAVE + lane] = 0;
         for (uint32_t i = r[j].n16; i & (TC_G - 1); i++) codes[(int64_t)r[j].base * TC_G + i] = (uint16_t)TC_PAD16;
         for (uint32_t i = r[j].n32; i & (TC_G - 1); i++) ids[(int64_t)r[j].base * TC_G + i] = TC_PAD;
     }
@@ -931,56 +933,67 @@ __device__ __forceinline__ uint32_t tc_common(const TcRow& s, const TcRow& l, co
     return c;
 }
 
-// Edges between two lists of at most TC_SMALL entries: a lane per edge, TC_SMALL
-// lanes per source.  The chain source row, entry, hub, row, list is what bounds
+// Edges between two lists of at most `most` entries: a lane per edge, TC_SMALL
+// lanes per source, twice where it has more.  The chain source row, entry, hub, row, list is what bounds
 // it, so a lane starts four of them at once; a thread per source, one entry after
 // the other, took 330 us on a graph of a thousand vertices.
+// An owner's task is a longer chain, 20 us for a handful of candidates, and its edges are
+// grouped first: 260 K vertices with 16 entries to others took 1.65 ms where lists of
+// 17 to 32 entries were owners', 0.60 so; 100 K, 718 and 307 us.  Not where few waves
+// share the work (R-MAT s12 oriented, 140 us, 182 so; s17 690 and 715), nor on symmetric
+// storage, where nothing is grouped (R-MAT s22 9.4 and 10.4 ms).
 // A wave's sources are those of `per` vertices, its lanes' own rows: 16, one step at
 // most, or 64 where there are waves enough all the same (16 M vertices with
 // a thousand edges: 186 us with every lane reading its source's row, 51 so; four million of
 // four entries: 975, 690; R-MAT s12 is 20 % slower with 64, 16 M vertices are so with 16).
 constexpr int TC_SRC = 4;
 constexpr int64_t TC_WIDE = 1 << 20;
-__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, const uint64_t* __restrict__ small,
+__global__ __launch_bounds__(BLOCK) void tc_small_kernel(int64_t nv, int per, uint32_t most, const uint64_t* __restrict__ small,
                                                          const TcRow* __restrict__ row,
                                                          const uint16_t* __restrict__ codes,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ hub, TcCtl* __restrict__ ctl,
                                                          unsigned long long* __restrict__ per_vertex) {
-    const int lane = __lane_id(), sub = lane % TC_SMALL, team = lane / TC_SMALL;
+    const int lane = __lane_id(), team = lane / TC_SMALL;
+    const uint32_t sub = lane % TC_SMALL;
     const int64_t w0 = ((int64_t)blockIdx.x * NWAVES + threadIdx.x / WAVE) * per;
     if (w0 >= nv) return;
     const bool has = lane < per && (small[w0 / WAVE] >> (w0 % WAVE) >> lane & 1u);   // (no bits from nv on)
     const uint64_t m = __ballot(has);
     if (m == 0) return;
     const TcRow own = has ? row[w0 + lane] : TcRow{0u, 0u, 0u, 0u};
-    const int nsrc = __popcll(m);
-    // lane k gets the k-th source's lane (the others fill up behind)
-    const int to = has ? __popcll(m & lanemask_lt()) : nsrc + __popcll(~m & lanemask_lt());
-    const int from = __builtin_amdgcn_ds_permute(to * 4, lane);
     uint64_t acc = 0;
-    for (int k0 = 0; k0 < nsrc; k0 += TC_SRC * (WAVE / TC_SMALL)) {
-        TcRow ru[TC_SRC], rv[TC_SRC];
-        uint32_t u[TC_SRC], v[TC_SRC];
+    // entries [i0, i0 + TC_SMALL) of the lists that have them
+    for (uint32_t i0 = 0; i0 < most; i0 += TC_SMALL) {
+        const bool src = own.len() > i0;
+        const uint64_t ms = __ballot(src);
+        const int nsrc = __popcll(ms);
+        // lane k gets the k-th source's lane (the others fill up behind)
+        const int to = src ? __popcll(ms & lanemask_lt()) : nsrc + __popcll(~ms & lanemask_lt());
+        const int from = __builtin_amdgcn_ds_permute(to * 4, lane);
+        for (int k0 = 0; k0 < nsrc; k0 += TC_SRC * (WAVE / TC_SMALL)) {
+            TcRow ru[TC_SRC], rv[TC_SRC];
+            uint32_t u[TC_SRC], v[TC_SRC];
 #pragma unroll
-        for (int j = 0; j < TC_SRC; j++) {
-            const int k = k0 + j * (WAVE / TC_SMALL) + team, l = __shfl(from, min(k, WAVE - 1), WAVE);
-            ru[j] = TcRow{(uint32_t)__shfl(own.base, l, WAVE), 0u, (uint32_t)__shfl(own.n16, l, WAVE),
-                          (uint32_t)__shfl(own.n32, l, WAVE)};
-            u[j] = (uint32_t)(w0 + l);
-            v[j] = k < nsrc && sub < (int)ru[j].len() ? tc_entry(ru[j], sub, codes, ids, hub) : TC_PAD;
-        }
+            for (int j = 0; j < TC_SRC; j++) {
+                const int k = k0 + j * (WAVE / TC_SMALL) + team, l = __shfl(from, min(k, WAVE - 1), WAVE);
+                ru[j] = TcRow{(uint32_t)__shfl(own.base, l, WAVE), 0u, (uint32_t)__shfl(own.n16, l, WAVE),
+                              (uint32_t)__shfl(own.n32, l, WAVE)};
+                u[j] = (uint32_t)(w0 + l);
+                v[j] = k < nsrc && i0 + sub < ru[j].len() ? tc_entry(ru[j], i0 + sub, codes, ids, hub) : TC_PAD;
+            }
 #pragma unroll
-        for (int j = 0; j < TC_SRC; j++) rv[j] = v[j] != TC_PAD && v[j] != u[j] ? row[v[j]] : TcRow{0u, 0u, 0u, 0u};
+            for (int j = 0; j < TC_SRC; j++) rv[j] = v[j] != TC_PAD && v[j] != u[j] ? row[v[j]] : TcRow{0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int j = 0; j < TC_SRC; j++) {
-            if (rv[j].len() == 0 || rv[j].len() > TC_SMALL) continue;
-            const bool mine = ru[j].len() < rv[j].len();   // the source's list is the shorter one (ties: the destination's)
-            const TcRow a = {mine ? ru[j].base : rv[j].base, 0u, mine ? ru[j].n16 : rv[j].n16, mine ? ru[j].n32 : rv[j].n32};
-            const TcRow b = {mine ? rv[j].base : ru[j].base, 0u, mine ? rv[j].n16 : ru[j].n16, mine ? rv[j].n32 : ru[j].n32};
-            const uint32_t c = tc_common(a, b, codes, ids);
-            if (c && per_vertex) atomicAdd(per_vertex + (mine ? u[j] : v[j]), (unsigned long long)c);
-            acc += c;
+            for (int j = 0; j < TC_SRC; j++) {
+                if (rv[j].len() == 0 || rv[j].len() > most) continue;
+                const bool mine = ru[j].len() < rv[j].len();   // the source's list is the shorter one (ties: the destination's)
+                const TcRow a = {mine ? ru[j].base : rv[j].base, 0u, mine ? ru[j].n16 : rv[j].n16, mine ? ru[j].n32 : rv[j].n32};
+                const TcRow b = {mine ? rv[j].base : ru[j].base, 0u, mine ? rv[j].n16 : ru[j].n16, mine ? rv[j].n32 : ru[j].n32};
+                const uint32_t c = tc_common(a, b, codes, ids);
+                if (c && per_vertex) atomicAdd(per_vertex + (mine ? u[j] : v[j]), (unsigned long long)c);
+                acc += c;
+            }
         }
     }
     acc = wave_reduce_sum(acc);
@@ -1013,6 +1026,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     const int64_t tasks = std::min(nv, ne / TC_SMALL) + 2 * ne / TC_CAND + 1;
     // what an owner's stored row says of its edges holds on symmetric storage only
     const int sym = orient && graph_known_symmetric(g) ? 1 : 0;
+    const uint32_t most = sym || nv <= (int64_t)TC_HUBS ? TC_SMALL : TC_SMALL_GROUPED;
     int64_t o = 0;
     auto take = [&](int64_t bytes) {
         const int64_t at = o;
@@ -1085,7 +1099,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     else
         tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
     HN_CHECK_LAUNCH();
-    tc_pad_kernel<<<(unsigned)ceil_div(nv, BLOCK * TC_PAD_WORDS), BLOCK, 0, st>>>(nv, some, row, codes, ids, owner, small, gcnt);
+    tc_pad_kernel<<<(unsigned)ceil_div(nv, BLOCK * TC_PAD_WORDS), BLOCK, 0, st>>>(nv, some, row, codes, ids, most, owner, small, gcnt);
     HN_CHECK_LAUNCH();
     // 3. edges owned by their destination
     tc_group_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, sym, ctl, row, owner, codes, ids, hub, gcnt, part, nhub,
@@ -1102,7 +1116,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
                                                                hub, gcnt, goff, members, ctl, per);
     HN_CHECK_LAUNCH();
     const int small_per = nv > TC_WIDE ? WAVE : TC_SRC * (WAVE / TC_SMALL);
-    tc_small_kernel<<<(unsigned)ceil_div(nv, (int64_t)small_per * NWAVES), BLOCK, 0, st>>>(nv, small_per, small, row, codes, ids,
+    tc_small_kernel<<<(unsigned)ceil_div(nv, (int64_t)small_per * NWAVES), BLOCK, 0, st>>>(nv, small_per, most, small, row, codes, ids,
                                                                                            hub, ctl, per);
     HN_CHECK_LAUNCH();
     TcSum sums[TC_SUMS];

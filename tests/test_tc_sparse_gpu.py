@@ -57,3 +57,30 @@ def test_edges_grouped_in_some_tiles(length):
     for _ in range(2):
         tc.run()
         assert tc.countTriangles() == int(want.sum()) and np.array_equal(tc.copyTCToHost(), want)
+
+
+@pytest.mark.parametrize("nv", [65535, 65536])
+@pytest.mark.parametrize("stored", [False, True])
+def test_lists_around_the_small_ones(nv, stored):
+    """Cliques whose lists have 15 to 18 and 30 to 34 entries, stored as they are and from a
+    CSR (not known to be symmetric), on both sides of where lists of 32 count as short."""
+    import torch
+
+    import hornet_amd.graph as G
+    print(f"case tc short lists nv={nv} stored={stored}", flush=True)
+    sizes = [16, 17, 18, 19, 31, 32, 33, 34, 35] * 2
+    at = np.cumsum([0] + [n + 7 for n in sizes])
+    src, dst = (np.concatenate([v + np.triu_indices(n, 1)[e] for v, n in zip(at, sizes)]) for e in (0, 1))
+    # and edges between lists of different lengths
+    rng = np.random.default_rng(5)
+    more = rng.integers(0, at[-1], (2, 400))
+    src, dst = np.concatenate([src, more[0]]), np.concatenate([dst, more[1]])
+    h = G.Hornet.from_coo_device(nv, *(torch.from_numpy(x.astype(np.int32)).cuda() for x in (src, dst)))
+    h = G.Hornet.from_device_csr(*h.getCSR())
+    off, adj = (x.cpu().numpy() for x in h.getCSR())
+    want = O.tc2_per_vertex(*((off, adj) if stored else O.directed_by_degree(off, adj)))
+    tc = G.TriangleCounting2(h)
+    tc.init()
+    for _ in range(2):
+        (tc.run if stored else tc.run_undirected)()
+        assert tc.countTriangles() == int(want.sum()) and np.array_equal(tc.copyTCToHost(), want)
