@@ -160,12 +160,16 @@ struct HubIn {
         return w > 1 && tc_bin(w) >= ctl->cut ? 1u : 0u;
     }
 };
-// (weight, code) side by side: the orientation looks up both of every entry
+// (weight, code) side by side: the orientation looks up both of every entry; and a bit
+// per vertex, for the passes that need a hub's code only (a wave has a word of `hubs`)
 struct HubOut {
     const uint32_t* weight;
     uint2* wc;
     uint32_t* hub;
+    uint64_t* hubs;
     __device__ __forceinline__ void operator()(int64_t v, uint32_t ex, uint32_t is) const {
+        const uint64_t any = __ballot(is != 0);
+        if (v % WAVE == 0) hubs[v / WAVE] = any;
         wc[v] = make_uint2(weight[v], is ? ex : (TC_ID | (uint32_t)v));
         if (is) hub[ex] = (uint32_t)v;
     }
@@ -317,6 +321,9 @@ __global__ __launch_bounds__(BLOCK) void tc_weight_freq_kernel(int64_t nv, const
 // claim its next places, in both of its rows, with one atomic, or none if they hold
 // all of it (four million rows of four entries: 461 us with one for each, 440 so;
 // of one entry: 457, 274).
+// Stored rows need the codes of hubs only, and the L2 holds a bit per vertex that says which
+// are (four million rows of four entries 442 us with a look-up for every entry, 272 so;
+// 16 M rows 1,880 and 1,230); degree orders need every entry's degree.
 typedef int32_t TcVec __attribute__((ext_vector_type(4)));
 template <bool ORIENT>
 __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32_t* __restrict__ ngroups,
@@ -324,7 +331,8 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
                                                         const uint32_t* __restrict__ tile_lo,
                                                         const hn_vrec* __restrict__ rec,
                                                         const int32_t* __restrict__ arena,
-                                                        const uint2* __restrict__ wc, TcRow* __restrict__ row,
+                                                        const uint2* __restrict__ wc,
+                                                        const uint64_t* __restrict__ hubs, TcRow* __restrict__ row,
                                                         uint16_t* __restrict__ codes, uint32_t* __restrict__ ids,
                                                         TcCtl* __restrict__ ctl) {
     __shared__ TcLb sh;
@@ -355,7 +363,17 @@ __global__ __launch_bounds__(BLOCK) void tc_rows_kernel(int64_t nv, const uint32
             const int32_t u = (int32_t)c.seg[j];
             uint2 x[TC_G];
 #pragma unroll
-            for (int e = 0; e < TC_G; e++) x[e] = wc[e < n ? a[j][e] : 0];
+            for (int e = 0; e < TC_G; e++) {
+                if constexpr (ORIENT) {
+                    x[e] = wc[e < n ? a[j][e] : 0];
+                } else {
+                    const uint32_t v = e < n ? (uint32_t)a[j][e] : 0u;
+                    x[e].x = !hubs || (hubs[v / WAVE] >> (v % WAVE) & 1u) ? 1u : 0u;   // (no bits: all are)
+                }
+            }
+            if constexpr (!ORIENT)
+#pragma unroll
+                for (int e = 0; e < TC_G; e++) x[e].y = !hubs ? (uint32_t)a[j][e] : x[e].x ? wc[e < n ? a[j][e] : 0].y : TC_ID;
             uint32_t keep = 0, hubs = 0;
 #pragma unroll
             for (int e = 0; e < TC_G; e++) {
@@ -1040,7 +1058,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     const int64_t o_row = take(nv * (int64_t)sizeof(TcRow)), o_P = take((nv + 1) * 4), o_tile = take(tiles * 4), o_placed = take(tiles * (TC_TILE / WAVE));
     const int64_t o_codes = take(groups * TC_G * 2), o_ids = take(groups * TC_G * 4), o_place = take(groups * TC_G * 4);
     const int64_t o_goff = take((nv + 1) * 4), o_mem = take(ne * 4), o_task = take(tasks * 8);
-    const int64_t bits = (nv + WAVE - 1) / WAVE * 8, o_some = take(bits), o_owner = take(bits), o_small = take(bits);
+    const int64_t bits = (nv + WAVE - 1) / WAVE * 8, o_some = take(bits), o_owner = take(bits), o_small = take(bits), o_hubs = take(bits);
     const int64_t o_scan = take((int64_t)scan_temp_bytes(nv));
     HN_TRY(g->s_tc.reserve((size_t)o));
     char* base = g->s_tc.as<char>();
@@ -1063,6 +1081,7 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
     uint32_t* members = at(o_mem, (uint32_t*)nullptr);
     uint2* task = at(o_task, (uint2*)nullptr);
     uint64_t* some = at(o_some, (uint64_t*)nullptr);
+    uint64_t* hubs = at(o_hubs, (uint64_t*)nullptr);
     uint64_t* owner = at(o_owner, (uint64_t*)nullptr);
     uint64_t* small = at(o_small, (uint64_t*)nullptr);
     void* tmp = base + o_scan;
@@ -1091,13 +1110,14 @@ static hn_status tc_run(hn_graph* g, bool orient, uint64_t* total_out, uint64_t*
         HN_CHECK_LAUNCH();
         tc_cut_kernel<<<1, BLOCK, 0, st>>>(hist, ctl);
         HN_CHECK_LAUNCH();
-        HN_TRY(exclusive_scan_fn<uint32_t>(HubIn{weight, ctl}, HubOut{weight, wc, hub}, &ctl->hubs, nv, tmp, st));
+        HN_TRY(exclusive_scan_fn<uint32_t>(HubIn{weight, ctl}, HubOut{weight, wc, hub, hubs}, &ctl->hubs, nv, tmp, st));
     }
     // 2. lists
     if (orient)
-        tc_rows_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
+        tc_rows_kernel<true><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, nullptr, row, codes, ids, ctl);
     else
-        tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, row, codes, ids, ctl);
+        tc_rows_kernel<false><<<gt, BLOCK, 0, st>>>(nv, P + nv, P, tile_lo, g->rec, g->arena, wc, all_hubs ? nullptr : hubs, row,
+                                                    codes, ids, ctl);
     HN_CHECK_LAUNCH();
     tc_pad_kernel<<<(unsigned)ceil_div(nv, BLOCK * TC_PAD_WORDS), BLOCK, 0, st>>>(nv, some, row, codes, ids, most, owner, small, gcnt);
     HN_CHECK_LAUNCH();
